@@ -78,8 +78,15 @@ def _draw(rng):
                 "dtype": rng.choice((half, half, half, "f32"))}
     if kind in ("encoder", "encode"):
         dim = rng.choice((32, 64, 64, 64, 128))
-        d = dim * rng.choice((4, 6, 8, 12, 16))
-        return {"kind": kind, "batch": _log(rng, 1, 32), "seq": _log(rng, 16, 1024), "d": d, "heads": d // dim, "ff": 4 * d, "dtype": rng.choice((half, half, half, "f32"))}
+        d = dim * rng.choice((4, 6, 8, 12, 16) if dim < 128 else (4, 6, 8))
+        c = {"kind": kind, "batch": _log(rng, 1, 32), "seq": _log(rng, 16, 1024), "d": d, "heads": d // dim, "ff": 4 * d, "dtype": rng.choice((half, half, half, "f32"))}
+        if kind == "encoder":
+            # A step's gradients are compared: on few tokens, and in bf16, one pre-activation that rounds to the other side
+            # of a ReLU is more than any tolerance can tell from a mistake (bf16 is in the listed cases and the other families).
+            c["batch"] = max(c["batch"], -(-512 // c["seq"]))
+            if c["dtype"] == "bf16":
+                c["dtype"] = "f16"
+        return c
     k, stride = rng.choice(((1, 1), (3, 1), (3, 1), (3, 1), (3, 2), (1, 2), (5, 1), (7, 2)))
     hw = rng.choice((7, 14, 28, 32, 56, 56, 64, 96, 112, 224))
     cin, cout = (rng.choice((16, 32, 64, 64, 96, 128, 192, 256, 512)) for _ in range(2))
