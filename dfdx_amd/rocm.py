@@ -87,6 +87,7 @@ EXPORTS = [
     "dfdx_rocm_scalar_mul_forward", "dfdx_rocm_scalar_mul_backward",
     "dfdx_rocm_softmax_forward", "dfdx_rocm_softmax_backward",
     "dfdx_rocm_reshape_forward", "dfdx_rocm_reshape_backward",
+    "dfdx_rocm_attention_forward", "dfdx_rocm_attention_backward",
     "dfdx_rocm_layer_norm_forward", "dfdx_rocm_layer_norm_backward",
     "dfdx_rocm_relu_forward", "dfdx_rocm_relu_backward",
     "dfdx_rocm_add_forward", "dfdx_rocm_add_backward",
@@ -594,6 +595,32 @@ class Rocm:
         vp = ctypes.c_void_p
         self._check(self.lib.dfdx_rocm_reshape_backward(self.ctx, DTYPES[x.dtype], len(x.shape), _i64arr(x.shape),
                                                         _i64arr(x.strides), vp(grad_inp.ptr), vp(grad_out.ptr)))
+
+    def attention_supported(self, dtype: str, head_dim: int) -> bool:
+        """Whether the fused attention takes this element type and head dimension (else: matmul, softmax, matmul)."""
+        return dtype in ("f16", "bf16") and head_dim in (32, 64, 128)
+
+    def attention_forward(self, q: View, k: View, v: View, scale: float, need_backward: bool = True):
+        """softmax(scale * q.k^T).v for (B, H, S, D) views sharing their strides; returns the result in token layout
+        (B, S, H * D) and the row statistics (f32) the backward takes (``None`` without ``need_backward``)."""
+        B, H, S, D = q.shape
+        assert k.shape == q.shape and v.shape == q.shape and k.strides == q.strides and v.strides == q.strides and q.strides[3] == 1
+        out = self.empty(q.dtype, (B, S, H * D))
+        lse = self.empty("f32", (B, H, S)) if need_backward else None
+        vp = ctypes.c_void_p
+        self._check(self.lib.dfdx_rocm_attention_forward(
+            self.ctx, DTYPES[q.dtype], _c(B), _c(H), _c(S), _c(D), vp(q.ptr), vp(k.ptr), vp(v.ptr), _i64arr(q.strides[:3]),
+            ctypes.c_float(scale), vp(out.ptr), _i64arr((S * H * D, D, H * D)), vp(lse.ptr if lse is not None else None)))
+        return out, lse
+
+    def attention_backward(self, q: View, grad_q: View, k: View, grad_k: View, v: View, grad_v: View, scale: float, out: View,
+                           grad_out: View, lse: View):
+        B, H, S, D = q.shape
+        vp = ctypes.c_void_p
+        self._check(self.lib.dfdx_rocm_attention_backward(
+            self.ctx, DTYPES[q.dtype], _c(B), _c(H), _c(S), _c(D), vp(q.ptr), vp(k.ptr), vp(v.ptr), _i64arr(q.strides[:3]),
+            ctypes.c_float(scale), vp(out.ptr), vp(grad_out.ptr), _i64arr((S * H * D, D, H * D)), vp(lse.ptr),
+            vp(grad_q.ptr), vp(grad_k.ptr), vp(grad_v.ptr)))
 
     # ------------------------------------------- ops between an encoder block's GEMMs --
     def layer_norm_forward(self, x: View, gamma: View, beta: View, epsilon: float = 1e-5) -> View:

@@ -356,6 +356,28 @@ int dfdx_rocm_reshape_forward(dfdx_rocm_ctx *ctx, int dtype, int rank, const int
 int dfdx_rocm_reshape_backward(dfdx_rocm_ctx *ctx, int dtype, int rank, const int64_t *shape, const int64_t *inp_strides,
                                void *grad_inp, const void *grad_out);
 
+/* The three ops of MultiHeadAttention between the projections in one:
+ * softmax(scale * q . k^T) . v per head (dfdx/src/nn/layers/
+ * multi_head_attention.rs:123-145), without the (seq, seq) matrices.  q, k and
+ * v are (batch, heads, seq, dim) views sharing one set of element strides for
+ * batch, head and row (dim contiguous); out has strides of its own, so it can
+ * be written straight into the (batch, seq, heads * dim) token layout.  lse
+ * (batch * heads * seq floats, contiguous; NULL when no backward follows)
+ * receives what the backward needs besides q, k, v and out: per row the base-2
+ * logarithm of the softmax denominator.  The scores stay in f32, the
+ * probabilities are rounded once as operands of the second product.  f16 and
+ * bf16, dim 32, 64 or 128, scale > 0, 16-byte-aligned rows; anything else is
+ * DFDX_ROCM_ERR_UNSUPPORTED before anything is launched, and the caller composes
+ * the ops above instead.  Backward: grad_q, grad_k, grad_v (strides of q, k, v)
+ * are accumulated into. */
+int dfdx_rocm_attention_forward(dfdx_rocm_ctx *ctx, int dtype, int64_t batch, int64_t heads, int64_t seq, int64_t dim,
+                                const void *q, const void *k, const void *v, const int64_t strides[3], float scale,
+                                void *out, const int64_t out_strides[3], float *lse);
+int dfdx_rocm_attention_backward(dfdx_rocm_ctx *ctx, int dtype, int64_t batch, int64_t heads, int64_t seq, int64_t dim,
+                                 const void *q, const void *k, const void *v, const int64_t strides[3], float scale,
+                                 const void *out, const void *grad_out, const int64_t out_strides[3], const float *lse,
+                                 void *grad_q, void *grad_k, void *grad_v);
+
 /* ---- The ops between a transformer encoder block's GEMMs ----------------------
  * TransformerEncoderBlock (dfdx/src/nn/layers/transformer.rs:24-48) is
  * ResidualAdd<MultiHeadAttention>, LayerNorm1D, ResidualAdd<(Linear, ReLU,
