@@ -489,6 +489,7 @@ int settle_operands(dfdx_rocm_ctx *ctx, GemmProblem *p, bool may_overwrite) {
         if (int e = settle(ctx, p->b)) return e;
     }
     if (int e = settle(ctx, p->bias)) return e;
+    if (int e = settle(ctx, p->with)) return e;
     const int64_t ext[4] = {p->reduce ? 1 : p->nb1, p->reduce ? 1 : p->nb2, p->m, p->n};
     const int64_t str[4] = {p->c_b1, p->c_b2, p->c_rs, p->c_cs};
     const size_t es = p->dtype == DT_F64 ? 8 : p->dtype == DT_F32 ? 4 : 2;
@@ -500,7 +501,52 @@ int settle_operands(dfdx_rocm_ctx *ctx, GemmProblem *p, bool may_overwrite) {
 
 }  // namespace
 
+namespace {
+// Which plans apply p.extra on the way into C.
+bool extra_supported(const GemmProblem &p, const Plan &plan) {
+    if (p.extra == EXTRA_NONE) return true;
+    if (plan.kernel != DFDX_ROCM_KERNEL_MFMA || p.nb1 * p.nb2 != 1) return false;
+    const bool is16 = p.dtype == DT_F16 || p.dtype == DT_BF16;
+    if (is16 && plan.variant == mfma16_small_variant()) return true;
+    if (p.dtype == DT_F64 && plan.variant == mfma64_small_variant()) return true;
+    if (is16 && plan.variant >= mfma16_dma_first_variant()) return mfma16dma_extra_supported(p, plan.variant - mfma16_dma_first_variant() + 1, plan.splits);
+    return plan.splits > 1;  // the reduce kernel does it
+}
+}  // namespace
+
 namespace dfdx_rocm {
+
+int gemm_beyond(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int extra, const void *with) {
+    if (int e = bind(ctx)) return e;
+    GemmProblem p;
+    if (int e = make_problem(desc, &p)) return e;
+    if (p.m == 0) return DFDX_ROCM_OK;
+    // C and `with` are one contiguous matrix each: what the separate ops below walk
+    if (p.nb1 * p.nb2 != 1 || p.c_cs != 1 || p.c_rs != p.n || (extra && (p.accumulate != 0) != (extra == EXTRA_FROM)) ||
+        (extra > EXTRA_RELU && !with))
+        return DFDX_ROCM_ERR_INVALID_ARG;
+    Plan plan;
+    if (int e = make_plan(ctx, desc, p, &plan)) return e;
+    if (int e = reserve_partials(ctx, p, plan, false)) return e;
+    p.extra = extra;
+    p.with = with;
+    const int64_t len = p.m * p.n;
+    const bool whole = extra_supported(p, plan);
+    if (!whole) {
+        if (extra == EXTRA_FROM)
+            if (int e = dfdx_rocm_copy_d2d(ctx, p.c, with, (size_t)len * dtype_size(p.dtype))) return e;
+        p.extra = EXTRA_NONE;
+    }
+    if (int e = settle_operands(ctx, &p, /*may_overwrite=*/extra != EXTRA_FROM)) return e;
+    if (int e = run_plan(ctx, p, plan)) return e;
+    if (whole) return DFDX_ROCM_OK;
+    switch (extra) {
+    case EXTRA_RELU: return dfdx_rocm_relu_forward(ctx, p.dtype, len, p.c, p.c);
+    case EXTRA_RESIDUAL: return dfdx_rocm_add_forward(ctx, p.dtype, len, p.c, with, p.c);
+    case EXTRA_MASK: return relu_mask(ctx, p.dtype, len, with, p.c);
+    default: return DFDX_ROCM_OK;
+    }
+}
 
 int gemm_with_colsum(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, void *colsum_b, bool *fused) {
     *fused = false;

@@ -75,6 +75,11 @@ size_t dense_bytes(int rank, const int64_t *extents, const int64_t *strides, siz
 // the batches of a reduced product) to colsum_b[0 .. n) in the element type: colsum_b[j] += sum_k B[k][j].  *fused tells
 // whether it did; when not, colsum_b has not been touched and the caller runs that reduction itself.
 int gemm_with_colsum(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, void *colsum_b, bool *fused);
+// dfdx_rocm_gemm(ctx, desc) for a contiguous C with one thing more on the way into it (EXTRA_* in gemm_internal.h; by a
+// separate op where the kernel picked cannot).
+int gemm_beyond(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int extra, const void *with);
+// x[i] = with[i] > 0 ? x[i] : 0, in place
+int relu_mask(dfdx_rocm_ctx *ctx, int dtype, int64_t len, const void *with, void *x);
 // Clears `bytes` bytes at `ptr` (any alignment) with a fill kernel on `stream`.
 hipError_t launch_zero_fill(void *ptr, size_t bytes, int compute_units, hipStream_t stream);
 

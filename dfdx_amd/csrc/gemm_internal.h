@@ -8,6 +8,11 @@ namespace dfdx_rocm {
 
 enum { DT_F32 = 0, DT_F16 = 1, DT_BF16 = 2, DT_F64 = 3 };
 enum { BIAS_NONE = 0, BIAS_PER_COL = 1, BIAS_PER_ROW = 2 };
+// What happens to a finished value on its way into C besides bias and beta (`with` has C's layout).  The last three are for
+// products that overwrite C; they take the value rounded to the element type, as the op they stand for would have read it.
+//   FROM (accumulate only): the old values of beta = 1 are read from `with`, not from C;
+//   RELU: max(value, 0);  RESIDUAL: value + with;  MASK: with > 0 ? value : 0 (the gradient of a ReLU whose output is `with`).
+enum { EXTRA_NONE = 0, EXTRA_RELU = 1, EXTRA_RESIDUAL = 2, EXTRA_MASK = 3, EXTRA_FROM = 4 };
 enum { KSUM_NONE = 0, KSUM_OF_A = 1, KSUM_OF_B = 2 };
 
 // One strided, batched GEMM:  C[b][i,j] = (accumulate ? C : 0) + bias + sum_k A[b][i,k] * B[b][k,j].
@@ -34,6 +39,8 @@ struct GemmProblem {
     void *ksum = nullptr;
     int ksum_of = KSUM_NONE;
     int ksum_accumulate = 0;
+    int extra = EXTRA_NONE;        // see above; kernels that have it: extra_supported in api.cpp
+    const void *with = nullptr;
     // split-k (filled in by the planner): `splits` workgroups share one C tile; f32 partials go to `workspace`
     int splits;
     float *workspace;
@@ -108,6 +115,9 @@ const char *mfma16dma_variant_name(int variant);
 bool mfma16dma_supported(const GemmProblem &p, int variant);
 int mfma16dma_pick_variant(const GemmProblem &p, int compute_units);
 hipError_t launch_mfma16dma(const GemmProblem &p, int variant, hipStream_t stream);
+struct DmaParams;
+bool mfma16dma_extra_supported(const GemmProblem &p, int variant, int splits);  // can this plan apply p.extra on the way into C?
+hipError_t launch_mfma16dma_extra(int variant, int dtype, int extra, const DmaParams &p, int compute_units, hipStream_t stream);  // gemm_mfma16_dma_extra.hip
 // Split-k planning for the LDS-DMA kernels: picks tile variant and split count together.  `forced_splits`
 // > 0 overrides the count (clamped to what the k extent allows).  `seconds` (may be null) receives the estimate.
 void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_variant, int forced_splits, int *variant,

@@ -37,6 +37,8 @@ struct SmallParams {
     int slice;         // k per wave, a multiple of the step (16 k; 32 for the 16-bit types)
     void *ksum;        // may be null: ksum[i] (+)= sum_k A[i][k]
     int ksum_accumulate;
+    const void *c_old, *with;  // old values of beta = 1 (c itself unless elsewhere); partner of `extra` (EXTRA_*), both like c
+    int extra;
 };
 
 // Per element type: the accumulator type, four k-values of one row as the MFMA wants them, the MFMA step, and which row
@@ -259,7 +261,14 @@ template <typename T, int WAVES, bool LONG> __global__ __launch_bounds__(WAVES *
         T *dst = (T *)p.c + (int64_t)orow * p.ldc + col;
         A v = sum[r] + cb;
         if (p.bias_mode == BIAS_PER_ROW) v += S::load((const T *)p.bias + orow);
-        if (p.accumulate) v += S::load(dst);
+        if (p.accumulate) v += S::load((const T *)p.c_old + (dst - (T *)p.c));
+        if (p.extra != EXTRA_NONE) {
+            T rounded;
+            S::store(&rounded, v);
+            v = S::load(&rounded);
+            const A w = p.extra == EXTRA_RELU ? A(0) : S::load((const T *)p.with + (dst - (T *)p.c));
+            v = p.extra == EXTRA_RELU ? (v > A(0) ? v : A(0)) : p.extra == EXTRA_RESIDUAL ? v + w : w > A(0) ? v : A(0);
+        }
         S::store(dst, v);
     }
 }
@@ -356,6 +365,9 @@ hipError_t launch_small(const GemmProblem &g, hipStream_t stream) {
     p.b_vec = g.b_rs == 1 && (g.n == 1 || g.b_cs % vq == 0) && ((uintptr_t)g.b & vmask) == 0;
     p.ksum = (g.ksum && g.ksum_of == KSUM_OF_A) ? g.ksum : nullptr;
     p.ksum_accumulate = g.ksum_accumulate;
+    p.c_old = g.extra == EXTRA_FROM ? g.with : g.c;
+    p.with = g.with;
+    p.extra = g.extra == EXTRA_FROM ? EXTRA_NONE : g.extra;
     const int waves = small_waves(g.dtype, g.k);
     const int step = 4 * kl;
     p.slice = (int)(((g.k + waves - 1) / waves + step - 1) / step * step);

@@ -21,6 +21,16 @@ template <> struct Cvt<__bf16> {
     static __device__ __forceinline__ void store(__bf16 *p, float v) { *p = (__bf16)v; }  // RNE, quiet NaNs (v_cvt_pk_bf16_f32)
 };
 
+// Where beta = 1 reads the old values, and what else is done to a finished value (EXTRA_RELU and on); both laid out like C.
+struct Beyond {
+    const void *c_old, *with;
+    int extra;
+};
+// `x` is a finished value, rounded to the element type; `w` its partner
+__device__ __forceinline__ float apply_extra(int extra, float x, float w) {
+    return extra == EXTRA_RELU ? fmaxf(x, 0.0f) : extra == EXTRA_RESIDUAL ? x + w : w > 0.0f ? x : 0.0f;
+}
+
 // The row sums that ride along with a split product (`ksum`, one value per row of C, `slots` partial sums each, stored
 // [slot][row]).  The first `blocks` workgroups of grid row 0 do nothing else: each takes 16 rows; thread t adds the
 // slots t / 16, t / 16 + 16, ... of row t % 16 in ascending order, four loads in flight at a time; the 16 partial sums
@@ -60,7 +70,7 @@ template <typename T> __device__ __forceinline__ void combine_ksum(const KsumPar
 template <typename T>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *ws, int splits, int64_t ws_ld, int64_t ws_split_stride,
                                                             T *c, int64_t c_rs, int m, int n, int accumulate, int bias_mode,
-                                                            const T *bias, int vec4, KsumParts ks) {
+                                                            const T *bias, int vec4, KsumParts ks, Beyond bd) {
     if (ks.ws && (int)blockIdx.x < ks.blocks) {   // uniform over the workgroup
         if (blockIdx.y == 0) combine_ksum<T>(ks, m);
         return;   // the same block index in the other grid rows has no work
@@ -82,12 +92,17 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *ws, int
             if (s0 + u < splits && s0 + u > 0) v += part[u];
     }
     T *dst = c + (int64_t)row * c_rs + col;
+    const T *from = (const T *)bd.c_old + (dst - c), *with = (const T *)bd.with + (dst - c);
     const float rb = (bias_mode == BIAS_PER_ROW) ? Cvt<T>::load(bias + row) : 0.0f;
     if constexpr (sizeof(T) == 4) {
         if (vec4 && col + 3 < n) {   // f32 rows aligned to 16 B: one load of the old values, one store
             f32x4 x = v + rb;
             if (bias_mode == BIAS_PER_COL) x += *(const f32x4 *)(bias + col);
-            if (accumulate) x += *(const f32x4 *)dst;
+            if (accumulate) x += *(const f32x4 *)from;
+            if (bd.extra) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[e] = apply_extra(bd.extra, x[e], bd.extra == EXTRA_RELU ? 0.0f : with[e]);
+            }
             *(f32x4 *)dst = x;
             return;
         }
@@ -97,7 +112,12 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *ws, int
         if (col + e >= n) break;
         float x = v[e] + rb;
         if (bias_mode == BIAS_PER_COL) x += Cvt<T>::load(bias + col + e);
-        if (accumulate) x += Cvt<T>::load(dst + e);
+        if (accumulate) x += Cvt<T>::load(from + e);
+        if (bd.extra) {
+            T rounded;
+            Cvt<T>::store(&rounded, x);
+            x = apply_extra(bd.extra, Cvt<T>::load(&rounded), bd.extra == EXTRA_RELU ? 0.0f : Cvt<T>::load(with + e));
+        }
         Cvt<T>::store(dst + e, x);
     }
 }
@@ -119,7 +139,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 template <typename T>
 __global__ __launch_bounds__(256) void splitk_reduce16_kernel(const float *ws, int splits, int64_t ws_ld, int64_t ws_split_stride,
                                                               uint16_t *c, int64_t c_rs, int m, int n, int accumulate,
-                                                              int bias_mode, const uint16_t *bias, KsumParts ks) {
+                                                              int bias_mode, const uint16_t *bias, KsumParts ks, Beyond bd) {
     if (ks.ws && (int)blockIdx.x < ks.blocks) {   // uniform over the workgroup
         if (blockIdx.y == 0) combine_ksum<T>(ks, m);
         return;   // the same block index in the other grid rows has no work
@@ -129,8 +149,9 @@ __global__ __launch_bounds__(256) void splitk_reduce16_kernel(const float *ws, i
     if (row >= m || col >= n) return;   // n is a multiple of 8: a thread's 8 columns are all inside or all outside
     const float *src = ws + (int64_t)row * ws_ld + col;
     uint16_t *dst = c + (int64_t)row * c_rs + col;
-    u32x4 old = {0u, 0u, 0u, 0u}, cb = {0u, 0u, 0u, 0u};
-    if (accumulate) old = *(const u32x4 *)dst;
+    u32x4 old = {0u, 0u, 0u, 0u}, cb = {0u, 0u, 0u, 0u}, with = {0u, 0u, 0u, 0u};
+    if (accumulate) old = *(const u32x4 *)((const uint16_t *)bd.c_old + (dst - c));
+    if (bd.extra > EXTRA_RELU) with = *(const u32x4 *)((const uint16_t *)bd.with + (dst - c));
     if (bias_mode == BIAS_PER_COL) cb = *(const u32x4 *)(bias + col);
     // eight splits requested at a time (a tail repeats the last one, unused) and added in ascending order: with the old
     // C values and the bias that is ONE round trip to memory for up to eight splits (a loop that waited for split after
@@ -163,7 +184,8 @@ __global__ __launch_bounds__(256) void splitk_reduce16_kernel(const float *ws, i
         const int sh = (e & 1) * 16;
         if (bias_mode == BIAS_PER_COL) x += Bits16<T>::widen((uint16_t)(cb[e / 2] >> sh));
         if (accumulate) x += Bits16<T>::widen((uint16_t)(old[e / 2] >> sh));
-        const uint32_t bits = Bits16<T>::narrow(x);
+        uint32_t bits = Bits16<T>::narrow(x);
+        if (bd.extra) bits = Bits16<T>::narrow(apply_extra(bd.extra, Bits16<T>::widen((uint16_t)bits), Bits16<T>::widen((uint16_t)(with[e / 2] >> sh))));
         out[e / 2] = (e & 1) ? (out[e / 2] | (bits << 16)) : bits;
     }
     *(u32x4 *)dst = out;
@@ -177,39 +199,42 @@ hipError_t launch_splitk_reduce(const GemmProblem &p, int64_t ws_ld, int64_t ws_
     const bool with_ksum = p.ksum && ws_ksum;
     const KsumParts ks{with_ksum ? ws_ksum : nullptr, ws_ksum_stride, p.ksum, p.ksum_accumulate, ksum_slots,
                        with_ksum ? (int)((p.m + KSUM_ROWS - 1) / KSUM_ROWS) : 0};
+    const bool from = p.extra == EXTRA_FROM;
+    const Beyond bd{from ? p.with : p.c, p.with, from ? EXTRA_NONE : p.extra};
     dim3 grid((unsigned)((p.m + 3) / 4 + ks.blocks), (unsigned)((p.n + 255) / 256)), block(256);
     if ((p.n + 255) / 256 > 65535) return hipErrorInvalidValue;  // 16.7 M columns: no planner splits such a product
     const int64_t c_rs = p.m == 1 ? p.n : p.c_rs;
     const int bias_mode = p.bias ? p.bias_mode : BIAS_NONE;
     const bool is16 = p.dtype == DT_F16 || p.dtype == DT_BF16;
     if (is16 && p.n % 8 == 0 && c_rs % 8 == 0 && ws_ld % 4 == 0 && ws_split_stride % 4 == 0 && ((uintptr_t)p.c & 15u) == 0 &&
-        ((uintptr_t)p.workspace & 15u) == 0 && (bias_mode != BIAS_PER_COL || ((uintptr_t)p.bias & 15u) == 0)) {
+        ((uintptr_t)p.workspace & 15u) == 0 && (((uintptr_t)bd.c_old | (uintptr_t)bd.with) & 15u) == 0 &&
+        (bias_mode != BIAS_PER_COL || ((uintptr_t)p.bias & 15u) == 0)) {
         dim3 grid16((unsigned)((p.m + 3) / 4 + ks.blocks), (unsigned)((p.n + 511) / 512));
         if (p.dtype == DT_F16)
             splitk_reduce16_kernel<_Float16><<<grid16, block, 0, stream>>>(p.workspace, p.splits, ws_ld, ws_split_stride, (uint16_t *)p.c,
                                                                             c_rs, (int)p.m, (int)p.n, p.accumulate, bias_mode,
-                                                                            (const uint16_t *)p.bias, ks);
+                                                                            (const uint16_t *)p.bias, ks, bd);
         else
             splitk_reduce16_kernel<__bf16><<<grid16, block, 0, stream>>>(p.workspace, p.splits, ws_ld, ws_split_stride, (uint16_t *)p.c,
                                                                           c_rs, (int)p.m, (int)p.n, p.accumulate, bias_mode,
-                                                                          (const uint16_t *)p.bias, ks);
+                                                                          (const uint16_t *)p.bias, ks, bd);
         return hipGetLastError();
     }
     const int vec4 = p.dtype == DT_F32 && c_rs % 4 == 0 && ((uintptr_t)p.c & 15u) == 0 && ws_ld % 4 == 0 && ws_split_stride % 4 == 0 &&
-                     ((uintptr_t)p.workspace & 15u) == 0 && (bias_mode != BIAS_PER_COL || ((uintptr_t)p.bias & 15u) == 0);
+                     (((uintptr_t)p.workspace | (uintptr_t)bd.c_old) & 15u) == 0 && (bias_mode != BIAS_PER_COL || ((uintptr_t)p.bias & 15u) == 0);
     switch (p.dtype) {
     case DT_F32:
         splitk_reduce_kernel<float><<<grid, block, 0, stream>>>(p.workspace, p.splits, ws_ld, ws_split_stride, (float *)p.c, c_rs,
-                                                                 (int)p.m, (int)p.n, p.accumulate, bias_mode, (const float *)p.bias, vec4, ks);
+                                                                 (int)p.m, (int)p.n, p.accumulate, bias_mode, (const float *)p.bias, vec4, ks, bd);
         break;
     case DT_F16:
         splitk_reduce_kernel<_Float16><<<grid, block, 0, stream>>>(p.workspace, p.splits, ws_ld, ws_split_stride, (_Float16 *)p.c,
                                                                     c_rs, (int)p.m, (int)p.n, p.accumulate, bias_mode,
-                                                                    (const _Float16 *)p.bias, 0, ks);
+                                                                    (const _Float16 *)p.bias, 0, ks, bd);
         break;
     case DT_BF16:
         splitk_reduce_kernel<__bf16><<<grid, block, 0, stream>>>(p.workspace, p.splits, ws_ld, ws_split_stride, (__bf16 *)p.c, c_rs,
-                                                                  (int)p.m, (int)p.n, p.accumulate, bias_mode, (const __bf16 *)p.bias, 0, ks);
+                                                                  (int)p.m, (int)p.n, p.accumulate, bias_mode, (const __bf16 *)p.bias, 0, ks, bd);
         break;
     default: return hipErrorInvalidValue;
     }

@@ -218,6 +218,17 @@ template <int OP> int dispatch_op(dfdx_rocm_ctx *ctx, int dtype, int64_t len, co
 }
 
 }  // namespace
+
+int relu_mask(dfdx_rocm_ctx *ctx, int dtype, int64_t len, const void *with, void *x) {
+    if (len == 0) return DFDX_ROCM_OK;
+    switch (dtype) {  // the gradient kernel storing over its own input, element by element
+    case DFDX_ROCM_F64: return launch_f64<F64_RELU_BWD>(ctx, len, with, x, x, nullptr, 0.0, true, false);
+    case DFDX_ROCM_F32: return launch_op<float, OP_RELU_BWD>(ctx, len, with, x, x, nullptr, true, false);
+    case DFDX_ROCM_F16: return launch_op<_Float16, OP_RELU_BWD>(ctx, len, with, x, x, nullptr, true, false);
+    default: return launch_op<__bf16, OP_RELU_BWD>(ctx, len, with, x, x, nullptr, true, false);
+    }
+}
+
 }  // namespace dfdx_rocm
 
 extern "C" {

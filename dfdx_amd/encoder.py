@@ -1,51 +1,97 @@
-"""Host-side mirror of dfdx's ``TransformerEncoderBlock`` on the Rocm device: every op is one call into the C ABI.
+"""Host-side mirror of dfdx's ``TransformerEncoderBlock`` on the Rocm device: one call into the C ABI forward, one backward.
 
     TransformerEncoderBlock   dfdx/src/nn/layers/transformer.rs:24-48
         = ResidualAdd<MultiHeadAttention>, LayerNorm1D, ResidualAdd<(Linear, ReLU, Linear)>, LayerNorm1D
     MultiHeadAttention        dfdx/src/nn/layers/multi_head_attention.rs:105-146
     Linear / LayerNorm1D / ResidualAdd   linear.rs:82-89, layer_norm1d.rs:87-91, residual_add.rs:38-45
 
-The forward keeps what the reference's tape would keep (the inputs of every op); the backward walks the ops in
-reverse; every gradient buffer starts as zeros and is accumulated into, as with
-``Gradients::get_or_alloc_mut`` (dfdx-core/src/tensor/gradients.rs:53-58) -- here all of a pass's buffers are carved
-from one allocation and declared zero without a fill (``dfdx_rocm_zero_deferred``): the first op that accumulates
-into a whole buffer stores 0 + value, so the step pays neither the fill nor the read of the zeros; a buffer whose
-first use is anything else is filled then.  ``deferred_zeros=False`` restores the single eager fill.  The
-multiplication by 1/sqrt(head dim) between q.k^T and the softmax (multi_head_attention.rs:133-134) is folded into the
-softmax kernel.  Where the fused attention takes the element type and head dimension, the (seq, seq) matrices are never
-formed, forward or backward; ``saved["probs"]`` and ``saved["tokens"]`` are then made when somebody asks for them.
+The library strings the block's ops together (``dfdx_rocm_encoder_forward`` / ``_backward``); here live the parameters, the
+storage and the names of what the forward keeps.  The forward keeps what the backward needs; the other values of the
+reference's tape (the attention probabilities where the fused attention runs, the pre-activation of the ReLU) are made
+when somebody asks for them.  Gradients are stored, not added into zeros, so the step pays neither a fill nor the read of
+the zeros.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Dict, Tuple
 
-import numpy as np
-
-from .rocm import Rocm, View
+from .rocm import DTYPES, ITEMSIZE, Encoder, EncoderLayout, Rocm, View, _row_major
 
 PARAMS = ("wq", "bq", "wk", "bk", "wv", "bv", "wo", "bo", "g1", "be1", "w1", "b1", "w2", "b2", "g2", "be2")
 
 
+class _Plan:
+    """What one (batch, seq) shape of a block needs to know: sizes and places, no data."""
+
+    def __init__(self, block: "EncoderBlock", B: int, S: int):
+        d, H, ff = block.d, block.h, block.ff
+        self.desc = Encoder(DTYPES[block.dtype], 0, B, S, d, H, ff)
+        self.layout = EncoderLayout()
+        dev = block.dev
+        dev._check(dev.lib.dfdx_rocm_encoder_plan(dev.ctx, ctypes.byref(self.desc), ctypes.byref(self.layout)))
+        self.shapes = {"wq": (d, d), "wk": (d, d), "wv": (d, d), "wo": (d, d), "w1": (ff, d), "w2": (d, ff), "b1": (ff,)}
+        self.shapes = {n: self.shapes.get(n, (d,)) for n in PARAMS}
+        # gradients: one allocation, the pieces in the order of PARAMS, then that of x, on 16-byte boundaries
+        es = ITEMSIZE[block.dtype]
+        self.pieces = []
+        for shape in list(self.shapes.values()) + [(B, S, d)]:
+            n = math.prod(shape) * es
+            self.pieces += [n, -n % 16]
+        self.grad_bytes = sum(self.pieces)
+        self.gapless = not any(self.pieces[1::2])
+        self.grad_views = [(n, s, _row_major(s)) for n, s in self.shapes.items()] + [("x", (B, S, d), _row_major((B, S, d)))]
+
+
 class _Saved(dict):
-    """What the backward needs, by name.  Two tensors that only the op-by-op attention has to keep are made on request."""
+    """What the forward keeps, by name: ``x`` and ``out``, and Views into the one allocation ``arena`` made on first use."""
+
+    def __init__(self, block: "EncoderBlock", plan: _Plan, x: View, arena):
+        super().__init__(x=x)
+        self.block, self.plan, self.arena = block, plan, arena
 
     def __missing__(self, name):
-        if name == "probs":
-            dev, q, k = self["dev"], self["qv"], self["kv"]
-            value = dev.softmax_forward(dev.forward(q, k), self["scale"])
-        elif name == "tokens":
-            tok, (B, H, S, D) = self["tok"], self["qv"].shape
-            value = View(tok.storage, tok.dtype, (B, S, H, D), (S * H * D, H * D, D, 1), tok.offset).permute(0, 2, 1, 3)
-        else:
-            raise KeyError(name)
-        self[name] = value
+        value = self[name] = self._make(name)
         return value
+
+    def _make(self, name):
+        dev, dtype, l = self.block.dev, self.block.dtype, self.plan.layout
+        B, S, d = self["x"].shape
+        H, D, ff = self.block.h, d // self.block.h, self.block.ff
+
+        def at(offset, shape, strides=None, kind=dtype):
+            n = math.prod(shape) * ITEMSIZE[kind]
+            return View(self.arena[offset:offset + n], kind, shape, strides or _row_major(shape))
+
+        heads = (S * d, D, d, 1)
+        if name in ("qv", "vv"):                     # (B, H, S, D), head-interleaved strides
+            return at(l.q if name == "qv" else l.v, (B, H, S, D), heads)
+        if name == "kv":                             # (B, H, D, S)
+            return at(l.k, (B, H, D, S), (S * d, D, 1, d))
+        if name in ("tok", "h1", "n1", "h2"):
+            return at(getattr(l, name), (B, S, d))
+        if name == "r1":
+            return at(l.r1, (B, S, ff))
+        if name == "f1":
+            return dev.linear_forward(self["n1"], self.block.p["w1"], self.block.p["b1"])
+        if name == "scale":
+            return 1.0 / math.sqrt(D)
+        if l.fused_attention:
+            if name == "lse":
+                return at(l.lse, (B, H, S), kind="f32")
+            if name == "probs":
+                return dev.softmax_forward(dev.forward(self["qv"], self["kv"]), self["scale"])
+            if name == "tokens":
+                return at(l.tok, (B, H, S, D), heads)
+        elif name in ("probs", "tokens"):
+            return at(getattr(l, name), (B, H, S, S if name == "probs" else D))
+        raise KeyError(name)
 
 
 class EncoderBlock:
     """Parameters are device ``View``s: w* are (out, in) row-major Linear weights, b* biases, g*/be* the LayerNorm
-    gamma / beta."""
+    gamma / beta.  ``deferred_zeros`` is kept for callers that pass it: there are no gradient zeros to fill either way."""
 
     def __init__(self, dev: Rocm, dtype: str, d_model: int, heads: int, d_ff: int, params: Dict[str, View],
                  deferred_zeros: bool = True):
@@ -54,94 +100,59 @@ class EncoderBlock:
         assert not missing, f"missing parameters: {missing}"
         self.dev, self.dtype, self.d, self.h, self.ff, self.p = dev, dtype, d_model, heads, d_ff, params
         self.deferred_zeros = deferred_zeros
+        self._plans: Dict[tuple, _Plan] = {}
+
+    def _plan(self, B: int, S: int) -> _Plan:
+        plan = self._plans.get((B, S))
+        if plan is None:
+            if len(self._plans) >= 64:   # shapes come and go: keep no more than a loader's buckets
+                self._plans.clear()
+            plan = self._plans[(B, S)] = _Plan(self, B, S)
+        return plan
+
+    def _desc(self, plan: _Plan) -> Encoder:
+        p, desc = self.p, Encoder.from_buffer_copy(plan.desc)
+        ptrs = []
+        for name, shape in plan.shapes.items():
+            v = p[name]
+            assert v.shape == shape and v.dtype == self.dtype and v.strides[-1] == 1 and (len(shape) == 1 or v.strides[0] == shape[1]), \
+                f"{name}: left: {v.shape}\n right: {shape}"
+            ptrs.append(v.ptr)
+        desc.params[:] = ptrs
+        return desc
 
     def forward(self, x: View) -> Tuple[View, dict]:
         """x: (batch, seq, d_model) contiguous.  Returns the block's output and the tensors the backward needs."""
-        dev, p = self.dev, self.p
+        dev, torch = self.dev, self.dev._torch
         B, S, d = x.shape
         assert d == self.d, f"left: {d}\n right: {self.d}"
-        H, D = self.h, self.d // self.h
-        q = dev.linear_forward(x, p["wq"], p["bq"])
-        k = dev.linear_forward(x, p["wk"], p["bk"])
-        v = dev.linear_forward(x, p["wv"], p["bv"])
-        heads = lambda t: View(t.storage, t.dtype, (B, S, H, D), (S * d, d, D, 1), t.offset)
-        qv = heads(q).permute(0, 2, 1, 3)          # (B, H, S, D), head-interleaved strides
-        kv = heads(k).permute(0, 2, 3, 1)          # (B, H, D, S)
-        vv = heads(v).permute(0, 2, 1, 3)
-        scale = 1.0 / math.sqrt(D)
-        attention = dict(scale=scale, folded=True)
-        if dev.attention_supported(self.dtype, D):
-            tok, attention["lse"] = dev.attention_forward(qv, heads(k).permute(0, 2, 1, 3), vv, scale)
-        else:
-            scores = dev.forward(qv, kv)               # (B, H, S, S)
-            # The softmax entry takes its scale as a C float.  An f64 block whose 1/sqrt(head dim) has no exact float value
-            # multiplies by the double scalar in an op of its own, as the reference does (multi_head_attention.rs:133-134).
-            folded = self.dtype != "f64" or float(np.float32(scale)) == scale
-            if not folded:
-                scores = dev.scalar_mul_forward(scores, scale)
-            probs = dev.softmax_forward(scores, scale if folded else 1.0)
-            tokens = dev.forward(probs, vv)            # (B, H, S, D)
-            tok = dev.reshape_forward(tokens.permute(0, 2, 1, 3), (B, S, d))
-            attention.update(probs=probs, tokens=tokens, folded=folded)
-        attn = dev.linear_forward(tok, p["wo"], p["bo"])
-        h1 = dev.add_forward(attn, x)
-        n1 = dev.layer_norm_forward(h1, p["g1"], p["be1"])
-        f1 = dev.linear_forward(n1, p["w1"], p["b1"])
-        r1 = dev.relu_forward(f1)
-        f2 = dev.linear_forward(r1, p["w2"], p["b2"])
-        h2 = dev.add_forward(f2, n1)
-        out = dev.layer_norm_forward(h2, p["g2"], p["be2"])
-        saved = _Saved(x=x, qv=qv, kv=kv, vv=vv, tok=tok, h1=h1, n1=n1, f1=f1, r1=r1, h2=h2, dev=dev, **attention)
-        return out, saved
+        strides = (S * d, d, 1)
+        assert x.strides == strides and x.dtype == self.dtype, "encoder input must be contiguous"
+        plan = self._plan(B, S)
+        l = plan.layout
+        out = torch.empty(max(B * S * d * ITEMSIZE[self.dtype], 16), dtype=torch.uint8, device=dev.device)
+        arena = torch.empty(l.saved_bytes, dtype=torch.uint8, device=dev.device)
+        scratch = torch.empty(l.forward_scratch_bytes, dtype=torch.uint8, device=dev.device) if l.forward_scratch_bytes else None
+        vp = ctypes.c_void_p
+        dev._check(dev.lib.dfdx_rocm_encoder_forward(dev.ctx, ctypes.byref(self._desc(plan)), vp(x.ptr), vp(out.data_ptr()), vp(arena.data_ptr()),
+                                                     vp(scratch.data_ptr() if scratch is not None else None)))
+        return View(out, self.dtype, (B, S, d), strides), _Saved(self, plan, x, arena)
 
     def backward(self, saved: dict, grad_out: View) -> Tuple[Dict[str, View], View]:
         """grad_out: d(loss)/d(out), contiguous like the output.  Returns ({parameter: gradient}, d(loss)/d(x))."""
-        dev, p, s = self.dev, self.p, saved
-        x, n1, tok = s["x"], s["n1"], s["tok"]
-        qv, kv, vv = s["qv"], s["kv"], s["vv"]
-        # every gradient buffer of the pass: one allocation, pieces aligned to 256 B, zero by declaration (or one fill)
-        acts = dict(gh2=s["h2"], gf2=s["h2"], gn1=n1, gr1=s["r1"], gf1=s["f1"], gh1=s["h1"], gattn=s["h1"], gx=x, gtok=tok,
-                    gq=x, gk=x, gv=x)   # gq, gk, gv: laid out like the q, k, v storages
-        fused = "lse" in s
-        if not fused:
-            probs, tokens = s["probs"], s["tokens"]
-            acts.update(gtokens=tokens, gp=probs, gscores=probs)
-            if not s["folded"]:
-                acts["gscaled"] = probs   # gradient of the scaled scores, between the softmax and the scalar multiply
-        bufs = dev.zeros_many([p[n] for n in PARAMS] + list(acts.values()), deferred=self.deferred_zeros)
-        grads = dict(zip(PARAMS, bufs[:len(PARAMS)]))
-        g = dict(zip(acts, bufs[len(PARAMS):]))
-        gh2, gf2, gn1, gr1, gf1, gh1, gattn, gx = (g[k] for k in ("gh2", "gf2", "gn1", "gr1", "gf1", "gh1", "gattn", "gx"))
-        gtok, gq, gk, gv = (g[k] for k in ("gtok", "gq", "gk", "gv"))
-        try:
-            dev.layer_norm_backward(s["h2"], p["g2"], gh2, grads["g2"], grads["be2"], grad_out)
-            dev.add_backward(gf2, gn1, gh2)            # h2 = f2 + n1
-            dev.linear_backward(s["r1"], gr1, p["w2"], grads["w2"], grads["b2"], gf2)
-            dev.relu_backward(s["f1"], gf1, gr1)
-            dev.linear_backward(n1, gn1, p["w1"], grads["w1"], grads["b1"], gf1)
-            dev.layer_norm_backward(s["h1"], p["g1"], gh1, grads["g1"], grads["be1"], gn1)
-            dev.add_backward(gattn, gx, gh1)           # h1 = attn + x
-            dev.linear_backward(tok, gtok, p["wo"], grads["wo"], grads["bo"], gattn)
-            if fused:
-                k = View(kv.storage, kv.dtype, qv.shape, qv.strides, kv.offset)
-                dev.attention_backward(qv, gq, k, gk, vv, gv, s["scale"], tok, gtok, s["lse"])
-            else:
-                gtokens, gp, gscores = g["gtokens"], g["gp"], g["gscores"]
-                dev.reshape_backward(tokens.permute(0, 2, 1, 3), gtokens, gtok)
-                dev.backward(probs, gp, vv, gv, gtokens)
-                if s["folded"]:
-                    dev.softmax_backward(probs, gscores, gp, s["scale"])
-                else:
-                    dev.softmax_backward(probs, g["gscaled"], gp, 1.0)
-                    dev.scalar_mul_backward(s["scale"], gscores, g["gscaled"])
-                dev.backward(qv, gq, kv, gk, gscores)
-            for w, b, gg in (("wq", "bq", gq), ("wk", "bk", gk), ("wv", "bv", gv)):   # x feeds three Linears: one buffer
-                dev.linear_backward(x, gx, p[w], grads[w], grads[b], gg)
-            dev.settle_zeros()   # nothing is left pending in this block; a gradient no op touched would be filled here
-        except BaseException:
-            # an op refused or raised in mid-pass: no declaration may outlive the pass unsettled, whoever still holds
-            # a View of the arena (the caller sees the exception, not zeros it could rely on)
-            if bufs and bufs[0].owner is not None:
-                bufs[0].owner.forget()
-            raise
-        return grads, gx
+        dev, torch = self.dev, self.dev._torch
+        plan, x, dtype = saved.plan, saved["x"], self.dtype
+        assert grad_out.shape == x.shape and grad_out.strides == x.strides and grad_out.dtype == dtype
+        grads = torch.empty(plan.grad_bytes, dtype=torch.uint8, device=dev.device)
+        scratch = torch.empty(plan.layout.backward_scratch_bytes, dtype=torch.uint8, device=dev.device)
+        base, ptrs = grads.data_ptr(), []
+        for n in range(0, len(plan.pieces), 2):
+            ptrs.append(base)
+            base += plan.pieces[n] + plan.pieces[n + 1]
+        vp = ctypes.c_void_p
+        dev._check(dev.lib.dfdx_rocm_encoder_backward(
+            dev.ctx, ctypes.byref(self._desc(plan)), vp(x.ptr), vp(saved.arena.data_ptr()), vp(grad_out.ptr), (vp * len(PARAMS))(*ptrs[:-1]),
+            vp(ptrs[-1]), vp(scratch.data_ptr())))
+        parts = grads.split(plan.pieces[::2]) if plan.gapless else grads.split(plan.pieces)[::2]
+        views = {name: View(part, dtype, shape, strides) for part, (name, shape, strides) in zip(parts, plan.grad_views)}
+        return views, views.pop("x")

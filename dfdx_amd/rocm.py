@@ -64,6 +64,23 @@ class Conv2DOp(ctypes.Structure):
                                                "chan_in", "chan_out", "h_in", "h_out", "w_in", "w_out")]
 
 
+ENCODER_PARAMS = 16   # DFDX_ROCM_ENCODER_PARAMS
+
+
+class Encoder(ctypes.Structure):
+    """``dfdx_rocm_encoder`` (include/dfdx_rocm.h)."""
+    _fields_ = [("dtype", ctypes.c_int32), ("reserved", ctypes.c_int32), ("batch", ctypes.c_int64), ("seq", ctypes.c_int64),
+                ("d_model", ctypes.c_int64), ("heads", ctypes.c_int64), ("d_ff", ctypes.c_int64),
+                ("params", ctypes.c_void_p * ENCODER_PARAMS)]
+
+
+class EncoderLayout(ctypes.Structure):
+    """``dfdx_rocm_encoder_layout``."""
+    _fields_ = [(n, ctypes.c_size_t) for n in ("saved_bytes", "forward_scratch_bytes", "backward_scratch_bytes", "q", "k", "v", "tok",
+                                               "h1", "n1", "h2", "r1", "lse", "probs", "tokens")] + \
+               [("fused_attention", ctypes.c_int32), ("reserved", ctypes.c_int32)]
+
+
 def lib_path() -> str:
     return os.path.join(_HERE, "lib", "libdfdx_rocm.so")
 
@@ -91,6 +108,7 @@ EXPORTS = [
     "dfdx_rocm_layer_norm_forward", "dfdx_rocm_layer_norm_backward",
     "dfdx_rocm_relu_forward", "dfdx_rocm_relu_backward",
     "dfdx_rocm_add_forward", "dfdx_rocm_add_backward",
+    "dfdx_rocm_encoder_plan", "dfdx_rocm_encoder_forward", "dfdx_rocm_encoder_backward",
     "dfdx_rocm_conv2d_forward", "dfdx_rocm_conv2d_backward",
 ]
 

@@ -416,6 +416,40 @@ int dfdx_rocm_relu_backward(dfdx_rocm_ctx *ctx, int dtype, int64_t len, const vo
 int dfdx_rocm_add_forward(dfdx_rocm_ctx *ctx, int dtype, int64_t len, const void *lhs, const void *rhs, void *out);
 int dfdx_rocm_add_backward(dfdx_rocm_ctx *ctx, int dtype, int64_t len, void *grad_lhs, void *grad_rhs, const void *grad_out);
 
+/* A whole TransformerEncoderBlock, forward and backward, as one call each
+ * (dfdx/src/nn/layers/transformer.rs:24-48): the sequence of the entry points
+ * above, with ReLU, the residual adds, ReLU's gradient and the sums of two
+ * gradient contributions done by the products they follow.  A value is rounded
+ * to the element type where the separate op would have read it rounded.
+ * `params` holds the 16 parameters in the order wq bq wk bk wv bv wo bo
+ * gamma1 beta1 w1 b1 w2 b2 gamma2 beta2; weights are (out, in) row-major
+ * Linear weights.  x, out, grad_out and grad_x are (batch, seq, d_model)
+ * contiguous.  The caller provides the storage: dfdx_rocm_encoder_plan tells how
+ * many bytes of it, and where in `saved` (16-byte-aligned; what the backward
+ * needs) the block's intermediate values lie: q, k, v and tok (the attention's
+ * result) in (batch, seq, d_model) token layout, h1 / h2 (inputs of the two
+ * LayerNorms), n1 (output of the first), r1 (ReLU's output), and, depending on
+ * fused_attention, lse (dfdx_rocm_attention_forward) or probs (batch, heads,
+ * seq, seq) and tokens (batch, heads, seq, dim).  `scratch` is free again when
+ * the work queued by the call is done.  Backward STORES its 16 gradients and
+ * grad_x (they need not be filled with zeros first). */
+#define DFDX_ROCM_ENCODER_PARAMS 16
+typedef struct dfdx_rocm_encoder {
+    int32_t dtype;
+    int32_t reserved;
+    int64_t batch, seq, d_model, heads, d_ff;
+    const void *params[DFDX_ROCM_ENCODER_PARAMS];
+} dfdx_rocm_encoder;
+typedef struct dfdx_rocm_encoder_layout {
+    size_t saved_bytes, forward_scratch_bytes, backward_scratch_bytes;
+    size_t q, k, v, tok, h1, n1, h2, r1, lse, probs, tokens; /* byte offsets in `saved` */
+    int32_t fused_attention, reserved;
+} dfdx_rocm_encoder_layout;
+int dfdx_rocm_encoder_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_encoder *block, dfdx_rocm_encoder_layout *layout);
+int dfdx_rocm_encoder_forward(dfdx_rocm_ctx *ctx, const dfdx_rocm_encoder *block, const void *x, void *out, void *saved, void *scratch);
+int dfdx_rocm_encoder_backward(dfdx_rocm_ctx *ctx, const dfdx_rocm_encoder *block, const void *x, const void *saved, const void *grad_out,
+                               void *const grads[DFDX_ROCM_ENCODER_PARAMS], void *grad_x, void *scratch);
+
 /* ---- conv2d: unfold + batched GEMM, and the forms that avoid its patch matrix -
  * Conv2DKernel (dfdx-core/src/tensor_ops/conv2d/mod.rs:31-55; Cpu impl
  * cpu_kernel.rs:40-278, Cuda impl cuda_kernel.rs:62-281).  The op struct has

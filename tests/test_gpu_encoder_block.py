@@ -1,0 +1,83 @@
+"""GPU: the encoder block's two calls against the same block strung together from the single entry points (Linear, the fused
+attention or its ops, LayerNorm, ReLU, add and their backward): every output and gradient equal bit for bit, since what the
+block's products do on the way into their results (ReLU, residual, ReLU's gradient, a first contribution read from elsewhere)
+rounds where the separate op would.  The shapes reach the small, the split and the tiled kernels, whole tiles and edges."""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import rng
+from gpu_util import announce, device
+
+pytestmark = pytest.mark.gpu
+
+from dfdx_amd import EncoderBlock, View  # noqa: E402
+from dfdx_amd.encoder import PARAMS  # noqa: E402
+
+
+def by_ops(dev, dtype, p, x, go, H):
+    B, S, d = x.shape
+    D, scale = d // H, (d // H) ** -0.5
+    zeros = lambda v: dev.zeros(dtype, v.shape)
+    q, k, v = (dev.linear_forward(x, p["w" + n], p["b" + n]) for n in "qkv")
+    heads = lambda t, *perm: View(t.storage, dtype, (B, S, H, D), (S * d, d, D, 1)).permute(*perm)
+    qv, vv, kv, kt = heads(q, 0, 2, 1, 3), heads(v, 0, 2, 1, 3), heads(k, 0, 2, 1, 3), heads(k, 0, 2, 3, 1)
+    fused = dev.attention_supported(dtype, D)
+    if fused:
+        tok, lse = dev.attention_forward(qv, kv, vv, scale)
+    else:
+        probs = dev.softmax_forward(dev.forward(qv, kt), scale)
+        tokens = dev.forward(probs, vv)
+        tok = dev.reshape_forward(tokens.permute(0, 2, 1, 3), (B, S, d))
+    h1 = dev.add_forward(dev.linear_forward(tok, p["wo"], p["bo"]), x)
+    n1 = dev.layer_norm_forward(h1, p["g1"], p["be1"])
+    r1 = dev.relu_forward(dev.linear_forward(n1, p["w1"], p["b1"]))
+    h2 = dev.add_forward(dev.linear_forward(r1, p["w2"], p["b2"]), n1)
+    out = dev.layer_norm_forward(h2, p["g2"], p["be2"])
+    g = {n: zeros(p[n]) for n in PARAMS}
+    gh2, gn1, gr1, gf1, gh1, gx, gtok, gq, gk, gv = (zeros(t) for t in (x, x, r1, r1, x, x, x, x, x, x))
+    dev.layer_norm_backward(h2, p["g2"], gh2, g["g2"], g["be2"], go)
+    dev.linear_backward(r1, gr1, p["w2"], g["w2"], g["b2"], gh2)
+    dev.relu_backward(r1, gf1, gr1)
+    dev.add_backward(gn1, zeros(x), gh2)
+    dev.linear_backward(n1, gn1, p["w1"], g["w1"], g["b1"], gf1)
+    dev.layer_norm_backward(h1, p["g1"], gh1, g["g1"], g["be1"], gn1)
+    dev.add_backward(gx, zeros(x), gh1)
+    dev.linear_backward(tok, gtok, p["wo"], g["wo"], g["bo"], gh1)
+    if fused:
+        dev.attention_backward(qv, gq, kv, gk, vv, gv, scale, tok, gtok, lse)
+    else:
+        gtokens, gp, gs = zeros(tokens), zeros(probs), zeros(probs)
+        dev.reshape_backward(tokens.permute(0, 2, 1, 3), gtokens, gtok)
+        dev.backward(probs, gp, vv, gv, gtokens)
+        dev.softmax_backward(probs, gs, gp, scale)
+        dev.backward(qv, gq, kt, gk, gs)
+    for n, gg in zip("qkv", (gq, gk, gv)):
+        dev.linear_backward(x, gx, p["w" + n], g["w" + n], g["b" + n], gg)
+    return out, g, gx
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("B,S,d,H,ff", [(1, 1, 64, 1, 64), (2, 33, 120, 3, 200), (3, 100, 256, 4, 1024), (1, 257, 512, 4, 2048), (4, 300, 1024, 16, 4096)])
+def test_block_equals_its_ops(dtype, B, S, d, H, ff):
+    dev = device()
+    announce("encoder block", dtype, (B, S, d, H, ff))
+    g = rng(d + S)
+    up = lambda shape, s: dev.tensor(oracle.to_storage((g.standard_normal(int(np.prod(shape))) * s).astype(np.float32), dtype), dtype, shape)
+    shapes = {n: (d, d) for n in ("wq", "wk", "wv", "wo")} | {"w1": (ff, d), "w2": (d, ff), "b1": (ff,)}
+    p = {n: up(shapes.get(n, (d,)), 1.0 if n in ("g1", "g2") else 0.05) for n in PARAMS}
+    x, go = up((B, S, d), 1.0), up((B, S, d), 1.0)
+    block = EncoderBlock(dev, dtype, d, H, ff, p)
+    out, saved = block.forward(x)
+    grads, gx = block.backward(saved, go)
+    want, wg, wgx = by_ops(dev, dtype, p, x, go, H)
+    dev.synchronize()
+    pairs = {"out": (out, want), "x": (gx, wgx)} | {n: (grads[n], wg[n]) for n in PARAMS}
+    tol = 5 * (4e-6 + {"f16": 2.0 ** -12, "bf16": 2.0 ** -9, "f32": 0.0}[dtype])
+    for n, (a, b) in pairs.items():
+        a, b = oracle.to_f64(dev.to_host(a), dtype), oracle.to_f64(dev.to_host(b), dtype)
+        if n == "out":
+            assert np.array_equal(a, b), np.abs(a - b).max()
+        elif n != "bk":   # a shift of all scores of a row: its gradient is the rounding of zero
+            assert np.linalg.norm(a - b) <= tol * np.linalg.norm(b), (n, np.linalg.norm(a - b) / np.linalg.norm(b))
+    assert saved["f1"].shape == (B, S, ff) and saved["probs"].shape == (B, H, S, S) and saved["tokens"].shape == (B, H, S, d // H)
