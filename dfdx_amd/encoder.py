@@ -19,6 +19,8 @@ from typing import Dict, Tuple
 
 from .rocm import DTYPES, ITEMSIZE, Encoder, EncoderLayout, Rocm, View, _row_major
 
+_POINTERS = ctypes.c_void_p * 16
+
 PARAMS = ("wq", "bq", "wk", "bk", "wv", "bv", "wo", "bo", "g1", "be1", "w1", "b1", "w2", "b2", "g2", "be2")
 
 
@@ -123,36 +125,33 @@ class EncoderBlock:
 
     def forward(self, x: View) -> Tuple[View, dict]:
         """x: (batch, seq, d_model) contiguous.  Returns the block's output and the tensors the backward needs."""
-        dev, torch = self.dev, self.dev._torch
+        dev = self.dev
         B, S, d = x.shape
         assert d == self.d, f"left: {d}\n right: {self.d}"
         strides = (S * d, d, 1)
         assert x.strides == strides and x.dtype == self.dtype, "encoder input must be contiguous"
         plan = self._plan(B, S)
         l = plan.layout
-        out = torch.empty(max(B * S * d * ITEMSIZE[self.dtype], 16), dtype=torch.uint8, device=dev.device)
-        arena = torch.empty(l.saved_bytes, dtype=torch.uint8, device=dev.device)
-        scratch = torch.empty(l.forward_scratch_bytes, dtype=torch.uint8, device=dev.device) if l.forward_scratch_bytes else None
-        vp = ctypes.c_void_p
-        dev._check(dev.lib.dfdx_rocm_encoder_forward(dev.ctx, ctypes.byref(self._desc(plan)), vp(x.ptr), vp(out.data_ptr()), vp(arena.data_ptr()),
-                                                     vp(scratch.data_ptr() if scratch is not None else None)))
+        out = dev._bytes(max(B * S * d * ITEMSIZE[self.dtype], 16))
+        arena = dev._bytes(l.saved_bytes)
+        scratch = dev._bytes(l.forward_scratch_bytes) if l.forward_scratch_bytes else None
+        dev._check(dev._f.encoder_forward(dev.ctx, ctypes.byref(self._desc(plan)), x.ptr, out.data_ptr(), arena.data_ptr(),
+                                          scratch.data_ptr() if scratch is not None else None))
         return View(out, self.dtype, (B, S, d), strides), _Saved(self, plan, x, arena)
 
     def backward(self, saved: dict, grad_out: View) -> Tuple[Dict[str, View], View]:
         """grad_out: d(loss)/d(out), contiguous like the output.  Returns ({parameter: gradient}, d(loss)/d(x))."""
-        dev, torch = self.dev, self.dev._torch
+        dev = self.dev
         plan, x, dtype = saved.plan, saved["x"], self.dtype
         assert grad_out.shape == x.shape and grad_out.strides == x.strides and grad_out.dtype == dtype
-        grads = torch.empty(plan.grad_bytes, dtype=torch.uint8, device=dev.device)
-        scratch = torch.empty(plan.layout.backward_scratch_bytes, dtype=torch.uint8, device=dev.device)
+        grads = dev._bytes(plan.grad_bytes)
+        scratch = dev._bytes(plan.layout.backward_scratch_bytes)
         base, ptrs = grads.data_ptr(), []
         for n in range(0, len(plan.pieces), 2):
             ptrs.append(base)
             base += plan.pieces[n] + plan.pieces[n + 1]
-        vp = ctypes.c_void_p
-        dev._check(dev.lib.dfdx_rocm_encoder_backward(
-            dev.ctx, ctypes.byref(self._desc(plan)), vp(x.ptr), vp(saved.arena.data_ptr()), vp(grad_out.ptr), (vp * len(PARAMS))(*ptrs[:-1]),
-            vp(ptrs[-1]), vp(scratch.data_ptr())))
+        dev._check(dev._f.encoder_backward(dev.ctx, ctypes.byref(self._desc(plan)), x.ptr, saved.arena.data_ptr(), grad_out.ptr,
+                                           _POINTERS(*ptrs[:-1]), ptrs[-1], scratch.data_ptr()))
         parts = grads.split(plan.pieces[::2]) if plan.gapless else grads.split(plan.pieces)[::2]
         views = {name: View(part, dtype, shape, strides) for part, (name, shape, strides) in zip(parts, plan.grad_views)}
         return views, views.pop("x")

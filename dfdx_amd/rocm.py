@@ -15,8 +15,9 @@ PyTorch is used for device memory only (allocation, host<->device copies).
 from __future__ import annotations
 
 import ctypes
+import math
 import os
-import weakref
+import struct
 from dataclasses import dataclass
 from typing import Optional, Sequence
 
@@ -132,6 +133,41 @@ def load_library() -> ctypes.CDLL:
     return _lib
 
 
+# The entry points a training or inference step goes through, with their argument types: a call then costs no wrapper
+# object per argument (3 us of the 10 us that a 64-row Linear used to take on the host).  p: pointer (an address, or the
+# packed bytes of a small array), i: int, l: int64_t, z: size_t, f: float, d: double.
+_KINDS = {"p": ctypes.c_void_p, "i": ctypes.c_int, "l": ctypes.c_int64, "z": ctypes.c_size_t, "f": ctypes.c_float, "d": ctypes.c_double}
+_TYPED = {
+    "memset_zero": "ppz", "zero_deferred": "ppz", "settle_zeros": "p", "forget_zeros": "ppz",
+    "matmat_forward": "pilllppppp", "matmat_backward": "pilllppppppp",
+    "matmat_br_forward": "pillllppppp", "matmat_br_backward": "pillllppppppp",
+    "matmat_batch3_forward": "pillllppppp", "matmat_batch3_backward": "pillllppppppp",
+    "matmat_batch4_forward": "pilllllppppp", "matmat_batch4_backward": "pilllllppppppp",
+    "linear_forward": "pilllppppp", "linear_backward": "pilllppppppp",
+    "bias_forward": "pillppp", "bias_backward": "pillpp",
+    "scalar_mul_forward": "pilpdp", "scalar_mul_backward": "pildpp",
+    "softmax_forward": "pillpfp", "softmax_backward": "pillpfpp",
+    "reshape_forward": "piipppp", "reshape_backward": "piipppp",
+    "attention_forward": "pillllppppfppp", "attention_backward": "pillllppppfppppppp",
+    "layer_norm_forward": "pillpppdp", "layer_norm_backward": "pillppdpppp",
+    "relu_forward": "pilpp", "relu_backward": "pilppp", "add_forward": "pilppp", "add_backward": "pilppp",
+    "conv2d_forward": "pipppp", "conv2d_backward": "pipppppp",
+    "encoder_forward": "pppppp", "encoder_backward": "pppppppp",
+}
+_PACK = {n: struct.Struct(f"{n}q").pack for n in range(1, 9)}
+
+
+class _Typed:
+    def __init__(self, lib):
+        for name, kinds in _TYPED.items():
+            setattr(self, name, ctypes.CFUNCTYPE(ctypes.c_int, *[_KINDS[k] for k in kinds])(("dfdx_rocm_" + name, lib)))
+
+
+def _i64s(v) -> bytes:
+    """A small int64_t array as an argument: the call reads it while the bytes object lives."""
+    return _PACK[len(v)](*v)
+
+
 @dataclass
 class View:
     """Device storage seen through a shape and element strides (a dfdx tensor's kernel-side face)."""
@@ -144,7 +180,7 @@ class View:
 
     @property
     def ptr(self) -> int:
-        return self.storage.data_ptr() + self.offset * ITEMSIZE[self.dtype]
+        return self.storage.data_ptr() + self.offset * ITEMSIZE[self.dtype] if self.offset else self.storage.data_ptr()
 
     def permute(self, *axes) -> "View":
         """Zero-copy permute (reference: tensor_ops/permute_to.rs:38-52)."""
@@ -158,28 +194,36 @@ class View:
 class _Arena:
     """One allocation that several Views are carved from.  When the last View of it goes, whatever zero declarations
     its pieces still carry are withdrawn (``dfdx_rocm_forget_zeros``) BEFORE torch gets the memory back, so that a later
-    settle cannot write zeros into memory that has a new owner by then."""
+    settle cannot write zeros into memory that has a new owner by then.  (At interpreter exit the context may go first; it
+    takes its declarations with it.)"""
+    __slots__ = ("dev", "raw")
 
     def __init__(self, dev: "Rocm", raw):
-        self.raw = raw
-        self._fin = weakref.finalize(self, _forget_range, weakref.ref(dev), raw, raw.data_ptr(), raw.numel())
-        self._fin.atexit = False   # at interpreter exit the context goes first and takes its declarations with it
+        self.dev, self.raw = dev, raw   # the views keep the device alive, which the declarations need anyway
 
     def forget(self):
-        self._fin()
+        dev, raw = self.dev, self.raw
+        if dev is not None and dev.ctx:
+            dev._f.forget_zeros(dev.ctx, raw.data_ptr(), raw.numel())
+        self.dev = None
 
-
-def _forget_range(dev_ref, raw, ptr, nbytes):
-    # `raw` is held by this callback's arguments: the memory is still allocated while the declarations are dropped
-    dev = dev_ref()
-    if dev is not None and getattr(dev, "ctx", None):
-        dev.lib.dfdx_rocm_forget_zeros(dev.ctx, ctypes.c_void_p(ptr), ctypes.c_size_t(nbytes))
-    del raw
+    def __del__(self):
+        try:
+            self.forget()
+        except Exception:   # at interpreter exit
+            pass
 
 
 def _row_major(shape):
-    s = [1] * len(shape)
-    for i in range(len(shape) - 2, -1, -1):
+    n = len(shape)
+    if n == 1:
+        return (1,)
+    if n == 2:
+        return (shape[1], 1)
+    if n == 3:
+        return (shape[1] * shape[2], shape[2], 1)
+    s = [1] * n
+    for i in range(n - 2, -1, -1):
         s[i] = s[i + 1] * shape[i + 1]
     return tuple(s)
 
@@ -198,6 +242,7 @@ class Rocm:
         if not torch.cuda.is_available():
             raise RuntimeError("no GPU visible: the Rocm device needs an MI355X (there is no CPU fallback)")
         self.lib = load_library()
+        self._f = _Typed(self.lib)
         self.ordinal = ordinal
         self.device = torch.device("cuda", ordinal)
         torch.cuda.set_device(ordinal)
@@ -205,6 +250,7 @@ class Rocm:
         ctx = ctypes.c_void_p()
         self._check(self.lib.dfdx_rocm_create(ordinal, ctypes.c_void_p(stream), ctypes.byref(ctx)))
         self.ctx = ctx
+        self._bytes = torch.empty(1, dtype=torch.uint8, device=self.device).new_empty   # uninitialised bytes on the device
 
     def close(self):
         if getattr(self, "ctx", None):
@@ -260,7 +306,7 @@ class Rocm:
     def zero_deferred(self, ptr: int, nbytes: int):
         """Declares ``nbytes`` at ``ptr`` zero without filling them (``dfdx_rocm_zero_deferred``): the first call that
         accumulates into the whole buffer stores 0 + value, any other first use runs the fill."""
-        self._check(self.lib.dfdx_rocm_zero_deferred(self.ctx, ctypes.c_void_p(ptr), ctypes.c_size_t(nbytes)))
+        self._check(self._f.zero_deferred(self.ctx, ptr, nbytes))
 
     def forget_zeros(self, ptr: int, nbytes: int):
         """Withdraws the zero declarations inside ``[ptr, ptr + nbytes)`` without filling (``dfdx_rocm_forget_zeros``):
@@ -269,7 +315,7 @@ class Rocm:
 
     def settle_zeros(self):
         """Runs every deferred fill still pending: needed before code outside the library reads such a buffer."""
-        self._check(self.lib.dfdx_rocm_settle_zeros(self.ctx))
+        self._check(self._f.settle_zeros(self.ctx))
 
     # --------------------------------------------------------------- storage --
     def tensor(self, host: np.ndarray, dtype: str, shape=None, strides=None) -> View:
@@ -302,39 +348,38 @@ class Rocm:
         accumulates into the whole of it stores instead -- read the results through this object (``to_host``) or
         call ``settle_zeros`` first.  The declarations are withdrawn when the last of the returned Views (and of the
         Views derived from them) is dropped, so the arena never goes back to the allocator with a fill still promised."""
-        sizes = [max(int(np.prod(v.shape, dtype=np.int64)) * ITEMSIZE[v.dtype], 16) for v in likes]
-        offs, total = [], 0
-        for n in sizes:
-            offs.append(total)
-            total += (n + 255) // 256 * 256
+        sizes, total, pieces = [], 0, []
+        for v in likes:
+            n = max(math.prod(v.shape) * ITEMSIZE[v.dtype], 16)
+            sizes.append((total, n))
+            pieces += (n, -n % 256)
+            total += n + -n % 256
         owner = None
         if deferred:
-            arena = self._torch.empty(max(total, 16), dtype=self._torch.uint8, device=self.device)
+            arena = self._bytes(max(total, 16))
             owner = _Arena(self, arena)
-            try:
-                for o, n in zip(offs, sizes):
-                    self.zero_deferred(arena.data_ptr() + o, n)
-            except Exception:
-                owner.forget()
-                raise
+            declare, ctx, base = self._f.zero_deferred, self.ctx, arena.data_ptr()
+            for o, n in sizes:
+                rc = declare(ctx, base + o, n)
+                if rc:
+                    owner.forget()
+                    self._check(rc)
         else:
             arena = self._zeroed_bytes(max(total, 16))
-        return [View(arena[o:o + n], v.dtype, tuple(v.shape), _row_major(tuple(v.shape)), 0, owner)
-                for v, o, n in zip(likes, offs, sizes)]
+        parts = arena.split(pieces)[::2] if pieces else ()
+        return [View(part, v.dtype, tuple(v.shape), _row_major(v.shape), 0, owner) for v, part in zip(likes, parts)]
 
     def _zeroed_bytes(self, nbytes: int):
         """Device memory from torch's allocator, cleared by the library's own fill kernel (``dfdx_rocm_memset_zero``)."""
-        raw = self._torch.empty(nbytes, dtype=self._torch.uint8, device=self.device)
-        self._check(self.lib.dfdx_rocm_memset_zero(self.ctx, ctypes.c_void_p(raw.data_ptr()), ctypes.c_size_t(nbytes)))
+        raw = self._bytes(nbytes)
+        self._check(self._f.memset_zero(self.ctx, raw.data_ptr(), nbytes))
         return raw
 
     def empty(self, dtype: str, shape) -> View:
         """Uninitialised storage for an output that a forward kernel overwrites (``alloc_empty``,
         tensor_ops/matmul/cuda_kernel.rs:253)."""
         shape = tuple(shape)
-        n = int(np.prod(shape, dtype=np.int64))
-        raw = self._torch.empty(max(n * ITEMSIZE[dtype], 16), dtype=self._torch.uint8, device=self.device)
-        return View(raw, dtype, shape, _row_major(shape))
+        return View(self._bytes(max(math.prod(shape) * ITEMSIZE[dtype], 16)), dtype, shape, _row_major(shape))
 
     def zeros_like_storage(self, v: View) -> View:
         """A gradient buffer for ``v``: zero-filled, same physical length, same strides (gradients.rs:53-58)."""
@@ -397,222 +442,170 @@ class Rocm:
     # --------------------------------------------------------- kernel traits --
     def forward(self, lhs: View, rhs: View) -> View:
         """Dispatch on rank like ``TryMatMul`` (mod.rs:133-311); rank-1 operands are reshapes (mod.rs:139-174)."""
-        dt = lhs.dtype
-        assert lhs.dtype == rhs.dtype
-        L, R = len(lhs.shape), len(rhs.shape)
-        vp = ctypes.c_void_p
-        if L == 1 and R == 1:      # outer product: (M,1) x (1,N)
-            m, n = lhs.shape[0], rhs.shape[0]
-            out = self.empty(dt, (m, n))
-            self._check(self.lib.dfdx_rocm_matmat_forward(
-                self.ctx, DTYPES[dt], _c(m), _c(1), _c(n), vp(lhs.ptr), _i64arr((lhs.strides[0], 1)),
-                vp(rhs.ptr), _i64arr((n * rhs.strides[0], rhs.strides[0])), vp(out.ptr)))
-            return out
-        if L == 1 and R == 2:      # (1,K) x (K,N) -> (N,)
-            assert lhs.shape[0] == rhs.shape[0], f"left: {lhs.shape[0]}\n right: {rhs.shape[0]}"
-            k, n = rhs.shape
-            out = self.empty(dt, (n,))
-            self._check(self.lib.dfdx_rocm_matmat_forward(
-                self.ctx, DTYPES[dt], _c(1), _c(k), _c(n), vp(lhs.ptr), _i64arr((k * lhs.strides[0], lhs.strides[0])),
-                vp(rhs.ptr), _i64arr(rhs.strides), vp(out.ptr)))
-            return out
-        if L == 2 and R == 1:      # (M,K) x (K,1) -> (M,)
-            assert lhs.shape[1] == rhs.shape[0], f"left: {lhs.shape[1]}\n right: {rhs.shape[0]}"
-            m, k = lhs.shape
-            out = self.empty(dt, (m,))
-            self._check(self.lib.dfdx_rocm_matmat_forward(
-                self.ctx, DTYPES[dt], _c(m), _c(k), _c(1), vp(lhs.ptr), _i64arr(lhs.strides),
-                vp(rhs.ptr), _i64arr((rhs.strides[0], 1)), vp(out.ptr)))
-            return out
-        if L == 2 and R == 2:
-            assert lhs.shape[1] == rhs.shape[0], f"left: {lhs.shape[1]}\n right: {rhs.shape[0]}"
-            (m, k), n = lhs.shape, rhs.shape[1]
-            out = self.empty(dt, (m, n))
-            self._check(self.lib.dfdx_rocm_matmat_forward(
-                self.ctx, DTYPES[dt], _c(m), _c(k), _c(n), vp(lhs.ptr), _i64arr(lhs.strides),
-                vp(rhs.ptr), _i64arr(rhs.strides), vp(out.ptr)))
-            return out
-        if L == 3 and R == 2:
-            assert lhs.shape[2] == rhs.shape[0], f"left: {lhs.shape[2]}\n right: {rhs.shape[0]}"
-            (b, m, k), n = lhs.shape, rhs.shape[1]
-            out = self.empty(dt, (b, m, n))
-            self._check(self.lib.dfdx_rocm_matmat_br_forward(
-                self.ctx, DTYPES[dt], _c(b), _c(m), _c(k), _c(n), vp(lhs.ptr), _i64arr(lhs.strides),
-                vp(rhs.ptr), _i64arr(rhs.strides), vp(out.ptr)))
-            return out
-        if L == 3 and R == 3:
-            assert lhs.shape[0] == rhs.shape[0], f"left: {lhs.shape[0]}\n right: {rhs.shape[0]}"
-            assert lhs.shape[2] == rhs.shape[1], f"left: {lhs.shape[2]}\n right: {rhs.shape[1]}"
-            (b, m, k), n = lhs.shape, rhs.shape[2]
-            out = self.empty(dt, (b, m, n))
-            self._check(self.lib.dfdx_rocm_matmat_batch3_forward(
-                self.ctx, DTYPES[dt], _c(b), _c(m), _c(k), _c(n), vp(lhs.ptr), _i64arr(lhs.strides),
-                vp(rhs.ptr), _i64arr(rhs.strides), vp(out.ptr)))
-            return out
-        if L == 4 and R == 4:
-            assert lhs.shape[0] == rhs.shape[0], f"left: {lhs.shape[0]}\n right: {rhs.shape[0]}"
-            assert lhs.shape[1] == rhs.shape[1], f"left: {lhs.shape[1]}\n right: {rhs.shape[1]}"
-            assert lhs.shape[3] == rhs.shape[2], f"left: {lhs.shape[3]}\n right: {rhs.shape[2]}"
-            (b, s, m, k), n = lhs.shape, rhs.shape[3]
-            out = self.empty(dt, (b, s, m, n))
-            self._check(self.lib.dfdx_rocm_matmat_batch4_forward(
-                self.ctx, DTYPES[dt], _c(b), _c(s), _c(m), _c(k), _c(n), vp(lhs.ptr), _i64arr(lhs.strides),
-                vp(rhs.ptr), _i64arr(rhs.strides), vp(out.ptr)))
-            return out
-        raise TypeError(f"matmul of rank {L} by rank {R} is not defined (mod.rs:133-311)")
+        dt, ls, rs, lt, rt = lhs.dtype, lhs.shape, rhs.shape, lhs.strides, rhs.strides
+        assert dt == rhs.dtype
+        L, R = len(ls), len(rs)
+        if L <= 2 and R <= 2:
+            if L == 2 and R == 2:
+                assert ls[1] == rs[0], f"left: {ls[1]}\n right: {rs[0]}"
+                (m, k), n = ls, rs[1]
+                shape = (m, n)
+            elif L == 1 and R == 1:      # outer product: (M,1) x (1,N)
+                m, k, n = ls[0], 1, rs[0]
+                shape, lt, rt = (m, n), (lt[0], 1), (n * rt[0], rt[0])
+            elif L == 1:                 # (1,K) x (K,N) -> (N,)
+                assert ls[0] == rs[0], f"left: {ls[0]}\n right: {rs[0]}"
+                m, (k, n) = 1, rs
+                shape, lt = (n,), (k * lt[0], lt[0])
+            else:                        # (M,K) x (K,1) -> (M,)
+                assert ls[1] == rs[0], f"left: {ls[1]}\n right: {rs[0]}"
+                (m, k), n = ls, 1
+                shape, rt = (m,), (rt[0], 1)
+            fn, dims = self._f.matmat_forward, (m, k, n)
+        elif L == 3 and R == 2:
+            assert ls[2] == rs[0], f"left: {ls[2]}\n right: {rs[0]}"
+            (b, m, k), n = ls, rs[1]
+            fn, dims, shape = self._f.matmat_br_forward, (b, m, k, n), (b, m, n)
+        elif L == 3 and R == 3:
+            assert ls[0] == rs[0], f"left: {ls[0]}\n right: {rs[0]}"
+            assert ls[2] == rs[1], f"left: {ls[2]}\n right: {rs[1]}"
+            (b, m, k), n = ls, rs[2]
+            fn, dims, shape = self._f.matmat_batch3_forward, (b, m, k, n), (b, m, n)
+        elif L == 4 and R == 4:
+            assert ls[0] == rs[0], f"left: {ls[0]}\n right: {rs[0]}"
+            assert ls[1] == rs[1], f"left: {ls[1]}\n right: {rs[1]}"
+            assert ls[3] == rs[2], f"left: {ls[3]}\n right: {rs[2]}"
+            (b, s, m, k), n = ls, rs[3]
+            fn, dims, shape = self._f.matmat_batch4_forward, (b, s, m, k, n), (b, s, m, n)
+        else:
+            raise TypeError(f"matmul of rank {L} by rank {R} is not defined (mod.rs:133-311)")
+        out = self.empty(dt, shape)
+        rc = fn(self.ctx, DTYPES[dt], *dims, lhs.ptr, _i64s(lt), rhs.ptr, _i64s(rt), out.storage.data_ptr())
+        if rc:
+            self._check(rc)
+        return out
 
     def backward(self, lhs: View, grad_lhs: View, rhs: View, grad_rhs: View, grad_out: View):
         """``D::backward(lhs, grad_lhs, rhs, grad_rhs, grad_out)``; grad_out contiguous; grads accumulate."""
-        dt = lhs.dtype
-        L, R = len(lhs.shape), len(rhs.shape)
-        vp = ctypes.c_void_p
+        ls, rs, lt, rt = lhs.shape, rhs.shape, lhs.strides, rhs.strides
+        L, R = len(ls), len(rs)
         if L <= 2 and R <= 2:
-            if L == 1 and R == 1:
-                m, k, n = lhs.shape[0], 1, rhs.shape[0]
-                ls, rs = (lhs.strides[0], 1), (n * rhs.strides[0], rhs.strides[0])
+            if L == 2 and R == 2:
+                dims = (*ls, rs[1])
+            elif L == 1 and R == 1:
+                n = rs[0]
+                dims, lt, rt = (ls[0], 1, n), (lt[0], 1), (n * rt[0], rt[0])
             elif L == 1:
-                (k, n), m = rhs.shape, 1
-                ls, rs = (k * lhs.strides[0], lhs.strides[0]), rhs.strides
-            elif R == 1:
-                (m, k), n = lhs.shape, 1
-                ls, rs = lhs.strides, (rhs.strides[0], 1)
+                k, n = rs
+                dims, lt = (1, k, n), (k * lt[0], lt[0])
             else:
-                (m, k), n = lhs.shape, rhs.shape[1]
-                ls, rs = lhs.strides, rhs.strides
-            self._check(self.lib.dfdx_rocm_matmat_backward(
-                self.ctx, DTYPES[dt], _c(m), _c(k), _c(n), vp(lhs.ptr), _i64arr(ls), vp(grad_lhs.ptr),
-                vp(rhs.ptr), _i64arr(rs), vp(grad_rhs.ptr), vp(grad_out.ptr)))
-            return
-        if L == 3 and R == 2:
-            (b, m, k), n = lhs.shape, rhs.shape[1]
-            fn, dims = self.lib.dfdx_rocm_matmat_br_backward, (b, m, k, n)
+                dims, rt = (*ls, 1), (rt[0], 1)
+            fn = self._f.matmat_backward
+        elif L == 3 and R == 2:
+            fn, dims = self._f.matmat_br_backward, (*ls, rs[1])
         elif L == 3 and R == 3:
-            (b, m, k), n = lhs.shape, rhs.shape[2]
-            fn, dims = self.lib.dfdx_rocm_matmat_batch3_backward, (b, m, k, n)
+            fn, dims = self._f.matmat_batch3_backward, (*ls, rs[2])
         elif L == 4 and R == 4:
-            (b, s, m, k), n = lhs.shape, rhs.shape[3]
-            fn, dims = self.lib.dfdx_rocm_matmat_batch4_backward, (b, s, m, k, n)
+            fn, dims = self._f.matmat_batch4_backward, (*ls, rs[3])
         else:
             raise TypeError(f"matmul of rank {L} by rank {R} is not defined")
-        self._check(fn(self.ctx, DTYPES[dt], *[_c(d) for d in dims], vp(lhs.ptr), _i64arr(lhs.strides),
-                       vp(grad_lhs.ptr), vp(rhs.ptr), _i64arr(rhs.strides), vp(grad_rhs.ptr), vp(grad_out.ptr)))
+        rc = fn(self.ctx, DTYPES[lhs.dtype], *dims, lhs.ptr, _i64s(lt), grad_lhs.ptr, rhs.ptr, _i64s(rt), grad_rhs.ptr, grad_out.ptr)
+        if rc:
+            self._check(rc)
 
     def linear_forward(self, x: View, weight: View, bias: Optional[View]) -> View:
         """``Linear::try_forward`` (dfdx/src/nn/layers/linear.rs:82-89); weight is the (O, I) storage."""
         o, i = weight.shape
         assert weight.strides == (i, 1), "Linear weight storage is (O, I) row-major"
-        assert x.shape[-1] == i, f"left: {x.shape[-1]}\n right: {i}"
-        if len(x.shape) == 1:
-            rows, xs = 1, (i * x.strides[0], x.strides[0])
-        elif len(x.shape) == 2:
-            rows, xs = x.shape[0], x.strides
-        else:
-            assert x.strides == _row_major(x.shape), "batched Linear input must be contiguous to fold its rows"
-            rows, xs = int(np.prod(x.shape[:-1])), (i, 1)
-        out = self.empty(x.dtype, tuple(x.shape[:-1]) + (o,))
-        self._check(self.lib.dfdx_rocm_linear_forward(
-            self.ctx, DTYPES[x.dtype], _c(rows), _c(i), _c(o), ctypes.c_void_p(x.ptr), _i64arr(xs),
-            ctypes.c_void_p(weight.ptr), ctypes.c_void_p(bias.ptr if bias is not None else None),
-            ctypes.c_void_p(out.ptr)))
+        shape = x.shape
+        assert shape[-1] == i, f"left: {shape[-1]}\n right: {i}"
+        rows, xs = self._linear_rows(x, i)
+        out = self.empty(x.dtype, (*shape[:-1], o))
+        rc = self._f.linear_forward(self.ctx, DTYPES[x.dtype], rows, i, o, x.ptr, _i64s(xs), weight.ptr,
+                                    bias.ptr if bias is not None else None, out.storage.data_ptr())
+        if rc:
+            self._check(rc)
         return out
 
     def _linear_rows(self, x: View, i: int):
-        if len(x.shape) == 1:
-            return 1, (i * x.strides[0], x.strides[0])
         if len(x.shape) == 2:
             return x.shape[0], x.strides
+        if len(x.shape) == 1:
+            return 1, (i * x.strides[0], x.strides[0])
         assert x.strides == _row_major(x.shape), "batched Linear input must be contiguous to fold its rows"
-        return int(np.prod(x.shape[:-1])), (i, 1)
+        return math.prod(x.shape[:-1]), (i, 1)
 
     def linear_backward(self, x: View, grad_x: View, weight: View, grad_weight: View, grad_bias: Optional[View],
                         grad_out: View):
         """Backward of ``Linear``: grad_x += go.W, grad_weight += go^T.x, grad_bias += column sums of go."""
         o, i = weight.shape
         assert weight.strides == (i, 1), "Linear weight storage is (O, I) row-major"
-        assert x.shape[-1] == i, f"left: {x.shape[-1]}\n right: {i}"
-        assert grad_out.shape == tuple(x.shape[:-1]) + (o,) and grad_out.strides == _row_major(grad_out.shape)
+        shape = x.shape
+        assert shape[-1] == i, f"left: {shape[-1]}\n right: {i}"
+        assert grad_out.shape == (*shape[:-1], o) and grad_out.strides == _row_major(grad_out.shape)
         rows, xs = self._linear_rows(x, i)
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_linear_backward(
-            self.ctx, DTYPES[x.dtype], _c(rows), _c(i), _c(o), vp(x.ptr), _i64arr(xs), vp(grad_x.ptr),
-            vp(weight.ptr), vp(grad_weight.ptr), vp(grad_bias.ptr if grad_bias is not None else None),
-            vp(grad_out.ptr)))
+        rc = self._f.linear_backward(self.ctx, DTYPES[x.dtype], rows, i, o, x.ptr, _i64s(xs), grad_x.ptr, weight.ptr, grad_weight.ptr,
+                                     grad_bias.ptr if grad_bias is not None else None, grad_out.ptr)
+        if rc:
+            self._check(rc)
 
     def bias_forward(self, x: View, bias: View) -> View:
         """``Bias1D::try_forward`` (dfdx/src/nn/layers/bias1d.rs:62-78) on a contiguous input."""
         cols = bias.shape[0]
         assert x.shape[-1] == cols, f"left: {x.shape[-1]}\n right: {cols}"
         assert x.strides == _row_major(x.shape) and bias.strides == (1,)
-        rows = int(np.prod(x.shape[:-1], dtype=np.int64))
         out = self.empty(x.dtype, x.shape)
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_bias_forward(self.ctx, DTYPES[x.dtype], _c(rows), _c(cols), vp(x.ptr),
-                                                    vp(bias.ptr), vp(out.ptr)))
+        self._check(self._f.bias_forward(self.ctx, DTYPES[x.dtype], math.prod(x.shape[:-1]), cols, x.ptr, bias.ptr, out.ptr))
         return out
 
     def bias_backward(self, grad_out: View, grad_bias: View):
         """grad_bias += column sums of grad_out (the broadcast operand's share of the add's backward)."""
         cols = grad_bias.shape[0]
         assert grad_out.shape[-1] == cols and grad_out.strides == _row_major(grad_out.shape)
-        rows = int(np.prod(grad_out.shape[:-1], dtype=np.int64))
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_bias_backward(self.ctx, DTYPES[grad_out.dtype], _c(rows), _c(cols),
-                                                     vp(grad_out.ptr), vp(grad_bias.ptr)))
+        self._check(self._f.bias_backward(self.ctx, DTYPES[grad_out.dtype], math.prod(grad_out.shape[:-1]), cols, grad_out.ptr, grad_bias.ptr))
 
     # ------------------------------------------------- ops between attention's GEMMs --
+    def _like(self, x: View) -> View:
+        """Uninitialised storage of the same physical length, seen the same way."""
+        return View(self._bytes(x.storage.numel()), x.dtype, x.shape, x.strides, x.offset)
+
     def scalar_mul_forward(self, x: View, scalar: float) -> View:
         """``x * scalar`` over the physical storage (unary kernel, utilities/cpu_kernels.rs:46-79); same strides."""
-        out = View(self._torch.empty_like(x.storage), x.dtype, x.shape, x.strides, x.offset)
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_scalar_mul_forward(self.ctx, DTYPES[x.dtype], _c(x.numel_storage()),
-                                                          vp(x.storage.data_ptr()), ctypes.c_double(scalar),
-                                                          vp(out.storage.data_ptr())))
+        out = self._like(x)
+        self._check(self._f.scalar_mul_forward(self.ctx, DTYPES[x.dtype], x.numel_storage(), x.storage.data_ptr(), scalar, out.storage.data_ptr()))
         return out
 
     def scalar_mul_backward(self, scalar: float, grad_inp: View, grad_out: View):
         assert grad_inp.numel_storage() == grad_out.numel_storage()
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_scalar_mul_backward(self.ctx, DTYPES[grad_inp.dtype], _c(grad_inp.numel_storage()),
-                                                           ctypes.c_double(scalar), vp(grad_inp.storage.data_ptr()),
-                                                           vp(grad_out.storage.data_ptr())))
+        self._check(self._f.scalar_mul_backward(self.ctx, DTYPES[grad_inp.dtype], grad_inp.numel_storage(), scalar,
+                                                grad_inp.storage.data_ptr(), grad_out.storage.data_ptr()))
 
     def softmax_forward(self, x: View, scale: float = 1.0) -> View:
         """softmax(scale * x) over the last axis of a contiguous tensor (softmax.rs:70-83)."""
         assert x.strides == _row_major(x.shape), "softmax input must be contiguous"
-        cols = x.shape[-1]
-        rows = int(np.prod(x.shape[:-1], dtype=np.int64))
-        out = View(self._torch.empty_like(x.storage), x.dtype, x.shape, x.strides)
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_softmax_forward(self.ctx, DTYPES[x.dtype], _c(rows), _c(cols), vp(x.ptr),
-                                                       ctypes.c_float(scale), vp(out.ptr)))
+        out = View(self._bytes(x.storage.numel()), x.dtype, x.shape, x.strides)
+        self._check(self._f.softmax_forward(self.ctx, DTYPES[x.dtype], math.prod(x.shape[:-1]), x.shape[-1], x.ptr, scale, out.ptr))
         return out
 
     def softmax_backward(self, out: View, grad_x: View, grad_out: View, scale: float = 1.0):
         assert out.strides == _row_major(out.shape) and grad_out.shape == out.shape and grad_x.shape == out.shape
-        cols = out.shape[-1]
-        rows = int(np.prod(out.shape[:-1], dtype=np.int64))
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_softmax_backward(self.ctx, DTYPES[out.dtype], _c(rows), _c(cols), vp(out.ptr),
-                                                        ctypes.c_float(scale), vp(grad_x.ptr), vp(grad_out.ptr)))
+        self._check(self._f.softmax_backward(self.ctx, DTYPES[out.dtype], math.prod(out.shape[:-1]), out.shape[-1], out.ptr, scale,
+                                             grad_x.ptr, grad_out.ptr))
 
     def reshape_forward(self, x: View, new_shape) -> View:
         """``try_reshape_like`` (reshape_to/mod.rs:90-115): free for a contiguous tensor, a copy otherwise."""
         new_shape = tuple(int(d) for d in new_shape)
-        assert int(np.prod(x.shape, dtype=np.int64)) == int(np.prod(new_shape, dtype=np.int64)), \
-            f"left: {int(np.prod(x.shape))}\n right: {int(np.prod(new_shape))}"
+        assert math.prod(x.shape) == math.prod(new_shape), f"left: {math.prod(x.shape)}\n right: {math.prod(new_shape)}"
         if x.strides == _row_major(x.shape):
             return View(x.storage, x.dtype, new_shape, _row_major(new_shape), x.offset, x.owner)
         out = self.empty(x.dtype, new_shape)
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_reshape_forward(self.ctx, DTYPES[x.dtype], len(x.shape), _i64arr(x.shape),
-                                                       _i64arr(x.strides), vp(x.ptr), vp(out.ptr)))
+        self._check(self._f.reshape_forward(self.ctx, DTYPES[x.dtype], len(x.shape), _i64arr(x.shape), _i64arr(x.strides), x.ptr, out.ptr))
         return out
 
     def reshape_backward(self, x: View, grad_inp: View, grad_out: View):
         """Backward of a copying reshape: grad_inp (laid out like x's storage) += grad_out through x's strides."""
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_reshape_backward(self.ctx, DTYPES[x.dtype], len(x.shape), _i64arr(x.shape),
-                                                        _i64arr(x.strides), vp(grad_inp.ptr), vp(grad_out.ptr)))
+        self._check(self._f.reshape_backward(self.ctx, DTYPES[x.dtype], len(x.shape), _i64arr(x.shape), _i64arr(x.strides),
+                                             grad_inp.ptr, grad_out.ptr))
 
     def attention_supported(self, dtype: str, head_dim: int) -> bool:
         """Whether the fused attention takes this element type and head dimension (else: matmul, softmax, matmul)."""
@@ -625,20 +618,15 @@ class Rocm:
         assert k.shape == q.shape and v.shape == q.shape and k.strides == q.strides and v.strides == q.strides and q.strides[3] == 1
         out = self.empty(q.dtype, (B, S, H * D))
         lse = self.empty("f32", (B, H, S)) if need_backward else None
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_attention_forward(
-            self.ctx, DTYPES[q.dtype], _c(B), _c(H), _c(S), _c(D), vp(q.ptr), vp(k.ptr), vp(v.ptr), _i64arr(q.strides[:3]),
-            ctypes.c_float(scale), vp(out.ptr), _i64arr((S * H * D, D, H * D)), vp(lse.ptr if lse is not None else None)))
+        self._check(self._f.attention_forward(self.ctx, DTYPES[q.dtype], B, H, S, D, q.ptr, k.ptr, v.ptr, _i64s(q.strides[:3]), scale,
+                                              out.ptr, _i64s((S * H * D, D, H * D)), lse.ptr if lse is not None else None))
         return out, lse
 
     def attention_backward(self, q: View, grad_q: View, k: View, grad_k: View, v: View, grad_v: View, scale: float, out: View,
                            grad_out: View, lse: View):
         B, H, S, D = q.shape
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_attention_backward(
-            self.ctx, DTYPES[q.dtype], _c(B), _c(H), _c(S), _c(D), vp(q.ptr), vp(k.ptr), vp(v.ptr), _i64arr(q.strides[:3]),
-            ctypes.c_float(scale), vp(out.ptr), vp(grad_out.ptr), _i64arr((S * H * D, D, H * D)), vp(lse.ptr),
-            vp(grad_q.ptr), vp(grad_k.ptr), vp(grad_v.ptr)))
+        self._check(self._f.attention_backward(self.ctx, DTYPES[q.dtype], B, H, S, D, q.ptr, k.ptr, v.ptr, _i64s(q.strides[:3]), scale,
+                                               out.ptr, grad_out.ptr, _i64s((S * H * D, D, H * D)), lse.ptr, grad_q.ptr, grad_k.ptr, grad_v.ptr))
 
     # ------------------------------------------- ops between an encoder block's GEMMs --
     def layer_norm_forward(self, x: View, gamma: View, beta: View, epsilon: float = 1e-5) -> View:
@@ -646,53 +634,40 @@ class Rocm:
         assert x.strides == _row_major(x.shape), "layer norm input must be contiguous"
         cols = x.shape[-1]
         assert gamma.shape == (cols,) and beta.shape == (cols,), f"left: {gamma.shape}\n right: {(cols,)}"
-        rows = int(np.prod(x.shape[:-1], dtype=np.int64))
-        out = View(self._torch.empty_like(x.storage), x.dtype, x.shape, x.strides)
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_layer_norm_forward(self.ctx, DTYPES[x.dtype], _c(rows), _c(cols), vp(x.ptr), vp(gamma.ptr),
-                                                          vp(beta.ptr), ctypes.c_double(epsilon), vp(out.ptr)))
+        out = View(self._bytes(x.storage.numel()), x.dtype, x.shape, x.strides)
+        self._check(self._f.layer_norm_forward(self.ctx, DTYPES[x.dtype], math.prod(x.shape[:-1]), cols, x.ptr, gamma.ptr, beta.ptr, epsilon, out.ptr))
         return out
 
     def layer_norm_backward(self, x: View, gamma: View, grad_x: View, grad_gamma: View, grad_beta: View, grad_out: View,
                             epsilon: float = 1e-5):
         assert x.strides == _row_major(x.shape) and grad_out.shape == x.shape and grad_x.shape == x.shape
-        cols = x.shape[-1]
-        rows = int(np.prod(x.shape[:-1], dtype=np.int64))
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_layer_norm_backward(self.ctx, DTYPES[x.dtype], _c(rows), _c(cols), vp(x.ptr), vp(gamma.ptr),
-                                                           ctypes.c_double(epsilon), vp(grad_x.ptr), vp(grad_gamma.ptr),
-                                                           vp(grad_beta.ptr), vp(grad_out.ptr)))
+        self._check(self._f.layer_norm_backward(self.ctx, DTYPES[x.dtype], math.prod(x.shape[:-1]), x.shape[-1], x.ptr, gamma.ptr, epsilon,
+                                                grad_x.ptr, grad_gamma.ptr, grad_beta.ptr, grad_out.ptr))
 
     def relu_forward(self, x: View) -> View:
         """``t.relu()`` over the physical storage (relu/cpu_kernel.rs:3-18); same strides."""
-        out = View(self._torch.empty_like(x.storage), x.dtype, x.shape, x.strides, x.offset)
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_relu_forward(self.ctx, DTYPES[x.dtype], _c(x.numel_storage()), vp(x.storage.data_ptr()),
-                                                    vp(out.storage.data_ptr())))
+        out = self._like(x)
+        self._check(self._f.relu_forward(self.ctx, DTYPES[x.dtype], x.numel_storage(), x.storage.data_ptr(), out.storage.data_ptr()))
         return out
 
     def relu_backward(self, x: View, grad_x: View, grad_out: View):
         assert grad_x.numel_storage() == grad_out.numel_storage() == x.numel_storage()
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_relu_backward(self.ctx, DTYPES[x.dtype], _c(x.numel_storage()), vp(x.storage.data_ptr()),
-                                                     vp(grad_x.storage.data_ptr()), vp(grad_out.storage.data_ptr())))
+        self._check(self._f.relu_backward(self.ctx, DTYPES[x.dtype], x.numel_storage(), x.storage.data_ptr(), grad_x.storage.data_ptr(),
+                                          grad_out.storage.data_ptr()))
 
     def add_forward(self, lhs: View, rhs: View) -> View:
         """``lhs + rhs`` for two tensors of one shape and layout (add/cpu_kernel.rs:4-26)."""
         assert lhs.shape == rhs.shape, f"left: {lhs.shape}\n right: {rhs.shape}"
         assert lhs.strides == rhs.strides and lhs.numel_storage() == rhs.numel_storage()
-        out = View(self._torch.empty_like(lhs.storage), lhs.dtype, lhs.shape, lhs.strides, lhs.offset)
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_add_forward(self.ctx, DTYPES[lhs.dtype], _c(lhs.numel_storage()), vp(lhs.storage.data_ptr()),
-                                                   vp(rhs.storage.data_ptr()), vp(out.storage.data_ptr())))
+        out = self._like(lhs)
+        self._check(self._f.add_forward(self.ctx, DTYPES[lhs.dtype], lhs.numel_storage(), lhs.storage.data_ptr(), rhs.storage.data_ptr(),
+                                        out.storage.data_ptr()))
         return out
 
     def add_backward(self, grad_lhs: View, grad_rhs: View, grad_out: View):
         assert grad_lhs.numel_storage() == grad_rhs.numel_storage() == grad_out.numel_storage()
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_add_backward(self.ctx, DTYPES[grad_out.dtype], _c(grad_out.numel_storage()),
-                                                    vp(grad_lhs.storage.data_ptr()), vp(grad_rhs.storage.data_ptr()),
-                                                    vp(grad_out.storage.data_ptr())))
+        self._check(self._f.add_backward(self.ctx, DTYPES[grad_out.dtype], grad_out.numel_storage(), grad_lhs.storage.data_ptr(),
+                                         grad_rhs.storage.data_ptr(), grad_out.storage.data_ptr()))
 
     # ---------------------------------------------------------------- conv2d --
     def _conv2d_op(self, img: View, filters: View, stride, padding, dilation, groups) -> Conv2DOp:
@@ -714,19 +689,11 @@ class Rocm:
         op = self._conv2d_op(img, filters, stride, padding, dilation, groups)
         lead = (op.batch,) if len(img.shape) == 4 else ()
         out = self.empty(img.dtype, lead + (op.chan_out, op.h_out, op.w_out))
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_conv2d_forward(self.ctx, DTYPES[img.dtype], ctypes.byref(op), vp(img.ptr),
-                                                      vp(filters.ptr), vp(out.ptr)))
+        self._check(self._f.conv2d_forward(self.ctx, DTYPES[img.dtype], ctypes.byref(op), img.ptr, filters.ptr, out.ptr))
         return out
 
     def conv2d_backward(self, img: View, grad_img: View, filters: View, grad_filters: View, grad_out: View,
                         stride=1, padding=0, dilation=1, groups=1):
         op = self._conv2d_op(img, filters, stride, padding, dilation, groups)
-        vp = ctypes.c_void_p
-        self._check(self.lib.dfdx_rocm_conv2d_backward(self.ctx, DTYPES[img.dtype], ctypes.byref(op), vp(img.ptr),
-                                                       vp(grad_img.ptr), vp(filters.ptr), vp(grad_filters.ptr),
-                                                       vp(grad_out.ptr)))
-
-
-def _c(v: int):
-    return ctypes.c_int64(int(v))
+        self._check(self._f.conv2d_backward(self.ctx, DTYPES[img.dtype], ctypes.byref(op), img.ptr, grad_img.ptr, filters.ptr,
+                                            grad_filters.ptr, grad_out.ptr))
