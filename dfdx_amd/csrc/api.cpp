@@ -272,6 +272,10 @@ int drop_cache(dfdx_rocm_ctx *ctx) {
 
 struct Plan {
     int kernel, variant, splits;
+    // An LDS-DMA variant on copies of the operands that are off its grid (realign.hip); the plan without copies is kept for
+    // calls that may not have the space for them.
+    bool realign = false;
+    int plain_kernel = 0, plain_variant = 0, plain_splits = 1;
 };
 
 // Rank-1 updates and k = 2 stream their rows on the vector ALUs; from k = 3 on the matrix-core form of the thin
@@ -399,8 +403,32 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
                  is32 ? mfma32_plan_splits(p, v, ctx->compute_units, forced_splits)
                       : is16 ? mfma16_plan_splits(p, v, ctx->compute_units, forced_splits) : 1};
         if (!is32) t_family = is16 ? mfma16_staged_time(p, v, plan->splits, ctx->compute_units) : mfma64_time(p, v, ctx->compute_units);
-        if (may_small && t_small < t_family) *plan = small_plan;
-        if (t_bw < std::min(t_small, t_family)) *plan = bw_plan;
+        Realign ra;
+        const bool realignable = is16 && plan_realign(p, &ra);
+        // The small-product kernel's estimate holds for rows on the 16-byte grid; an operand stored along k whose rows are off it
+        // is gathered value by value (f16, 76 x 6298 x 100, both such: 62 us for an estimate of 13, 13 us in 64 x 64 tiles;
+        // 118 x 2413 x 481, one such: 20 against 13 us).
+        const double t_small_here = realignable && ra.off_grid_k ? 2.5e-6 + (t_small - 2.5e-6) * (1.0 + 1.9 * ra.off_grid_k) : t_small;
+        if (may_small && t_small_here < t_family) *plan = small_plan;
+        if (t_bw < std::min(t_small_here, t_family)) *plan = bw_plan;
+        // Operands off the grid of the LDS-DMA kernels: copies of them and those kernels, where the two together are expected
+        // to be faster.  The register-staged family's estimate ranks its own tiles; against the clock the 64 x 64 tile runs at
+        // 0.6 of it with operands on the 16-byte grid and at 0.9 - 1.6 off it, the larger tiles at about 1 and 1.4 - 3, and those
+        // write a large C at 2.2 TB/s.  f16, staged and on copies: 2048 x 50257 x 1024 563 and 325 us, 4095^3 293 and 143, 1315 x
+        // 2340 x 3033 150 and 52, 530 x 3231 x 1057 84 and 28, 6928 x 106 x 7330 80 and 43; and where the line leaves the
+        // staged kernels: 1000^3 12.0 and 18.8, 304 x 611 x 4120 11.0 and 16.4, 448 x 315 x 4890 13.2 and 14.5.
+        if (realignable) {
+            int dv = 0, splits = 1;
+            double t_dma = 1e300;
+            mfma16dma_plan_split(ra.problem, ctx->compute_units, 0, forced_splits, &dv, &splits, &t_dma);
+            const bool small_tile = v == mfma16_skinny_variant();
+            const double t_staged = t_family * (small_tile ? (ra.off_grid ? 1.0 : 0.6) : ra.off_grid ? 1.4 : 0.95) +
+                                    (small_tile ? 0.0 : 2.0 * (double)p.m * (double)p.n * (double)(p.reduce ? 1 : p.nb1 * p.nb2) / 2.2e12);
+            if (dv && t_dma + ra.seconds < std::min(std::min(t_small_here, t_staged), t_bw)) {
+                const Plan plain = *plan;
+                *plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits, true, plain.kernel, plain.variant, plain.splits};
+            }
+        }
         return DFDX_ROCM_OK;
     }
     if (bw) {  // no tiled kernel takes these strides, the multi-vector kernel does
@@ -430,8 +458,15 @@ int partials_buffer(dfdx_rocm_ctx *ctx, size_t need, bool static_scratch, float 
     return DFDX_ROCM_OK;
 }
 
-// The f32 partial sums `plan` needs for `p`, in bytes (0: none).
-size_t partials_bytes(const GemmProblem &p, const Plan &plan) {
+// The f32 partial sums `plan` needs for `p`, in bytes (0: none), and, behind them, the copies of its operands.
+size_t partials_bytes(const GemmProblem &p, const Plan &plan, Realign *ra = nullptr) {
+    if (plan.realign) {
+        Realign here;
+        if (!ra) ra = &here;
+        if (!plan_realign(p, ra)) return 0;
+        return ((mfma16dma_workspace_bytes(ra->problem, plan.variant - mfma16_dma_first_variant() + 1, plan.splits) + 255) & ~(size_t)255) +
+               ra->a_bytes + ra->b_bytes;
+    }
     if (plan.kernel == DFDX_ROCM_KERNEL_MFMA && plan.splits > 1)
         return p.dtype == DT_F32 ? mfma32_workspace_bytes(p, plan.variant, plan.splits)
                : plan.variant < mfma16_dma_first_variant()
@@ -444,10 +479,25 @@ size_t partials_bytes(const GemmProblem &p, const Plan &plan) {
 
 // Makes sure the partial sums of `plan` have a place, BEFORE the caller resolves pending zero fills among the operands:
 // a call that is refused here (scratch too small, out of memory) must leave every declaration as it found it.
-int reserve_partials(dfdx_rocm_ctx *ctx, const GemmProblem &problem, const Plan &plan, bool static_scratch) {
+// Copies of operands are left out, and the plan changed to the one without them, where they cannot have their space: under
+// a fixed scratch array, when memory has run out, and while the stream is being captured into a graph, where nothing is
+// allocated that the call could do without.
+int reserve_partials(dfdx_rocm_ctx *ctx, const GemmProblem &problem, Plan &plan, bool static_scratch) {
     GemmProblem p = problem;
     p.compute_units = ctx->compute_units;
     float *unused = nullptr;
+    if (plan.realign) {
+        CtxLock lock(ctx->mu);
+        const size_t need = partials_bytes(p, plan);
+        bool room = !static_scratch;
+        if (room && need > ctx->workspace_bytes) {
+            hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess) (void)hipGetLastError();
+            room = capturing == hipStreamCaptureStatusNone && ensure_workspace(ctx, need) == DFDX_ROCM_OK;
+        }
+        if (room) return DFDX_ROCM_OK;
+        plan = {plan.plain_kernel, plan.plain_variant, plan.plain_splits};
+    }
     const size_t need = partials_bytes(p, plan);
     return need ? partials_buffer(ctx, need, static_scratch, &unused) : DFDX_ROCM_OK;
 }
@@ -458,9 +508,15 @@ int run_plan(dfdx_rocm_ctx *ctx, const GemmProblem &problem, const Plan &plan, b
     p.splits = 1;
     p.workspace = nullptr;
     p.compute_units = ctx->compute_units;
-    if (const size_t need = partials_bytes(p, plan)) {
+    Realign ra;
+    if (const size_t need = partials_bytes(p, plan, &ra)) {
         if (int rc = partials_buffer(ctx, need, static_scratch, &p.workspace)) return rc;
+        if (plan.realign) {
+            ra.problem.workspace = p.workspace;
+            HIP_TRY(launch_realign(p, &ra, (char *)p.workspace + (need - ra.a_bytes - ra.b_bytes), ctx->stream));
+        }
     }
+    if (plan.realign) p = ra.problem;
     if (plan.kernel == DFDX_ROCM_KERNEL_MFMA && plan.splits > 1) p.splits = plan.splits;
     hipError_t e;
     switch (plan.kernel) {
@@ -505,6 +561,7 @@ namespace {
 // Which plans apply p.extra on the way into C.
 bool extra_supported(const GemmProblem &p, const Plan &plan) {
     if (p.extra == EXTRA_NONE) return true;
+    if (plan.realign) return false;
     if (plan.kernel != DFDX_ROCM_KERNEL_MFMA || p.nb1 * p.nb2 != 1) return false;
     const bool is16 = p.dtype == DT_F16 || p.dtype == DT_BF16;
     if (is16 && plan.variant == mfma16_small_variant()) return true;
@@ -558,7 +615,7 @@ int gemm_with_colsum(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, void *
     if (int e = make_plan(ctx, desc, p, &plan)) return e;
     if (int e = reserve_partials(ctx, p, plan, false)) return e;
     if (int e = settle_operands(ctx, &p, /*may_overwrite=*/true)) return e;
-    bool can = p.ksum && plan.kernel == DFDX_ROCM_KERNEL_MFMA;
+    bool can = p.ksum && plan.kernel == DFDX_ROCM_KERNEL_MFMA && !plan.realign;
     if (can && (p.dtype == DT_F16 || p.dtype == DT_BF16))
         can = plan.variant == mfma16_small_variant()
                   ? small_ksum_supported(p)
@@ -887,13 +944,13 @@ int dfdx_rocm_gemm_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int
     if (variant) *variant = plan.kernel == DFDX_ROCM_KERNEL_GEMV ? 0 : plan.variant;  // (a tile variant; the bandwidth kernels have none)
     if (name && name_len) {
         if (plan.kernel == DFDX_ROCM_KERNEL_MFMA && plan.splits > 1)
-            std::snprintf(name, name_len, "%s_%s_splitk%d", p.dtype == DT_F32 ? "mfma32" : "mfma16",
-                          p.dtype == DT_F32 ? mfma32_variant_name(plan.variant) : mfma16_variant_name(plan.variant), plan.splits);
+            std::snprintf(name, name_len, "%s_%s%s_splitk%d", p.dtype == DT_F32 ? "mfma32" : "mfma16",
+                          p.dtype == DT_F32 ? mfma32_variant_name(plan.variant) : mfma16_variant_name(plan.variant), plan.realign ? "_realigned" : "", plan.splits);
         else if (plan.kernel == DFDX_ROCM_KERNEL_MFMA && p.dtype == DT_F64)
             std::snprintf(name, name_len, "mfma64_%s", mfma64_variant_name(plan.variant));
         else if (plan.kernel == DFDX_ROCM_KERNEL_MFMA)
-            std::snprintf(name, name_len, "%s_%s", p.dtype == DT_F32 ? "mfma32" : "mfma16",
-                          p.dtype == DT_F32 ? mfma32_variant_name(plan.variant) : mfma16_variant_name(plan.variant));
+            std::snprintf(name, name_len, "%s_%s%s", p.dtype == DT_F32 ? "mfma32" : "mfma16",
+                          p.dtype == DT_F32 ? mfma32_variant_name(plan.variant) : mfma16_variant_name(plan.variant), plan.realign ? "_realigned" : "");
         else
             std::snprintf(name, name_len, "%s", plan.kernel != DFDX_ROCM_KERNEL_GEMV ? "generic" : bandwidth_kernel_name(p, plan.variant));
     }
@@ -920,6 +977,7 @@ int dfdx_rocm_gemm_time_rotating(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *
             return DFDX_ROCM_OK;
         }
         if (int e = make_plan(ctx, &descs[i], problems[(size_t)i], &plans[(size_t)i])) return e;
+        if (int e = reserve_partials(ctx, problems[(size_t)i], plans[(size_t)i], false)) return e;
         if (int e = settle_operands(ctx, &problems[(size_t)i], /*may_overwrite=*/false)) return e;
     }
     for (int i = 0; i < warmup; i++)

@@ -27,7 +27,9 @@ __global__ __launch_bounds__(256) void bias_forward_kernel(const T *x, const T *
 // a row when N is a 16-byte vector), the other 256 / LPR lane groups walk the rows of the slice; their partial
 // sums meet in LDS and are added in a fixed order.  With several row slices the strip sums go to an f32 workspace
 // [slices][cols] and a second kernel adds them, again in a fixed order, so the result does not depend on timing.
-template <typename T, int N, int LPR>
+// ANY: rows off the 16-byte grid, read as element-aligned vectors, the columns behind the last whole one by themselves
+// (2048 x 50257 f16: 74 us one column per lane, 56 so).
+template <typename T, int N, int LPR, bool ANY = false>
 __global__ __launch_bounds__(256) void bias_backward_kernel(const T *go, int rows, int cols, int rows_per_slice,
                                                             float *partial, T *grad_bias, bool fresh) {
     constexpr int RL = 256 / LPR;  // row lanes
@@ -38,21 +40,33 @@ __global__ __launch_bounds__(256) void bias_backward_kernel(const T *go, int row
     float acc[N];
 #pragma unroll
     for (int i = 0; i < N; i++) acc[i] = 0.0f;
+    auto load = [&](const T *p, float (&v)[N]) {
+        if constexpr (ANY) {
+            if (col + N <= cols) {
+                load_elems_unaligned<T, N>(p, v);
+            } else {
+#pragma unroll
+                for (int i = 0; i < N; i++) v[i] = col + i < cols ? Elem<T>::load(p + i) : 0.0f;
+            }
+        } else {
+            load_elems<T, N>(p, v);
+        }
+    };
     if (col < cols) {
         const T *src = go + (int64_t)col;
         int r = r0 + r_lane;
         for (; r + 3 * RL < r1; r += 4 * RL) {  // four independent loads in flight
             float v0[N], v1[N], v2[N], v3[N];
-            load_elems<T, N>(src + (int64_t)r * cols, v0);
-            load_elems<T, N>(src + (int64_t)(r + RL) * cols, v1);
-            load_elems<T, N>(src + (int64_t)(r + 2 * RL) * cols, v2);
-            load_elems<T, N>(src + (int64_t)(r + 3 * RL) * cols, v3);
+            load(src + (int64_t)r * cols, v0);
+            load(src + (int64_t)(r + RL) * cols, v1);
+            load(src + (int64_t)(r + 2 * RL) * cols, v2);
+            load(src + (int64_t)(r + 3 * RL) * cols, v3);
 #pragma unroll
             for (int i = 0; i < N; i++) acc[i] += (v0[i] + v1[i]) + (v2[i] + v3[i]);
         }
         for (; r < r1; r += RL) {
             float v[N];
-            load_elems<T, N>(src + (int64_t)r * cols, v);
+            load(src + (int64_t)r * cols, v);
 #pragma unroll
             for (int i = 0; i < N; i++) acc[i] += v[i];
         }
@@ -124,11 +138,13 @@ int bias_backward_t(dfdx_rocm_ctx *ctx, int64_t rows, int64_t cols, const void *
     constexpr int V = Elem<T>::VEC;
     const bool vec = cols % V == 0 && aligned16(go);
     constexpr int LPR_VEC = 16, LPR_SCALAR = 64;
-    const int strip = vec ? LPR_VEC * V : LPR_SCALAR;
-    const int row_lanes = 256 / (vec ? LPR_VEC : LPR_SCALAR);
+    const bool any = !vec && sizeof(T) == 2 && cols >= LPR_VEC * V;  // (fewer columns leave most of a strip's lanes idle)
+    const int strip = vec || any ? LPR_VEC * V : LPR_SCALAR;
+    const int row_lanes = 256 / (vec || any ? LPR_VEC : LPR_SCALAR);
     const int64_t strips = (cols + strip - 1) / strip;
     // two workgroups per compute unit, but at least 8 rows per lane group and slice
-    int64_t slices = std::max<int64_t>(1, (int64_t)ctx->compute_units * 2 / strips);
+    // (eight where every load straddles two lines)
+    int64_t slices = std::max<int64_t>(1, (int64_t)ctx->compute_units * (any ? 8 : 2) / strips);
     slices = std::min<int64_t>(slices, std::max<int64_t>(1, rows / (8 * row_lanes)));
     slices = std::min<int64_t>(slices, 65535);
     const int64_t rows_per_slice = (rows + slices - 1) / slices;
@@ -142,6 +158,8 @@ int bias_backward_t(dfdx_rocm_ctx *ctx, int64_t rows, int64_t cols, const void *
     dim3 grid((unsigned)strips, (unsigned)slices);
     if (vec)
         bias_backward_kernel<T, V, LPR_VEC><<<grid, 256, 0, ctx->stream>>>((const T *)go, (int)rows, (int)cols, (int)rows_per_slice, partial, (T *)gb, fresh);
+    else if (any)
+        bias_backward_kernel<T, V, LPR_VEC, true><<<grid, 256, 0, ctx->stream>>>((const T *)go, (int)rows, (int)cols, (int)rows_per_slice, partial, (T *)gb, fresh);
     else
         bias_backward_kernel<T, 1, LPR_SCALAR><<<grid, 256, 0, ctx->stream>>>((const T *)go, (int)rows, (int)cols, (int)rows_per_slice, partial, (T *)gb, fresh);
     HIP_TRY(hipGetLastError());

@@ -41,6 +41,9 @@ struct GemmProblem {
     int ksum_accumulate = 0;
     int extra = EXTRA_NONE;        // see above; kernels that have it: extra_supported in api.cpp
     const void *with = nullptr;
+    // Operands laid out by launch_realign: an operand whose rows lie along memory is readable up to the next multiple of eight
+    // of them, and C may lie anywhere.
+    bool ragged = false;
     // split-k (filled in by the planner): `splits` workgroups share one C tile; f32 partials go to `workspace`
     int splits;
     float *workspace;
@@ -101,6 +104,7 @@ int mfma16_plan_splits(const GemmProblem &p, int variant, int compute_units, int
 size_t mfma16_workspace_bytes(const GemmProblem &p, int variant, int splits);
 double mfma16_staged_time(const GemmProblem &p, int variant, int splits, int compute_units);  // estimated seconds
 // a few rows or columns against a large matrix: the 64 x 64 register-staged tile with split-k (0 = does not apply)
+int mfma16_skinny_variant();  // that tile
 int mfma16_skinny_plan(const GemmProblem &p, int compute_units, int forced_splits, int *splits, double *seconds);
 hipError_t launch_mfma16(const GemmProblem &p, int variant, hipStream_t stream);
 // The same product with B given as a patch matrix (`p.b` = channel 0 of the first image, b_b1 / b_b2 = image and group
@@ -118,6 +122,17 @@ hipError_t launch_mfma16dma(const GemmProblem &p, int variant, hipStream_t strea
 struct DmaParams;
 bool mfma16dma_extra_supported(const GemmProblem &p, int variant, int splits);  // can this plan apply p.extra on the way into C?
 hipError_t launch_mfma16dma_extra(int variant, int dtype, int extra, const DmaParams &p, int compute_units, hipStream_t stream);  // gemm_mfma16_dma_extra.hip
+hipError_t launch_mfma16dma_ragged(int variant, int dtype, const DmaParams &p, int compute_units, bool a_kc, bool b_kc, hipStream_t stream);  // gemm_mfma16_dma_ragged.hip
+// ---- operands of the 16-bit types laid out for those kernels (realign.hip) ----
+struct Realign {
+    bool a, b;                 // which operands are copied
+    GemmProblem problem;       // what the kernels are given (operand addresses: see realign_into)
+    size_t a_bytes, b_bytes;   // space for the copies, multiples of 256
+    double seconds;            // estimated time of the copies
+    int off_grid, off_grid_k;  // operands whose rows are off the 16-byte grid; those of them that are stored along k
+};
+bool plan_realign(const GemmProblem &p, Realign *r);  // false where a copy does not help (strides, sizes)
+hipError_t launch_realign(const GemmProblem &p, Realign *r, void *space, hipStream_t stream);  // copies and fills in the addresses
 // Split-k planning for the LDS-DMA kernels: picks tile variant and split count together.  `forced_splits`
 // > 0 overrides the count (clamped to what the k extent allows).  `seconds` (may be null) receives the estimate.
 void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_variant, int forced_splits, int *variant,

@@ -677,13 +677,16 @@ double mfma16_staged_time(const GemmProblem &p, int variant, int splits, int com
     return 2.5e-6 + std::max(1.0, blocks / cus) * (double)((total_iters + splits - 1) / splits) * step + (splits > 1 ? 4e-6 : 0.0);
 }
 
+constexpr int kSkinnyVariant = 6;  // 64x64x64_w2x2
+int mfma16_skinny_variant() { return kSkinnyVariant; }
+
 // A few rows (or columns) against a large matrix, streamed by the 64 x 64 tile with the contraction split: the tile wastes
 // the least of its rows on such a product and its small LDS footprint puts several workgroups on a compute unit, which
 // is what streaming at the rate of HBM takes (16 x 8192 x 8192 A.B^T: 26.7 us where the 128-row LDS-DMA tiles take 30.6
 // and the k-sliced small kernel 33.5; 8 x 4096 x 4096 A.B: 13.7 us against 15.8).  Returns the variant and its split
 // count with an estimate in seconds, or 0 where the candidate does not apply.
 int mfma16_skinny_plan(const GemmProblem &p, int compute_units, int forced_splits, int *splits, double *seconds) {
-    constexpr int V = 6;  // 64x64x64_w2x2
+    constexpr int V = kSkinnyVariant;
     static_assert(kNumVariants >= V, "variant table");
     *splits = 1;
     *seconds = 1e300;

@@ -59,6 +59,22 @@ typedef DmaParams Params;
 // cached form is up to 6 % faster (256 x (512 x 64 x 512): 29.1 vs 30.9 us) -- a state no training step is in.
 __device__ __forceinline__ void stream16(void *p, u32x4 v) { __builtin_nontemporal_store(v, (u32x4 *)p); }
 
+// 16 bytes of C at any element (ANY) or on the 16-byte grid.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+typedef u32x2 u32x2_any __attribute__((aligned(2)));
+template <bool ANY> __device__ __forceinline__ u32x4 load16(const void *p) {
+    if constexpr (ANY) return *(const u32x4_any *)p;
+    else return *(const u32x4 *)p;
+}
+template <bool ANY> __device__ __forceinline__ void store16(void *p, u32x4 v) {
+    if constexpr (ANY) *(u32x4_any *)p = v;
+    else *(u32x4 *)p = v;
+}
+template <bool ANY> __device__ __forceinline__ void stream16_at(void *p, u32x4 v) {
+    if constexpr (ANY) *(u32x4_any *)p = v;
+    else stream16(p, v);
+}
+
 template <typename T> struct Mma;
 template <> struct Mma<_Float16> {
     static __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
@@ -156,6 +172,10 @@ constexpr int dma_waves_per_simd(int bm, int bn, int waves) {
 // fragment registers against a load of that form it cannot prove complete, with a wait for ALL memory traffic in the
 // middle of the k loop -- where every wave then stalls on the tile prefetched for the step after.
 //
+// EDGE = 2 is the edge form for a C off the 16-byte grid (odd extents or leading dimensions, any address): the same pieces of
+// eight columns as element-aligned accesses, which global memory allows at the cost of the lines they straddle, and the
+// last columns of a row one by one.  These stores take the cached form, so that the two writers of a straddled line meet in L2.
+//
 // EXTRA: what is done with a finished value besides bias and beta (EXTRA_* in gemm_internal.h): what the op behind a Linear layer, or in front of its backward, would otherwise read and write C once more for.
 //
 // KSUM = true (A stored [k][m] only, split-k only) adds a second result: the sums of A's rows over the contraction --
@@ -165,7 +185,7 @@ constexpr int dma_waves_per_simd(int bm, int bn, int waves) {
 // 64 * BM / 8 pieces; the workgroups of a tile row all hold the same A tiles, so tile column q < BM / 64 takes the q-th
 // 512 pieces and the others none.  At the end of a work item lanes that hold the same 8 columns are added up and each
 // wave leaves its sums in a workspace slot of its own; the split-k reduce kernel adds the slots.
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, bool EDGE, bool KSUM = false, int EXTRA = EXTRA_NONE>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, bool A_KC, bool B_KC, int EDGE, bool KSUM = false, int EXTRA = EXTRA_NONE>
 __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, WAVES_M *WAVES_N)) void gemm_mfma16_dma_kernel(const Params p) {
     constexpr int NW = WAVES_M * WAVES_N;
     constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
@@ -241,8 +261,9 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
         // are recomputed here instead of being carried through the k loop
         int f_wave = wave, f_lane = lane;
         asm volatile("" : "+v"(f_wave), "+v"(f_lane));
-        ta.init(p.lda, p.m - fw.bm0, f_wave, f_lane);
-        tb.init(p.ldb, p.n - fw.bn0, f_wave, f_lane);
+        // (rows that lie along memory are read in whole pieces: the stored rows go on to the next multiple of eight)
+        ta.init(p.lda, (A_KC ? p.m : (p.m + 7) & ~7) - fw.bm0, f_wave, f_lane);
+        tb.init(p.ldb, (B_KC ? p.n : (p.n + 7) & ~7) - fw.bn0, f_wave, f_lane);
     };
     begin_fetch();
     bool fetching = true;
@@ -552,6 +573,15 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
         return ST_SPLIT;
     }
     if constexpr (!KSUM) {
+    constexpr bool ANY = EDGE == 2;
+    static_assert(!ANY || (EXTRA == EXTRA_NONE && TN % 2 == 0), "see launch_mfma16dma_ragged");
+    [[maybe_unused]] auto columns_left = [](const uint16_t *q, int left) -> u32x4 {  // up to seven values, zeros behind them
+        u32x4 r = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int e = 0; e < 7; e++)
+            if (e < left) r[e / 2] |= (uint32_t)q[e] << (e % 2 * 16);
+        return r;
+    };
     const int cb = p.kbatches > 1 ? 0 : batch;
     uint16_t *cbase = p.c + (int64_t)(cb / p.nb2) * p.c_b1 + (int64_t)(cb % p.nb2) * p.c_b2;
     // two finished values (rounded, packed) and their partners; see EXTRA_*
@@ -577,8 +607,15 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
                 float rbias_all[TM];
                 if (p.bias_mode == BIAS_PER_COL) {
 #pragma unroll
-                    for (int jp = 0; jp < TN / 2; jp++)
-                        cbias[jp] = *(const u32x4 *)(p.bias + min(bn0 + wn0 + (PERM ? jp * 32 + lq * 8 : (2 * jp + (lq & 1)) * 16 + (lq >> 1) * 8), p.n - 8));
+                    for (int jp = 0; jp < TN / 2; jp++) {
+                        const int gn = bn0 + wn0 + (PERM ? jp * 32 + lq * 8 : (2 * jp + (lq & 1)) * 16 + (lq >> 1) * 8);
+                        if constexpr (ANY) {
+                            if (gn + 8 <= p.n) cbias[jp] = load16<true>(p.bias + gn);
+                            else cbias[jp] = columns_left(p.bias + gn, p.n - gn);
+                        } else {
+                            cbias[jp] = *(const u32x4 *)(p.bias + min(gn, p.n - 8));
+                        }
+                    }
                 }
                 if (p.bias_mode == BIAS_PER_ROW) {
 #pragma unroll
@@ -605,7 +642,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
                             }
                         }
                         const int gn = bn0 + wn0 + (PERM ? jp * 32 + lq * 8 : (2 * jp + (lq & 1)) * 16 + (lq >> 1) * 8);
-                        if (!row_ok || gn >= p.n) continue;  // n % 8 == 0 here: all 8 columns are in range
+                        if (!row_ok || gn >= p.n) continue;  // (n % 8 == 0 unless ANY: all 8 columns are in range)
+                        const bool whole = !ANY || gn + 8 <= p.n;
                         if (p.bias_mode == BIAS_PER_ROW) {
 #pragma unroll
                             for (int e = 0; e < 8; e++) v[e] += rbias_all[i];
@@ -619,7 +657,9 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
                             }
                         }
                         if (p.accumulate) {
-                            const u32x4 old = *(const u32x4 *)(EXTRA == EXTRA_FROM ? p.with + (crow + gn - p.c) : crow + gn);
+                            u32x4 old;
+                            if (whole) old = load16<ANY>(EXTRA == EXTRA_FROM ? p.with + (crow + gn - p.c) : crow + gn);
+                            else old = columns_left(crow + gn, p.n - gn);
 #pragma unroll
                             for (int e = 0; e < 4; e++) {
                                 v[2 * e] += Mma<T>::to_f32((uint16_t)(old[e] & 0xffffu));
@@ -629,13 +669,19 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
                         u32x4 o;
 #pragma unroll
                         for (int e = 0; e < 4; e++) o[e] = Mma<T>::pack2(v[2 * e], v[2 * e + 1]);
-                        if constexpr (EXTRA != EXTRA_NONE && EXTRA != EXTRA_FROM) {
+                        if constexpr (EXTRA != EXTRA_NONE && EXTRA != EXTRA_FROM) {  // (never together with ANY)
                             u32x4 w = {0u, 0u, 0u, 0u};
                             if constexpr (EXTRA != EXTRA_RELU) w = *(const u32x4 *)(p.with + (crow + gn - p.c));
 #pragma unroll
                             for (int e = 0; e < 4; e++) o[e] = extra(o[e], w[e]);
                         }
-                        *(u32x4 *)(crow + gn) = o;
+                        if (whole) {
+                            store16<ANY>(crow + gn, o);
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 7; e++)
+                                if (gn + e < p.n) crow[gn + e] = (uint16_t)(o[e / 2] >> (e % 2 * 16));
+                        }
                     }
                 }
             };
@@ -667,7 +713,10 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
                 if constexpr (BIAS) {
 #pragma unroll
                     for (int j = 0; j < TN; j++) {
-                        const u32x2 bv = *(const u32x2 *)(p.bias + bn0 + wn0 + (PERM ? (j / 2) * 32 + lq * 8 + (j % 2) * 4 : j * 16 + lq * 4));
+                        u32x2 bv;
+                        const uint16_t *const bias_at = p.bias + bn0 + wn0 + (PERM ? (j / 2) * 32 + lq * 8 + (j % 2) * 4 : j * 16 + lq * 4);
+                        if constexpr (ANY) bv = *(const u32x2_any *)bias_at;
+                        else bv = *(const u32x2 *)bias_at;
                         cb[j][0] = Mma<T>::to_f32((uint16_t)(bv[0] & 0xffffu));
                         cb[j][1] = Mma<T>::to_f32((uint16_t)(bv[0] >> 16));
                         cb[j][2] = Mma<T>::to_f32((uint16_t)(bv[1] & 0xffffu));
@@ -730,8 +779,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
                                 hi[e] = extra(hi[e], with[WITH ? i % IG : 0][1][e]);
                             }
                         }
-                        stream16(tile_base + i * row_step + line_off, lo);
-                        stream16(tile_base + i * row_step + half_step + line_off, hi);
+                        stream16_at<ANY>(tile_base + i * row_step + line_off, lo);
+                        stream16_at<ANY>(tile_base + i * row_step + half_step + line_off, hi);
                     } else {
 #pragma unroll
                         for (int jp = 0; jp < TN / 2; jp++) {
@@ -739,7 +788,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
 #pragma unroll
                                 for (int e = 0; e < 4; e++) o[jp][e] = extra(o[jp][e], with[WITH ? i % IG : 0][jp][e]);
                             }
-                            stream16(tile_base + i * row_step + jp * 64 + lane_off, o[jp]);
+                            stream16_at<ANY>(tile_base + i * row_step + jp * 64 + lane_off, o[jp]);
                         }
                     }
                 }
@@ -759,8 +808,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
                     for (int i = 0; i < IG; i++)
 #pragma unroll
                         for (int jp = 0; jp < TN / 2; jp++) {
-                            if constexpr (TN == 4) old[i][jp] = *(const u32x4 *)(old_base + (i0 + i) * row_step + jp * half_step + line_off);
-                            else old[i][jp] = *(const u32x4 *)(old_base + (i0 + i) * row_step + jp * 64 + lane_off);
+                            if constexpr (TN == 4) old[i][jp] = load16<ANY>(old_base + (i0 + i) * row_step + jp * half_step + line_off);
+                            else old[i][jp] = load16<ANY>(old_base + (i0 + i) * row_step + jp * 64 + lane_off);
                         }
 #pragma unroll
                     for (int i = 0; i < IG; i++) {
@@ -794,8 +843,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
                             for (int e = 0; e < 4; e++)
                                 o[e] = Mma<T>::pack2(v[jp][2 * e] + Mma<T>::to_f32((uint16_t)(old[i][jp][e] & 0xffffu)),
                                                      v[jp][2 * e + 1] + Mma<T>::to_f32((uint16_t)(old[i][jp][e] >> 16)));
-                            if constexpr (TN == 4) *(u32x4 *)(base + (i0 + i) * row_step + jp * half_step + line_off) = o;
-                            else *(u32x4 *)(base + (i0 + i) * row_step + jp * 64 + lane_off) = o;
+                            if constexpr (TN == 4) store16<ANY>(base + (i0 + i) * row_step + jp * half_step + line_off, o);
+                            else store16<ANY>(base + (i0 + i) * row_step + jp * 64 + lane_off, o);
                         }
                     }
                 }

@@ -80,14 +80,27 @@ struct OperandLayout {
     bool ok, kc;
     int64_t ld;
 };
-inline OperandLayout classify(int64_t rows, int64_t kdim, int64_t row_stride, int64_t k_stride) {
+// `ragged`: rows that lie along memory may end off the grid of eight (GemmProblem::ragged: what follows them is readable)
+inline OperandLayout classify(int64_t rows, int64_t kdim, int64_t row_stride, int64_t k_stride, bool ragged = false) {
     OperandLayout r{false, false, 0};
-    if (k_stride == 1 && kdim % 8 == 0 && (rows == 1 || (row_stride % 8 == 0 && row_stride >= kdim))) {
+    if (ragged && row_stride == 1 && k_stride % 8 == 0 && k_stride >= ((rows + 7) & ~(int64_t)7)) {
+        r.ok = true; r.kc = false; r.ld = k_stride;
+    } else if (k_stride == 1 && kdim % 8 == 0 && (rows == 1 || (row_stride % 8 == 0 && row_stride >= kdim))) {
         r.ok = true; r.kc = true; r.ld = rows == 1 ? kdim : row_stride;
     } else if (row_stride == 1 && rows % 8 == 0 && (kdim == 1 || (k_stride % 8 == 0 && k_stride >= rows))) {
         r.ok = true; r.kc = false; r.ld = kdim == 1 ? rows : k_stride;
     }
     return r;
+}
+
+// The epilogue stores whole 16 B (8 B for the 16-column wave tile) pieces of C rows and nothing narrower; the instances for
+// everything else are in gemm_mfma16_dma_ragged.hip.
+inline bool c_on_grid(const GemmProblem &p, const Variant &v) {
+    const int vecw = (v.bn / v.waves_n) % 32 == 0 ? 8 : 4;
+    const int64_t ldc = p.m == 1 ? p.n : p.c_rs;
+    const uintptr_t mask = (uintptr_t)vecw * 2 - 1;
+    if (p.n % vecw || ldc % vecw || ((uintptr_t)p.c & mask) || p.c_b1 % vecw || p.c_b2 % vecw) return false;
+    return !p.bias || !((uintptr_t)p.bias & mask);
 }
 
 }  // namespace
@@ -102,19 +115,13 @@ bool mfma16dma_supported(const GemmProblem &p, int variant) {
     if (p.m > (1 << 30) || p.n > (1 << 30) || p.k > (1 << 30)) return false;
     if (p.c_cs != 1 && p.n != 1) return false;
     if (p.n > 1 && p.m > 1 && p.c_rs < p.n) return false;
-    const OperandLayout la = classify(p.m, p.k, p.a_rs, p.a_cs);
-    const OperandLayout lb = classify(p.n, p.k, p.b_cs, p.b_rs);
+    const OperandLayout la = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged);
+    const OperandLayout lb = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged);
     if (!la.ok || !lb.ok) return false;
     const Variant &v = kVariants[variant - 1];
     if (la.ld * (la.kc ? v.bm : BK) >= (1ll << 30) || lb.ld * (lb.kc ? v.bn : BK) >= (1ll << 30)) return false;
     if (!aligned16(p.a) || !aligned16(p.b)) return false;
-    {   // the epilogue stores whole 16 B (8 B for the 16-column wave tile) pieces of C rows and nothing narrower
-        const int vecw = (v.bn / v.waves_n) % 32 == 0 ? 8 : 4;
-        const int64_t ldc = p.m == 1 ? p.n : p.c_rs;
-        const uintptr_t mask = (uintptr_t)vecw * 2 - 1;
-        if (p.n % vecw || ldc % vecw || ((uintptr_t)p.c & mask) || p.c_b1 % vecw || p.c_b2 % vecw) return false;
-        if (p.bias && ((uintptr_t)p.bias & mask)) return false;
-    }
+    if (!c_on_grid(p, v) && !(p.ragged && (v.bn / v.waves_n) % 32 == 0)) return false;
     if (p.nb1 * p.nb2 > 1) {
         if (p.a_b1 % 8 || p.a_b2 % 8 || p.b_b1 % 8 || p.b_b2 % 8) return false;
         if (p.a_b1 < 0 || p.a_b2 < 0 || p.b_b1 < 0 || p.b_b2 < 0) return false;
@@ -179,7 +186,7 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
     const int64_t nbatch = p.reduce ? 1 : p.nb1 * p.nb2;
     const bool may_split = nbatch == 1 && p.c_cs == 1;
     const int64_t total_iters = (p.k / BK) * (p.reduce ? p.nb1 * p.nb2 : 1);
-    const bool a_kc = classify(p.m, p.k, p.a_rs, p.a_cs).kc, b_kc = classify(p.n, p.k, p.b_cs, p.b_rs).kc;
+    const bool a_kc = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged).kc, b_kc = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged).kc;
     const double elem = 2.0, out_elems = (double)p.m * p.n * nbatch;
     double best = 1e300;
     for (int v = 1; v <= kNumVariants; v++) {
@@ -253,22 +260,22 @@ bool mfma16dma_ksum_supported(const GemmProblem &p, int variant, int splits) {
     if ((uintptr_t)p.ksum & 1u) return false;
     const Variant &v = kVariants[variant - 1];
     if ((p.n + v.bn - 1) / v.bn < v.bm / 64) return false;  // too few tile columns to share a tile's pieces
-    return !classify(p.m, p.k, p.a_rs, p.a_cs).kc && !classify(p.n, p.k, p.b_cs, p.b_rs).kc;
+    return !classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged).kc && !classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged).kc;
 }
 
 bool mfma16dma_extra_supported(const GemmProblem &p, int variant, int splits) {
     if ((p.accumulate != 0) != (p.extra == EXTRA_FROM) || p.nb1 * p.nb2 != 1 || !mfma16dma_supported(p, variant)) return false;
     if (p.extra != EXTRA_RELU && (!p.with || !aligned16(p.with))) return false;
     if (splits > 1) return true;  // the reduce kernel applies it
-    const bool a_kc = classify(p.m, p.k, p.a_rs, p.a_cs).kc, b_kc = classify(p.n, p.k, p.b_cs, p.b_rs).kc;
+    const bool a_kc = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged).kc, b_kc = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged).kc;
     return a_kc && b_kc == (p.extra == EXTRA_RELU || p.extra == EXTRA_RESIDUAL);
 }
 
 hipError_t launch_mfma16dma(const GemmProblem &g, int variant, hipStream_t stream) {
     if (!mfma16dma_supported(g, variant)) return hipErrorInvalidValue;
     const Variant &v = kVariants[variant - 1];
-    const OperandLayout la = classify(g.m, g.k, g.a_rs, g.a_cs);
-    const OperandLayout lb = classify(g.n, g.k, g.b_cs, g.b_rs);
+    const OperandLayout la = classify(g.m, g.k, g.a_rs, g.a_cs, g.ragged);
+    const OperandLayout lb = classify(g.n, g.k, g.b_cs, g.b_rs, g.ragged);
     Params p;
     p.a = (const uint16_t *)g.a; p.b = (const uint16_t *)g.b; p.c = (uint16_t *)g.c; p.bias = (const uint16_t *)g.bias;
     p.m = (int)g.m; p.n = (int)g.n; p.k = (int)g.k;
@@ -306,6 +313,7 @@ hipError_t launch_mfma16dma(const GemmProblem &g, int variant, hipStream_t strea
     p.with = (const uint16_t *)g.with;
     if (g.extra != EXTRA_NONE && !mfma16dma_extra_supported(g, variant, g.splits)) return hipErrorInvalidValue;
     if (g.extra != EXTRA_NONE && g.splits <= 1) return launch_mfma16dma_extra(variant, g.dtype, g.extra, p, g.compute_units, stream);
+    if (g.splits <= 1 && !c_on_grid(g, v)) return launch_mfma16dma_ragged(variant, g.dtype, p, g.compute_units, la.kc, lb.kc, stream);
     hipError_t e = (g.dtype == DT_F16) ? launch_variant<_Float16>(variant, p, g.compute_units, la.kc, lb.kc, stream)
                                        : launch_variant<__bf16>(variant, p, g.compute_units, la.kc, lb.kc, stream);
     if (e != hipSuccess || g.splits <= 1) return e;

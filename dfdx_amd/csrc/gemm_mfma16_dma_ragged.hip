@@ -1,0 +1,38 @@
+// The instances of the LDS-DMA kernel whose C lies off the 16-byte grid (odd extents or leading dimensions).  The operands are on
+// it: such a product's were laid out by launch_realign, or have always been.
+#include "gemm_mfma16_dma.h"
+
+namespace dfdx_rocm {
+namespace {
+
+template <typename T, int BM, int BN, int WM, int WN>
+hipError_t launch_layout(Params p, int compute_units, bool a_kc, bool b_kc, hipStream_t stream) {
+    constexpr int NT = WM * WN * 64;
+    constexpr size_t lds = (size_t)STAGES * (BM + BN) * BK * 2;
+    if (a_kc && b_kc) DFDX_LAUNCH(true, true, 2);
+    else if (a_kc && !b_kc) DFDX_LAUNCH(true, false, 2);
+    else if (!a_kc && b_kc) DFDX_LAUNCH(false, true, 2);
+    else DFDX_LAUNCH(false, false, 2);
+    return hipGetLastError();
+}
+
+template <typename T> hipError_t launch_variant(int variant, const Params &p, int compute_units, bool a_kc, bool b_kc, hipStream_t s) {
+    switch (variant) {
+#define X(id, bm, bn, wm, wn)                                                                             \
+    case id:                                                                                              \
+        if constexpr ((bn / wn) % 32 == 0) return launch_layout<T, bm, bn, wm, wn>(p, compute_units, a_kc, b_kc, s); \
+        else return hipErrorInvalidValue;
+        DFDX_MFMA16_DMA_VARIANTS(X)
+#undef X
+    default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace
+
+hipError_t launch_mfma16dma_ragged(int variant, int dtype, const DmaParams &p, int compute_units, bool a_kc, bool b_kc, hipStream_t stream) {
+    return dtype == DT_F16 ? launch_variant<_Float16>(variant, p, compute_units, a_kc, b_kc, stream)
+                           : launch_variant<__bf16>(variant, p, compute_units, a_kc, b_kc, stream);
+}
+
+}  // namespace dfdx_rocm

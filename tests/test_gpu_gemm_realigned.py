@@ -1,0 +1,89 @@
+"""Products of the 16-bit types whose operands are copied onto the 16-byte grid for the LDS-DMA kernels: odd extents in each
+place, contractions that end inside a k tile, a C at any address, padded leading dimensions, batches, shared operands."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from helpers import assert_within, rng
+from gpu_util import announce, device
+
+from dfdx_amd import View
+from dfdx_amd.rocm import KERNEL_AUTO
+from test_gpu_gemm import run_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("m,k,n,layout,pads", [
+    (2049, 1153, 1031, "nn", (0, 0, 0)),     # every extent odd, both copies
+    (2047, 1217, 2049, "nt", (1, 3, 1)),     # odd leading dimensions
+    (1025, 2111, 1279, "tn", (0, 5, 3)),     # A across k: zero rows behind the last
+    (2305, 1024, 2051, "nt", (0, 0, 0)),     # no copy at all: only C is off the grid
+    (2048, 1001, 2048, "nn", (0, 0, 0)),     # only the contraction is off the k tile
+    (261, 6795, 871, "tn", (0, 0, 0)),       # split contraction
+    (16384, 2048, 50, "tn", (0, 0, 0)),      # narrow output: the 64-column tile
+])
+@pytest.mark.parametrize("accumulate,bias,colmajor", [(False, True, False), (True, False, False), (True, False, True), (False, True, True)])
+def test_operands_off_the_grid(dtype, m, k, n, layout, pads, accumulate, bias, colmajor):
+    name = run_case(dtype, m, k, n, layout, accumulate, KERNEL_AUTO, 0, bias=bias, c_colmajor=colmajor, pads=pads, seed=m + k)
+    if not colmajor:
+        assert "_dma_" in name and "_realigned" in name, name
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_batches_and_addresses_off_the_grid(dtype, shared, shift):
+    """A batch whose matrices start anywhere, one operand shared by all of them, every pointer `shift` elements off."""
+    dev, g = device(), rng(91)
+    nb, m, k, n = 3, 2049, 1027, 2051
+    a = oracle.to_storage(g.standard_normal(shift + nb * m * k), dtype)
+    b = oracle.to_storage(g.standard_normal(shift + (1 if shared else nb) * k * n), dtype)
+    c = oracle.to_storage(g.standard_normal(shift + nb * m * n + 8), dtype)
+    da, db, dc = (dev.tensor(t, dtype) for t in (a, b, c))
+    desc = dev.gemm_desc(dtype, m, k, n, da.ptr + 2 * shift, (k, 1), db.ptr + 2 * shift, (n, 1), dc.ptr + 2 * shift, (n, 1), accumulate=True,
+                         batch=(nb, 1), a_batch=(m * k, 0), b_batch=(0 if shared else k * n, 0), c_batch=(m * n, 0))
+    name = dev.gemm_plan(desc)[2]
+    announce("realigned batch", dtype, shared, shift, name)
+    assert "_realigned" in name, name
+    dev.gemm(desc)
+    got = oracle.to_f64(dev.to_host(dc), dtype)
+    A = oracle.to_f64(a, dtype)[shift:].reshape(nb, m, k)
+    B = oracle.to_f64(b, dtype)[shift:].reshape(-1, k, n)
+    C = oracle.to_f64(c, dtype)
+    assert np.array_equal(got[:shift], C[:shift]) and np.array_equal(got[shift + nb * m * n:], C[shift + nb * m * n:])
+    ulp = 2.0 ** (-11 if dtype == "f16" else -8)
+    for i in range(nb):
+        Bi = B[0 if shared else i]
+        want = A[i] @ Bi + C[shift + i * m * n: shift + (i + 1) * m * n].reshape(m, n)
+        assert_within(dtype, k, got[shift + i * m * n: shift + (i + 1) * m * n].reshape(m, n), want, A[i], Bi, extra=ulp * float(np.abs(want).max()))
+
+
+def test_infinities_stay_in_their_row_and_column():
+    """The zeros that pad a copy meet zeros only: an infinite value in the last place of A reaches its row and nothing else."""
+    dev = device()
+    m, k, n, dtype = 2049, 1153, 1031, "f16"
+    a = torch.randn(m, k, device="cuda").half()
+    b = torch.rand(k, n, device="cuda").half() + 0.5
+    a[m - 1, k - 1] = float("inf")
+    view = lambda t: View(t.view(torch.uint8).reshape(-1), dtype, tuple(t.shape), tuple(t.stride()))
+    y = dev.forward(view(a), view(b)).storage.view(torch.float16).reshape(m, n)
+    assert bool(torch.isfinite(y[:-1]).all()) and bool((y[-1] == float("inf")).all())
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("rows,cols", [(2048, 50257), (3, 129), (77, 1001), (512, 135)])
+def test_bias_gradient_of_odd_rows(dtype, rows, cols):
+    """Column sums of rows off the 16-byte grid; f32 sums, one rounding: half an ulp of the result and rows * 2^-24 of the sum of magnitudes."""
+    dev = device()
+    t = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    g = torch.randn(rows, cols, device="cuda").to(t)
+    old = torch.randn(cols, device="cuda").to(t)
+    gb = old.clone()
+    view = lambda t_: View(t_.view(torch.uint8).reshape(-1), dtype, tuple(t_.shape), tuple(t_.stride()))
+    dev.bias_backward(view(g), view(gb))
+    want = g.double().sum(0) + old.double()
+    bound = want.abs() * 2.0 ** (-11 if dtype == "f16" else -8) + (g.double().abs().sum(0) + old.double().abs()) * rows * 2.0 ** -24 + 1e-7
+    assert bool(((gb.double() - want).abs() <= bound).all())
