@@ -8,6 +8,7 @@
 #include "elem.h"
 #include "gemm_internal.h"
 #include "conv3x3.h"
+#include "conv_few.h"
 
 #include <cstring>
 
@@ -546,6 +547,18 @@ bool implicit_forward(dfdx_rocm_ctx *ctx, int dtype, const Op &op, const void *f
     return true;
 }
 
+// The first layer of a network: one or three channels, half-size padding, 16-bit types (conv_few.hip).
+template <typename T> bool few_channels(dfdx_rocm_ctx *ctx, int dtype, const Op &op, ConvFew *c) {
+    if (sizeof(T) != 2 || op.groups != 1 || op.dilation != 1 || op.padding != op.kernel / 2) return false;
+    *c = ConvFew{};
+    c->dtype = dtype == DFDX_ROCM_F16 ? DT_F16 : DT_BF16;
+    c->kernel = op.kernel; c->stride = op.stride;
+    c->batch = op.batch; c->chan_in = op.chan_in; c->chan_out = op.chan_out;
+    c->h_in = op.h_in; c->w_in = op.w_in; c->h_out = op.h_out; c->w_out = op.w_out;
+    c->compute_units = ctx->compute_units;
+    return true;
+}
+
 // 3 x 3 filters at unit stride with padding 1, f16 / bf16 / f32, channel counts in whole chunks: the kernel that keeps a band
 // of the image in LDS and reads every tap's operand from it (conv3x3.hip).  The filters go through the patch buffer in
 // the order that kernel wants.
@@ -822,6 +835,11 @@ int forward_t(dfdx_rocm_ctx *ctx, int dtype, Op op, const void *img, const void 
         return (int)hipGetLastError();
     }
     if (per_image >= (1ll << 31) || (int64_t)op.chan_out * np >= (1ll << 31)) return DFDX_ROCM_ERR_UNSUPPORTED;
+    ConvFew few;
+    if (few_channels<T>(ctx, dtype, op, &few)) {
+        few.img = img; few.filters = filters; few.out = out;
+        if (conv_few_forward_supported(few)) return (int)launch_conv_few_forward(few, ctx->stream);
+    }
     if (op.kernel > 1) {  // (1x1 filters have no patch matrix to avoid: see `pointwise` below)
         int rc = 0;
         if (tiled3x3_forward<T>(ctx, dtype, op, filters, img, out, &rc)) return rc;
@@ -1126,6 +1144,17 @@ int backward_t(dfdx_rocm_ctx *ctx, int dtype, Op op, const void *img, void *grad
         depthwise_grad_filters_kernel<T><<<(unsigned)op.chan_out, 256, 0, ctx->stream>>>(op, (const T *)img, (const T *)grad_out, (T *)grad_filters,
                                                                                       magic_of(op.w_out));
         return (int)hipGetLastError();
+    }
+    ConvFew few;
+    if (few_channels<T>(ctx, dtype, op, &few)) {
+        few.img = img; few.filters = filters; few.grad_out = grad_out;
+        few.grad_img = grad_img; few.grad_filters = grad_filters;
+        few.fresh_img = fresh_img;
+        if (conv_few_backward_supported(few)) {
+            CtxLock lock(ctx->mu);  // the patch buffer is shared by every conv2d call on this context
+            if (int rc = ensure_patches(ctx, round256(conv_few_workspace_bytes(few)))) return rc;
+            return (int)launch_conv_few_backward(few, ctx->patches, ctx->stream);
+        }
     }
     // (also at unit stride when the image has far fewer channels than the output -- a first layer, 3 -> 64: the forward patch
     // matrix is O / C times smaller than the one over grad_out, and the products with three rows of filters disappear)
