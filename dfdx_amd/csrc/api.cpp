@@ -605,6 +605,60 @@ int gemm_beyond(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int extra, 
     }
 }
 
+int gemm_three(dfdx_rocm_ctx *ctx, const GemmProblem &problem, bool *done) {
+    *done = false;
+    GemmProblem p = problem;
+    if ((p.dtype != DT_F16 && p.dtype != DT_BF16) || p.k % 64) return DFDX_ROCM_OK;
+    p.compute_units = ctx->compute_units;
+    int dv = 0, splits = 1, dv1 = 0, splits1 = 1;
+    double t3 = 1e300, t1 = 1e300;
+    mfma16dma_plan_split(p, ctx->compute_units, 0, 0, &dv, &splits, &t3);
+    if (!dv || (p.ksum && !mfma16dma_ksum_supported(p, dv, splits)) || (p.extra != EXTRA_NONE && !mfma16dma_extra_supported(p, dv, splits)))
+        return DFDX_ROCM_OK;
+    GemmProblem q = p;
+    q.batches = 0;
+    q.nb1 = q.nb2 = 1;
+    q.reduce = 0;
+    mfma16dma_plan_split(q, ctx->compute_units, 0, 0, &dv1, &splits1, &t1);
+    t1 -= splits1 > 1 ? 6.5e-6 : 1.0e-6;  // (as in make_plan)
+    t3 -= splits > 1 ? 6.5e-6 : 1.0e-6;
+    const double t_small = small_supported(q) ? small_time(q, ctx->compute_units) : 1e300;
+    // Results that replace those of three calls have the bits of those: the order of the contraction is that of the tiles, so the
+    // small kernel and split plans are no match.  (Sums that join what three calls round one by one are free of that.)
+    if (!p.accumulate && (t_small < t1 || splits1 > 1 || splits > 1)) return DFDX_ROCM_OK;
+    if (t3 >= 3.0 * std::min(t1, t_small)) return DFDX_ROCM_OK;
+    Plan plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
+    if (int e = reserve_partials(ctx, p, plan, false)) return e;
+    // deferred zero fills: as settle_operands, for each of the three
+    const size_t es = dtype_size(p.dtype), c_bytes = (size_t)(p.m * p.n) * es, k_bytes = (size_t)p.m * es;
+    auto at = [&](const void *ptr, int64_t b1, int64_t b2, int i) -> char * {
+        return ptr ? (char *)ptr + (i == 1 ? b2 : i == 2 ? b1 : 0) * (int64_t)es : nullptr;
+    };
+    if (int e = settle(ctx, p.with)) return e;
+    bool fresh[2][3] = {};
+    for (int i = 0; i < 3; i++) {
+        if (int e = settle(ctx, at(p.a, p.a_b1, p.a_b2, i))) return e;
+        if (int e = settle(ctx, at(p.b, p.b_b1, p.b_b2, i))) return e;
+        if (int e = settle(ctx, at(p.bias, p.bias_b1, p.bias_b2, i))) return e;
+        if (i > 0 && p.reduce) continue;
+        if (int e = settle_output(ctx, at(p.c, p.c_b1, p.c_b2, i), c_bytes, p.accumulate, p.extra == EXTRA_FROM ? nullptr : &fresh[0][i])) return e;
+        if (p.ksum)
+            if (int e = settle_output(ctx, at(p.ksum, p.ksum_b1, p.ksum_b2, i), k_bytes, true, &fresh[1][i])) return e;
+    }
+    // gradients are stored where all three count as zero; a mixture is filled after all
+    for (int r = 0; r < 2; r++) {
+        const bool all = fresh[r][0] && fresh[r][1] && fresh[r][2];
+        if (all && r == 0) p.accumulate = 0;
+        if (all && r == 1) p.ksum_accumulate = 0;
+        for (int i = 0; i < 3 && !all; i++)
+            if (fresh[r][i])
+                HIP_TRY(launch_zero_fill(r == 0 ? at(p.c, p.c_b1, p.c_b2, i) : at(p.ksum, p.ksum_b1, p.ksum_b2, i), r == 0 ? c_bytes : k_bytes,
+                                         ctx->compute_units, ctx->stream));
+    }
+    *done = true;
+    return run_plan(ctx, p, plan);
+}
+
 int gemm_with_colsum(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, void *colsum_b, bool *fused) {
     *fused = false;
     if (int e = bind(ctx)) return e;

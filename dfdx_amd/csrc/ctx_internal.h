@@ -78,6 +78,9 @@ int gemm_with_colsum(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, void *
 // dfdx_rocm_gemm(ctx, desc) for a contiguous C with one thing more on the way into it (EXTRA_* in gemm_internal.h; by a
 // separate op where the kernel picked cannot).
 int gemm_beyond(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int extra, const void *with);
+// Three products of the same shape in one launch (GemmProblem::batches = 3, or their sum: `reduce`), where the LDS-DMA kernels take
+// them and one launch is expected to be faster than three.  *done tells whether it ran; when not, nothing has been touched.
+int gemm_three(dfdx_rocm_ctx *ctx, const struct GemmProblem &problem, bool *done);
 // x[i] = with[i] > 0 ? x[i] : 0, in place
 int relu_mask(dfdx_rocm_ctx *ctx, int dtype, int64_t len, const void *with, void *x);
 // Clears `bytes` bytes at `ptr` (any alignment) with a fill kernel on `stream`.

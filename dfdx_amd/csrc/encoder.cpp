@@ -117,6 +117,27 @@ int weight_grad(dfdx_rocm_ctx *ctx, const Shape &s, int64_t i, int64_t o, const 
     return done ? DFDX_ROCM_OK : dfdx_rocm_bias_backward(ctx, s.dtype, s.T, o, gy, gb);
 }
 
+// The products of the query, key and value projections as one launch: same shapes, matrices wherever they are (addresses from
+// the first to the second and to the third).  False where the distances are not whole elements.
+bool apart(const void *first, const void *second, const void *third, size_t es, int64_t *b1, int64_t *b2) {
+    const int64_t to2 = (const char *)second - (const char *)first, to3 = (const char *)third - (const char *)first;
+    *b2 = to2 / (int64_t)es;
+    *b1 = to3 / (int64_t)es;
+    return to2 % (int64_t)es == 0 && to3 % (int64_t)es == 0;
+}
+GemmProblem three(int dtype, int64_t m, int64_t k, int64_t n, const void *a, int64_t a_rs, int64_t a_cs, const void *b, int64_t b_rs, int64_t b_cs, void *c) {
+    GemmProblem p{};
+    p.dtype = dtype;
+    p.m = m; p.k = k; p.n = n;
+    p.nb1 = p.nb2 = 2;
+    p.batches = 3;
+    p.a = a; p.a_rs = a_rs; p.a_cs = a_cs;
+    p.b = b; p.b_rs = b_rs; p.b_cs = b_cs;
+    p.c = c; p.c_rs = n; p.c_cs = 1;
+    p.splits = 1;
+    return p;
+}
+
 #define TRY(call)                \
     do {                         \
         if (int e__ = (call)) return e__; \
@@ -128,9 +149,18 @@ int forward(dfdx_rocm_ctx *ctx, const Shape &s, const dfdx_rocm_encoder *e, cons
     void *q = saved + l.q, *k = saved + l.k, *v = saved + l.v, *tok = saved + l.tok, *h1 = saved + l.h1, *n1 = saved + l.n1,
          *h2 = saved + l.h2, *r1 = saved + l.r1;
     const int64_t row[2] = {s.d, 1};
-    TRY(dfdx_rocm_linear_forward(ctx, s.dtype, s.T, s.d, s.d, x, row, p[WQ], p[BQ], q));
-    TRY(dfdx_rocm_linear_forward(ctx, s.dtype, s.T, s.d, s.d, x, row, p[WK], p[BK_], k));
-    TRY(dfdx_rocm_linear_forward(ctx, s.dtype, s.T, s.d, s.d, x, row, p[WV], p[BV], v));
+    bool done = false;
+    GemmProblem all = three(s.dtype, s.T, s.d, s.d, x, s.d, 1, p[WQ], 1, s.d, q);
+    all.bias = p[BQ];
+    all.bias_mode = BIAS_PER_COL;
+    if (apart(p[WQ], p[WK], p[WV], s.es, &all.b_b1, &all.b_b2) && apart(p[BQ], p[BK_], p[BV], s.es, &all.bias_b1, &all.bias_b2) &&
+        apart(q, k, v, s.es, &all.c_b1, &all.c_b2))
+        TRY(gemm_three(ctx, all, &done));
+    if (!done) {
+        TRY(dfdx_rocm_linear_forward(ctx, s.dtype, s.T, s.d, s.d, x, row, p[WQ], p[BQ], q));
+        TRY(dfdx_rocm_linear_forward(ctx, s.dtype, s.T, s.d, s.d, x, row, p[WK], p[BK_], k));
+        TRY(dfdx_rocm_linear_forward(ctx, s.dtype, s.T, s.d, s.d, x, row, p[WV], p[BV], v));
+    }
     if (s.fused) {
         TRY(dfdx_rocm_attention_forward(ctx, s.dtype, s.B, s.H, s.S, s.D, q, k, v, s.token, (float)s.scale, tok, s.token, (float *)(saved + l.lse)));
     } else {
@@ -202,14 +232,31 @@ int backward(dfdx_rocm_ctx *ctx, const Shape &s, const dfdx_rocm_encoder *e, con
         if (!s.folded) TRY(dfdx_rocm_scalar_mul_backward(ctx, s.dtype, s.B * s.H * s.S * s.S, s.scale, gscores, gscaled));
         TRY(dfdx_rocm_matmat_batch4_backward(ctx, s.dtype, s.B, s.H, s.S, s.D, s.S, q, qs, gq, k, ks, gk, gscores));
     }
-    // x feeds the three projections and the residual
+    // x feeds the three projections and the residual: grad_x is one sum over their 3 d columns, rounded once
+    bool summed = false, weights = false;
+    GemmProblem all = three(s.dtype, s.T, s.d, s.d, gq, s.d, 1, p[WQ], s.d, 1, grad_x);
+    all.reduce = 1;
+    all.accumulate = 1;
+    all.extra = EXTRA_FROM;
+    all.with = gh1;
+    if (apart(gq, gk, gv, s.es, &all.a_b1, &all.a_b2) && apart(p[WQ], p[WK], p[WV], s.es, &all.b_b1, &all.b_b2)) TRY(gemm_three(ctx, all, &summed));
+    all = three(s.dtype, s.d, s.T, s.d, gq, 1, s.d, x, s.d, 1, grads[WQ]);  // weight (o, i) += grad_y^T . x, bias += sums of grad_y
+    all.accumulate = 1;
+    all.ksum = grads[BQ];
+    all.ksum_of = KSUM_OF_A;
+    all.ksum_accumulate = 1;
+    if (apart(gq, gk, gv, s.es, &all.a_b1, &all.a_b2) && apart(grads[WQ], grads[WK], grads[WV], s.es, &all.c_b1, &all.c_b2) &&
+        apart(grads[BQ], grads[BK_], grads[BV], s.es, &all.ksum_b1, &all.ksum_b2))
+        TRY(gemm_three(ctx, all, &weights));
     for (int i = 0; i < 3; i++) {
         const int w = i == 0 ? WQ : i == 1 ? WK : WV;
         const void *gy = i == 0 ? gq : i == 1 ? gk : gv;
-        g = input_grad(s, s.d, s.d, gy, p[w], grad_x);
-        g.accumulate = 1;
-        TRY(gemm_beyond(ctx, &g, i == 0 ? EXTRA_FROM : EXTRA_NONE, i == 0 ? gh1 : nullptr));
-        TRY(weight_grad(ctx, s, s.d, s.d, x, gy, grads[w], grads[w + 1]));
+        if (!summed) {
+            g = input_grad(s, s.d, s.d, gy, p[w], grad_x);
+            g.accumulate = 1;
+            TRY(gemm_beyond(ctx, &g, i == 0 ? EXTRA_FROM : EXTRA_NONE, i == 0 ? gh1 : nullptr));
+        }
+        if (!weights) TRY(weight_grad(ctx, s, s.d, s.d, x, gy, grads[w], grads[w + 1]));
     }
     return DFDX_ROCM_OK;
 }

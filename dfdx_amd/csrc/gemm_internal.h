@@ -24,6 +24,12 @@ struct GemmProblem {
     int bias_mode;
     int64_t m, n, k;
     int64_t nb1, nb2;
+    // The batches are walked in the order (0, 0), (0, 1) .. (0, nb2 - 1), (1, 0) ..; `batches` > 0 stops after that many of them
+    // (LDS-DMA kernels only).  Three matrices that lie anywhere are nb1 = nb2 = 2, batches = 3: batch stride 2 leads to the
+    // second, batch stride 1 to the third, and either may be negative.
+    int64_t batches = 0;
+    int64_t bias_b1 = 0, bias_b2 = 0;
+    int64_t batch_count() const { return batches > 0 ? batches : nb1 * nb2; }
     const void *a;
     int64_t a_rs, a_cs, a_b1, a_b2;
     const void *b;
@@ -39,6 +45,7 @@ struct GemmProblem {
     void *ksum = nullptr;
     int ksum_of = KSUM_NONE;
     int ksum_accumulate = 0;
+    int64_t ksum_b1 = 0, ksum_b2 = 0;  // where `batches` says how many
     int extra = EXTRA_NONE;        // see above; kernels that have it: extra_supported in api.cpp
     const void *with = nullptr;
     // Operands laid out by launch_realign: an operand whose rows lie along memory is readable up to the next multiple of eight

@@ -31,7 +31,7 @@ struct DmaParams {
     int m, n, k;
     int lda, ldb;
     int64_t ldc;
-    int64_t a_b1, a_b2, b_b1, b_b2, c_b1, c_b2;
+    int64_t a_b1, a_b2, b_b1, b_b2, c_b1, c_b2, bias_b1, bias_b2;
     int nb2, kbatches;
     int tiles_m, tiles_n, tiles_per_batch, total_blocks;
     int accumulate, bias_mode;
@@ -211,14 +211,22 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
     // A work item is one C tile (of one batch, or of one k split).  The workgroup is persistent: it walks the
     // work items blockIdx.x, blockIdx.x + gridDim.x, ... and keeps ONE load pipeline running across them, so
     // the stores of a finished tile overlap with the loads (already in flight) and MFMAs of the next one.
+    // The arguments that only a work item's start and end need are read from memory there, not held in scalar registers
+    // through the k loop (4096^3 f16, registers spilled to vector lanes: 17 - 32 with all arguments held, none now).
+    typedef const __attribute__((address_space(4))) Params ArgParams;
+    auto late_args = [&]() -> ArgParams * {
+        ArgParams *args = (ArgParams *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(args));
+        return args;
+    };
     struct Work {
         int batch, split, bm0, bn0, it0, iters;
     };
     const int ktiles = p.k / BK;
-    auto decode = [&](int index) -> Work {
+    auto decode = [&](auto &p, int index) -> Work {
         Work w;
         const int work = xcd_remap(index, p.total_blocks);
-        const int bidx = work / p.tiles_per_batch;  // batch, or k split
+        const int bidx = work / p.tiles_per_batch;  // k pieces of a batch, batch after batch
         const int tile = work % p.tiles_per_batch;
         const int gsize = p.group_m * p.tiles_n;
         const int group = tile / gsize;
@@ -226,8 +234,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
         const int gm = min(p.tiles_m - first_m, p.group_m);
         w.bm0 = (first_m + (tile % gsize) % gm) * BM;
         w.bn0 = ((tile % gsize) / gm) * BN;
-        w.split = p.splits > 1 ? bidx : 0;
-        w.batch = p.splits > 1 ? 0 : bidx;
+        w.batch = p.splits > 1 ? bidx / p.splits : bidx;
+        w.split = p.splits > 1 ? bidx - w.batch * p.splits : 0;
         // k-loop steps run over (batch, k-tile) pairs; with split-k this item owns steps [it0, it0 + iters)
         w.it0 = w.split * p.chunk;
         w.iters = min(ktiles * p.kbatches - w.it0, p.chunk);
@@ -238,7 +246,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
     const int64_t a_step = A_KC ? BK : (int64_t)BK * p.lda;
     const int64_t b_step = B_KC ? BK : (int64_t)BK * p.ldb;
     int f_index = blockIdx.x;   // work item whose tiles are being requested
-    Work fw = decode(f_index);
+    Work fw = decode(p, f_index);
     int f_left = 0, f_kb = 0, f_kt = 0, f_stage = 0;
     const uint16_t *a_next = nullptr, *b_next = nullptr;
     TA ta;
@@ -279,7 +287,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
             f_index += gridDim.x;
             fetching = f_index < p.total_blocks;
             if (fetching) {
-                fw = decode(f_index);
+                fw = decode(*late_args(), f_index);
                 begin_fetch();
             }
             return;
@@ -540,6 +548,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
     // ---- epilogue of one work item: lane holds m = l16 (per tile), n = 4*lq + 0..3 -------------
     // Returns the number of stores it issued after its last load (see sync_tile), 0 when that is not a fixed count.
     auto store_tile = [&](const Work &w) -> int {
+        ArgParams &p = *late_args();
         const int bm0 = w.bm0, bn0 = w.bn0, split = w.split, batch = w.batch;
         if constexpr (KSUM) {
             // Lanes that hold the same 8 columns (they differ in the k-row) are added up; the first CH lanes of each wave
@@ -552,7 +561,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
                     for (int d = CH; d < 64; d *= 2) ks_sum[e] += __shfl_xor(ks_sum[e], d, 64);
                 }
                 if (lane < CH) {
-                    float *slot = p.ws_ksum + (int64_t)((split * KS_SHARE + bn0 / BN) * 8 + wave) * p.ws_ksum_stride + bm0 + ks_chunk * 8;
+                    float *slot = p.ws_ksum + (int64_t)(((batch * p.splits + split) * KS_SHARE + bn0 / BN) * 8 + wave) * p.ws_ksum_stride + bm0 + ks_chunk * 8;
                     *(f32x4 *)slot = f32x4{ks_sum[0], ks_sum[1], ks_sum[2], ks_sum[3]};  // rows padded to whole tiles
                     *(f32x4 *)(slot + 4) = f32x4{ks_sum[4], ks_sum[5], ks_sum[6], ks_sum[7]};
                 }
@@ -563,7 +572,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
     // f32 partial tile into the workspace (padded to whole tiles: no bounds checks).  KSUM instances run for split plans
     // only: without the other forms of the epilogue the bf16 256 x 256 instance spills far fewer registers in its k loop.
     if (KSUM || p.splits > 1) {
-        float *wbase = p.ws + split * p.ws_split_stride;
+        float *wbase = p.ws + (int64_t)(batch * p.splits + split) * p.ws_split_stride;
 #pragma unroll
         for (int i = 0; i < TM; i++) {
             float *wrow = wbase + (int64_t)(bm0 + wm0 + i * 16 + l16) * p.ws_ld + bn0 + wn0 + lq * (PERM ? 8 : 4);
@@ -584,6 +593,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
     };
     const int cb = p.kbatches > 1 ? 0 : batch;
     uint16_t *cbase = p.c + (int64_t)(cb / p.nb2) * p.c_b1 + (int64_t)(cb % p.nb2) * p.c_b2;
+    const uint16_t *const bias = p.bias + (int64_t)(cb / p.nb2) * p.bias_b1 + (int64_t)(cb % p.nb2) * p.bias_b2;
     // two finished values (rounded, packed) and their partners; see EXTRA_*
     [[maybe_unused]] auto extra = [](uint32_t o, uint32_t w) -> uint32_t {
         const float lo = Mma<T>::to_f32((uint16_t)(o & 0xffffu)), hi = Mma<T>::to_f32((uint16_t)(o >> 16));
@@ -610,16 +620,16 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
                     for (int jp = 0; jp < TN / 2; jp++) {
                         const int gn = bn0 + wn0 + (PERM ? jp * 32 + lq * 8 : (2 * jp + (lq & 1)) * 16 + (lq >> 1) * 8);
                         if constexpr (ANY) {
-                            if (gn + 8 <= p.n) cbias[jp] = load16<true>(p.bias + gn);
-                            else cbias[jp] = columns_left(p.bias + gn, p.n - gn);
+                            if (gn + 8 <= p.n) cbias[jp] = load16<true>(bias + gn);
+                            else cbias[jp] = columns_left(bias + gn, p.n - gn);
                         } else {
-                            cbias[jp] = *(const u32x4 *)(p.bias + min(gn, p.n - 8));
+                            cbias[jp] = *(const u32x4 *)(bias + min(gn, p.n - 8));
                         }
                     }
                 }
                 if (p.bias_mode == BIAS_PER_ROW) {
 #pragma unroll
-                    for (int i = 0; i < TM; i++) rbias_all[i] = Mma<T>::to_f32(p.bias[min(bm0 + wm0 + i * 16 + l16, p.m - 1)]);
+                    for (int i = 0; i < TM; i++) rbias_all[i] = Mma<T>::to_f32(bias[min(bm0 + wm0 + i * 16 + l16, p.m - 1)]);
                 }
 #pragma unroll
                 for (int i = 0; i < TM; i++) {
@@ -714,7 +724,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
 #pragma unroll
                     for (int j = 0; j < TN; j++) {
                         u32x2 bv;
-                        const uint16_t *const bias_at = p.bias + bn0 + wn0 + (PERM ? (j / 2) * 32 + lq * 8 + (j % 2) * 4 : j * 16 + lq * 4);
+                        const uint16_t *const bias_at = bias + bn0 + wn0 + (PERM ? (j / 2) * 32 + lq * 8 + (j % 2) * 4 : j * 16 + lq * 4);
                         if constexpr (ANY) bv = *(const u32x2_any *)bias_at;
                         else bv = *(const u32x2 *)bias_at;
                         cb[j][0] = Mma<T>::to_f32((uint16_t)(bv[0] & 0xffffu));
@@ -879,7 +889,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
             const int gm_row = bm0 + wm0 + i * 16 + l16;
             if (gm_row >= p.m) continue;
             uint16_t *crow = cbase + (int64_t)gm_row * p.ldc;
-            const float rbias = (p.bias_mode == BIAS_PER_ROW) ? Mma<T>::to_f32(p.bias[gm_row]) : 0.0f;
+            const float rbias = (p.bias_mode == BIAS_PER_ROW) ? Mma<T>::to_f32(bias[gm_row]) : 0.0f;
 #pragma unroll
             for (int j = 0; j < TN; j++) {
                 const int gn = bn0 + wn0 + j * 16 + lq * 4;
@@ -888,7 +898,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
 #pragma unroll
                 for (int e = 0; e < 4; e++) v[e] = acc[i][j][e] + rbias;
                 if (p.bias_mode == BIAS_PER_COL) {
-                    const u32x2 bv = *(const u32x2 *)(p.bias + gn);
+                    const u32x2 bv = *(const u32x2 *)(bias + gn);
                     v[0] += Mma<T>::to_f32((uint16_t)(bv[0] & 0xffffu));
                     v[1] += Mma<T>::to_f32((uint16_t)(bv[0] >> 16));
                     v[2] += Mma<T>::to_f32((uint16_t)(bv[1] & 0xffffu));
@@ -917,7 +927,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
 
     // ---- compute state ---------------------------------------------------------------------------------------
     int c_index = blockIdx.x;
-    Work cw = decode(c_index);
+    Work cw = fw;
     int c_left = cw.iters, c_stage = 0;
     int behind = 0;  // stores of the previous work item that may still be in flight
     if constexpr (KSUM) ks_begin(cw.bn0);
@@ -947,7 +957,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
 #pragma unroll
                 for (int v = 0; v < 4; v++) acc[i][j][v] = 0.0f;
         c_index += gridDim.x;
-        cw = decode(c_index);
+        cw = decode(*late_args(), c_index);
         c_left = cw.iters;
         if constexpr (KSUM) ks_begin(cw.bn0);
         read_first(smem + c_stage * STAGE_BYTES);

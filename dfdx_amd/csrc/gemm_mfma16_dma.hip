@@ -122,20 +122,21 @@ bool mfma16dma_supported(const GemmProblem &p, int variant) {
     if (la.ld * (la.kc ? v.bm : BK) >= (1ll << 30) || lb.ld * (lb.kc ? v.bn : BK) >= (1ll << 30)) return false;
     if (!aligned16(p.a) || !aligned16(p.b)) return false;
     if (!c_on_grid(p, v) && !(p.ragged && (v.bn / v.waves_n) % 32 == 0)) return false;
-    if (p.nb1 * p.nb2 > 1) {
+    if (p.batch_count() > 1) {
         if (p.a_b1 % 8 || p.a_b2 % 8 || p.b_b1 % 8 || p.b_b2 % 8) return false;
-        if (p.a_b1 < 0 || p.a_b2 < 0 || p.b_b1 < 0 || p.b_b2 < 0) return false;
+        if (!p.batches && (p.a_b1 < 0 || p.a_b2 < 0 || p.b_b1 < 0 || p.b_b2 < 0)) return false;
+        if (p.bias_b1 % 8 || p.bias_b2 % 8) return false;
     }
     const int64_t tiles = ((p.m + v.bm - 1) / v.bm) * ((p.n + v.bn - 1) / v.bn);
-    const int64_t blocks = tiles * (p.reduce ? 1 : p.nb1 * p.nb2);
-    if (blocks >= (1ll << 31) || p.nb1 * p.nb2 >= (1ll << 31)) return false;
-    if (p.k * (p.reduce ? p.nb1 * p.nb2 : 1) >= (1ll << 31)) return false;
+    const int64_t blocks = tiles * (p.reduce ? 1 : p.batch_count());
+    if (blocks >= (1ll << 31) || p.batch_count() >= (1ll << 31)) return false;
+    if (p.k * (p.reduce ? p.batch_count() : 1) >= (1ll << 31)) return false;
     return true;
 }
 
 int mfma16dma_pick_variant(const GemmProblem &p, int compute_units) {
     // Largest tile that still gives every compute unit a workgroup; BN = 64 tiles only for narrow outputs.
-    const int64_t nbatch = p.reduce ? 1 : p.nb1 * p.nb2;
+    const int64_t nbatch = p.reduce ? 1 : p.batch_count();
     const int wide[] = {1, 2, 3}, narrow[] = {4, 5};
     if (p.n <= 64) {
         for (int v : narrow) {
@@ -183,9 +184,9 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
     *variant = 0;
     *splits = 1;
     const int cus = std::max(1, compute_units);
-    const int64_t nbatch = p.reduce ? 1 : p.nb1 * p.nb2;
-    const bool may_split = nbatch == 1 && p.c_cs == 1;
-    const int64_t total_iters = (p.k / BK) * (p.reduce ? p.nb1 * p.nb2 : 1);
+    const int64_t nbatch = p.reduce ? 1 : p.batch_count();
+    const bool may_split = (nbatch == 1 || p.batches > 0) && p.c_cs == 1;
+    const int64_t total_iters = (p.k / BK) * (p.reduce ? p.batch_count() : 1);
     const bool a_kc = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged).kc, b_kc = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged).kc;
     const double elem = 2.0, out_elems = (double)p.m * p.n * nbatch;
     double best = 1e300;
@@ -248,7 +249,7 @@ size_t mfma16dma_workspace_bytes(const GemmProblem &p, int variant, int splits) 
     int64_t ld, stride, ks;
     ws_layout(p, variant, &ld, &stride, &ks);
     const int64_t slots = p.ksum ? ksum_slots(variant, splits) : 0;
-    return (size_t)(stride * splits + ks * slots) * sizeof(float);
+    return (size_t)(stride * splits + ks * slots) * (size_t)(p.reduce ? 1 : p.batch_count()) * sizeof(float);
 }
 
 // The sums of A's rows ride along only where A and B are both stored contraction-major (m- and n-contiguous: the
@@ -256,7 +257,7 @@ size_t mfma16dma_workspace_bytes(const GemmProblem &p, int variant, int splits) 
 // combined by the reduce kernel that runs then anyway).
 bool mfma16dma_ksum_supported(const GemmProblem &p, int variant, int splits) {
     if (!p.ksum || p.ksum_of != KSUM_OF_A || splits <= 1 || !mfma16dma_supported(p, variant)) return false;
-    if (!p.reduce && p.nb1 * p.nb2 != 1) return false;
+    if (!p.reduce && p.batch_count() != 1 && !p.batches) return false;
     if ((uintptr_t)p.ksum & 1u) return false;
     const Variant &v = kVariants[variant - 1];
     if ((p.n + v.bn - 1) / v.bn < v.bm / 64) return false;  // too few tile columns to share a tile's pieces
@@ -264,7 +265,7 @@ bool mfma16dma_ksum_supported(const GemmProblem &p, int variant, int splits) {
 }
 
 bool mfma16dma_extra_supported(const GemmProblem &p, int variant, int splits) {
-    if ((p.accumulate != 0) != (p.extra == EXTRA_FROM) || p.nb1 * p.nb2 != 1 || !mfma16dma_supported(p, variant)) return false;
+    if ((p.accumulate != 0) != (p.extra == EXTRA_FROM) || (p.batch_count() != 1 && !p.reduce) || !mfma16dma_supported(p, variant)) return false;
     if (p.extra != EXTRA_RELU && (!p.with || !aligned16(p.with))) return false;
     if (splits > 1) return true;  // the reduce kernel applies it
     const bool a_kc = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged).kc, b_kc = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged).kc;
@@ -283,7 +284,8 @@ hipError_t launch_mfma16dma(const GemmProblem &g, int variant, hipStream_t strea
     p.ldc = g.m == 1 ? g.n : g.c_rs;
     p.a_b1 = g.a_b1; p.a_b2 = g.a_b2; p.b_b1 = g.b_b1; p.b_b2 = g.b_b2; p.c_b1 = g.c_b1; p.c_b2 = g.c_b2;
     p.nb2 = (int)g.nb2;
-    const int nbatch = (int)(g.nb1 * g.nb2);
+    p.bias_b1 = g.bias_b1; p.bias_b2 = g.bias_b2;
+    const int nbatch = (int)(g.batch_count());
     p.kbatches = g.reduce ? nbatch : 1;
     p.tiles_m = (int)((g.m + v.bm - 1) / v.bm);
     p.tiles_n = (int)((g.n + v.bn - 1) / v.bn);
@@ -296,7 +298,7 @@ hipError_t launch_mfma16dma(const GemmProblem &g, int variant, hipStream_t strea
     p.ws_ksum = nullptr; p.ws_ksum_stride = 0;
     if (g.ksum && !mfma16dma_ksum_supported(g, variant, g.splits)) return hipErrorInvalidValue;
     if (g.splits > 1) {
-        if (!g.workspace || p.total_blocks != p.tiles_per_batch) return hipErrorInvalidValue;
+        if (!g.workspace || (p.total_blocks != p.tiles_per_batch && !g.batches)) return hipErrorInvalidValue;
         p.splits = g.splits;
         p.chunk = (total_iters + g.splits - 1) / g.splits;
         if ((int64_t)(g.splits - 1) * p.chunk >= total_iters) return hipErrorInvalidValue;
@@ -304,10 +306,10 @@ hipError_t launch_mfma16dma(const GemmProblem &g, int variant, hipStream_t strea
         int64_t ks_stride = 0;
         ws_layout(g, variant, &p.ws_ld, &p.ws_split_stride, &ks_stride);
         if (g.ksum) {
-            p.ws_ksum = g.workspace + p.ws_split_stride * g.splits;
+            p.ws_ksum = g.workspace + p.ws_split_stride * g.splits * (g.reduce ? 1 : nbatch);
             p.ws_ksum_stride = (int)ks_stride;
         }
-        p.total_blocks = p.tiles_per_batch * g.splits;
+        p.total_blocks *= g.splits;
     }
     p.grid = 0;  // set per kernel instantiation at launch
     p.with = (const uint16_t *)g.with;

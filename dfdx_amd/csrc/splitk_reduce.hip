@@ -66,11 +66,28 @@ template <typename T> __device__ __forceinline__ void combine_ksum(const KsumPar
     }
 }
 
+// Where the results of batch blockIdx.z lie (elements): several split products in one launch (GemmProblem::batches).
+struct Batches {
+    int nb2, splits;
+    int64_t c_b1, c_b2, k_b1, k_b2;
+};
+template <typename T> __device__ __forceinline__ void to_batch(const Batches &bt, const float *&ws, int64_t ws_split_stride, T *&c, KsumParts &ks, Beyond &bd) {
+    const int z = blockIdx.z, z1 = z / bt.nb2, z2 = z - z1 * bt.nb2;
+    const int64_t off = z1 * bt.c_b1 + z2 * bt.c_b2;
+    ws += (int64_t)z * bt.splits * ws_split_stride;
+    c += off;
+    bd.c_old = (const T *)bd.c_old + off;
+    bd.with = (const T *)bd.with + off;
+    ks.ws = ks.ws ? ks.ws + (int64_t)z * ks.slots * ks.stride : nullptr;
+    ks.out = (T *)ks.out + (z1 * bt.k_b1 + z2 * bt.k_b2);
+}
+
 // one thread: 4 consecutive columns of one row
 template <typename T>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *ws, int splits, int64_t ws_ld, int64_t ws_split_stride,
                                                             T *c, int64_t c_rs, int m, int n, int accumulate, int bias_mode,
-                                                            const T *bias, int vec4, KsumParts ks, Beyond bd) {
+                                                            const T *bias, int vec4, KsumParts ks, Beyond bd, Batches bt) {
+    to_batch<T>(bt, ws, ws_split_stride, c, ks, bd);
     if (ks.ws && (int)blockIdx.x < ks.blocks) {   // uniform over the workgroup
         if (blockIdx.y == 0) combine_ksum<T>(ks, m);
         return;   // the same block index in the other grid rows has no work
@@ -139,7 +156,8 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 template <typename T>
 __global__ __launch_bounds__(256) void splitk_reduce16_kernel(const float *ws, int splits, int64_t ws_ld, int64_t ws_split_stride,
                                                               uint16_t *c, int64_t c_rs, int m, int n, int accumulate,
-                                                              int bias_mode, const uint16_t *bias, KsumParts ks, Beyond bd) {
+                                                              int bias_mode, const uint16_t *bias, KsumParts ks, Beyond bd, Batches bt) {
+    to_batch<uint16_t>(bt, ws, ws_split_stride, c, ks, bd);
     if (ks.ws && (int)blockIdx.x < ks.blocks) {   // uniform over the workgroup
         if (blockIdx.y == 0) combine_ksum<T>(ks, m);
         return;   // the same block index in the other grid rows has no work
@@ -193,7 +211,7 @@ __global__ __launch_bounds__(256) void splitk_reduce16_kernel(const float *ws, i
 
 }  // namespace
 
-// C of `p` must have unit column stride and no batch (the planner only splits such problems).
+// C of `p` must have unit column stride and no batch (the planner only splits such problems), or `batches`.
 hipError_t launch_splitk_reduce(const GemmProblem &p, int64_t ws_ld, int64_t ws_split_stride, hipStream_t stream,
                                 const float *ws_ksum, int64_t ws_ksum_stride, int ksum_slots) {
     const bool with_ksum = p.ksum && ws_ksum;
@@ -201,23 +219,25 @@ hipError_t launch_splitk_reduce(const GemmProblem &p, int64_t ws_ld, int64_t ws_
                        with_ksum ? (int)((p.m + KSUM_ROWS - 1) / KSUM_ROWS) : 0};
     const bool from = p.extra == EXTRA_FROM;
     const Beyond bd{from ? p.with : p.c, p.with, from ? EXTRA_NONE : p.extra};
-    dim3 grid((unsigned)((p.m + 3) / 4 + ks.blocks), (unsigned)((p.n + 255) / 256)), block(256);
+    const unsigned products = p.reduce ? 1u : (unsigned)p.batch_count();
+    const Batches bt{products > 1 ? (int)p.nb2 : 1, p.splits, p.c_b1, p.c_b2, p.ksum_b1, p.ksum_b2};
+    dim3 grid((unsigned)((p.m + 3) / 4 + ks.blocks), (unsigned)((p.n + 255) / 256), products), block(256);
     if ((p.n + 255) / 256 > 65535) return hipErrorInvalidValue;  // 16.7 M columns: no planner splits such a product
     const int64_t c_rs = p.m == 1 ? p.n : p.c_rs;
     const int bias_mode = p.bias ? p.bias_mode : BIAS_NONE;
     const bool is16 = p.dtype == DT_F16 || p.dtype == DT_BF16;
-    if (is16 && p.n % 8 == 0 && c_rs % 8 == 0 && ws_ld % 4 == 0 && ws_split_stride % 4 == 0 && ((uintptr_t)p.c & 15u) == 0 &&
+    if (is16 && p.n % 8 == 0 && c_rs % 8 == 0 && p.c_b1 % 8 == 0 && p.c_b2 % 8 == 0 && ws_ld % 4 == 0 && ws_split_stride % 4 == 0 && ((uintptr_t)p.c & 15u) == 0 &&
         ((uintptr_t)p.workspace & 15u) == 0 && (((uintptr_t)bd.c_old | (uintptr_t)bd.with) & 15u) == 0 &&
         (bias_mode != BIAS_PER_COL || ((uintptr_t)p.bias & 15u) == 0)) {
-        dim3 grid16((unsigned)((p.m + 3) / 4 + ks.blocks), (unsigned)((p.n + 511) / 512));
+        dim3 grid16((unsigned)((p.m + 3) / 4 + ks.blocks), (unsigned)((p.n + 511) / 512), products);
         if (p.dtype == DT_F16)
             splitk_reduce16_kernel<_Float16><<<grid16, block, 0, stream>>>(p.workspace, p.splits, ws_ld, ws_split_stride, (uint16_t *)p.c,
                                                                             c_rs, (int)p.m, (int)p.n, p.accumulate, bias_mode,
-                                                                            (const uint16_t *)p.bias, ks, bd);
+                                                                            (const uint16_t *)p.bias, ks, bd, bt);
         else
             splitk_reduce16_kernel<__bf16><<<grid16, block, 0, stream>>>(p.workspace, p.splits, ws_ld, ws_split_stride, (uint16_t *)p.c,
                                                                           c_rs, (int)p.m, (int)p.n, p.accumulate, bias_mode,
-                                                                          (const uint16_t *)p.bias, ks, bd);
+                                                                          (const uint16_t *)p.bias, ks, bd, bt);
         return hipGetLastError();
     }
     const int vec4 = p.dtype == DT_F32 && c_rs % 4 == 0 && ((uintptr_t)p.c & 15u) == 0 && ws_ld % 4 == 0 && ws_split_stride % 4 == 0 &&
@@ -225,16 +245,16 @@ hipError_t launch_splitk_reduce(const GemmProblem &p, int64_t ws_ld, int64_t ws_
     switch (p.dtype) {
     case DT_F32:
         splitk_reduce_kernel<float><<<grid, block, 0, stream>>>(p.workspace, p.splits, ws_ld, ws_split_stride, (float *)p.c, c_rs,
-                                                                 (int)p.m, (int)p.n, p.accumulate, bias_mode, (const float *)p.bias, vec4, ks, bd);
+                                                                 (int)p.m, (int)p.n, p.accumulate, bias_mode, (const float *)p.bias, vec4, ks, bd, bt);
         break;
     case DT_F16:
         splitk_reduce_kernel<_Float16><<<grid, block, 0, stream>>>(p.workspace, p.splits, ws_ld, ws_split_stride, (_Float16 *)p.c,
                                                                     c_rs, (int)p.m, (int)p.n, p.accumulate, bias_mode,
-                                                                    (const _Float16 *)p.bias, 0, ks, bd);
+                                                                    (const _Float16 *)p.bias, 0, ks, bd, bt);
         break;
     case DT_BF16:
         splitk_reduce_kernel<__bf16><<<grid, block, 0, stream>>>(p.workspace, p.splits, ws_ld, ws_split_stride, (__bf16 *)p.c, c_rs,
-                                                                  (int)p.m, (int)p.n, p.accumulate, bias_mode, (const __bf16 *)p.bias, 0, ks, bd);
+                                                                  (int)p.m, (int)p.n, p.accumulate, bias_mode, (const __bf16 *)p.bias, 0, ks, bd, bt);
         break;
     default: return hipErrorInvalidValue;
     }

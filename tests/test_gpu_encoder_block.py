@@ -81,3 +81,32 @@ def test_block_equals_its_ops(dtype, B, S, d, H, ff):
         elif n != "bk":   # a shift of all scores of a row: its gradient is the rounding of zero
             assert np.linalg.norm(a - b) <= tol * np.linalg.norm(b), (n, np.linalg.norm(a - b) / np.linalg.norm(b))
     assert saved["f1"].shape == (B, S, ff) and saved["probs"].shape == (B, H, S, S) and saved["tokens"].shape == (B, H, S, d // H)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("B,S,d,H", [(2, 64, 256, 4), (16, 128, 512, 8), (3, 100, 256, 4)])
+def test_block_does_not_depend_on_where_its_parameters_lie(dtype, B, S, d, H):
+    """The three projections run as one launch that walks from one matrix to the next by their distance: the same bits with
+    the parameters in one buffer in reverse order (negative distances, gaps) as with each in its own."""
+    dev, g, ff = device(), rng(d + S), 2 * d
+    shapes = {n: (d, d) for n in ("wq", "wk", "wv", "wo")} | {"w1": (ff, d), "w2": (d, ff), "b1": (ff,)}
+    host = {n: oracle.to_storage((g.standard_normal(int(np.prod(shapes.get(n, (d,))))) * 0.05 + (n in ("g1", "g2"))).astype(np.float32), dtype) for n in PARAMS}
+    own = {n: dev.tensor(host[n], dtype, shapes.get(n, (d,))) for n in PARAMS}
+    order, at, pos = list(PARAMS)[::-1], {}, 0
+    for i, n in enumerate(order):
+        at[n] = pos
+        pos += host[n].size + 8 * (i % 3)
+    flat = np.zeros(pos, dtype=host["wq"].dtype)
+    for n in order:
+        flat[at[n]:at[n] + host[n].size] = host[n]
+    arena = dev.tensor(flat, dtype)
+    one = {n: View(arena.storage[2 * at[n]:2 * (at[n] + host[n].size)], dtype, own[n].shape, own[n].strides) for n in PARAMS}
+    x, go = (dev.tensor(oracle.to_storage(g.standard_normal(B * S * d).astype(np.float32), dtype), dtype, (B, S, d)) for _ in range(2))
+    results = []
+    for p in (own, one):
+        block = EncoderBlock(dev, dtype, d, H, ff, p)
+        out, saved = block.forward(x)
+        grads, gx = block.backward(saved, go)
+        results.append([dev.to_host(t) for t in (out, gx, *(grads[n] for n in PARAMS))])
+    for a, b in zip(*results):
+        assert np.array_equal(a.view(np.uint16), b.view(np.uint16))
