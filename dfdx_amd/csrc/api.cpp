@@ -605,6 +605,60 @@ int gemm_beyond(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int extra, 
     }
 }
 
+int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_rocm_gemm_desc *second, const void *grad_out, int64_t rows, int64_t cols,
+              void *colsum, bool *fused) {
+    auto apart = [&]() -> int {
+        if (int e = dfdx_rocm_gemm(ctx, first)) return e;
+        return fused ? gemm_with_colsum(ctx, second, colsum, fused) : dfdx_rocm_gemm(ctx, second);
+    };
+    if (fused) *fused = false;
+    // (a copy of less than 4 MB costs little more than its launch)
+    const bool off = cols % 64 || rows % 64 || ((uintptr_t)grad_out & 15u);
+    if ((first->dtype != DFDX_ROCM_F16 && first->dtype != DFDX_ROCM_BF16) || !off || (double)rows * (double)cols < 2097152.0) return apart();
+    if (int e = bind(ctx)) return e;
+    GemmProblem p[2];
+    Plan plan[2];
+    Realign ra;
+    bool both = true;
+    for (int i = 0; i < 2; i++) {
+        const dfdx_rocm_gemm_desc *d = i ? second : first;
+        if (int e = make_problem(d, &p[i])) return e;
+        if (p[i].m == 0) return apart();
+        if (int e = make_plan(ctx, d, p[i], &plan[i])) return e;
+        both = both && plan[i].realign && p[i].a != p[i].b && plan_realign(p[i], &ra) && (p[i].a == grad_out ? ra.a : ra.b);
+    }
+    CtxLock lock(ctx->mu);  // the copy lives in the patch buffer until the second product has been launched
+    int64_t ld = 0;
+    const size_t bytes = realign_shared_bytes(rows, cols, &ld);
+    if (!both || bytes == 0) return apart();
+    if (bytes > ctx->patches_bytes) {
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess) (void)hipGetLastError();
+        if (capturing != hipStreamCaptureStatusNone || ensure_patches(ctx, bytes) != DFDX_ROCM_OK) return apart();
+    }
+    for (int i = 0; i < 2; i++) {  // with everything reserved, nothing below turns to another plan
+        if (int e = reserve_partials(ctx, p[i], plan[i], false)) return e;
+        if (!plan[i].realign) return apart();
+    }
+    if (int e = settle(ctx, grad_out)) return e;
+    HIP_TRY(launch_realign_shared(grad_out, rows, cols, ctx->patches, ctx->stream));
+    for (int i = 0; i < 2; i++) {
+        GemmProblem &q = p[i];
+        if (q.a == grad_out) {
+            (q.a_rs == 1 ? q.a_cs : q.a_rs) = ld;
+            q.a = ctx->patches;
+            q.a_laid = true;
+        } else {
+            (q.b_cs == 1 ? q.b_rs : q.b_cs) = ld;
+            q.b = ctx->patches;
+            q.b_laid = true;
+        }
+        if (int e = settle_operands(ctx, &q, /*may_overwrite=*/true)) return e;
+        if (int e = run_plan(ctx, q, plan[i])) return e;
+    }
+    return DFDX_ROCM_OK;
+}
+
 int gemm_three(dfdx_rocm_ctx *ctx, const GemmProblem &problem, bool *done) {
     *done = false;
     GemmProblem p = problem;

@@ -51,6 +51,7 @@ struct GemmProblem {
     // Operands laid out by launch_realign: an operand whose rows lie along memory is readable up to the next multiple of eight
     // of them, and C may lie anywhere.
     bool ragged = false;
+    bool a_laid = false, b_laid = false;  // that operand is a copy of launch_realign_shared already
     // split-k (filled in by the planner): `splits` workgroups share one C tile; f32 partials go to `workspace`
     int splits;
     float *workspace;
@@ -90,6 +91,7 @@ static inline GemmProblem transposed(const GemmProblem &p) {
     t.c_rs = p.c_cs; t.c_cs = p.c_rs;
     if (p.bias_mode == BIAS_PER_COL) t.bias_mode = BIAS_PER_ROW;
     else if (p.bias_mode == BIAS_PER_ROW) t.bias_mode = BIAS_PER_COL;
+    t.a_laid = p.b_laid; t.b_laid = p.a_laid;
     if (p.ksum_of == KSUM_OF_A) t.ksum_of = KSUM_OF_B;
     else if (p.ksum_of == KSUM_OF_B) t.ksum_of = KSUM_OF_A;
     return t;
@@ -140,6 +142,10 @@ struct Realign {
 };
 bool plan_realign(const GemmProblem &p, Realign *r);  // false where a copy does not help (strides, sizes)
 hipError_t launch_realign(const GemmProblem &p, Realign *r, void *space, hipStream_t stream);  // copies and fills in the addresses
+// One rows x cols matrix (rows of `cols` elements, one behind the other) as an operand of either orientation: rows and columns
+// padded with zeros to multiples of 64.
+size_t realign_shared_bytes(int64_t rows, int64_t cols, int64_t *ld);
+hipError_t launch_realign_shared(const void *src, int64_t rows, int64_t cols, void *dst, hipStream_t stream);
 // Split-k planning for the LDS-DMA kernels: picks tile variant and split count together.  `forced_splits`
 // > 0 overrides the count (clamped to what the k extent allows).  `seconds` (may be null) receives the estimate.
 void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_variant, int forced_splits, int *variant,

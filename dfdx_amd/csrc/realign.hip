@@ -66,7 +66,7 @@ struct Operand {
     int64_t pieces() const { return n1 * n2 * lines_out * (ld_out / 8); }
 };
 // False where no stride is 1 or the copy would be out of range.
-bool operand(const void *ptr, int64_t rows, int64_t k, int64_t row_stride, int64_t k_stride, int64_t b1, int64_t b2, int64_t nb1, int64_t nb2, Operand *o) {
+bool operand(const void *ptr, int64_t rows, int64_t k, int64_t row_stride, int64_t k_stride, int64_t b1, int64_t b2, int64_t nb1, int64_t nb2, bool laid, Operand *o) {
     const int64_t kp = up(k, 64);
     if (b1 < 0 || b2 < 0 || row_stride < 0 || k_stride < 0) return false;
     if (k_stride == 1 && (rows == 1 || row_stride >= k)) {
@@ -89,6 +89,7 @@ bool operand(const void *ptr, int64_t rows, int64_t k, int64_t row_stride, int64
     o->n2 = b2 == 0 ? 1 : nb2;
     o->off = o->src_ld % 8 != 0 || (!o->kc && rows % 8 != 0) || ((uintptr_t)ptr & 15u) != 0 || (o->n1 > 1 && b1 % 8 != 0) || (o->n2 > 1 && b2 % 8 != 0);
     o->copy = o->off || kp != k;
+    if (laid) o->off = o->copy = false;
     return !o->copy || (o->pieces() < (1ll << 31) && o->lines_out < (1ll << 31) && o->ld_out < (1ll << 31));
 }
 void describe(const Operand &o, const void *src, void *dst, int64_t b1, int64_t b2, Side *s) {
@@ -118,8 +119,8 @@ void strides(const Operand &o, int64_t *row_stride, int64_t *k_stride, int64_t *
 bool plan_realign(const GemmProblem &p, Realign *r) {
     if ((p.dtype != DT_F16 && p.dtype != DT_BF16) || p.k < 1 || p.extra != EXTRA_NONE) return false;
     Operand a, b;
-    if (!operand(p.a, p.m, p.k, p.a_rs, p.a_cs, p.a_b1, p.a_b2, p.nb1, p.nb2, &a)) return false;
-    if (!operand(p.b, p.n, p.k, p.b_cs, p.b_rs, p.b_b1, p.b_b2, p.nb1, p.nb2, &b)) return false;
+    if (!operand(p.a, p.m, p.k, p.a_rs, p.a_cs, p.a_b1, p.a_b2, p.nb1, p.nb2, p.a_laid, &a)) return false;
+    if (!operand(p.b, p.n, p.k, p.b_cs, p.b_rs, p.b_b1, p.b_b2, p.nb1, p.nb2, p.b_laid, &b)) return false;
     r->a = a.copy;
     r->b = b.copy;
     r->problem = p;
@@ -147,10 +148,33 @@ bool plan_realign(const GemmProblem &p, Realign *r) {
     return true;
 }
 
+size_t realign_shared_bytes(int64_t rows, int64_t cols, int64_t *ld) {
+    *ld = up(cols, 64);
+    const int64_t pieces = up(rows, 64) * (*ld / 8);
+    return pieces < (1ll << 31) ? (size_t)pieces * 16 : 0;
+}
+
+hipError_t launch_realign_shared(const void *src, int64_t rows, int64_t cols, void *dst, hipStream_t stream) {
+    Sides both{};
+    Side &s = both.s[0];
+    s.src = (const uint16_t *)src;
+    s.dst = (uint16_t *)dst;
+    s.ld = cols;
+    s.rows = (uint32_t)rows;
+    s.cols = (uint32_t)cols;
+    s.rows_out = (uint32_t)up(rows, 64);
+    s.pieces = (uint32_t)(up(cols, 64) / 8);
+    s.n2 = 1;
+    s.total = s.rows_out * s.pieces;
+    both.first_blocks = (s.total + PER_BLOCK - 1) / PER_BLOCK;
+    realign_kernel<<<dim3(both.first_blocks), dim3(256), 0, stream>>>(both);
+    return hipGetLastError();
+}
+
 hipError_t launch_realign(const GemmProblem &p, Realign *r, void *space, hipStream_t stream) {
     Operand a, b;
-    if (!operand(p.a, p.m, p.k, p.a_rs, p.a_cs, p.a_b1, p.a_b2, p.nb1, p.nb2, &a) ||
-        !operand(p.b, p.n, p.k, p.b_cs, p.b_rs, p.b_b1, p.b_b2, p.nb1, p.nb2, &b) || a.copy != r->a || b.copy != r->b)
+    if (!operand(p.a, p.m, p.k, p.a_rs, p.a_cs, p.a_b1, p.a_b2, p.nb1, p.nb2, p.a_laid, &a) ||
+        !operand(p.b, p.n, p.k, p.b_cs, p.b_rs, p.b_b1, p.b_b2, p.nb1, p.nb2, p.b_laid, &b) || a.copy != r->a || b.copy != r->b)
         return hipErrorInvalidValue;
     Sides both{};
     describe(a, p.a, space, p.a_b1, p.a_b2, &both.s[0]);

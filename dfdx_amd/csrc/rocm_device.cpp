@@ -53,14 +53,14 @@ int dfdx_rocm_matmat_backward(dfdx_rocm_ctx *ctx, int dtype, int64_t m, int64_t 
     d.a = grad_out; d.a_rs = n; d.a_cs = 1;
     d.b = rhs; d.b_rs = rs[1]; d.b_cs = rs[0];
     d.c = grad_lhs; d.c_rs = ls[0]; d.c_cs = ls[1];
-    if (int e = dfdx_rocm_gemm(ctx, &d)) return e;
+    const dfdx_rocm_gemm_desc left = d;
     // grad_rhs (k,n) += lhs^T (k,m) . grad_out (m,n)
     d = blank(dtype, k, m, n);
     d.accumulate = 1;
     d.a = lhs; d.a_rs = ls[1]; d.a_cs = ls[0];
     d.b = grad_out; d.b_rs = n; d.b_cs = 1;
     d.c = grad_rhs; d.c_rs = rs[0]; d.c_cs = rs[1];
-    return dfdx_rocm_gemm(ctx, &d);
+    return dfdx_rocm::gemm_pair(ctx, &left, &d, grad_out, m, n, nullptr, nullptr);
 }
 
 // MatMatBrKernel::forward (cpu_kernel.rs:294-316): (B,M,K) x (K,N).
@@ -104,7 +104,9 @@ int dfdx_rocm_matmat_br_backward(dfdx_rocm_ctx *ctx, int dtype, int64_t batch, i
         d.a_b1 = m * n;
         d.c_b1 = ls[0];
     }
-    if (int e = dfdx_rocm_gemm(ctx, &d)) return e;
+    const dfdx_rocm_gemm_desc left = d;
+    if (!fold)
+        if (int e = dfdx_rocm_gemm(ctx, &d)) return e;
     // grad_rhs (k,n) += sum_i lhs[i]^T (k,m) . grad_out[i] (m,n): the batch extends the contraction
     if (fold) {
         d = blank(dtype, k, batch * m, n);
@@ -119,7 +121,7 @@ int dfdx_rocm_matmat_br_backward(dfdx_rocm_ctx *ctx, int dtype, int64_t batch, i
     d.a = lhs; d.a_rs = ls[2]; d.a_cs = ls[1];
     d.b = grad_out; d.b_rs = n; d.b_cs = 1;
     d.c = grad_rhs; d.c_rs = rs[0]; d.c_cs = rs[1];
-    return dfdx_rocm_gemm(ctx, &d);
+    return fold ? dfdx_rocm::gemm_pair(ctx, &left, &d, grad_out, batch * m, n, nullptr, nullptr) : dfdx_rocm_gemm(ctx, &d);
 }
 
 // MatMatBatch3Kernel::forward (cpu_kernel.rs:358-382): (B,M,K) x (B,K,N).
@@ -227,14 +229,14 @@ int dfdx_rocm_linear_backward(dfdx_rocm_ctx *ctx, int dtype, int64_t rows, int64
     d.a = grad_out; d.a_rs = out_dim; d.a_cs = 1;
     d.b = weight; d.b_rs = ws[1]; d.b_cs = ws[0];
     d.c = grad_x; d.c_rs = xs[0]; d.c_cs = xs[1];
-    if (int e = dfdx_rocm_gemm(ctx, &d)) return e;
+    const dfdx_rocm_gemm_desc left = d;
     d = blank(dtype, in_dim, rows, out_dim);
     d.accumulate = 1;
     d.a = x; d.a_rs = xs[1]; d.a_cs = xs[0];
     d.b = grad_out; d.b_rs = out_dim; d.b_cs = 1;
     d.c = grad_weight; d.c_rs = ws[0]; d.c_cs = ws[1];
     bool fused = false;
-    if (int e = dfdx_rocm::gemm_with_colsum(ctx, &d, grad_bias, &fused)) return e;
+    if (int e = dfdx_rocm::gemm_pair(ctx, &left, &d, grad_out, rows, out_dim, grad_bias, &fused)) return e;
     return fused ? DFDX_ROCM_OK : dfdx_rocm_bias_backward(ctx, dtype, rows, out_dim, grad_out, grad_bias);
 }
 

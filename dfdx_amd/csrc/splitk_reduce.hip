@@ -72,6 +72,7 @@ struct Batches {
     int64_t c_b1, c_b2, k_b1, k_b2;
 };
 template <typename T> __device__ __forceinline__ void to_batch(const Batches &bt, const float *&ws, int64_t ws_split_stride, T *&c, KsumParts &ks, Beyond &bd) {
+    if (gridDim.z == 1) return;
     const int z = blockIdx.z, z1 = z / bt.nb2, z2 = z - z1 * bt.nb2;
     const int64_t off = z1 * bt.c_b1 + z2 * bt.c_b2;
     ws += (int64_t)z * bt.splits * ws_split_stride;

@@ -87,3 +87,33 @@ def test_bias_gradient_of_odd_rows(dtype, rows, cols):
     want = g.double().sum(0) + old.double()
     bound = want.abs() * 2.0 ** (-11 if dtype == "f16" else -8) + (g.double().abs().sum(0) + old.double().abs()) * rows * 2.0 ** -24 + 1e-7
     assert bool(((gb.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("rows,inp,out", [(2048, 1024, 3001), (2113, 1024, 2112), (1500, 1111, 3333)])
+def test_backward_products_share_one_copy_of_grad_out(dtype, rows, inp, out):
+    """Both products of a backward call read grad_out; off the grid it is copied once for both, in Linear, the plain product and the
+    broadcast one.  Against the two products as single calls, each with its own copies: the same kernels, the same bits."""
+    dev = device()
+    t = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    view = lambda t_: View(t_.view(torch.uint8).reshape(-1), dtype, tuple(t_.shape), tuple(t_.stride()))
+    rnd = lambda *s: torch.randn(*s, device="cuda").to(t)
+    x, w, b, g = rnd(rows, inp), rnd(out, inp) / 32, rnd(out), rnd(rows, out)
+    wt = view(w).permute(1, 0)
+    flat = lambda v: v.storage.view(t)
+    gx, gw = torch.zeros_like(x), torch.zeros_like(w)
+    for d in (dev.gemm_desc(dtype, rows, out, inp, g.data_ptr(), (out, 1), w.data_ptr(), (inp, 1), gx.data_ptr(), (inp, 1), accumulate=True),
+              dev.gemm_desc(dtype, inp, rows, out, x.data_ptr(), (1, inp), g.data_ptr(), (out, 1), gw.data_ptr(), (1, inp), accumulate=True)):
+        announce("shared copy", dtype, rows, inp, out, dev.gemm_plan(d)[2])
+        dev.gemm(d)
+    for fresh in (True, False):
+        ox, ow, ob = view(torch.zeros_like(x)), view(torch.zeros_like(w)), view(torch.zeros_like(b))
+        if fresh:
+            ox, ow, ob = dev.zeros_many([view(x), view(w), view(b)], deferred=True)
+        dev.linear_backward(view(x), ox, view(w), ow, ob, view(g))
+        dev.settle_zeros()
+        assert torch.equal(flat(ox), gx.view(-1)) and torch.equal(flat(ow), gw.view(-1))
+        assert torch.allclose(flat(ob).double(), g.double().sum(0), rtol=2.0 ** -7 if dtype == "bf16" else 2.0 ** -10, atol=1e-2)
+        px, pw = view(torch.zeros_like(x)), view(torch.zeros_like(w)).permute(1, 0)
+        dev.backward(view(x), px, wt, pw, view(g))
+        assert torch.equal(flat(px), gx.view(-1)) and torch.equal(pw.storage.view(t), gw.view(-1))
