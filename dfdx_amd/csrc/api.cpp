@@ -631,17 +631,29 @@ int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_r
     int64_t ld = 0;
     const size_t bytes = realign_shared_bytes(rows, cols, &ld);
     if (!both || bytes == 0) return apart();
-    if (bytes > ctx->patches_bytes) {
+    const size_t sums_bytes = fused && colsum ? bias_backward_copy_partials(ctx->compute_units, rows, cols, ld) : 0;
+    bool sums = sums_bytes > 0;
+    if (bytes > ctx->patches_bytes || sums_bytes > ctx->workspace_bytes) {
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess) (void)hipGetLastError();
-        if (capturing != hipStreamCaptureStatusNone || ensure_patches(ctx, bytes) != DFDX_ROCM_OK) return apart();
+        const bool may_grow = capturing == hipStreamCaptureStatusNone;
+        if (bytes > ctx->patches_bytes && (!may_grow || ensure_patches(ctx, bytes) != DFDX_ROCM_OK)) return apart();
+        if (sums_bytes > ctx->workspace_bytes) sums = may_grow && ensure_workspace(ctx, sums_bytes) == DFDX_ROCM_OK;
     }
     for (int i = 0; i < 2; i++) {  // with everything reserved, nothing below turns to another plan
         if (int e = reserve_partials(ctx, p[i], plan[i], false)) return e;
         if (!plan[i].realign) return apart();
     }
     if (int e = settle(ctx, grad_out)) return e;
-    HIP_TRY(launch_realign_shared(grad_out, rows, cols, ctx->patches, ctx->stream));
+    if (sums) {  // on the way into the copy; their partials are done with the workspace before the products write it
+        bool fresh = false;
+        if (int e = settle_output(ctx, colsum, (size_t)cols * dtype_size(first->dtype), true, &fresh)) return e;
+        HIP_TRY(launch_bias_backward_copy(first->dtype, ctx->compute_units, rows, cols, grad_out, ctx->patches, ld, (rows + 63) / 64 * 64, colsum, fresh,
+                                          (float *)ctx->workspace, ctx->stream));
+        *fused = true;
+    } else {
+        HIP_TRY(launch_realign_shared(grad_out, rows, cols, ctx->patches, ctx->stream));
+    }
     for (int i = 0; i < 2; i++) {
         GemmProblem &q = p[i];
         if (q.a == grad_out) {

@@ -3,6 +3,7 @@
 // the forward one write) of the matrix.
 #include "ctx_internal.h"
 #include "elem.h"
+#include "gemm_internal.h"
 
 namespace dfdx_rocm {
 namespace {
@@ -104,6 +105,72 @@ __global__ __launch_bounds__(64) void bias_backward_combine_kernel(const float *
     Elem<T>::store(grad_bias + c, (fresh ? 0.0f : Elem<T>::load(grad_bias + c)) + s);
 }
 
+// ---- backward of rows off the 16-byte grid that the products behind it read as a padded copy ---------------------
+// The same strips, slices and sums as bias_backward_kernel, on the way from grad_out to the copy (`ld` elements per row, rows up to
+// `rows_out`, zeros where grad_out has nothing): grad_out is read once instead of twice.  Bound by HBM, one read and one write.
+// Linear 2048 x 1024 x 50257 f16, forward and backward: 847 -> 804 us (a copy of 75 us and sums of 54 + 5 us behind each other before).
+template <typename T>
+__global__ __launch_bounds__(256) void bias_backward_copy_kernel(const T *go, int rows, int cols, int rows_per_slice, uint16_t *copy, int ld, int rows_out,
+                                                                 float *partial, T *grad_bias, bool fresh) {
+    constexpr int N = 8, LPR = 16, RL = 256 / LPR;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    typedef u32x4 u32x4_any __attribute__((aligned(2)));
+    __shared__ float red[RL][LPR * N + 1];
+    const int c_lane = threadIdx.x % LPR, r_lane = threadIdx.x / LPR;
+    const int col = (blockIdx.x * LPR + c_lane) * N;
+    const int r0 = blockIdx.y * rows_per_slice, r1 = min(rows, r0 + rows_per_slice);
+    float acc[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) acc[i] = 0.0f;
+    auto load = [&](int r) -> u32x4 {
+        const uint16_t *p = (const uint16_t *)go + (int64_t)r * cols + col;
+        if (col + N <= cols) return *(const u32x4_any *)p;
+        u32x4 v = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int i = 0; i < N - 1; i++)
+            if (col + i < cols) v[i / 2] |= (uint32_t)p[i] << (i % 2 * 16);
+        return v;
+    };
+    auto store = [&](int r, u32x4 v) { *(u32x4 *)(copy + (int64_t)r * ld + col) = v; };
+    auto value = [&](const u32x4 &v, int i) -> float {
+        const uint16_t bits = (uint16_t)(v[i / 2] >> (i % 2 * 16));
+        return Elem<T>::load((const T *)&bits);
+    };
+    if (col < ld) {  // (ld % 8 == 0)
+        int r = r0 + r_lane;
+        for (; r + 3 * RL < r1; r += 4 * RL) {  // four independent loads in flight
+            const u32x4 v0 = load(r), v1 = load(r + RL), v2 = load(r + 2 * RL), v3 = load(r + 3 * RL);
+            store(r, v0);
+            store(r + RL, v1);
+            store(r + 2 * RL, v2);
+            store(r + 3 * RL, v3);
+#pragma unroll
+            for (int i = 0; i < N; i++) acc[i] += (value(v0, i) + value(v1, i)) + (value(v2, i) + value(v3, i));
+        }
+        for (; r < r1; r += RL) {
+            const u32x4 v = load(r);
+            store(r, v);
+#pragma unroll
+            for (int i = 0; i < N; i++) acc[i] += value(v, i);
+        }
+        if (blockIdx.y == gridDim.y - 1)
+            for (r = rows + r_lane; r < rows_out; r += RL) store(r, u32x4{0u, 0u, 0u, 0u});
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) red[r_lane][c_lane * N + i] = acc[i];
+    __syncthreads();
+    if (threadIdx.x < LPR * N) {
+        const int c = blockIdx.x * LPR * N + threadIdx.x;
+        if (c < cols) {
+            float s = 0.0f;
+#pragma unroll
+            for (int j = 0; j < RL; j++) s += red[j][threadIdx.x];
+            if (partial) partial[(int64_t)blockIdx.y * cols + c] = s;
+            else Elem<T>::store(grad_bias + c, (fresh ? 0.0f : Elem<T>::load(grad_bias + c)) + s);
+        }
+    }
+}
+
 // ---- f64 (the reference runs its whole test suite in f64 as well): plain kernels, f64 arithmetic -----------------
 __global__ __launch_bounds__(256) void bias_forward_f64_kernel(const double *x, const double *bias, double *out, int64_t total, int64_t cols) {
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) out[i] = x[i] + bias[i % cols];
@@ -170,10 +237,41 @@ int bias_backward_t(dfdx_rocm_ctx *ctx, int64_t rows, int64_t cols, const void *
     return DFDX_ROCM_OK;
 }
 
+// Eight workgroups per compute unit, but at least four rows per lane group and slice.
+int64_t copy_rows_per_slice(int compute_units, int64_t rows, int64_t ld) {
+    const int64_t strips = (ld + 127) / 128;
+    const int64_t slices = std::max<int64_t>(1, std::min<int64_t>({(int64_t)compute_units * 8 / strips, rows / 64, 65535}));
+    return (rows + slices - 1) / slices;
+}
+
+template <typename T>
+hipError_t bias_backward_copy_t(int compute_units, int64_t rows, int64_t cols, const void *go, void *copy, int64_t ld, int64_t rows_out, void *gb, bool fresh,
+                                float *partial, hipStream_t stream) {
+    const int64_t per_slice = copy_rows_per_slice(compute_units, rows, ld), slices = (rows + per_slice - 1) / per_slice;
+    const dim3 grid((unsigned)((ld + 127) / 128), (unsigned)slices);
+    bias_backward_copy_kernel<T><<<grid, 256, 0, stream>>>((const T *)go, (int)rows, (int)cols, (int)per_slice, (uint16_t *)copy, (int)ld, (int)rows_out,
+                                                           slices > 1 ? partial : nullptr, (T *)gb, fresh);
+    if (const hipError_t e = hipGetLastError()) return e;
+    if (slices > 1) bias_backward_combine_kernel<T><<<(unsigned)((cols + 63) / 64), 64, 0, stream>>>(partial, (int)slices, (int)cols, (T *)gb, fresh);
+    return hipGetLastError();
+}
+
 size_t elem_bytes(int dtype) { return dtype == DFDX_ROCM_F64 ? 8 : dtype == DFDX_ROCM_F32 ? 4 : 2; }
 bool dims_ok(int64_t rows, int64_t cols) { return rows >= 0 && cols >= 0 && rows < (1ll << 31) && cols < (1ll << 31); }
 
 }  // namespace
+
+size_t bias_backward_copy_partials(int compute_units, int64_t rows, int64_t cols, int64_t ld) {
+    const int64_t per_slice = copy_rows_per_slice(compute_units, rows, ld);
+    return (size_t)((rows + per_slice - 1) / per_slice) * cols * sizeof(float);
+}
+
+hipError_t launch_bias_backward_copy(int dtype, int compute_units, int64_t rows, int64_t cols, const void *go, void *copy, int64_t ld, int64_t rows_out,
+                                     void *grad_bias, bool fresh, float *partial, hipStream_t stream) {
+    return dtype == DFDX_ROCM_BF16 ? bias_backward_copy_t<__bf16>(compute_units, rows, cols, go, copy, ld, rows_out, grad_bias, fresh, partial, stream)
+                                   : bias_backward_copy_t<_Float16>(compute_units, rows, cols, go, copy, ld, rows_out, grad_bias, fresh, partial, stream);
+}
+
 }  // namespace dfdx_rocm
 
 using namespace dfdx_rocm;

@@ -80,7 +80,7 @@ int gemm_with_colsum(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, void *
 int gemm_beyond(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int extra, const void *with);
 // The two products of a backward pass, both of which read grad_out (rows x cols, contiguous): as dfdx_rocm_gemm(first) and
 // dfdx_rocm_gemm(second) -- or gemm_with_colsum(second, colsum, fused) where `fused` is not null -- but a grad_out that both would
-// copy onto the 16-byte grid is copied once.
+// copy onto the 16-byte grid is copied once, with the column sums taken on the way.
 int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_rocm_gemm_desc *second, const void *grad_out, int64_t rows, int64_t cols,
               void *colsum, bool *fused);
 // Three products of the same shape in one launch (GemmProblem::batches = 3, or their sum: `reduce`), where the LDS-DMA kernels take

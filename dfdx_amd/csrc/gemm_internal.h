@@ -146,6 +146,11 @@ hipError_t launch_realign(const GemmProblem &p, Realign *r, void *space, hipStre
 // padded with zeros to multiples of 64.
 size_t realign_shared_bytes(int64_t rows, int64_t cols, int64_t *ld);
 hipError_t launch_realign_shared(const void *src, int64_t rows, int64_t cols, void *dst, hipStream_t stream);
+// The same copy with grad_bias[c] += sum of column c on the way (grad_bias stored where `fresh`); `partial` holds
+// bias_backward_copy_partials() bytes.
+size_t bias_backward_copy_partials(int compute_units, int64_t rows, int64_t cols, int64_t ld);
+hipError_t launch_bias_backward_copy(int dtype, int compute_units, int64_t rows, int64_t cols, const void *go, void *copy, int64_t ld, int64_t rows_out,
+                                     void *grad_bias, bool fresh, float *partial, hipStream_t stream);
 // Split-k planning for the LDS-DMA kernels: picks tile variant and split count together.  `forced_splits`
 // > 0 overrides the count (clamped to what the k extent allows).  `seconds` (may be null) receives the estimate.
 void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_variant, int forced_splits, int *variant,

@@ -117,3 +117,25 @@ def test_backward_products_share_one_copy_of_grad_out(dtype, rows, inp, out):
         px, pw = view(torch.zeros_like(x)), view(torch.zeros_like(w)).permute(1, 0)
         dev.backward(view(x), px, wt, pw, view(g))
         assert torch.equal(flat(px), gx.view(-1)) and torch.equal(pw.storage.view(t), gw.view(-1))
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("rows,inp,out", [(2048, 1024, 3001), (2113, 1024, 2112), (1537, 1024, 1367), (513, 1024, 50257)])
+def test_bias_gradient_taken_on_the_way_into_the_copy(dtype, rows, inp, out):
+    """Column sums that ride on the copy of grad_out, added to an old gradient and stored into a fresh one, at ragged rows, ragged
+    columns and both; f32 sums, one rounding: half an ulp of the result and rows * 2^-24 of the sum of magnitudes."""
+    dev = device()
+    t = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    view = lambda t_: View(t_.view(torch.uint8).reshape(-1), dtype, tuple(t_.shape), tuple(t_.stride()))
+    rnd = lambda *s: torch.randn(*s, device="cuda").to(t)
+    x, w, old, g = rnd(rows, inp), rnd(out, inp) / 32, rnd(out), rnd(rows, out)
+    for start in (old, None):
+        ox, ow, ob = dev.zeros_many([view(x), view(w), view(old)], deferred=True)
+        if start is not None:
+            ob = view(old.clone())
+        dev.linear_backward(view(x), ox, view(w), ow, ob, view(g))
+        dev.settle_zeros()
+        before = old.double() if start is not None else torch.zeros_like(old).double()
+        want = g.double().sum(0) + before
+        bound = want.abs() * 2.0 ** (-11 if dtype == "f16" else -8) + (g.double().abs().sum(0) + before.abs()) * rows * 2.0 ** -24 + 1e-7
+        assert bool(((ob.storage.view(t).double() - want).abs() <= bound).all())
