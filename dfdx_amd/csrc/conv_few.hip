@@ -24,6 +24,7 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 template <typename T> struct Mma;
@@ -195,7 +196,9 @@ __global__ __launch_bounds__(256, 3) void conv_few_forward_kernel(const Params p
 // its columns, 32 output channels one step; every position of grad_out that any pixel of a cell reads -- WIN x WIN of them, 4 x 4
 // for 7 x 7 filters at stride 2 -- is one product with its own filter matrix (zero where a pixel has no tap there).  grad_out is
 // transposed on its way into LDS, [pixel][32 channels], so that a lane's operand is 16 bytes at any shift of the window.  All sums in
-// f32, one rounding.  LDS reads bound it: one operand per product of 16 rows, 12 of them in use.
+// f32, one rounding.  No single unit bounds it: LDS and the vector ALU are each busy a third of the time (74 us at the size above)
+// and the phases between barriers -- transpose, products -- do not overlap inside a workgroup.  XORing slots and pieces of the LDS
+// tile against bank conflicts of the stores measured level (73.7 us).
 // A tile that holds an infinity or a NaN goes through plain sums instead: those zeros would spread it over its cell.
 template <int C, int K, int S> struct GradImg {
     static constexpr int PAD = K / 2, Q = 2 / S;                                // positions of grad_out per cell
@@ -268,10 +271,27 @@ __global__ __launch_bounds__(256, 2) void conv_few_grad_img_kernel(const Params 
             if (chunks > G::KEEP || item == (int)blockIdx.x) {
                 uint16_t *raw = (uint16_t *)go_lds;
                 uint32_t nf = 0;
-                for (int i = tid; i < 32 * C * KK; i += 256) {
-                    const uint16_t v = o0 + i / (C * KK) < p.chan_out ? p.filters[(int64_t)o0 * C * KK + i] : (uint16_t)0;
-                    nf |= not_finite<T>(v);
-                    raw[i] = v;
+                constexpr int PIECES = 32 * C * KK / 8;  // 16 bytes each, all of a thread's in flight: element by element the kernel took 88 us instead of 82
+                const int have = min(32, p.chan_out - o0) * C * KK;
+                const uint16_t *src = p.filters + (int64_t)o0 * C * KK;
+                u32x4 piece[(PIECES + 255) / 256];
+#pragma unroll
+                for (int n = 0; n < (PIECES + 255) / 256; n++) {
+                    const int i = (n * 256 + tid) * 8;
+                    piece[n] = u32x4{0u, 0u, 0u, 0u};
+                    if (i + 8 <= have) {
+                        piece[n] = *(const u32x4_any *)(src + i);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 7; e++)
+                            if (i + e < have) piece[n][e / 2] |= (uint32_t)src[i + e] << (e % 2 * 16);
+                    }
+                }
+#pragma unroll
+                for (int n = 0; n < (PIECES + 255) / 256; n++) {
+#pragma unroll
+                    for (int w = 0; w < 4; w++) nf |= not_finite<T>(piece[n][w]);
+                    if (n * 256 + tid < PIECES) *(u32x4 *)(raw + (n * 256 + tid) * 8) = piece[n];
                 }
                 bad_filters |= __syncthreads_or(nf != 0) != 0;
                 for (int e = tid; e < G::WIN * G::WIN * 256; e += 256) {  // words: [position][lane][channel pair]
@@ -310,19 +330,20 @@ __global__ __launch_bounds__(256, 2) void conv_few_grad_img_kernel(const Params 
             bad |= __syncthreads_or(nf != 0) != 0;
             if (ch + 1 < chunks) fetch(at, o0 + 32);
             else if (item + (int)gridDim.x < p.items) fetch(place(item + gridDim.x), 0);
-            const uint8_t *go_at[G::PER_WAVE];
+            // Fully unrolled with every address a constant away from one of the lane: tiles in different rows read the same operands
+            // one filter row apart, and the compiler keeps them (LDS reads 2.5 -> 1.8 million, 82 -> 74 us at 7 x 7, stride 2).
+            constexpr int TW = G::CELLS / 16;
+            const int row = wave * G::PER_WAVE / TW, tile0 = wave * G::PER_WAVE % TW;
+            const uint8_t *const go_at = go_lds + (G::Q * row * G::LINE + tile0 * 16 + l16) * 64 + lq * 16;
 #pragma unroll
-            for (int t = 0; t < G::PER_WAVE; t++) {
-                const int tile = wave * G::PER_WAVE + t, r = tile / (G::CELLS / 16), cx = tile % (G::CELLS / 16) * 16 + l16;
-                go_at[t] = go_lds + (G::Q * r * G::LINE + cx) * 64 + lq * 16;
-            }
             for (int u = 0; u < G::WIN; u++)
 #pragma unroll
                 for (int v = 0; v < G::WIN; v++) {
                     const u32x4 f = *(const u32x4 *)(f_lds + ((u * G::WIN + v) * 64 + lane) * 16);
-                    const int off = (u * G::LINE + (G::Q == 2 ? (v & 1) * G::HALF + (v >> 1) : v)) * 64;
+                    const int slot = G::Q == 2 ? (v & 1) * G::HALF + (v >> 1) : v;
 #pragma unroll
-                    for (int t = 0; t < G::PER_WAVE; t++) acc[t] = Mma<T>::mfma16(f, *(const u32x4 *)(go_at[t] + off), acc[t]);
+                    for (int t = 0; t < G::PER_WAVE; t++)
+                        acc[t] = Mma<T>::mfma16(f, *(const u32x4 *)(go_at + ((u + G::Q * (t / TW)) * G::LINE + slot + t % TW * 16) * 64), acc[t]);
                 }
         }
         // lane: channel lq of cell l16 of every tile, its four pixels in the accumulator
