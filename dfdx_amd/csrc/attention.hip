@@ -28,6 +28,7 @@
 #include "ctx_internal.h"
 #include "gemm_internal.h"
 #include <type_traits>
+#include <utility>
 
 namespace dfdx_rocm {
 namespace {
@@ -485,12 +486,29 @@ template <typename T, int D> __global__ __launch_bounds__(256, D == 128 ? 1 : 2)
 inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 // strides of (batch, head, row): what 16-byte pieces of a head's row can walk
 inline bool walkable(const int64_t s[3]) { return s[0] >= 0 && s[1] >= 0 && s[2] > 0 && s[0] % 8 == 0 && s[1] % 8 == 0 && s[2] % 8 == 0 && s[2] < (1ll << 31); }
+// What is written through these strides: two workgroups that share a row would store (or load, add and store) it without order.
+// Sorted by stride, every axis has to step past all that the shorter ones reach.
+bool rows_apart(int64_t batch, int64_t heads, int64_t seq, int64_t dim, const int64_t s[3]) {
+    int64_t ext[3] = {batch, heads, seq}, str[3] = {s[0], s[1], s[2]}, reach = dim;
+    for (int i = 0; i < 3; i++) {
+        int low = i;
+        for (int j = i + 1; j < 3; j++)
+            if (str[j] < str[low]) low = j;
+        std::swap(ext[i], ext[low]);
+        std::swap(str[i], str[low]);
+        if (ext[i] == 1) continue;
+        if (str[i] < reach) return false;
+        reach += (ext[i] - 1) * str[i];
+    }
+    return true;
+}
 
 }  // namespace
 
 bool attention_supported(int dtype, int64_t batch, int64_t heads, int64_t seq, int64_t dim) {
     return (dtype == DT_F16 || dtype == DT_BF16) && (dim == 32 || dim == 64 || dim == 128) && batch >= 1 && heads >= 1 && seq >= 1 &&
-           seq < (1ll << 30) && batch * heads * ((seq + ROWS - 1) / ROWS) < (1ll << 31);
+           seq < (1ll << 30) && batch < (1ll << 24) && heads < (1ll << 24) && batch * heads < (1ll << 24) &&
+           batch * heads * ((seq + ROWS - 1) / ROWS) < (1ll << 24);  // (workgroups of 256: a launch holds fewer than 2^32 threads)
 }
 
 namespace {
@@ -526,6 +544,7 @@ int dfdx_rocm_attention_forward(dfdx_rocm_ctx *ctx, int dtype, int64_t batch, in
     if (batch == 0 || heads == 0 || seq == 0) return DFDX_ROCM_OK;
     if (int e = fill(p, dtype, batch, heads, seq, dim, q, k, v, strides, scale, out_strides)) return e;
     if (!out || !aligned16(out)) return out ? DFDX_ROCM_ERR_UNSUPPORTED : DFDX_ROCM_ERR_INVALID_ARG;
+    if (!rows_apart(batch, heads, seq, dim, out_strides)) return DFDX_ROCM_ERR_ALIASED_OUTPUT;
     for (const void *ptr : {q, k, v})
         if (int e = settle(ctx, ptr)) return e;
     const int64_t ext[4] = {batch, heads, seq, dim}, str[4] = {out_strides[0], out_strides[1], out_strides[2], 1};
@@ -561,6 +580,7 @@ int dfdx_rocm_attention_backward(dfdx_rocm_ctx *ctx, int dtype, int64_t batch, i
     if (!out || !grad_out || !lse || !grad_q || !grad_k || !grad_v) return DFDX_ROCM_ERR_INVALID_ARG;
     for (const void *ptr : {out, grad_out, (const void *)grad_q, (const void *)grad_k, (const void *)grad_v})
         if (!aligned16(ptr)) return DFDX_ROCM_ERR_UNSUPPORTED;
+    if (!rows_apart(batch, heads, seq, dim, strides)) return DFDX_ROCM_ERR_ALIASED_OUTPUT;  // the gradients have the inputs' strides
     CtxLock lock(ctx->mu);  // delta lives in the shared workspace between the two launches
     if (int e = ensure_workspace(ctx, (size_t)(batch * heads * seq) * sizeof(float))) return e;
     for (const void *ptr : {q, k, v, out, grad_out, (const void *)lse})

@@ -32,7 +32,7 @@ NP_DTYPES = {"f32": np.float32, "f16": np.float16, "bf16": np.uint16, "f64": np.
 KERNEL_AUTO, KERNEL_GENERIC, KERNEL_MFMA, KERNEL_GEMV = 0, 1, 2, 3
 ZERO_DEFERRED = 2   # dfdx_rocm_alloc: zero as far as the library can tell, fill only if needed
 NOALLOC_SCRATCH_BYTES = 32 << 20   # DFDX_ROCM_NOALLOC_SCRATCH_BYTES
-ERR_SCRATCH_TOO_SMALL = -5
+ERR_ALIASED_OUTPUT, ERR_SCRATCH_TOO_SMALL = -4, -5
 
 
 class RocmError(RuntimeError):
@@ -624,7 +624,16 @@ class Rocm:
 
     def attention_backward(self, q: View, grad_q: View, k: View, grad_k: View, v: View, grad_v: View, scale: float, out: View,
                            grad_out: View, lse: View):
+        """Gradients of ``attention_forward``: added into grad_q, grad_k, grad_v, each laid out like the storage of q, k, v (one
+        set of strides, no broadcast axis); out, lse: what the forward returned; grad_out: like out."""
         B, H, S, D = q.shape
+        assert k.shape == q.shape and v.shape == q.shape and k.strides == q.strides and v.strides == q.strides and q.strides[3] == 1
+        tokens = (B, S, H * D)
+        assert out.shape == tokens and grad_out.shape == tokens and out.strides == grad_out.strides == _row_major(tokens), \
+            f"left: {out.shape}, {grad_out.shape}\n right: {tokens}"
+        assert lse.shape == (B, H, S) and lse.dtype == "f32" and all(t.dtype == q.dtype for t in (grad_q, k, grad_k, v, grad_v, out, grad_out))
+        reach = 1 + sum((n - 1) * s for n, s in zip(q.shape, q.strides)) if B * H * S else 0
+        assert all(t.numel_storage() - t.offset >= reach for t in (grad_q, grad_k, grad_v)), "gradients smaller than what their strides reach"
         self._check(self._f.attention_backward(self.ctx, DTYPES[q.dtype], B, H, S, D, q.ptr, k.ptr, v.ptr, _i64s(q.strides[:3]), scale,
                                                out.ptr, grad_out.ptr, _i64s((S * H * D, D, H * D)), lse.ptr, grad_q.ptr, grad_k.ptr, grad_v.ptr))
 

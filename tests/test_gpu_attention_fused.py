@@ -65,3 +65,61 @@ def test_fused_attention_refuses_what_it_does_not_take():
         with pytest.raises(RocmError):
             dev.attention_forward(x, x, x, 0.125)
         assert not dev.attention_supported(dtype, D)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("strides", [(0, 64, 128), (8192, 0, 128), (8192, 64, 56), (8192, 32, 128)],
+                         ids=["one batch for all", "one head for all", "rows shorter than a head", "heads inside each other"])
+def test_gradients_that_would_share_rows_are_refused(dtype, strides):
+    """Views of q, k, v whose rows overlap are read by the forward (the same as on copies of them); their gradients would be
+    added by several workgroups without order, and are refused with nothing written."""
+    from dfdx_amd import RocmError
+    from dfdx_amd.rocm import ERR_ALIASED_OUTPUT
+
+    dev = device()
+    B, H, S, D = 2, 2, 64, 64
+    announce("attention, aliased", dtype, strides)
+    g = rng(5)
+    size = 1 + sum((n - 1) * s for n, s in zip((B, H, S, D), (*strides, 1)))
+    st = [oracle.to_storage(g.standard_normal(size), dtype) for _ in range(3)]
+    q, k, v = (dev.tensor(t, dtype, (B, H, S, D), (*strides, 1)) for t in st)
+    flat = [np.lib.stride_tricks.as_strided(t, (B, H, S, D), [x * t.itemsize for x in (*strides, 1)]).copy().reshape(-1) for t in st]
+    out, lse = dev.attention_forward(q, k, v, 0.125)
+    same, _ = dev.attention_forward(*(dev.tensor(t, dtype, (B, H, S, D)) for t in flat), 0.125)
+    assert np.array_equal(dev.to_host(out), dev.to_host(same))
+    grads = [dev.tensor(np.zeros_like(st[0]), dtype) for _ in range(3)]
+    with pytest.raises(RocmError) as err:
+        dev.attention_backward(q, grads[0], k, grads[1], v, grads[2], 0.125, out, out, lse)
+    assert err.value.code == ERR_ALIASED_OUTPUT
+    assert all(not dev.to_host(t).any() for t in grads)
+
+
+def test_results_that_would_share_rows_are_refused():
+    dev = device()
+    announce("attention, aliased result")
+    B, H, S, D = 2, 2, 16, 64
+    x = dev.zeros("f16", (B, H, S, D))
+    from dfdx_amd.rocm import DTYPES, ERR_ALIASED_OUTPUT, _i64s
+
+    for strides in ((0, D, H * D), (S * H * D, 0, H * D), (S * H * D, D, D)):
+        rc = dev._f.attention_forward(dev.ctx, DTYPES["f16"], B, H, S, D, x.ptr, x.ptr, x.ptr, _i64s(x.strides[:3]), 0.125, x.ptr, _i64s(strides), None)
+        assert rc == ERR_ALIASED_OUTPUT, strides
+
+
+@pytest.mark.parametrize("wrong", ["grad_out", "lse", "small gradient", "strides of v"])
+def test_backward_looks_at_its_arguments(wrong):
+    dev = device()
+    B, H, S, D = 1, 2, 16, 64
+    x, rows = dev.zeros("f16", (B, H, S, D)), dev.zeros("f16", (B, S, H * D))
+    lse = dev.zeros("f32", (B, H, S))
+    v, go, gv = x, rows, dev.zeros("f16", (B, H, S, D))
+    if wrong == "grad_out":
+        go = dev.zeros("f16", (B, H, S, D))
+    elif wrong == "lse":
+        lse = dev.zeros("f16", (B, H, S))
+    elif wrong == "small gradient":
+        gv = dev.zeros("f16", (B, 1, S, D))
+    else:
+        v = dev.zeros("f16", (B, S, H, D)).permute(0, 2, 1, 3)
+    with pytest.raises(AssertionError):
+        dev.attention_backward(x, dev.zeros("f16", (B, H, S, D)), x, dev.zeros("f16", (B, H, S, D)), v, gv, 0.125, rows, go, lse)
