@@ -88,15 +88,20 @@ template <int D> __device__ __forceinline__ int swizzle(int r) {
 }
 
 // One [64][D] tile: 16-byte pieces, D / 32 of them per thread, held in registers between the load and the LDS store.
-template <int D> struct Stage {
+template <int D, bool ZERO = false> struct Stage {
     static constexpr int CPR = D / 8, N = TILE * CPR / 256, BYTES = TILE * D * 2;
+    static constexpr int OUTSIDE = 0x7ffffff0;  // past every offset in a tile: see walkable
     u32x4 piece[N];
+    // Rows past the end repeat the last one, or are ZERO: what the second products take meets probabilities of 0 there, and 0 times an
+    // infinity is not 0.  What the scores are formed of repeats: zeros would make NaN of a key's infinity where its rows make -infinity.
     __device__ __forceinline__ void load(const uint16_t *base, int row_stride, int row0, int rows) {
+        // (a buffer descriptor reads zeros at offsets past its end)
+        const auto tile = __builtin_amdgcn_make_buffer_rsrc((void *)(base + (int64_t)row0 * row_stride), 0, OUTSIDE, 0x00020000);
 #pragma unroll
         for (int i = 0; i < N; i++) {
-            const int slot = i * 256 + (int)threadIdx.x;
-            const int r = min(row0 + slot / CPR, rows - 1);  // rows past the end repeat the last one; what they give is masked
-            piece[i] = *(const u32x4 *)(base + (int64_t)r * row_stride + slot % CPR * 8);
+            const int slot = i * 256 + (int)threadIdx.x, r = ZERO ? slot / CPR : min(slot / CPR, rows - row0 - 1);
+            const int at = (r * row_stride + slot % CPR * 8) * 2;
+            piece[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(tile, !ZERO || r < rows - row0 ? at : OUTSIDE, 0, 0));
         }
     }
     __device__ __forceinline__ void store(uint8_t *lds) const {
@@ -223,7 +228,8 @@ template <typename T, int D> __global__ __launch_bounds__(256, D == 128 ? 2 : 3)
     const bool row_ok = row < p.seq;
     u32x4 qf[D / 16];
     own_rows<D>(p.q + b.in, p.in_r, min(row, p.seq - 1), qf);
-    Stage<D> sk, sv;
+    Stage<D> sk;
+    Stage<D, true> sv;
     sk.load(p.k + b.in, p.in_r, 0, p.seq);
     sv.load(p.v + b.in, p.in_r, 0, p.seq);
     f32x16 acc[D / 32];
@@ -231,7 +237,7 @@ template <typename T, int D> __global__ __launch_bounds__(256, D == 128 ? 2 : 3)
     for (int dt = 0; dt < D / 32; dt++)
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[dt][i] = 0.0f;
-    float m = -INFINITY, l = 0.0f;
+    float m = -__FLT_MAX__, l = 0.0f;  // (finite: where all scores so far are -infinity the exponentials are 0, not NaN)
     sk.store(smem[0][0]);
     sv.store(smem[0][1]);
     __syncthreads();
@@ -308,7 +314,8 @@ template <typename T, int D> __global__ __launch_bounds__(256, D == 128 ? 1 : 2)
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, h = lane / 32;
     const int row = b.row0 + wave * 32 + lane % 32, rowc = min(row, p.seq - 1);
     const bool row_ok = row < p.seq;
-    Stage<D> sk, sv;
+    Stage<D> sv;
+    Stage<D, true> sk;
     sk.load(p.k + b.in, p.in_r, 0, p.seq);
     sv.load(p.v + b.in, p.in_r, 0, p.seq);
     u32x4 qf[D / 16], gf[D / 16];
@@ -395,7 +402,8 @@ template <typename T, int D> __global__ __launch_bounds__(256, D == 128 ? 1 : 2)
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, h = lane / 32;
     const int row = b.row0 + wave * 32 + lane % 32, rowc = min(row, p.seq - 1);
     const bool row_ok = row < p.seq;
-    Stage<D> sq, sg;
+    Stage<D> sq;
+    Stage<D, true> sg;
     float st = 0.0f;
     auto load_stats = [&](int row0) {  // threads 0..63: lse, 64..127: -delta
         if (threadIdx.x < 2 * TILE) {
@@ -484,8 +492,8 @@ template <typename T, int D> __global__ __launch_bounds__(256, D == 128 ? 1 : 2)
 
 // ---- host side ------------------------------------------------------------------------------------------------------
 inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
-// strides of (batch, head, row): what 16-byte pieces of a head's row can walk
-inline bool walkable(const int64_t s[3]) { return s[0] >= 0 && s[1] >= 0 && s[2] > 0 && s[0] % 8 == 0 && s[1] % 8 == 0 && s[2] % 8 == 0 && s[2] < (1ll << 31); }
+// strides of (batch, head, row): what 16-byte pieces of a head's row can walk; offsets in a tile of 64 rows stay below 2^31 bytes
+inline bool walkable(const int64_t s[3]) { return s[0] >= 0 && s[1] >= 0 && s[2] > 0 && s[0] % 8 == 0 && s[1] % 8 == 0 && s[2] % 8 == 0 && s[2] < (1ll << 24); }
 // What is written through these strides: two workgroups that share a row would store (or load, add and store) it without order.
 // Sorted by stride, every axis has to step past all that the shorter ones reach.
 bool rows_apart(int64_t batch, int64_t heads, int64_t seq, int64_t dim, const int64_t s[3]) {

@@ -43,7 +43,7 @@ int shape_of(const dfdx_rocm_encoder *e, Shape *s) {
     s->D = s->d / s->H;
     s->T = s->B * s->S;
     s->es = dtype_size(s->dtype);
-    s->fused = attention_supported(s->dtype, s->B, s->H, s->S, s->D);
+    s->fused = attention_supported(s->dtype, s->B, s->H, s->S, s->D) && s->d < (1ll << 24);  // (the rows it walks are d_model apart)
     s->scale = 1.0 / std::sqrt((double)s->D);
     s->folded = s->dtype != DFDX_ROCM_F64 || (double)(float)s->scale == s->scale;
     s->token[0] = s->S * s->d; s->token[1] = s->D; s->token[2] = s->d;

@@ -123,3 +123,53 @@ def test_backward_looks_at_its_arguments(wrong):
         v = dev.zeros("f16", (B, S, H, D)).permute(0, 2, 1, 3)
     with pytest.raises(AssertionError):
         dev.attention_backward(x, dev.zeros("f16", (B, H, S, D)), x, dev.zeros("f16", (B, H, S, D)), v, gv, 0.125, rows, go, lse)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("case,S", [("last value", 65), ("last value", 200), ("first tile of keys", 130), ("first tile of keys", 64 + 17), ("last key", 65),
+                                    ("last gradient", 65), ("last gradient", 127)])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_infinities_reach_what_depends_on_them_and_nothing_else(dtype, case, S, D):
+    """The kernels work in tiles of 64 rows: what fills a tile up, and what a row's maximum starts from, may not meet an infinity.
+    Infinities and NaN as in the float64 formulas, finite values within the tolerance above (with one rounding of the largest finite one)."""
+    dev = device()
+    announce("attention, infinities", dtype, case, S, D)
+    B, H = 1, 2
+    d = H * D
+    g = rng(S + D)
+    st = [oracle.to_storage(np.abs(g.standard_normal(B * S * d)) * w, dtype) for w in (0.5, 0.5, 1.0, 1.0)]
+    at = lambda t, rows: t.reshape(S, d)[rows, 3:4]   # one column of the first head
+    inf = oracle.to_storage(np.array([np.inf]), dtype)[0]
+    minus = oracle.to_storage(np.array([-np.inf]), dtype)[0]
+    if case == "last value":
+        at(st[2], slice(S - 1, S))[:] = inf
+    elif case == "first tile of keys":
+        at(st[1], slice(0, 64))[:] = minus     # (the queries are positive: scores of -infinity)
+    elif case == "last key":
+        at(st[1], slice(S - 1, S))[:] = minus
+    else:
+        at(st[3], slice(S - 1, S))[:] = inf
+    qv, kv, vv, gv = (oracle.to_f64(t, dtype).reshape(B, S, H, D).swapaxes(1, 2) for t in st)
+    scale = D ** -0.5
+    with np.errstate(invalid="ignore"):
+        want = reference(qv, kv, vv, gv, scale)
+    q, k, v = (dev.tensor(t, dtype, (B, H, S, D), (S * d, D, d, 1)) for t in st[:3])
+    go = dev.tensor(st[3], dtype, (B, S, d))
+    out, lse = dev.attention_forward(q, k, v, scale)
+    grads = dev.zeros_many([go, go, go], deferred=True)
+    dev.attention_backward(q, grads[0], k, grads[1], v, grads[2], scale, out, go, lse)
+    eps = 2.0 ** -11 if dtype == "f16" else 2.0 ** -8
+    for name, got, ref in zip(("out", "dq", "dk", "dv"), (out, *grads), want):
+        if case == "last value" and name != "out":
+            continue   # (the gradients of an infinite result: out * grad_out and grad_out . v differ in which of them are NaN)
+        ref = ref.swapaxes(1, 2).reshape(-1)
+        got = oracle.to_f64(dev.to_host(got), dtype)
+        assert np.array_equal(np.isnan(got), np.isnan(ref)), (name, np.isnan(got).sum(), np.isnan(ref).sum())
+        assert np.array_equal(got[np.isinf(got)], ref[np.isinf(ref)]) and np.array_equal(np.isinf(got), np.isinf(ref)), name
+        ok = np.isfinite(ref)
+        assert ok.any() or name != "out"
+        most = lambda t: np.abs(t[np.isfinite(t)]).max()
+        floor = D * 2.0 ** -24 * D * most(vv) * most(gv) * scale * max(most(qv), most(kv))   # as in test_fused_attention
+        if ok.any():
+            err = np.abs(got[ok] - ref[ok]).max()
+            assert err <= 8 * eps * np.abs(ref[ok]).max() + floor * (name in ("dq", "dk")), (name, err)
