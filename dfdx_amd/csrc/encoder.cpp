@@ -37,7 +37,7 @@ struct Shape {
 
 int shape_of(const dfdx_rocm_encoder *e, Shape *s) {
     if (!e || e->dtype < DFDX_ROCM_F32 || e->dtype > DFDX_ROCM_F64) return DFDX_ROCM_ERR_INVALID_ARG;
-    if (e->batch < 1 || e->seq < 1 || e->d_model < 1 || e->heads < 1 || e->d_ff < 1 || e->d_model % e->heads) return DFDX_ROCM_ERR_INVALID_ARG;
+    if (e->batch < 0 || e->seq < 0 || e->d_model < 1 || e->heads < 1 || e->d_ff < 1 || e->d_model % e->heads) return DFDX_ROCM_ERR_INVALID_ARG;
     s->dtype = e->dtype;
     s->B = e->batch; s->S = e->seq; s->d = e->d_model; s->H = e->heads; s->ff = e->d_ff;
     s->D = s->d / s->H;
@@ -48,6 +48,15 @@ int shape_of(const dfdx_rocm_encoder *e, Shape *s) {
     s->folded = s->dtype != DFDX_ROCM_F64 || (double)(float)s->scale == s->scale;
     s->token[0] = s->S * s->d; s->token[1] = s->D; s->token[2] = s->d;
     return DFDX_ROCM_OK;
+}
+
+int64_t param_size(const Shape &s, int i) {
+    switch (i) {
+    case WQ: case WK: case WV: case WO: return s.d * s.d;
+    case W1: case W2: return s.ff * s.d;
+    case B1: return s.ff;
+    default: return s.d;
+    }
 }
 
 // Pieces of one buffer, each on a 256-byte boundary.
@@ -194,8 +203,7 @@ int backward(dfdx_rocm_ctx *ctx, const Shape &s, const dfdx_rocm_encoder *e, con
     void *gh2 = scratch + at.take(act), *gn1 = scratch + at.take(act), *gh1 = scratch + at.take(act), *gtok = scratch + at.take(act),
          *gq = scratch + at.take(act), *gk = scratch + at.take(act), *gv = scratch + at.take(act);
     // what the entry points below accumulate into counts as zero: every one of these is stored by its first use
-    const int64_t sizes[PARAM_COUNT] = {s.d * s.d, s.d, s.d * s.d, s.d, s.d * s.d, s.d, s.d * s.d, s.d, s.d, s.d, s.ff * s.d, s.ff, s.d * s.ff, s.d, s.d, s.d};
-    for (int i = 0; i < PARAM_COUNT; i++) TRY(dfdx_rocm_zero_deferred(ctx, grads[i], (size_t)sizes[i] * s.es));
+    for (int i = 0; i < PARAM_COUNT; i++) TRY(dfdx_rocm_zero_deferred(ctx, grads[i], (size_t)param_size(s, i) * s.es));
     for (void *g : {gh2, gh1, gtok, gq, gk, gv}) TRY(dfdx_rocm_zero_deferred(ctx, g, act));
 
     TRY(dfdx_rocm_layer_norm_backward(ctx, s.dtype, s.T, s.d, h2, p[G2], 1e-5, gh2, grads[G2], grads[BE2], grad_out));
@@ -279,6 +287,7 @@ int dfdx_rocm_encoder_forward(dfdx_rocm_ctx *ctx, const dfdx_rocm_encoder *e, co
     TRY(shape_of(e, &s));
     dfdx_rocm_encoder_layout l;
     saved_layout(s, &l);
+    if (s.T == 0) return DFDX_ROCM_OK;  // an empty batch has an empty result
     if (!x || !out || !saved || (l.forward_scratch_bytes && !scratch)) return DFDX_ROCM_ERR_INVALID_ARG;
     for (int i = 0; i < PARAM_COUNT; i++)
         if (!e->params[i]) return DFDX_ROCM_ERR_INVALID_ARG;
@@ -292,13 +301,16 @@ int dfdx_rocm_encoder_backward(dfdx_rocm_ctx *ctx, const dfdx_rocm_encoder *e, c
     TRY(shape_of(e, &s));
     dfdx_rocm_encoder_layout l;
     saved_layout(s, &l);
-    if (!x || !saved || !grad_out || !grads || !grad_x || !scratch) return DFDX_ROCM_ERR_INVALID_ARG;
+    if (!grads || (s.T && (!x || !saved || !grad_out || !grad_x || !scratch))) return DFDX_ROCM_ERR_INVALID_ARG;
     for (int i = 0; i < PARAM_COUNT; i++)
         if (!e->params[i] || !grads[i]) return DFDX_ROCM_ERR_INVALID_ARG;
+    if (s.T == 0) {  // sums over no token
+        for (int i = 0; i < PARAM_COUNT; i++) TRY(dfdx_rocm_memset_zero(ctx, grads[i], (size_t)param_size(s, i) * s.es));
+        return DFDX_ROCM_OK;
+    }
     const int rc = backward(ctx, s, e, l, x, (const char *)saved, grad_out, grads, grad_x, (char *)scratch);
     if (rc) {  // refused in mid-pass: no declaration made here outlives the call
-        const int64_t sizes[PARAM_COUNT] = {s.d * s.d, s.d, s.d * s.d, s.d, s.d * s.d, s.d, s.d * s.d, s.d, s.d, s.d, s.ff * s.d, s.ff, s.d * s.ff, s.d, s.d, s.d};
-        for (int i = 0; i < PARAM_COUNT; i++) (void)dfdx_rocm_forget_zeros(ctx, grads[i], (size_t)sizes[i] * s.es);
+        for (int i = 0; i < PARAM_COUNT; i++) (void)dfdx_rocm_forget_zeros(ctx, grads[i], (size_t)param_size(s, i) * s.es);
         (void)dfdx_rocm_forget_zeros(ctx, scratch, l.backward_scratch_bytes);
     }
     return rc;

@@ -39,7 +39,7 @@ class _Plan:
         es = ITEMSIZE[block.dtype]
         self.pieces = []
         for shape in list(self.shapes.values()) + [(B, S, d)]:
-            n = math.prod(shape) * es
+            n = math.prod(shape) * es or 16   # (an empty batch's gradient has an address all the same)
             self.pieces += [n, -n % 16]
         self.grad_bytes = sum(self.pieces)
         self.gapless = not any(self.pieces[1::2])

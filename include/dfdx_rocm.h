@@ -435,7 +435,8 @@ int dfdx_rocm_add_backward(dfdx_rocm_ctx *ctx, int dtype, int64_t len, void *gra
  * fused_attention, lse (dfdx_rocm_attention_forward) or probs (batch, heads,
  * seq, seq) and tokens (batch, heads, seq, dim).  `scratch` is free again when
  * the work queued by the call is done.  Backward STORES its 16 gradients and
- * grad_x (they need not be filled with zeros first). */
+ * grad_x (they need not be filled with zeros first).  Without tokens (batch or
+ * seq 0) the forward does nothing and the gradients are zeros. */
 #define DFDX_ROCM_ENCODER_PARAMS 16
 typedef struct dfdx_rocm_encoder {
     int32_t dtype;

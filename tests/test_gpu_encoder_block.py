@@ -110,3 +110,20 @@ def test_block_does_not_depend_on_where_its_parameters_lie(dtype, B, S, d, H):
         results.append([dev.to_host(t) for t in (out, gx, *(grads[n] for n in PARAMS))])
     for a, b in zip(*results):
         assert np.array_equal(a.view(np.uint16), b.view(np.uint16))
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32", "f64"])
+@pytest.mark.parametrize("B,S", [(0, 5), (2, 0), (0, 0)])
+def test_no_tokens(dtype, B, S):
+    """An empty batch: an empty result, and gradients that are sums over nothing."""
+    dev, d, ff, H = device(), 64, 128, 2
+    announce("encoder block, no tokens", dtype, B, S)
+    shapes = {n: (d, d) for n in ("wq", "wk", "wv", "wo")} | {"w1": (ff, d), "w2": (d, ff), "b1": (ff,)}
+    p = {n: dev.zeros(dtype, shapes.get(n, (d,))) for n in PARAMS}
+    block = EncoderBlock(dev, dtype, d, H, ff, p)
+    out, saved = block.forward(dev.zeros(dtype, (B, S, d)))
+    grads, gx = block.backward(saved, dev.zeros(dtype, (B, S, d)))
+    dev.synchronize()
+    assert out.shape == gx.shape == (B, S, d)
+    for n in PARAMS:
+        assert grads[n].shape == p[n].shape and not dev.to_host(grads[n]).any(), n
