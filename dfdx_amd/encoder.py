@@ -9,12 +9,13 @@ The library strings the block's ops together (``dfdx_rocm_encoder_forward`` / ``
 storage and the names of what the forward keeps.  The forward keeps what the backward needs; the other values of the
 reference's tape (the attention probabilities where the fused attention runs, the pre-activation of the ReLU) are made
 when somebody asks for them.  Gradients are stored, not added into zeros, so the step pays neither a fill nor the read of
-the zeros.
+the zeros.  A backward from other values than the forward's own goes op by op.
 """
 from __future__ import annotations
 
 import ctypes
 import math
+from collections.abc import ItemsView, KeysView, ValuesView
 from typing import Dict, Tuple
 
 from .rocm import DTYPES, ITEMSIZE, Encoder, EncoderLayout, Rocm, View, _row_major
@@ -46,24 +47,47 @@ class _Plan:
         self.grad_views = [(n, s, _row_major(s)) for n, s in self.shapes.items()] + [("x", (B, S, d), _row_major((B, S, d)))]
 
 
+KEPT = ("x", "qv", "kv", "vv", "probs", "tokens", "tok", "h1", "n1", "f1", "r1", "h2", "scale", "folded")
+
+
+def _version(storage):
+    """torch's count of changes in place (``None`` where it keeps none)."""
+    return None if storage.is_inference() else storage._version
+
+
 class _Saved(dict):
-    """What the forward keeps, by name: ``x`` and ``out``, and Views into the one allocation ``arena`` made on first use."""
+    """What the forward keeps, by name (``KEPT``; ``lse`` too where the fused attention ran): a dict whose values are made when somebody
+    asks for them, most of them Views into the one allocation ``arena``.  ``backward`` takes it as it is, or with values replaced or
+    changed, or any dict with the same names."""
 
     def __init__(self, block: "EncoderBlock", plan: _Plan, x: View, arena):
         super().__init__(x=x)
         self.block, self.plan, self.arena = block, plan, arena
+        self.made = {"x": x}
+        self.versions = {None: (arena, _version(arena))}   # storages whose contents stand for what the forward left
+        self.behind_f1 = [(block.p[n], _version(block.p[n].storage)) for n in ("w1", "b1")]
 
     def __missing__(self, name):
-        value = self[name] = self._make(name)
+        value = self._make(name)
+        self.made[name] = self[name] = value
+        if name in ("probs", "f1"):   # (made from what the forward left: changing them changes nothing that it left)
+            self.versions[name] = value.storage, _version(value.storage)
         return value
+
+    def untouched(self) -> bool:
+        """Whether the names still stand for what the forward left."""
+        return all(dict.get(self, n, v) is v for n, v in self.made.items()) and \
+            all(n in self.made for n in dict.keys(self) if n in KEPT) and \
+            all(_version(storage) == v for storage, v in self.versions.values())
 
     def _make(self, name):
         dev, dtype, l = self.block.dev, self.block.dtype, self.plan.layout
-        B, S, d = self["x"].shape
-        H, D, ff = self.block.h, d // self.block.h, self.block.ff
+        B, S, d = self.made["x"].shape
+        H = self.plan.desc.heads
+        D, ff = d // H, self.plan.desc.d_ff
 
         def at(offset, shape, strides=None, kind=dtype):
-            n = math.prod(shape) * ITEMSIZE[kind]
+            n = max(math.prod(shape) * ITEMSIZE[kind], 16)
             return View(self.arena[offset:offset + n], kind, shape, strides or _row_major(shape))
 
         heads = (S * d, D, d, 1)
@@ -76,24 +100,64 @@ class _Saved(dict):
         if name == "r1":
             return at(l.r1, (B, S, ff))
         if name == "f1":
+            if any(self.block.p[n] is not v or _version(v.storage) != at_forward for n, (v, at_forward) in zip(("w1", "b1"), self.behind_f1)):
+                raise RuntimeError("f1 is formed on request, from w1 and b1: they have changed since the forward")
             return dev.linear_forward(self["n1"], self.block.p["w1"], self.block.p["b1"])
         if name == "scale":
             return 1.0 / math.sqrt(D)
+        if name == "folded":
+            return _folded(dtype, D)
         if l.fused_attention:
             if name == "lse":
                 return at(l.lse, (B, H, S), kind="f32")
             if name == "probs":
                 return dev.softmax_forward(dev.forward(self["qv"], self["kv"]), self["scale"])
             if name == "tokens":
-                return at(l.tok, (B, H, S, D), heads)
+                return dev.reshape_forward(at(l.tok, (B, H, S, D), heads), (B, H, S, D))
         elif name in ("probs", "tokens"):
             return at(getattr(l, name), (B, H, S, S if name == "probs" else D))
         raise KeyError(name)
 
+    # the names are there whether or not their values have been made
+    def __contains__(self, name):
+        return name in KEPT or dict.__contains__(self, name)
+
+    def __iter__(self):
+        yield from KEPT
+        yield from [n for n in dict.keys(self) if n not in KEPT]
+
+    def __len__(self):
+        return len(list(iter(self)))
+
+    def get(self, name, default=None):
+        return self[name] if name in self else default
+
+    def keys(self):
+        return KeysView(self)
+
+    def values(self):
+        return ValuesView(self)
+
+    def items(self):
+        return ItemsView(self)
+
+    def copy(self):
+        return dict(self)
+
+    __copy__ = copy
+
+
+def _folded(dtype: str, head_dim: int) -> bool:
+    """Whether the softmax entry, which takes its scale as a C float, may scale: not for an f64 block whose 1/sqrt(head dim) has no
+    exact float value, which multiplies by the double scalar in an op of its own, as the reference does
+    (multi_head_attention.rs:133-134)."""
+    scale = 1.0 / math.sqrt(head_dim)
+    return dtype != "f64" or ctypes.c_float(scale).value == scale
+
 
 class EncoderBlock:
     """Parameters are device ``View``s: w* are (out, in) row-major Linear weights, b* biases, g*/be* the LayerNorm
-    gamma / beta.  ``deferred_zeros`` is kept for callers that pass it: there are no gradient zeros to fill either way."""
+    gamma / beta.  ``deferred_zeros``: where the backward adds into zeros (``_backward_by_ops``), whether they are declared or filled."""
 
     def __init__(self, dev: Rocm, dtype: str, d_model: int, heads: int, d_ff: int, params: Dict[str, View],
                  deferred_zeros: bool = True):
@@ -133,16 +197,19 @@ class EncoderBlock:
         plan = self._plan(B, S)
         l = plan.layout
         out = dev._bytes(max(B * S * d * ITEMSIZE[self.dtype], 16))
-        arena = dev._bytes(l.saved_bytes)
+        arena = dev._bytes(max(l.saved_bytes, 16))
         scratch = dev._bytes(l.forward_scratch_bytes) if l.forward_scratch_bytes else None
         dev._check(dev._f.encoder_forward(dev.ctx, ctypes.byref(self._desc(plan)), x.ptr, out.data_ptr(), arena.data_ptr(),
                                           scratch.data_ptr() if scratch is not None else None))
         return View(out, self.dtype, (B, S, d), strides), _Saved(self, plan, x, arena)
 
     def backward(self, saved: dict, grad_out: View) -> Tuple[Dict[str, View], View]:
-        """grad_out: d(loss)/d(out), contiguous like the output.  Returns ({parameter: gradient}, d(loss)/d(x))."""
+        """grad_out: d(loss)/d(out), contiguous like the output.  Returns ({parameter: gradient}, d(loss)/d(x)).  ``saved``: what the
+        forward returned, or a dict of the same names."""
+        if not (isinstance(saved, _Saved) and saved.untouched()):
+            return self._backward_by_ops(saved, grad_out)
         dev = self.dev
-        plan, x, dtype = saved.plan, saved["x"], self.dtype
+        plan, x, dtype = saved.plan, saved.made["x"], self.dtype
         assert grad_out.shape == x.shape and grad_out.strides == x.strides and grad_out.dtype == dtype
         grads = dev._bytes(plan.grad_bytes)
         scratch = dev._bytes(plan.layout.backward_scratch_bytes)
@@ -155,3 +222,46 @@ class EncoderBlock:
         parts = grads.split(plan.pieces[::2]) if plan.gapless else grads.split(plan.pieces)[::2]
         views = {name: View(part, dtype, shape, strides) for part, (name, shape, strides) in zip(parts, plan.grad_views)}
         return views, views.pop("x")
+
+    def _backward_by_ops(self, s: dict, grad_out: View) -> Tuple[Dict[str, View], View]:
+        """The same, op by op from the values in ``s``: what the caller has put in the place of the forward's own."""
+        dev, p, dtype = self.dev, self.p, self.dtype
+        x, n1, tok, probs, qv, kv, vv, r1 = (s[n] for n in ("x", "n1", "tok", "probs", "qv", "kv", "vv", "r1"))
+        B, H, S, D = qv.shape
+        f1 = r1 if isinstance(s, _Saved) and "f1" not in s.made and not dict.__contains__(s, "f1") else s["f1"]   # (positive in the same places)
+        tokens = View(tok.storage, dtype, (B, H, S, D), _row_major((B, H, S, D)))   # (its shape is all that counts)
+        # every gradient buffer of the pass: one allocation, pieces aligned to 256 B, zero by declaration (or one fill)
+        acts = dict(gh2=s["h2"], gf2=s["h2"], gn1=n1, gr1=r1, gf1=r1, gh1=s["h1"], gattn=s["h1"], gx=x, gtok=tok, gtokens=tokens, gp=probs,
+                    gscores=probs, gq=x, gk=x, gv=x)   # gq, gk, gv: laid out like the q, k, v storages
+        if not s["folded"]:
+            acts["gscaled"] = probs   # gradient of the scaled scores, between the softmax and the scalar multiply
+        bufs = dev.zeros_many([p[n] for n in PARAMS] + list(acts.values()), deferred=self.deferred_zeros)
+        grads = dict(zip(PARAMS, bufs[:len(PARAMS)]))
+        g = dict(zip(acts, bufs[len(PARAMS):]))
+        try:
+            dev.layer_norm_backward(s["h2"], p["g2"], g["gh2"], grads["g2"], grads["be2"], grad_out)
+            dev.add_backward(g["gf2"], g["gn1"], g["gh2"])            # h2 = f2 + n1
+            dev.linear_backward(r1, g["gr1"], p["w2"], grads["w2"], grads["b2"], g["gf2"])
+            dev.relu_backward(f1, g["gf1"], g["gr1"])
+            dev.linear_backward(n1, g["gn1"], p["w1"], grads["w1"], grads["b1"], g["gf1"])
+            dev.layer_norm_backward(s["h1"], p["g1"], g["gh1"], grads["g1"], grads["be1"], g["gn1"])
+            dev.add_backward(g["gattn"], g["gx"], g["gh1"])           # h1 = attn + x
+            dev.linear_backward(tok, g["gtok"], p["wo"], grads["wo"], grads["bo"], g["gattn"])
+            dev.reshape_backward(tokens.permute(0, 2, 1, 3), g["gtokens"], g["gtok"])
+            dev.backward(probs, g["gp"], vv, g["gv"], g["gtokens"])
+            if s["folded"]:
+                dev.softmax_backward(probs, g["gscores"], g["gp"], s["scale"])
+            else:
+                dev.softmax_backward(probs, g["gscaled"], g["gp"], 1.0)
+                dev.scalar_mul_backward(s["scale"], g["gscores"], g["gscaled"])
+            dev.backward(qv, g["gq"], kv, g["gk"], g["gscores"])
+            for w, b, gg in (("wq", "bq", "gq"), ("wk", "bk", "gk"), ("wv", "bv", "gv")):   # x feeds three Linears: one buffer
+                dev.linear_backward(x, g["gx"], p[w], grads[w], grads[b], g[gg])
+            dev.settle_zeros()   # nothing is left pending in this block; a gradient no op touched would be filled here
+        except BaseException:
+            # an op refused or raised in mid-pass: no declaration may outlive the pass unsettled, whoever still holds
+            # a View of the arena (the caller sees the exception, not zeros it could rely on)
+            if bufs[0].owner is not None:
+                bufs[0].owner.forget()
+            raise
+        return grads, g["gx"]

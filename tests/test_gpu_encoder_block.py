@@ -127,3 +127,74 @@ def test_no_tokens(dtype, B, S):
     assert out.shape == gx.shape == (B, S, d)
     for n in PARAMS:
         assert grads[n].shape == p[n].shape and not dev.to_host(grads[n]).any(), n
+
+
+def a_block(dtype, B, S, d, H, ff, seed=3, **more):
+    dev, g = device(), rng(seed)
+    up = lambda shape, s: dev.tensor(oracle.to_storage((g.standard_normal(int(np.prod(shape))) * s).astype(np.float32), dtype), dtype, shape)
+    shapes = {n: (d, d) for n in ("wq", "wk", "wv", "wo")} | {"w1": (ff, d), "w2": (d, ff), "b1": (ff,)}
+    p = {n: up(shapes.get(n, (d,)), 1.0 if n in ("g1", "g2") else 0.05) for n in PARAMS}
+    return EncoderBlock(dev, dtype, d, H, ff, p, **more), up((B, S, d), 1.0), up((B, S, d), 1.0)
+
+
+KEPT = {"x", "qv", "kv", "vv", "probs", "tokens", "tok", "h1", "n1", "f1", "r1", "h2", "scale", "folded"}
+
+
+@pytest.mark.parametrize("dtype,d,H", [("f16", 128, 2), ("bf16", 128, 2), ("f32", 128, 2), ("f64", 96, 2), ("f16", 96, 4), ("f32", 4, 1)])
+@pytest.mark.parametrize("deferred", [True, False])
+def test_backward_takes_any_dict_of_the_names(dtype, d, H, deferred):
+    """A plain copy of what the forward returned goes through the single ops: the same gradients up to the roundings in between
+    (the bound of test_block_equals_its_ops; the probabilities are rounded there)."""
+    dev = device()
+    B, S, ff = 2, 33, 2 * d
+    announce("encoder block, plain dict", dtype, d, H, deferred)
+    block, x, go = a_block(dtype, B, S, d, H, ff, deferred_zeros=deferred)
+    _, saved = block.forward(x)
+    want, wx = block.backward(saved, go)
+    assert set(saved) == set(saved.keys()) == KEPT and len(saved) == len(KEPT) and all(n in saved for n in KEPT) and saved.get("nothing", 7) == 7
+    plain = dict(saved)
+    assert type(plain) is dict and set(plain) == KEPT and saved["tokens"].strides == (H * S * (d // H), S * (d // H), d // H, 1)
+    got, gx = block.backward(plain, go)
+    dev.synchronize()
+    eps = {"f16": 2.0 ** -12, "bf16": 2.0 ** -9, "f32": 2.0 ** -24, "f64": 2.0 ** -53}[dtype]
+    for n, a, b in [("x", gx, wx)] + [(n, got[n], want[n]) for n in PARAMS if n != "bk"]:
+        a, b = (oracle.to_f64(dev.to_host(t), dtype)[:int(np.prod(b.shape))] for t in (a, b))
+        # scores and probabilities rounded to the type on one side: two more roundings in front of the gradients of the attention
+        assert np.linalg.norm(a - b) <= 20 * eps * np.linalg.norm(b) + 1e-6 * (dtype == "f32") * np.linalg.norm(b), (n, np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+@pytest.mark.parametrize("how", ["replaced", "changed in place", "changed in the arena"])
+def test_backward_uses_what_the_caller_put_there(how):
+    """Zeros in the place of the ReLU's output (or of the probabilities) leave no gradient for what is behind it."""
+    dev = device()
+    block, x, go = a_block("f16", 2, 33, 128, 2, 256)
+    announce("encoder block, saved values", how)
+    _, saved = block.forward(x)
+    if how == "replaced":
+        saved["r1"] = dev.zeros("f16", saved["r1"].shape)
+        none = ("w2", "w1", "b1")
+    elif how == "changed in the arena":
+        saved["r1"].storage.zero_()
+        none = ("w2", "w1", "b1")
+    else:
+        saved["probs"].storage.zero_()
+        none = ("wv", "bv", "wq", "bq", "wk")
+    grads, _ = block.backward(saved, go)
+    dev.synchronize()
+    for n in PARAMS:
+        if n != "bk":
+            assert bool(dev.to_host(grads[n]).astype(np.float32).any()) == (n not in none), n
+
+
+def test_no_stale_value_is_made():
+    """f1 is not kept: asked for after its weights have changed, it is refused instead of made from other weights."""
+    block, x, go = a_block("f16", 1, 9, 64, 1, 128)
+    _, saved = block.forward(x)
+    before = device().to_host(saved["f1"]).copy()
+    _, late = block.forward(x)
+    want, _ = block.backward(late, go)
+    block.p["w1"].storage.zero_()
+    with pytest.raises(RuntimeError):
+        late["f1"]
+    assert np.array_equal(device().to_host(saved["f1"]), before)
+    assert set(late) == KEPT
