@@ -567,7 +567,7 @@ class Rocm:
     # ------------------------------------------------- ops between attention's GEMMs --
     def _like(self, x: View) -> View:
         """Uninitialised storage of the same physical length, seen the same way."""
-        return View(self._bytes(x.storage.numel()), x.dtype, x.shape, x.strides, x.offset)
+        return View(self._bytes(x.storage.nbytes), x.dtype, x.shape, x.strides, x.offset)
 
     def scalar_mul_forward(self, x: View, scalar: float) -> View:
         """``x * scalar`` over the physical storage (unary kernel, utilities/cpu_kernels.rs:46-79); same strides."""
@@ -583,7 +583,7 @@ class Rocm:
     def softmax_forward(self, x: View, scale: float = 1.0) -> View:
         """softmax(scale * x) over the last axis of a contiguous tensor (softmax.rs:70-83)."""
         assert x.strides == _row_major(x.shape), "softmax input must be contiguous"
-        out = View(self._bytes(x.storage.numel()), x.dtype, x.shape, x.strides)
+        out = View(self._bytes(x.storage.nbytes), x.dtype, x.shape, x.strides)
         self._check(self._f.softmax_forward(self.ctx, DTYPES[x.dtype], math.prod(x.shape[:-1]), x.shape[-1], x.ptr, scale, out.ptr))
         return out
 
@@ -643,7 +643,7 @@ class Rocm:
         assert x.strides == _row_major(x.shape), "layer norm input must be contiguous"
         cols = x.shape[-1]
         assert gamma.shape == (cols,) and beta.shape == (cols,), f"left: {gamma.shape}\n right: {(cols,)}"
-        out = View(self._bytes(x.storage.numel()), x.dtype, x.shape, x.strides)
+        out = View(self._bytes(x.storage.nbytes), x.dtype, x.shape, x.strides)
         self._check(self._f.layer_norm_forward(self.ctx, DTYPES[x.dtype], math.prod(x.shape[:-1]), cols, x.ptr, gamma.ptr, beta.ptr, epsilon, out.ptr))
         return out
 

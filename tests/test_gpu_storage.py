@@ -7,6 +7,7 @@ import ctypes
 import numpy as np
 import pytest
 
+from helpers import rng
 from gpu_util import announce, device
 
 pytestmark = pytest.mark.gpu
@@ -119,3 +120,21 @@ def test_workspace_growth_does_not_disturb_queued_work():
     dev.synchronize()
     for dc, A, B, (m, k, n), _keep in outs:
         assert_within("f32", k, dev.to_host(dc).astype(np.float64).reshape(m, n), A @ B, A, B, extra=1e-5)
+
+
+def test_results_take_as_many_bytes_as_their_inputs():
+    """Storage of another torch type than uint8 counts its elements in other units: the result has its bytes, not its count."""
+    import torch
+
+    from dfdx_amd import View
+
+    dev, (rows, cols) = device(), (37, 130)
+    announce("typed storage")
+    host = rng(4).standard_normal((rows, cols)).astype(np.float16)
+    typed = View(torch.from_numpy(host.reshape(-1)).to(dev.device), "f16", (rows, cols), (cols, 1))
+    plain = dev.tensor(host, "f16")
+    one, zero = dev.tensor(np.ones(cols, np.float16), "f16"), dev.tensor(np.zeros(cols, np.float16), "f16")
+    for op in (lambda x: dev.softmax_forward(x), lambda x: dev.layer_norm_forward(x, one, zero)):
+        out = op(typed)
+        assert out.storage.nbytes == host.nbytes
+        assert np.array_equal(dev.to_host(out), dev.to_host(op(plain)))
