@@ -270,11 +270,16 @@ int drop_cache(dfdx_rocm_ctx *ctx) {
     return (int)first;
 }
 
+struct Plan;
+size_t partials_bytes(const GemmProblem &p, const Plan &plan, Realign *ra = nullptr);
+
 struct Plan {
     int kernel, variant, splits;
-    // An LDS-DMA variant on copies of the operands that are off its grid (realign.hip); the plan without copies is kept for
-    // calls that may not have the space for them.
+    // An LDS-DMA variant on copies of the operands that are off its grid (realign.hip).  Where the copies cannot have their space the
+    // register-staged tile `staged` runs on the operands as they lie, with the same splits: every 16-bit tile walks the
+    // contraction in the same order, so it leaves the same bits.  Where its partial sums have no space either: the plain plan.
     bool realign = false;
+    int staged = 0;
     int plain_kernel = 0, plain_variant = 0, plain_splits = 1;
 };
 
@@ -421,12 +426,16 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
             int dv = 0, splits = 1;
             double t_dma = 1e300;
             mfma16dma_plan_split(ra.problem, ctx->compute_units, 0, forced_splits, &dv, &splits, &t_dma);
+            // (a product whose plan without copies fits the fixed scratch array fits it in this form too: see dfdx_rocm_gemm_noalloc)
+            const size_t piece = mfma16_workspace_bytes(p, v, 2) / 2, most = DFDX_ROCM_NOALLOC_SCRATCH_BYTES;
+            if (dv && splits > 1 && !forced_splits && piece * (size_t)splits > most && partials_bytes(p, *plan) <= most)
+                mfma16dma_plan_split(ra.problem, ctx->compute_units, 0, (int)std::max<size_t>(1, most / piece), &dv, &splits, &t_dma);
             const bool small_tile = v == mfma16_skinny_variant();
             const double t_staged = t_family * (small_tile ? (ra.off_grid ? 1.0 : 0.6) : ra.off_grid ? 1.4 : 0.95) +
                                     (small_tile ? 0.0 : 2.0 * (double)p.m * (double)p.n * (double)(p.reduce ? 1 : p.nb1 * p.nb2) / 2.2e12);
             if (dv && t_dma + ra.seconds < std::min(std::min(t_small_here, t_staged), t_bw)) {
                 const Plan plain = *plan;
-                *plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits, true, plain.kernel, plain.variant, plain.splits};
+                *plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits, true, v, plain.kernel, plain.variant, plain.splits};
             }
         }
         return DFDX_ROCM_OK;
@@ -459,7 +468,7 @@ int partials_buffer(dfdx_rocm_ctx *ctx, size_t need, bool static_scratch, float 
 }
 
 // The f32 partial sums `plan` needs for `p`, in bytes (0: none), and, behind them, the copies of its operands.
-size_t partials_bytes(const GemmProblem &p, const Plan &plan, Realign *ra = nullptr) {
+size_t partials_bytes(const GemmProblem &p, const Plan &plan, Realign *ra) {
     if (plan.realign) {
         Realign here;
         if (!ra) ra = &here;
@@ -477,26 +486,32 @@ size_t partials_bytes(const GemmProblem &p, const Plan &plan, Realign *ra = null
     return 0;
 }
 
+// Nothing is allocated while the stream is being captured into a graph that the call could do without.
+bool may_grow(dfdx_rocm_ctx *ctx) {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess) (void)hipGetLastError();
+    return capturing == hipStreamCaptureStatusNone;
+}
+
 // Makes sure the partial sums of `plan` have a place, BEFORE the caller resolves pending zero fills among the operands:
 // a call that is refused here (scratch too small, out of memory) must leave every declaration as it found it.
-// Copies of operands are left out, and the plan changed to the one without them, where they cannot have their space: under
-// a fixed scratch array, when memory has run out, and while the stream is being captured into a graph, where nothing is
-// allocated that the call could do without.
+// A plan with copies of operands that cannot have their space -- they do not fit the fixed scratch array, memory has run out, or
+// the stream is being captured -- is changed to one without them (see Plan).
 int reserve_partials(dfdx_rocm_ctx *ctx, const GemmProblem &problem, Plan &plan, bool static_scratch) {
     GemmProblem p = problem;
     p.compute_units = ctx->compute_units;
     float *unused = nullptr;
     if (plan.realign) {
         CtxLock lock(ctx->mu);
-        const size_t need = partials_bytes(p, plan);
-        bool room = !static_scratch;
-        if (room && need > ctx->workspace_bytes) {
-            hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-            if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess) (void)hipGetLastError();
-            room = capturing == hipStreamCaptureStatusNone && ensure_workspace(ctx, need) == DFDX_ROCM_OK;
-        }
-        if (room) return DFDX_ROCM_OK;
-        plan = {plan.plain_kernel, plan.plain_variant, plan.plain_splits};
+        auto room = [&](size_t need) {
+            if (static_scratch) return need <= (size_t)DFDX_ROCM_NOALLOC_SCRATCH_BYTES;
+            return need <= ctx->workspace_bytes || (may_grow(ctx) && ensure_workspace(ctx, need) == DFDX_ROCM_OK);
+        };
+        if (room(partials_bytes(p, plan))) return DFDX_ROCM_OK;
+        const Plan plain = {plan.plain_kernel, plan.plain_variant, plan.plain_splits};
+        plan = {DFDX_ROCM_KERNEL_MFMA, plan.staged, plan.splits};
+        if (room(partials_bytes(p, plan))) return DFDX_ROCM_OK;
+        plan = plain;
     }
     const size_t need = partials_bytes(p, plan);
     return need ? partials_buffer(ctx, need, static_scratch, &unused) : DFDX_ROCM_OK;

@@ -197,15 +197,21 @@ int dfdx_rocm_gemm(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc);
  * No counterpart in the reference (its devices allocate freely).
  * dfdx_rocm_gemm grows a context-owned buffer on demand for the f32 partial
  * sums of a split reduction (split-k weight gradients, k-sliced vector
- * products); this entry point plans exactly as dfdx_rocm_gemm does -- same
- * kernels, same bits -- but keeps those partial sums in a fixed array of
+ * products) and, for 16-bit operands off the 16-byte grid, for padded copies of
+ * them; this entry point plans exactly as dfdx_rocm_gemm does and leaves the
+ * same bits, but keeps partial sums and copies in a fixed array of
  * DFDX_ROCM_NOALLOC_SCRATCH_BYTES that lives in the library's device image
  * (one copy per GPU, held until the process ends) and calls no hipMalloc /
- * hipFree or any other allocating routine.  A plan whose partial sums do not
- * fit is refused with DFDX_ROCM_ERR_SCRATCH_TOO_SMALL before anything is
- * launched and before any pending zero declaration of an operand is touched
- * (the caller may then lower or forbid the split through `flags`, or call
- * dfdx_rocm_gemm with the same descriptor).
+ * hipFree or any other allocating routine.  Copies that do not fit are left
+ * out: a kernel that reads the operands where they lie, in the same order of
+ * the contraction, takes their place (slower, the same bits).  A plan whose
+ * partial sums do not fit is refused with DFDX_ROCM_ERR_SCRATCH_TOO_SMALL
+ * before anything is launched and before any pending zero declaration of an
+ * operand is touched (the caller may then lower or forbid the split through
+ * `flags`, or call dfdx_rocm_gemm with the same descriptor).
+ * dfdx_rocm_gemm on a stream that is being captured into a graph does the same
+ * with the buffer that the context has by then: call once before the capture
+ * for the plan with copies.
  * Nothing in the array has to start at zero: every partial sum that is read
  * has been written by the same call.  All calls on one GPU share the array,
  * so calls that overlap on one GPU (two contexts, two streams, two threads)

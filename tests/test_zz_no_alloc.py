@@ -1,8 +1,8 @@
 """GPU: the entry point that allocates nothing (`dfdx_rocm_gemm_noalloc`) against `dfdx_rocm_gemm`.
 
-Both plan the same kernels; the only difference is where the f32 partial sums of a split reduction live (the
-library's fixed per-GPU scratch array instead of a context-owned buffer that grows on demand), so the two results
-must be identical bit for bit -- and both within the stated tolerance of the oracle
+Both plan the same products; the difference is where the f32 partial sums of a split reduction, and the padded copies of
+16-bit operands off the 16-byte grid, live (the library's fixed per-GPU scratch array instead of a context-owned buffer
+that grows on demand), and that copies which do not fit are left out; the two results must be identical bit for bit -- and both within the stated tolerance of the oracle
 (max|err| <= 2e-3*sqrt(K)*max|a|*max|b| for f16 / bf16, 1e-5*sqrt(K)*... for f32).  Every case makes two calls in a
 row, the second on a smaller product, because all calls on a GPU share the one array and it keeps the last call's
 contents.  Runs last (file name) so that a failure here cannot hide another test.
@@ -97,3 +97,62 @@ def test_full_size_scratch_and_refusal_beyond_it():
     dev.gemm(desc)
     dev.synchronize()
     assert not np.array_equal(dev.to_host(dc), c)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("m,k,n,layout,accumulate,copies", [
+    (2305, 1024, 2051, (False, True), False, "none"),      # only C is off the grid: no space needed
+    (2049, 1153, 1031, (False, False), False, "fit"),
+    (4095, 4095, 4097, (False, False), True, "too large"), # 67 MB of copies
+    (8193, 2049, 2047, (False, True), False, "too large"),
+    (261, 6795, 871, (True, False), True, "fit"),          # split contraction
+    (361, 2469, 4606, (False, False), False, "fit"),
+    (1023, 9001, 1021, (True, False), True, "too large"),  # split contraction
+])
+def test_operands_off_the_grid(dtype, m, k, n, layout, accumulate, copies):
+    """The same bits with the copies in the array, with none, and with the operands read where they lie because the copies do not fit."""
+    dev = device()
+    at, bt = layout
+    sizes = [x * 64 * -(-y // 64) * 2 for x, y in ((m, k), (n, k))] if k % 64 else [0]
+    assert copies == "none" or (sum(sizes) > NOALLOC_SCRATCH_BYTES) == (copies == "too large")
+    desc = dev.gemm_desc(dtype, m, k, n, 256, (1, m) if at else (k, 1), 512, (1, k) if bt else (n, 1), 1024, (n, 1), accumulate=accumulate)
+    plan = dev.gemm_plan(desc)[2]
+    assert "_realigned" in plan, plan
+    both_entries(dtype, m, k, n, layout, accumulate, seed=m + k, expect_split=False, check_oracle=m * k * n < 1 << 33)
+
+
+@pytest.mark.parametrize("m,k,n,at", [(2049, 1153, 1031, False), (261, 6795, 871, True), (2305, 1024, 2051, False)])
+def test_captured_into_a_graph_with_a_cold_context(m, k, n, at):
+    """A context that has no buffer yet allocates none while its stream is captured: the operands are read where they lie (a split
+    needs its partial sums, so that context has run a small split product before), and every replay leaves the bits of the eager call."""
+    import torch
+
+    from dfdx_amd import Rocm
+
+    dev, g, dtype = device(), rng(7), "f16"
+    a, astr = make_operand(g, m, k, at, dtype, dist="uniform")
+    b, bstr = make_operand(g, k, n, False, dtype, dist="uniform")
+    da, db, want = dev.tensor(a, dtype), dev.tensor(b, dtype), dev.zeros(dtype, (m, n))
+    desc = lambda d, c: d.gemm_desc(dtype, m, k, n, da.ptr, astr, db.ptr, bstr, c.ptr, (n, 1))
+    name = dev.gemm_plan(desc(dev, want))[2]
+    assert "_realigned" in name, name
+    announce("captured", (m, k, n), name)
+    dev.gemm(desc(dev, want))
+    dev.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        own = Rocm(0)
+        if "splitk" in name:   # 16 MB of partial sums, less than the copies need besides
+            x = own.zeros("f32", (1024, 1024))
+            own.gemm(own.gemm_desc("f32", 512, 1024, 1024, x.ptr, (1024, 1), x.ptr, (1024, 1), own.zeros("f32", (512, 1024)).ptr, (1024, 1), split_k=8, kernel=2, variant=4))
+        out = own.zeros(dtype, (m, n))
+        own.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            own.gemm(desc(own, out))
+        for _ in range(3):
+            out.storage.fill_(0x55)
+            graph.replay()
+            own.synchronize()
+            assert np.array_equal(own.to_host(out).view(np.uint16), dev.to_host(want).view(np.uint16))
+    own.close()
