@@ -584,6 +584,43 @@ bool extra_supported(const GemmProblem &p, const Plan &plan) {
     if (is16 && plan.variant >= mfma16_dma_first_variant()) return mfma16dma_extra_supported(p, plan.variant - mfma16_dma_first_variant() + 1, plan.splits);
     return plan.splits > 1;  // the reduce kernel does it
 }
+
+// A product with its plan made: space, pending fills, launches.
+int run_planned(dfdx_rocm_ctx *ctx, GemmProblem &p, Plan &plan, bool static_scratch = false) {
+    if (int e = reserve_partials(ctx, p, plan, static_scratch)) return e;
+    if (int e = settle_operands(ctx, &p, /*may_overwrite=*/true)) return e;
+    return run_plan(ctx, p, plan, static_scratch);
+}
+
+// The same with the sums that `p` asks for (ksum) where the plan can take them along: *fused.
+int run_with_colsum(dfdx_rocm_ctx *ctx, GemmProblem &p, Plan &plan, bool *fused) {
+    if (int e = reserve_partials(ctx, p, plan, false)) return e;
+    if (int e = settle_operands(ctx, &p, /*may_overwrite=*/true)) return e;
+    bool can = p.ksum && plan.kernel == DFDX_ROCM_KERNEL_MFMA && !plan.realign;
+    if (can && (p.dtype == DT_F16 || p.dtype == DT_BF16))
+        can = plan.variant == mfma16_small_variant()
+                  ? small_ksum_supported(p)
+                  : plan.variant >= mfma16_dma_first_variant() &&
+                        mfma16dma_ksum_supported(p, plan.variant - mfma16_dma_first_variant() + 1, plan.splits);
+    else if (can && p.dtype == DT_F32)
+        can = plan.splits <= 1 && mfma32_ksum_supported(p, plan.variant);
+    else if (can && p.dtype == DT_F64)
+        can = plan.variant == mfma64_small_variant() && small_ksum_supported(p);
+    else
+        can = false;
+    if (can) {
+        bool fresh = false;
+        const int64_t len = p.ksum_of == KSUM_OF_A ? p.m : p.n;
+        if (int e = settle_output(ctx, p.ksum, (size_t)len * dtype_size(p.dtype), true, &fresh)) return e;
+        p.ksum_accumulate = !fresh;
+        *fused = true;
+    } else {
+        p.ksum = nullptr;
+        p.ksum_of = KSUM_NONE;
+    }
+    return run_plan(ctx, p, plan);
+}
+
 }  // namespace
 
 namespace dfdx_rocm {
@@ -622,14 +659,13 @@ int gemm_beyond(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int extra, 
 
 int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_rocm_gemm_desc *second, const void *grad_out, int64_t rows, int64_t cols,
               void *colsum, bool *fused) {
-    auto apart = [&]() -> int {
-        if (int e = dfdx_rocm_gemm(ctx, first)) return e;
-        return fused ? gemm_with_colsum(ctx, second, colsum, fused) : dfdx_rocm_gemm(ctx, second);
-    };
     if (fused) *fused = false;
     // (a copy of less than 4 MB costs little more than its launch)
     const bool off = cols % 64 || rows % 64 || ((uintptr_t)grad_out & 15u);
-    if ((first->dtype != DFDX_ROCM_F16 && first->dtype != DFDX_ROCM_BF16) || !off || (double)rows * (double)cols < 2097152.0) return apart();
+    if ((first->dtype != DFDX_ROCM_F16 && first->dtype != DFDX_ROCM_BF16) || !off || (double)rows * (double)cols < 2097152.0) {
+        if (int e = dfdx_rocm_gemm(ctx, first)) return e;
+        return fused ? gemm_with_colsum(ctx, second, colsum, fused) : dfdx_rocm_gemm(ctx, second);
+    }
     if (int e = bind(ctx)) return e;
     GemmProblem p[2];
     Plan plan[2];
@@ -637,28 +673,44 @@ int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_r
     bool both = true;
     for (int i = 0; i < 2; i++) {
         const dfdx_rocm_gemm_desc *d = i ? second : first;
-        if (int e = make_problem(d, &p[i])) return e;
-        if (p[i].m == 0) return apart();
+        if (int e = make_problem(d, &p[i], i && fused ? colsum : nullptr)) return e;
+        if (p[i].m == 0) {
+            both = false;
+            continue;
+        }
         if (int e = make_plan(ctx, d, p[i], &plan[i])) return e;
         both = both && plan[i].realign && p[i].a != p[i].b && plan_realign(p[i], &ra) && (p[i].a == grad_out ? ra.a : ra.b);
     }
+    auto apart = [&]() -> int {
+        if (p[0].m)
+            if (int e = run_planned(ctx, p[0], plan[0])) return e;
+        if (!p[1].m) return DFDX_ROCM_OK;
+        return fused ? run_with_colsum(ctx, p[1], plan[1], fused) : run_planned(ctx, p[1], plan[1]);
+    };
     CtxLock lock(ctx->mu);  // the copy lives in the patch buffer until the second product has been launched
     int64_t ld = 0;
     const size_t bytes = realign_shared_bytes(rows, cols, &ld);
-    if (!both || bytes == 0) return apart();
+    if (!both || bytes == 0 || (bytes > ctx->patches_bytes && (!may_grow(ctx) || ensure_patches(ctx, bytes) != DFDX_ROCM_OK))) return apart();
+    // each product with grad_out replaced by the copy: the space of its own copy is not asked for
+    GemmProblem q[2] = {p[0], p[1]};
+    for (int i = 0; i < 2; i++) {
+        q[i].ksum = nullptr;
+        q[i].ksum_of = KSUM_NONE;
+        if (q[i].a == grad_out) {
+            (q[i].a_rs == 1 ? q[i].a_cs : q[i].a_rs) = ld;
+            q[i].a = ctx->patches;
+            q[i].a_laid = true;
+        } else {
+            (q[i].b_cs == 1 ? q[i].b_rs : q[i].b_cs) = ld;
+            q[i].b = ctx->patches;
+            q[i].b_laid = true;
+        }
+        Plan reserved = plan[i];
+        if (int e = reserve_partials(ctx, q[i], reserved, false)) return e;
+        if (!reserved.realign) return apart();
+    }
     const size_t sums_bytes = fused && colsum ? bias_backward_copy_partials(ctx->compute_units, rows, cols, ld) : 0;
-    bool sums = sums_bytes > 0;
-    if (bytes > ctx->patches_bytes || sums_bytes > ctx->workspace_bytes) {
-        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess) (void)hipGetLastError();
-        const bool may_grow = capturing == hipStreamCaptureStatusNone;
-        if (bytes > ctx->patches_bytes && (!may_grow || ensure_patches(ctx, bytes) != DFDX_ROCM_OK)) return apart();
-        if (sums_bytes > ctx->workspace_bytes) sums = may_grow && ensure_workspace(ctx, sums_bytes) == DFDX_ROCM_OK;
-    }
-    for (int i = 0; i < 2; i++) {  // with everything reserved, nothing below turns to another plan
-        if (int e = reserve_partials(ctx, p[i], plan[i], false)) return e;
-        if (!plan[i].realign) return apart();
-    }
+    const bool sums = sums_bytes > 0 && (sums_bytes <= ctx->workspace_bytes || (may_grow(ctx) && ensure_workspace(ctx, sums_bytes) == DFDX_ROCM_OK));
     if (int e = settle(ctx, grad_out)) return e;
     if (sums) {  // on the way into the copy; their partials are done with the workspace before the products write it
         bool fresh = false;
@@ -670,18 +722,8 @@ int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_r
         HIP_TRY(launch_realign_shared(grad_out, rows, cols, ctx->patches, ctx->stream));
     }
     for (int i = 0; i < 2; i++) {
-        GemmProblem &q = p[i];
-        if (q.a == grad_out) {
-            (q.a_rs == 1 ? q.a_cs : q.a_rs) = ld;
-            q.a = ctx->patches;
-            q.a_laid = true;
-        } else {
-            (q.b_cs == 1 ? q.b_rs : q.b_cs) = ld;
-            q.b = ctx->patches;
-            q.b_laid = true;
-        }
-        if (int e = settle_operands(ctx, &q, /*may_overwrite=*/true)) return e;
-        if (int e = run_plan(ctx, q, plan[i])) return e;
+        if (int e = settle_operands(ctx, &q[i], /*may_overwrite=*/true)) return e;
+        if (int e = run_plan(ctx, q[i], plan[i])) return e;
     }
     return DFDX_ROCM_OK;
 }
@@ -748,31 +790,7 @@ int gemm_with_colsum(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, void *
     if (p.m == 0) return DFDX_ROCM_OK;
     Plan plan;  // from the product as the caller states it: a pending zero fill of C must not change which kernel runs
     if (int e = make_plan(ctx, desc, p, &plan)) return e;
-    if (int e = reserve_partials(ctx, p, plan, false)) return e;
-    if (int e = settle_operands(ctx, &p, /*may_overwrite=*/true)) return e;
-    bool can = p.ksum && plan.kernel == DFDX_ROCM_KERNEL_MFMA && !plan.realign;
-    if (can && (p.dtype == DT_F16 || p.dtype == DT_BF16))
-        can = plan.variant == mfma16_small_variant()
-                  ? small_ksum_supported(p)
-                  : plan.variant >= mfma16_dma_first_variant() &&
-                        mfma16dma_ksum_supported(p, plan.variant - mfma16_dma_first_variant() + 1, plan.splits);
-    else if (can && p.dtype == DT_F32)
-        can = plan.splits <= 1 && mfma32_ksum_supported(p, plan.variant);
-    else if (can && p.dtype == DT_F64)
-        can = plan.variant == mfma64_small_variant() && small_ksum_supported(p);
-    else
-        can = false;
-    if (can) {
-        bool fresh = false;
-        const int64_t len = p.ksum_of == KSUM_OF_A ? p.m : p.n;
-        if (int e = settle_output(ctx, p.ksum, (size_t)len * dtype_size(p.dtype), true, &fresh)) return e;
-        p.ksum_accumulate = !fresh;
-        *fused = true;
-    } else {
-        p.ksum = nullptr;
-        p.ksum_of = KSUM_NONE;
-    }
-    return run_plan(ctx, p, plan);
+    return run_with_colsum(ctx, p, plan, fused);
 }
 
 }  // namespace dfdx_rocm
@@ -1050,9 +1068,7 @@ int dfdx_rocm_gemm(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc) {
     if (p.m == 0) return DFDX_ROCM_OK;
     Plan plan;  // from the product as the caller states it: a pending zero fill of C must not change which kernel runs
     if (int e = make_plan(ctx, desc, p, &plan)) return e;
-    if (int e = reserve_partials(ctx, p, plan, false)) return e;
-    if (int e = settle_operands(ctx, &p, /*may_overwrite=*/true)) return e;
-    return run_plan(ctx, p, plan);
+    return run_planned(ctx, p, plan);
 }
 
 int dfdx_rocm_gemm_noalloc(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc) {
@@ -1062,9 +1078,7 @@ int dfdx_rocm_gemm_noalloc(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc) 
     if (p.m == 0) return DFDX_ROCM_OK;
     Plan plan;  // from the product as the caller states it: a pending zero fill of C must not change which kernel runs
     if (int e = make_plan(ctx, desc, p, &plan)) return e;
-    if (int e = reserve_partials(ctx, p, plan, /*static_scratch=*/true)) return e;
-    if (int e = settle_operands(ctx, &p, /*may_overwrite=*/true)) return e;
-    return run_plan(ctx, p, plan, /*static_scratch=*/true);
+    return run_planned(ctx, p, plan, /*static_scratch=*/true);
 }
 
 int dfdx_rocm_gemm_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int *kernel, int *variant, char *name,

@@ -1,5 +1,7 @@
 """Products of the 16-bit types whose operands are copied onto the 16-byte grid for the LDS-DMA kernels: odd extents in each
 place, contractions that end inside a k tile, a C at any address, padded leading dimensions, batches, shared operands."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -8,7 +10,7 @@ import oracle
 from helpers import assert_within, rng
 from gpu_util import announce, device
 
-from dfdx_amd import View
+from dfdx_amd import Rocm, View
 from dfdx_amd.rocm import KERNEL_AUTO
 from test_gpu_gemm import run_case
 
@@ -104,7 +106,9 @@ def test_backward_products_share_one_copy_of_grad_out(dtype, rows, inp, out):
     gx, gw = torch.zeros_like(x), torch.zeros_like(w)
     for d in (dev.gemm_desc(dtype, rows, out, inp, g.data_ptr(), (out, 1), w.data_ptr(), (inp, 1), gx.data_ptr(), (inp, 1), accumulate=True),
               dev.gemm_desc(dtype, inp, rows, out, x.data_ptr(), (1, inp), g.data_ptr(), (out, 1), gw.data_ptr(), (1, inp), accumulate=True)):
-        announce("shared copy", dtype, rows, inp, out, dev.gemm_plan(d)[2])
+        name = dev.gemm_plan(d)[2]
+        announce("shared copy", dtype, rows, inp, out, name)
+        assert "_realigned" in name or out == 2112, name   # (2112 columns are whole k tiles: only one product needs a copy)
         dev.gemm(d)
     for fresh in (True, False):
         ox, ow, ob = view(torch.zeros_like(x)), view(torch.zeros_like(w)), view(torch.zeros_like(b))
@@ -139,3 +143,86 @@ def test_bias_gradient_taken_on_the_way_into_the_copy(dtype, rows, inp, out):
         want = g.double().sum(0) + before
         bound = want.abs() * 2.0 ** (-11 if dtype == "f16" else -8) + (g.double().abs().sum(0) + before.abs()) * rows * 2.0 ** -24 + 1e-7
         assert bool(((ob.storage.view(t).double() - want).abs() <= bound).all())
+
+
+def linear_operands(rows, inp, out):
+    view = lambda t: View(t.view(torch.uint8).reshape(-1), "f16", tuple(t.shape), tuple(t.stride()))
+    rnd = lambda *s: torch.randn(*s, device="cuda").half()
+    return [view(t) for t in (rnd(rows, inp), rnd(out, inp) / 32, rnd(out), rnd(rows, out))]
+
+
+def linear_gradients(dev, x, w, b, g):
+    grads = dev.zeros_many([x, w, b], deferred=True)
+    dev.linear_backward(x, grads[0], w, grads[1], grads[2], g)
+    dev.settle_zeros()
+    return grads
+
+
+def test_the_shared_copy_has_its_space_once():
+    """grad_out (4096 x 20001) is copied into one buffer; the input gradient's own space holds the weight's copy (41 MB) and partial sums
+    (at most 64 MB), and no second copy of grad_out (164 MB)."""
+    operands = linear_operands(4096, 1024, 20001)
+    linear_gradients(device(), *operands)
+    torch.cuda.synchronize()
+    announce("space of a shared copy")
+    own = Rocm(0)   # a context without buffers
+    grads = own.zeros_many(operands[:3], deferred=True)
+    own.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    own.linear_backward(operands[0], grads[0], operands[1], grads[1], grads[2], operands[3])
+    own.synchronize()
+    taken = before - torch.cuda.mem_get_info()[0]
+    own.close()
+    assert 160 << 20 < taken < 300 << 20, taken >> 20
+
+
+def test_shared_copy_without_room_for_it():
+    """On a stream that is being captured the context allocates nothing: each product reads its operands where they lie, with the same
+    bits; the bias gradient is summed by itself (f32 sums, one rounding)."""
+    dev = device()
+    operands = linear_operands(2048, 1024, 3001)
+    want = [dev.to_host(t).copy() for t in linear_gradients(dev, *operands)]
+    announce("shared copy, captured")
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        own = Rocm(0)
+        own.bias_backward(operands[3], own.zeros("f16", (3001,)))   # (room for the sums, 16 rows of them, and no more)
+        grads = [own.zeros("f16", t.shape) for t in operands[:3]]
+        own.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            own.linear_backward(operands[0], grads[0], operands[1], grads[1], grads[2], operands[3])
+        for _ in range(3):
+            for t in grads:
+                t.storage.zero_()
+            graph.replay()
+            own.synchronize()
+            got = [own.to_host(t) for t in grads]
+            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+            assert np.abs(got[2].astype(np.float64) - want[2].astype(np.float64)).max() <= 2.0 ** -10 * np.abs(want[2].astype(np.float64)).max()
+    own.close()
+
+
+def test_shared_copies_of_two_threads():
+    """The copy of grad_out lives in the context's buffer until both products have been launched: calls of other threads stay out."""
+    dev = device()
+    announce("shared copy, threads")
+    jobs = [linear_operands(2048 + 64 * t, 512, 2001 + 2 * t) for t in range(3)]
+    want = [[dev.to_host(t).copy() for t in linear_gradients(dev, *j)] for j in jobs]
+    got, errors = [[] for _ in jobs], []
+
+    def worker(i):
+        try:
+            for _ in range(8):
+                got[i].append([dev.to_host(t).copy() for t in linear_gradients(dev, *jobs[i])])
+        except Exception as e:  # surfaced in the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=worker, args=(i,)) for i in range(len(jobs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for runs, ref in zip(got, want):
+        assert len(runs) == 8 and all(np.array_equal(a, b) for run in runs for a, b in zip(run, ref))
