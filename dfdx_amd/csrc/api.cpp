@@ -24,33 +24,48 @@ static hipError_t free_retired(dfdx_rocm_ctx *ctx) {
         if (first == hipSuccess) first = e;
     }
     ctx->retired.clear();
+    ctx->retired_bytes = 0;
+    ctx->copies_refused = SIZE_MAX;  // (there may be room again)
     return first;
 }
 
 // The stream is not drained here: work already queued keeps the old buffer, which is retired, and the call in hand
-// gets a new one (only a failed allocation drains, frees what is retired and tries once more).
+// gets a new one.  (Drained all the same: when an allocation fails, which then is tried once more with everything retired freed, and
+// when the retired buffers hold kRetiredBytes.)  A buffer grows by half of itself at least, up to kGrowthBytes more than asked for, so that
+// sizes that rise step by step do not leave a buffer behind at every step.
 static int grow(dfdx_rocm_ctx *ctx, void **buf, size_t *have, size_t bytes) {
+    constexpr size_t kRetiredBytes = size_t(1) << 30, kGrowthBytes = size_t(256) << 20, kMb = size_t(1) << 20;
     CtxLock lock(ctx->mu);
     if (bytes <= *have) return DFDX_ROCM_OK;
+    bytes = (bytes + kMb - 1) & ~(kMb - 1);
+    const size_t roomy = std::max(bytes, std::min(*have + *have / 2, bytes + kGrowthBytes) & ~(kMb - 1));
     if (*buf) {
         ctx->retired.push_back(*buf);
+        ctx->retired_bytes += *have;
         *buf = nullptr;
         *have = 0;
     }
-    bytes = (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);
-    hipError_t e = hipMalloc(buf, bytes);
-    if (e == hipErrorOutOfMemory && !ctx->retired.empty()) {
-        (void)hipGetLastError();
+    if (ctx->retired_bytes >= kRetiredBytes) {
         HIP_TRY(hipStreamSynchronize(ctx->stream));
         (void)free_retired(ctx);
-        e = hipMalloc(buf, bytes);
+    }
+    size_t got = roomy;
+    hipError_t e = hipMalloc(buf, got);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        if (!ctx->retired.empty()) {
+            HIP_TRY(hipStreamSynchronize(ctx->stream));
+            (void)free_retired(ctx);
+        }
+        got = bytes;
+        e = hipMalloc(buf, got);
     }
     if (e != hipSuccess) {
         (void)hipGetLastError();  // the failed allocation must not surface again in the next launch check
         *buf = nullptr;
         return (int)e;
     }
-    *have = bytes;
+    *have = got;
     return DFDX_ROCM_OK;
 }
 
@@ -486,11 +501,16 @@ size_t partials_bytes(const GemmProblem &p, const Plan &plan, Realign *ra) {
     return 0;
 }
 
-// Nothing is allocated while the stream is being captured into a graph that the call could do without.
-bool may_grow(dfdx_rocm_ctx *ctx) {
+// Space that the call could do without is not asked for while the stream is being captured into a graph, nor where as much has been
+// refused since memory was last freed.
+bool grow_for_copies(dfdx_rocm_ctx *ctx, int (*ensure)(dfdx_rocm_ctx *, size_t), size_t bytes) {
+    if (bytes >= ctx->copies_refused) return false;
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess) (void)hipGetLastError();
-    return capturing == hipStreamCaptureStatusNone;
+    if (capturing != hipStreamCaptureStatusNone) return false;
+    if (ensure(ctx, bytes) == DFDX_ROCM_OK) return true;
+    ctx->copies_refused = bytes;
+    return false;
 }
 
 // Makes sure the partial sums of `plan` have a place, BEFORE the caller resolves pending zero fills among the operands:
@@ -505,7 +525,7 @@ int reserve_partials(dfdx_rocm_ctx *ctx, const GemmProblem &problem, Plan &plan,
         CtxLock lock(ctx->mu);
         auto room = [&](size_t need) {
             if (static_scratch) return need <= (size_t)DFDX_ROCM_NOALLOC_SCRATCH_BYTES;
-            return need <= ctx->workspace_bytes || (may_grow(ctx) && ensure_workspace(ctx, need) == DFDX_ROCM_OK);
+            return need <= ctx->workspace_bytes || grow_for_copies(ctx, ensure_workspace, need);
         };
         if (room(partials_bytes(p, plan))) return DFDX_ROCM_OK;
         const Plan plain = {plan.plain_kernel, plan.plain_variant, plan.plain_splits};
@@ -690,7 +710,7 @@ int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_r
     CtxLock lock(ctx->mu);  // the copy lives in the patch buffer until the second product has been launched
     int64_t ld = 0;
     const size_t bytes = realign_shared_bytes(rows, cols, &ld);
-    if (!both || bytes == 0 || (bytes > ctx->patches_bytes && (!may_grow(ctx) || ensure_patches(ctx, bytes) != DFDX_ROCM_OK))) return apart();
+    if (!both || bytes == 0 || (bytes > ctx->patches_bytes && !grow_for_copies(ctx, ensure_patches, bytes))) return apart();
     // each product with grad_out replaced by the copy: the space of its own copy is not asked for
     GemmProblem q[2] = {p[0], p[1]};
     for (int i = 0; i < 2; i++) {
@@ -710,7 +730,7 @@ int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_r
         if (!reserved.realign) return apart();
     }
     const size_t sums_bytes = fused && colsum ? bias_backward_copy_partials(ctx->compute_units, rows, cols, ld) : 0;
-    const bool sums = sums_bytes > 0 && (sums_bytes <= ctx->workspace_bytes || (may_grow(ctx) && ensure_workspace(ctx, sums_bytes) == DFDX_ROCM_OK));
+    const bool sums = sums_bytes > 0 && (sums_bytes <= ctx->workspace_bytes || grow_for_copies(ctx, ensure_workspace, sums_bytes));
     if (int e = settle(ctx, grad_out)) return e;
     if (sums) {  // on the way into the copy; their partials are done with the workspace before the products write it
         bool fresh = false;

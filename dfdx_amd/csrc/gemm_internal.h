@@ -140,6 +140,8 @@ struct Realign {
     double seconds;            // estimated time of the copies
     int off_grid, off_grid_k;  // operands whose rows are off the 16-byte grid; those of them that are stored along k
 };
+// The copies of one product: at most 2 GB of context memory (a batch of 16384 x a vocabulary of 50257 in 16 bits is 1.6 GB).
+constexpr size_t REALIGN_MAX_BYTES = size_t(2) << 30;
 bool plan_realign(const GemmProblem &p, Realign *r);  // false where a copy does not help (strides, sizes)
 hipError_t launch_realign(const GemmProblem &p, Realign *r, void *space, hipStream_t stream);  // copies and fills in the addresses
 // One rows x cols matrix (rows of `cols` elements, one behind the other) as an operand of either orientation: rows and columns

@@ -141,6 +141,7 @@ bool plan_realign(const GemmProblem &p, Realign *r) {
         q.b = (const void *)256;
         r->b_bytes = (size_t)up(b.pieces() * 16, 256);
     }
+    if (r->a_bytes + r->b_bytes > REALIGN_MAX_BYTES) return false;
     r->off_grid = a.off + b.off;
     r->off_grid_k = (a.off && a.kc) + (b.off && b.kc);
     // a launch and the gap behind it, a read and a write (2048 x 50257 and 50257 x 1024: 140 us)
@@ -151,7 +152,7 @@ bool plan_realign(const GemmProblem &p, Realign *r) {
 size_t realign_shared_bytes(int64_t rows, int64_t cols, int64_t *ld) {
     *ld = up(cols, 64);
     const int64_t pieces = up(rows, 64) * (*ld / 8);
-    return pieces < (1ll << 31) ? (size_t)pieces * 16 : 0;
+    return pieces < (1ll << 31) && (size_t)pieces * 16 <= REALIGN_MAX_BYTES ? (size_t)pieces * 16 : 0;
 }
 
 hipError_t launch_realign_shared(const void *src, int64_t rows, int64_t cols, void *dst, hipStream_t stream) {

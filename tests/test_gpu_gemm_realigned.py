@@ -226,3 +226,29 @@ def test_shared_copies_of_two_threads():
     assert not errors, errors
     for runs, ref in zip(got, want):
         assert len(runs) == 8 and all(np.array_equal(a, b) for run in runs for a, b in zip(run, ref))
+
+
+def test_copies_are_bounded():
+    """Two gigabytes of copies at most; beyond, and at leading dimensions that the copies need not, the operands are read where they lie."""
+    dev = device()
+    plan = lambda m, k, n: dev.gemm_plan(dev.gemm_desc("f16", m, k, n, 256, (k, 1), 512, (n, 1), 1024, (n, 1)))[2]   # (no launch)
+    assert "_realigned" in plan(20001, 20001, 20001) and "_realigned" not in plan(30001, 30001, 30001)
+
+
+def test_rising_sizes_do_not_leave_a_buffer_behind_at_every_step():
+    """Linear backward with a wide odd output and ever more rows, nothing synchronized through the library: the buffers grow by half of
+    themselves at least (copies of grad_out: 82, 123 and 185 MB; without that, 17 of 82 to 164 MB, and as many workspaces)."""
+    rows, out = 4096, 20001
+    x, w, b, g = linear_operands(rows, 1024, out)
+    part = lambda v, n: View(v.storage[:2 * n * v.shape[1]], v.dtype, (n, v.shape[1]), v.strides)
+    announce("rising sizes")
+    own = Rocm(0)
+    gx, gw, gb = (own.zeros("f16", v.shape) for v in (x, w, b))
+    own.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    for n in range(2048, rows + 1, 128):
+        own.linear_backward(part(x, n), part(gx, n), w, gw, gb, part(g, n))
+    torch.cuda.synchronize()
+    taken = before - torch.cuda.mem_get_info()[0]
+    own.close()
+    assert taken < 1000 << 20, taken >> 20
