@@ -199,7 +199,8 @@ __global__ __launch_bounds__(256, 3) void conv_few_forward_kernel(const Params p
 // f32, one rounding.  No single unit bounds it: LDS and the vector ALU are each busy a third of the time (74 us at the size above)
 // and the phases between barriers -- transpose, products -- do not overlap inside a workgroup.  XORing slots and pieces of the LDS
 // tile against bank conflicts of the stores measured level (73.7 us).
-// A tile that holds an infinity or a NaN goes through plain sums instead: those zeros would spread it over its cell.
+// Where a tile or the filters hold an infinity or a NaN, which those zeros would spread over its cell, the products are added position by
+// position: 147 -> 211 us for the whole backward at the size above with one infinite filter value (18.3 ms with plain sums of all taps).
 template <int C, int K, int S> struct GradImg {
     static constexpr int PAD = K / 2, Q = 2 / S;                                // positions of grad_out per cell
     static constexpr int WIN = S == 2 ? (K + 1) / 2 : K + 1, D0 = S == 2 ? -((K - 1 - PAD) / 2) : PAD - K + 1;  // window size, first offset
@@ -243,9 +244,11 @@ __global__ __launch_bounds__(256, 2) void conv_few_grad_img_kernel(const Params 
     // 32 channels are loaded while the products of these run.
     u32x4 next[G::UNITS][8];
     auto fetch = [&](const Place &t, int o0) {
+        int id = tid;
+        asm volatile("" : "+v"(id));  // (what is formed of it is formed here, not kept in registers under the products)
 #pragma unroll
         for (int n = 0; n < G::UNITS; n++) {
-            const int u = n * 256 + tid, g = u % 4, rest = u / 4, r = rest / t.octs, oct = t.oct0 + rest - r * t.octs, y = t.row0 + r;
+            const int u = n * 256 + id, g = u % 4, rest = u / 4, r = rest / t.octs, oct = t.oct0 + rest - r * t.octs, y = t.row0 + r;
             const bool ok = r < G::GO_ROWS && y >= 0 && y < p.h_out && oct >= 0 && oct * 8 < p.w_out;
             const uint16_t *src = p.go + ((int64_t)t.b * p.chan_out + o0 + g * 8) * plane + (int64_t)y * p.w_out + oct * 8;
 #pragma unroll
@@ -263,7 +266,6 @@ __global__ __launch_bounds__(256, 2) void conv_few_grad_img_kernel(const Params 
         f32x4 acc[G::PER_WAVE];
 #pragma unroll
         for (int t = 0; t < G::PER_WAVE; t++) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        bool bad = false;
         for (int ch = 0; ch < chunks; ch++) {
             uint8_t *const f_lds = smem + (ch % G::KEEP) * G::F_BYTES;
             const int o0 = ch * 32;
@@ -307,9 +309,11 @@ __global__ __launch_bounds__(256, 2) void conv_few_grad_img_kernel(const Params 
                 __syncthreads();
             }
             uint32_t nf = 0;
+            int id = tid;
+            asm volatile("" : "+v"(id));  // (as in fetch)
 #pragma unroll
             for (int n = 0; n < G::UNITS; n++) {
-                const int u = n * 256 + tid, g = u % 4, rest = u / 4, r = rest / at.octs, oct = at.oct0 + rest - r * at.octs;
+                const int u = n * 256 + id, g = u % 4, rest = u / 4, r = rest / at.octs, oct = at.oct0 + rest - r * at.octs;
 #pragma unroll
                 for (int j = 0; j < 8; j++)
 #pragma unroll
@@ -327,7 +331,7 @@ __global__ __launch_bounds__(256, 2) void conv_few_grad_img_kernel(const Params 
                     *(u32x4 *)(go_lds + (r * G::LINE + slot) * 64 + g * 16) = q;
                 }
             }
-            bad |= __syncthreads_or(nf != 0) != 0;
+            const bool masked = __syncthreads_or(nf != 0) != 0 || bad_filters;
             if (ch + 1 < chunks) fetch(at, o0 + 32);
             else if (item + (int)gridDim.x < p.items) fetch(place(item + gridDim.x), 0);
             // Fully unrolled with every address a constant away from one of the lane: tiles in different rows read the same operands
@@ -335,16 +339,39 @@ __global__ __launch_bounds__(256, 2) void conv_few_grad_img_kernel(const Params 
             constexpr int TW = G::CELLS / 16;
             const int row = wave * G::PER_WAVE / TW, tile0 = wave * G::PER_WAVE % TW;
             const uint8_t *const go_at = go_lds + (G::Q * row * G::LINE + tile0 * 16 + l16) * 64 + lq * 16;
+            if (__builtin_expect(!masked, 1)) {
 #pragma unroll
-            for (int u = 0; u < G::WIN; u++)
+                for (int u = 0; u < G::WIN; u++)
 #pragma unroll
-                for (int v = 0; v < G::WIN; v++) {
-                    const u32x4 f = *(const u32x4 *)(f_lds + ((u * G::WIN + v) * 64 + lane) * 16);
+                    for (int v = 0; v < G::WIN; v++) {
+                        const u32x4 f = *(const u32x4 *)(f_lds + ((u * G::WIN + v) * 64 + lane) * 16);
+                        const int slot = G::Q == 2 ? (v & 1) * G::HALF + (v >> 1) : v;
+#pragma unroll
+                        for (int t = 0; t < G::PER_WAVE; t++)
+                            acc[t] = Mma<T>::mfma16(f, *(const u32x4 *)(go_at + ((u + G::Q * (t / TW)) * G::LINE + slot + t % TW * 16) * 64), acc[t]);
+                    }
+            } else {
+                // An infinity or a NaN in the tile: every position's product by itself, added where a pixel has a tap at a position of
+                // grad_out, so that neither the zeros of the filter matrices nor those around grad_out meet it.
+#pragma unroll 1
+                for (int pos = 0; pos < G::WIN * G::WIN; pos++) {
+                    const int u = pos / G::WIN, v = pos % G::WIN;
+                    const u32x4 f = *(const u32x4 *)(f_lds + (pos * 64 + lane) * 16);
                     const int slot = G::Q == 2 ? (v & 1) * G::HALF + (v >> 1) : v;
+                    const int k1 = G::PAD - S * (G::D0 + u), k2 = G::PAD - S * (G::D0 + v);  // taps of a cell's first pixel
+                    int y0 = at.row0 + G::Q * row + u, x0 = at.col0 + G::Q * (tile0 * 16 + l16) + v;
+                    asm volatile("" : "+v"(y0), "+v"(x0));  // (formed here, not kept: the registers are the other loop's)
 #pragma unroll
-                    for (int t = 0; t < G::PER_WAVE; t++)
-                        acc[t] = Mma<T>::mfma16(f, *(const u32x4 *)(go_at + ((u + G::Q * (t / TW)) * G::LINE + slot + t % TW * 16) * 64), acc[t]);
+                    for (int t = 0; t < G::PER_WAVE; t++) {
+                        const f32x4 one = Mma<T>::mfma16(f, *(const u32x4 *)(go_at + ((u + G::Q * (t / TW)) * G::LINE + slot + t % TW * 16) * 64), f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+                        const int y = y0 + G::Q * (t / TW), x = x0 + G::Q * 16 * (t % TW);
+                        const bool inside = y >= 0 && y < p.h_out && x >= 0 && x < p.w_out;
+#pragma unroll
+                        for (int i = 0; i < 4; i++)
+                            if (inside && k1 + i / 2 >= 0 && k1 + i / 2 < K && k2 + i % 2 >= 0 && k2 + i % 2 < K) acc[t][i] += one[i];
+                    }
                 }
+            }
         }
         // lane: channel lq of cell l16 of every tile, its four pixels in the accumulator
 #pragma unroll
@@ -356,23 +383,6 @@ __global__ __launch_bounds__(256, 2) void conv_few_grad_img_kernel(const Params 
                 const int y = 2 * cy + a;
                 if (y >= p.h_in) continue;
                 float v[2] = {acc[t][2 * a], acc[t][2 * a + 1]};
-                if (bad || bad_filters) {
-                    for (int e = 0; e < 2; e++) {
-                        float sum = 0.0f;
-                        for (int o = 0; o < p.chan_out; o++)
-                            for (int k1 = 0; k1 < K; k1++) {
-                                const int ty = y + G::PAD - k1, oh = ty / S;
-                                if (ty < 0 || ty % S || oh >= p.h_out) continue;
-                                for (int k2 = 0; k2 < K; k2++) {
-                                    const int tx = 2 * cx + e + G::PAD - k2, ow = tx / S;
-                                    if (tx < 0 || tx % S || ow >= p.w_out) continue;
-                                    sum += Mma<T>::to_f32(p.filters[((int64_t)(o * C + lq) * K + k1) * K + k2]) *
-                                           Mma<T>::to_f32(p.go[((int64_t)b * p.chan_out + o) * plane + (int64_t)oh * p.w_out + ow]);
-                                }
-                            }
-                        v[e] = sum;
-                    }
-                }
                 uint32_t *dst = (uint32_t *)(p.grad_img + ((int64_t)(b * C + lq) * p.h_in + y) * p.w_in + 2 * cx);
                 if (!p.fresh) {
                     const uint32_t old = *dst;

@@ -41,11 +41,11 @@ def check(what, got, want, mag, terms, dtype, old=None):
 @pytest.mark.parametrize("batch,cin,cout,h,w,k,stride", [
     (2, 3, 64, 32, 224, 7, 2),
     (3, 3, 64, 37, 48, 7, 2),      # odd height: a cell row cut in half, a last band of few rows
-    (1, 1, 70, 18, 272, 7, 2),     # a second group of 64 channels, a third block of 32, 136 cells
+    (1, 1, 70, 18, 272, 7, 2),     # a second group of 64 channels in the forward (the backward goes through the patch matrix), 136 cells
     (2, 3, 33, 16, 32, 5, 2),
     (2, 1, 16, 9, 16, 3, 2),
     (2, 3, 64, 21, 40, 3, 1),
-    (1, 3, 130, 16, 72, 3, 1),
+    (1, 3, 130, 16, 72, 3, 1),     # (so does the backward of this one)
     (2, 3, 24, 13, 64, 5, 1),
     (1, 1, 10, 28, 32, 5, 1),
     (1, 3, 32, 10, 24, 7, 1),      # (the backward of this one goes through the patch matrix)
@@ -107,3 +107,67 @@ def test_infinities_reach_what_reads_them_and_nothing_else(stride, k):
     assert torch.allclose(torch.where(reach, 0, a).float(), torch.where(reach, 0, b).float(), rtol=2e-3, atol=2e-3)
     other = torch.arange(64) != 5
     assert torch.equal(fa[other], fb[other]) and bool(torch.isnan(fb[5]).all())
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("k,stride,hw", [(7, 2, (37, 48)), (5, 2, (18, 32)), (3, 2, (9, 16)), (5, 1, (13, 64)), (3, 1, (21, 40))])
+@pytest.mark.parametrize("where", ["filter", "gradient", "corner", "both"])
+def test_image_gradient_of_infinities(dtype, k, stride, hw, where):
+    """An infinite filter value or gradient: infinities and NaN where the sums over a pixel's taps have them (and not where a tap
+    lies outside of the output), and the other pixels within the bound of finite values."""
+    dev, (batch, cin, cout), pad = device(), (2, 3, 40), k // 2
+    h, w = hw
+    announce("conv few, infinities", dtype, k, stride, where)
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, f = rnd(batch, cin, h, w).to(TYPES[dtype]), (rnd(cout, cin, k, k) / 10).to(TYPES[dtype])
+    ho, wo = (h - 1) // stride + 1, (w - 1) // stride + 1
+    g = rnd(batch, cout, ho, wo).to(TYPES[dtype])
+    if where in ("filter", "both"):
+        f[35, 1, 0, k - 1] = float("inf")
+    if where in ("gradient", "both"):
+        g[1, 7, ho // 2, wo // 2] = float("-inf")
+    if where == "corner":
+        g[0, 39, 0, 0], g[1, 0, ho - 1, wo - 1] = float("inf"), float("-inf")
+    gi, gf = dev.zeros_many([view(x, dtype), view(f, dtype)], deferred=True)
+    dev.conv2d_backward(view(x, dtype), gi, view(f, dtype), gf, view(g, dtype), stride=stride, padding=pad)
+    dev.settle_zeros()
+    got = gi.storage.view(TYPES[dtype]).reshape(x.shape).double().cpu()
+    want, mag = torch.zeros(x.shape, dtype=torch.float64), torch.zeros(x.shape, dtype=torch.float64)
+    f64, g64 = f.double().cpu(), g.double().cpu()
+    for k1 in range(k):   # tap by tap, over the outputs that a tap reads from inside of the image
+        rows = [o for o in range(ho) if 0 <= o * stride + k1 - pad < h]
+        for k2 in range(k):
+            cols = [o for o in range(wo) if 0 <= o * stride + k2 - pad < w]
+            part = g64[:, :, rows][:, :, :, cols]
+            y, z = rows[0] * stride + k1 - pad, cols[0] * stride + k2 - pad
+            at = (slice(None), slice(None), slice(y, y + (len(rows) - 1) * stride + 1, stride), slice(z, z + (len(cols) - 1) * stride + 1, stride))
+            want[at] += torch.stack([(f64[None, :, c, k1, k2, None, None] * part).sum(1) for c in range(cin)], 1)
+            mag[at] += torch.stack([(f64[None, :, c, k1, k2, None, None] * part).abs().sum(1) for c in range(cin)], 1)
+    finite = torch.isfinite(want)
+    assert bool((~finite).any()) and bool(finite.any())
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
+    check("grad_img", got[finite], want[finite], mag[finite], cout * k * k, dtype)
+
+
+def test_an_infinite_filter_does_not_stall_the_step():
+    """A step whose values have overflowed is worth nothing and has to end all the same: within four times a finite one's time."""
+    dev, dtype = device(), "f16"
+    x, f, g = torch.randn(16, 3, 224, 224, device="cuda").half(), torch.randn(64, 3, 7, 7, device="cuda").half(), torch.randn(16, 64, 112, 112, device="cuda").half()
+    gi, gf = dev.zeros(dtype, x.shape), dev.zeros(dtype, f.shape)
+
+    def best():
+        times = []
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            dev.conv2d_backward(view(x, dtype), gi, view(f, dtype), gf, view(g, dtype), stride=2, padding=3)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    announce("conv few, time of an infinite filter")
+    finite = best()
+    f[3, 1, 2, 2] = float("inf")
+    assert best() < 4 * finite + 0.1
