@@ -408,7 +408,7 @@ __global__ __launch_bounds__(256, 2) void conv_few_grad_filters_kernel(const Par
     constexpr int KK = K * K, TAPS = C * KK, NB = (TAPS + 31) / 32, PAD = K / 2;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, h = lane / 32, l32 = lane % 32, ob = wave / 2;
-    const int o0 = blockIdx.y * 64, channels = min(64, p.chan_out - o0);
+    const int channels = p.chan_out;  // at most 64
     const int in_max = (p.band - 1) * S + K, plane_pitch = S == 2 ? p.w_in / 2 + 8 : p.w_in + 16, pitch = S * plane_pitch;
     const int go_pitch = p.band * p.w_out + 8, octs_row = p.w_out / 8, octs_line = p.w_in / 8 + 2;
     uint16_t *const go_lds = (uint16_t *)smem, *const img_lds = go_lds + 64 * go_pitch;
@@ -441,7 +441,7 @@ __global__ __launch_bounds__(256, 2) void conv_few_grad_filters_kernel(const Par
 #pragma unroll
         for (int n = 0; n < GO_UNITS; n++) {
             const int u = n * 256 + tid, o = u / t.octs, oct = u - o * t.octs;
-            if (o < channels) go_next[n] = *(const u32x4 *)(p.go + ((int64_t)(t.b * p.chan_out + o0 + o) * p.h_out + t.first) * p.w_out + oct * 8);
+            if (o < channels) go_next[n] = *(const u32x4 *)(p.go + ((int64_t)(t.b * channels + o) * p.h_out + t.first) * p.w_out + oct * 8);
         }
         const int in_rows = (t.rows - 1) * S + K, y0 = t.first * S - PAD;
 #pragma unroll
@@ -515,16 +515,16 @@ __global__ __launch_bounds__(256, 2) void conv_few_grad_filters_kernel(const Par
         }
     }
     __syncthreads();
-    float *ws = p.ws + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 64 * TAPS;
+    float *ws = p.ws + (int64_t)blockIdx.x * 64 * TAPS;
     for (int i = tid; i < channels * TAPS; i += 256) ws[i] = sums[i / TAPS * (32 * NB) + i % TAPS];
 }
 
-// 32 sums of one 64-channel group per workgroup, the workgroups' shares in eight runs, in order.
+// 32 sums per workgroup, the workgroups' shares in eight runs, in order.
 template <typename T>
 __global__ __launch_bounds__(256) void conv_few_grad_filters_add_kernel(const float *ws, int shares, int taps, int chan_out, uint16_t *grad_filters) {
     __shared__ float part[8][32];
-    const int lane = threadIdx.x % 32, run = threadIdx.x / 32, i = blockIdx.x * 32 + lane, n = min(64, chan_out - (int)blockIdx.y * 64) * taps;
-    const float *src = ws + (int64_t)blockIdx.y * shares * 64 * taps + min(i, n - 1);
+    const int lane = threadIdx.x % 32, run = threadIdx.x / 32, i = blockIdx.x * 32 + lane, n = chan_out * taps;
+    const float *src = ws + min(i, n - 1);
     const int per = (shares + 7) / 8, s1 = min(shares, (run + 1) * per);
     float sum = 0.0f;
     int s = run * per;
@@ -541,7 +541,7 @@ __global__ __launch_bounds__(256) void conv_few_grad_filters_add_kernel(const fl
     if (run == 0 && i < n) {
 #pragma unroll
         for (int r = 1; r < 8; r++) sum += part[r][lane];
-        uint16_t *dst = grad_filters + (int64_t)blockIdx.y * 64 * taps + i;
+        uint16_t *dst = grad_filters + i;
         *dst = (uint16_t)Mma<T>::pack2(Mma<T>::to_f32(*dst) + sum, 0.0f);
     }
 }
@@ -633,10 +633,10 @@ template <typename T, int C, int K, int S> hipError_t backward_run(const ConvFew
     p.ws = (float *)workspace;
     const size_t lds = grad_filters_lds(c, p.band);
     if (hipError_t e = allow_lds<conv_few_grad_filters_kernel<T, C, K, S>>(lds)) return e;
-    const int shares = grad_filters_shares(c), groups = (c.chan_out + 63) / 64, taps = C * K * K;
-    conv_few_grad_filters_kernel<T, C, K, S><<<dim3((unsigned)shares, (unsigned)groups), 256, lds, stream>>>(p);
+    const int shares = grad_filters_shares(c), taps = C * K * K;
+    conv_few_grad_filters_kernel<T, C, K, S><<<(unsigned)shares, 256, lds, stream>>>(p);
     if (hipError_t e = hipGetLastError()) return e;
-    conv_few_grad_filters_add_kernel<T><<<dim3((unsigned)((64 * taps + 31) / 32), (unsigned)groups), 256, 0, stream>>>(p.ws, shares, taps, c.chan_out, p.grad_filters);
+    conv_few_grad_filters_add_kernel<T><<<(unsigned)((c.chan_out * taps + 31) / 32), 256, 0, stream>>>(p.ws, shares, taps, c.chan_out, p.grad_filters);
     return hipGetLastError();
 }
 
@@ -677,7 +677,7 @@ bool conv_few_backward_supported(const ConvFew &c) {
     return shape_ok(c) && !(c.kernel == 7 && c.stride == 1) && c.chan_out <= 64 && aligned16(c.grad_out) && ((uintptr_t)c.grad_img & 3u) == 0 && grad_filters_band(c) > 0;
 }
 size_t conv_few_workspace_bytes(const ConvFew &c) {
-    return (size_t)grad_filters_shares(c) * ((c.chan_out + 63) / 64) * 64 * c.chan_in * c.kernel * c.kernel * sizeof(float);
+    return (size_t)grad_filters_shares(c) * 64 * c.chan_in * c.kernel * c.kernel * sizeof(float);
 }
 
 hipError_t launch_conv_few_backward(const ConvFew &c, void *workspace, hipStream_t stream) {

@@ -32,7 +32,7 @@ struct Shape {
     bool fused;    // attention without the (seq, seq) matrices
     double scale;  // 1 / sqrt(D)
     bool folded;   // the softmax entry's float scale is exact enough (f64: only when the value is)
-    int64_t token[3], none;
+    int64_t token[3];
 };
 
 int shape_of(const dfdx_rocm_encoder *e, Shape *s) {
@@ -224,8 +224,7 @@ int backward(dfdx_rocm_ctx *ctx, const Shape &s, const dfdx_rocm_encoder *e, con
         TRY(dfdx_rocm_attention_backward(ctx, s.dtype, s.B, s.H, s.S, s.D, q, k, v, s.token, (float)s.scale, tok, gtok, s.token,
                                          (const float *)(saved + l.lse), gq, gk, gv));
     } else {
-        const void *probs = saved + l.probs, *tokens = saved + l.tokens;
-        (void)tokens;
+        const void *probs = saved + l.probs;
         void *gtokens = scratch + at.take(act), *gp = scratch + at.take(mat), *gscores = scratch + at.take(mat);
         void *gscaled = s.folded ? gscores : scratch + at.take(mat);
         TRY(dfdx_rocm_zero_deferred(ctx, gtokens, act));
