@@ -1,9 +1,15 @@
 """GPU: the encoder block's two calls against the same block strung together from the single entry points (Linear, the fused
-attention or its ops, LayerNorm, ReLU, add and their backward): every output and gradient equal bit for bit, since what the
-block's products do on the way into their results (ReLU, residual, ReLU's gradient, a first contribution read from elsewhere)
-rounds where the separate op would.  The shapes reach the small, the split and the tiled kernels, whole tiles and edges."""
+attention or its ops, LayerNorm, ReLU, add and their backward).  What the block's products do on the way into their results (ReLU,
+residual, ReLU's gradient, a first contribution read from elsewhere) rounds where the separate op would, so the output and the
+gradients are equal bit for bit, but for two things.  In 16 bits grad_x is one f32 sum rounded once where the single calls round four;
+and where ReLU's gradient is cheap enough as a small product on its own, the plan differs from that of a product that adds
+to its result, and with it the order of the sum.  These are bounded per element and in the norm.  The shapes reach the small, the split and
+the tiled kernels, whole tiles and edges."""
+import ctypes
+
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from helpers import rng
@@ -11,7 +17,7 @@ from gpu_util import announce, device
 
 pytestmark = pytest.mark.gpu
 
-from dfdx_amd import EncoderBlock, View  # noqa: E402
+from dfdx_amd import EncoderBlock, Rocm, View  # noqa: E402
 from dfdx_amd.encoder import PARAMS  # noqa: E402
 
 
@@ -73,13 +79,16 @@ def test_block_equals_its_ops(dtype, B, S, d, H, ff):
     want, wg, wgx = by_ops(dev, dtype, p, x, go, H)
     dev.synchronize()
     pairs = {"out": (out, want), "x": (gx, wgx)} | {n: (grads[n], wg[n]) for n in PARAMS}
-    tol = 5 * (4e-6 + {"f16": 2.0 ** -12, "bf16": 2.0 ** -9, "f32": 0.0}[dtype])
+    eps = {"f16": 2.0 ** -12, "bf16": 2.0 ** -9, "f32": 0.0}[dtype]
+    behind_relu = ("wq", "bq", "wk", "bk", "wv", "bv", "wo", "bo", "g1", "be1", "w1", "b1")   # what ReLU's gradient reaches
     for n, (a, b) in pairs.items():
-        a, b = oracle.to_f64(dev.to_host(a), dtype), oracle.to_f64(dev.to_host(b), dtype)
-        if n == "out":
-            assert np.array_equal(a, b), np.abs(a - b).max()
+        a, b = (oracle.to_f64(dev.to_host(t), dtype)[:int(np.prod(b.shape))] for t in (a, b))
+        if dtype == "f32" or not (n == "x" or (n in behind_relu and (B, S, d) == (3, 100, 256))):
+            assert np.array_equal(a, b), (n, np.abs(a - b).max())
         elif n != "bk":   # a shift of all scores of a row: its gradient is the rounding of zero
-            assert np.linalg.norm(a - b) <= tol * np.linalg.norm(b), (n, np.linalg.norm(a - b) / np.linalg.norm(b))
+            assert np.linalg.norm(a - b) <= 5 * (4e-6 + eps) * np.linalg.norm(b), (n, np.linalg.norm(a - b) / np.linalg.norm(b))
+            # five roundings of sums that are twice the largest result at most, each half a unit in the last place (2 eps)
+            assert np.abs(a - b).max() <= 20 * eps * np.abs(b).max(), (n, np.abs(a - b).max() / np.abs(b).max())
     assert saved["f1"].shape == (B, S, ff) and saved["probs"].shape == (B, H, S, S) and saved["tokens"].shape == (B, H, S, d // H)
 
 
@@ -198,3 +207,36 @@ def test_no_stale_value_is_made():
         late["f1"]
     assert np.array_equal(device().to_host(saved["f1"]), before)
     assert set(late) == KEPT
+
+
+def graph_nodes(run, stream):
+    """Launches of `run`: the nodes of the graph it is captured into."""
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=stream):
+        keep = run()
+    with open("/proc/self/maps") as maps:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    n = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    del keep
+    return n.value
+
+
+@pytest.mark.parametrize("shape,forward,backward", [((16, 128, 512, 8, 1024), 7, None), ((16, 512, 1024, 16, 4096), 7, 18)])
+def test_three_projections_are_one_launch(shape, forward, backward):
+    """Forward: the projections, the attention, three products and two LayerNorms.  Backward: two launches for each LayerNorm
+    and for the attention, four input gradients (one for all projections) and four weight gradients with their combines."""
+    block, x, go = a_block("bf16", *shape)
+    announce("encoder block, launches", shape)
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        own = Rocm(0)
+        block = EncoderBlock(own, "bf16", *shape[2:], block.p)
+        _, saved = block.forward(x)
+        block.backward(saved, go)   # (the workspaces have their sizes before a capture)
+        own.synchronize()
+        assert graph_nodes(lambda: block.forward(x), stream) == forward
+        assert backward is None or graph_nodes(lambda: block.backward(saved, go), stream) == backward
+        own.synchronize()
+    own.close()
