@@ -12,6 +12,8 @@ from gpu_util import announce, device
 
 pytestmark = pytest.mark.gpu
 
+from dfdx_amd import View  # noqa: E402
+
 
 def reference(q, k, v, g, scale):
     s = scale * q @ k.swapaxes(-1, -2)
@@ -173,3 +175,61 @@ def test_infinities_reach_what_depends_on_them_and_nothing_else(dtype, case, S, 
         if ok.any():
             err = np.abs(got[ok] - ref[ok]).max()
             assert err <= 8 * eps * np.abs(ref[ok]).max() + floor * (name in ("dq", "dk")), (name, err)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("S,D", [(65, 64), (130, 32), (33, 128)])
+@pytest.mark.parametrize("layout", ["heads in front", "one of three in a row", "padded rows"])
+def test_strides_and_offsets(dtype, S, D, layout):
+    """Views of other strides than the token layout, offsets of whole 16-byte pieces included: the same sums in the same order, so
+    the bits of contiguous tokens, and nothing written between the rows of a gradient."""
+    dev = device()
+    B, H = 2, 3
+    announce("attention, strides", dtype, S, D, layout)
+    d = H * D
+    strides, offset, size = {"heads in front": ((H * S * D, S * D, D), 0, B * S * d), "one of three in a row": ((S * 3 * d, D, 3 * d), d, B * S * 3 * d),
+                             "padded rows": ((S * (d + 16), D, d + 16), 8, B * S * (d + 16) + 8)}[layout]
+    g = rng(S + D)
+    at = offset + sum(np.arange(n).reshape([-1 if i == j else 1 for j in range(4)]) * s for i, (n, s) in enumerate(zip((B, H, S, D), (*strides, 1))))
+    tokens = [oracle.to_storage(g.standard_normal(B * S * d), dtype) for _ in range(4)]
+    spread = []
+    for t in tokens[:3]:
+        u = np.zeros(size, t.dtype)
+        u[at] = t.reshape(B, S, H, D).swapaxes(1, 2)
+        spread.append(u)
+    token = (S * d, D, d, 1)
+    go = dev.tensor(tokens[3], dtype, (B, S, d))
+
+    def both(storages, st, off):
+        q, k, v = (View(dev.tensor(t, dtype).storage, dtype, (B, H, S, D), st, off) for t in storages)
+        out, lse = dev.attention_forward(q, k, v, D ** -0.5)
+        grads = [View(dev.zeros(dtype, (len(storages[0]),)).storage, dtype, (B, H, S, D), st, off) for _ in range(3)]
+        dev.attention_backward(q, grads[0], k, grads[1], v, grads[2], D ** -0.5, out, go, lse)
+        return dev.to_host(out), [dev.to_host(View(t.storage, dtype, (), ())) for t in grads]
+
+    out, grads = both(spread, (*strides, 1), offset)
+    want, wgrads = both(tokens[:3], token, 0)
+    assert np.array_equal(out.view(np.uint16), want.view(np.uint16))
+    for a, b in zip(grads, wgrads):
+        assert np.array_equal(a[at].view(np.uint16), b.reshape(B, S, H, D).swapaxes(1, 2).view(np.uint16))
+        a[at] = 0
+        assert not a.any()
+
+
+@pytest.mark.parametrize("wrong", ["address", "row stride", "scale", "result's address"])
+def test_what_the_pieces_of_16_bytes_cannot_walk_is_refused(wrong):
+    from dfdx_amd import RocmError
+    from dfdx_amd.rocm import DTYPES, _i64s
+
+    dev = device()
+    B, H, S, D = 1, 2, 16, 64
+    room = dev.zeros("f16", (B, S, H * (D + 8) + 64))
+    strides = (S * H * D, D, H * D + (4 if wrong == "row stride" else 0))
+    x = View(room.storage, "f16", (B, H, S, D), (*strides, 1), 1 if wrong == "address" else 0)
+    scale, out = 0.0 if wrong == "scale" else 0.125, dev.zeros("f16", (B, S, H * D + 8))
+    rc = dev._f.attention_forward(dev.ctx, DTYPES["f16"], B, H, S, D, x.ptr, x.ptr, x.ptr, _i64s(strides), scale,
+                                  out.ptr + (2 if wrong == "result's address" else 0), _i64s((S * H * D, D, H * D)), None)
+    assert rc == -2   # DFDX_ROCM_ERR_UNSUPPORTED
+    if wrong != "result's address":
+        with pytest.raises(RocmError):
+            dev.attention_forward(x, x, x, scale)
