@@ -52,7 +52,10 @@ KEPT = ("x", "qv", "kv", "vv", "probs", "tokens", "tok", "h1", "n1", "f1", "r1",
 
 def _version(storage):
     """torch's count of changes in place (``None`` where it keeps none)."""
-    return None if storage.is_inference() else storage._version
+    try:
+        return storage._version
+    except RuntimeError:   # an inference tensor
+        return None
 
 
 class _Saved(dict):
@@ -60,12 +63,16 @@ class _Saved(dict):
     asks for them, most of them Views into the one allocation ``arena``.  ``backward`` takes it as it is, or with values replaced or
     changed, or any dict with the same names."""
 
+    __slots__ = ("made", "block", "plan", "arena", "version", "versions", "behind_f1")
+
     def __init__(self, block: "EncoderBlock", plan: _Plan, x: View, arena):
-        super().__init__(x=x)
-        self.block, self.plan, self.arena = block, plan, arena
         self.made = {"x": x}
-        self.versions = {None: (arena, _version(arena))}   # storages whose contents stand for what the forward left
-        self.behind_f1 = [(block.p[n], _version(block.p[n].storage)) for n in ("w1", "b1")]
+        super().__init__(self.made)
+        self.block, self.plan, self.arena = block, plan, arena
+        self.version = _version(arena)   # its contents stand for what the forward left, and those of `versions`
+        self.versions = {}
+        w1, b1 = block.p["w1"], block.p["b1"]
+        self.behind_f1 = w1, _version(w1.storage), b1, _version(b1.storage)
 
     def __missing__(self, name):
         value = self._make(name)
@@ -76,8 +83,12 @@ class _Saved(dict):
 
     def untouched(self) -> bool:
         """Whether the names still stand for what the forward left."""
-        return all(dict.get(self, n, v) is v for n, v in self.made.items()) and \
-            all(n in self.made for n in dict.keys(self) if n in KEPT) and \
+        if _version(self.arena) != self.version:
+            return False
+        made = self.made
+        if len(made) == dict.__len__(self) == 1:   # (x, which nobody has asked about)
+            return dict.get(self, "x") is made["x"]
+        return all(dict.get(self, n, v) is v for n, v in made.items()) and all(n in made for n in dict.keys(self) if n in KEPT) and \
             all(_version(storage) == v for storage, v in self.versions.values())
 
     def _make(self, name):
@@ -100,7 +111,9 @@ class _Saved(dict):
         if name == "r1":
             return at(l.r1, (B, S, ff))
         if name == "f1":
-            if any(self.block.p[n] is not v or _version(v.storage) != at_forward for n, (v, at_forward) in zip(("w1", "b1"), self.behind_f1)):
+            w1, b1 = self.block.p["w1"], self.block.p["b1"]
+            at_w1, version_w1, at_b1, version_b1 = self.behind_f1
+            if w1 is not at_w1 or b1 is not at_b1 or (_version(w1.storage), _version(b1.storage)) != (version_w1, version_b1):
                 raise RuntimeError("f1 is formed on request, from w1 and b1: they have changed since the forward")
             return dev.linear_forward(self["n1"], self.block.p["w1"], self.block.p["b1"])
         if name == "scale":
