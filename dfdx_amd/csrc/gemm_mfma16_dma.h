@@ -212,7 +212,9 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
     // work items blockIdx.x, blockIdx.x + gridDim.x, ... and keeps ONE load pipeline running across them, so
     // the stores of a finished tile overlap with the loads (already in flight) and MFMAs of the next one.
     // The arguments that only a work item's start and end need are read from memory there, not held in scalar registers
-    // through the k loop (4096^3 f16, registers spilled to vector lanes: 17 - 32 with all arguments held, none now).
+    // through the k loop (4096^3 f16, registers spilled to vector lanes: 17 - 32 with all arguments held, none now).  Small tiles gain:
+    // 1024^3 f16 12.2 -> 11.6 us, 8192 x 1024 x 64 12.4 -> 11.9; with the plain instances holding them 12.0 and 12.3, and the large
+    // products, which lost 0.5 - 1.7 % when batches that lie anywhere came in, level (4096^3 103.2 and 103.2, the 256-row ones 0.5 % slower).
     typedef const __attribute__((address_space(4))) Params ArgParams;
     auto late_args = [&]() -> ArgParams * {
         ArgParams *args = (ArgParams *)__builtin_amdgcn_kernarg_segment_ptr();
