@@ -699,7 +699,8 @@ int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_r
             continue;
         }
         if (int e = make_plan(ctx, d, p[i], &plan[i])) return e;
-        both = both && plan[i].realign && p[i].a != p[i].b && plan_realign(p[i], &ra) && (p[i].a == grad_out ? ra.a : ra.b);
+        // (one matrix each: the batches that a broadcast gradient is summed over step through grad_out by strides of their own)
+        both = both && plan[i].realign && p[i].nb1 * p[i].nb2 == 1 && p[i].a != p[i].b && plan_realign(p[i], &ra) && (p[i].a == grad_out ? ra.a : ra.b);
     }
     auto apart = [&]() -> int {
         if (p[0].m)
