@@ -393,14 +393,16 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
     const bool may_small = forced_splits == 0 && (is16 || is64) && small_supported(p);
     const double t_small = may_small ? small_time(p, ctx->compute_units) : 1e300;
     const Plan small_plan = {DFDX_ROCM_KERNEL_MFMA, is16 ? mfma16_small_variant() : mfma64_small_variant(), 1};
+    Plan ring_plan = {};
+    double t_ring = 1e300;
     if (is16) {
         int dv = 0, splits = 1;
         double t_dma = 1e300;
         mfma16dma_plan_split(p, ctx->compute_units, 0, forced_splits, &dv, &splits, &t_dma);
-        if (dv) {
-            // that family's estimate ranks its own tiles and split counts; on products of a few microseconds it runs
-            // 1 - 2 us above the clock, and 8 us above it for a split plan
-            t_dma -= splits > 1 ? 6.5e-6 : 1.0e-6;
+        if (dv && p.k % 64) {  // (one of the tiles that take any k: weighed against the families below)
+            t_ring = t_dma;
+            ring_plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
+        } else if (dv) {
             *plan = t_small < t_dma ? small_plan : Plan{DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
             double t_best = std::min(t_small, t_dma);
             int skinny_splits = 1;
@@ -437,22 +439,32 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         // write a large C at 2.2 TB/s.  f16, staged and on copies: 2048 x 50257 x 1024 563 and 325 us, 4095^3 293 and 143, 1315 x
         // 2340 x 3033 150 and 52, 530 x 3231 x 1057 84 and 28, 6928 x 106 x 7330 80 and 43; and where the line leaves the
         // staged kernels: 1000^3 12.0 and 18.8, 304 x 611 x 4120 11.0 and 16.4, 448 x 315 x 4890 13.2 and 14.5.
+        double t_copies = 1e300;
         if (realignable) {
             int dv = 0, splits = 1;
-            double t_dma = 1e300;
-            mfma16dma_plan_split(ra.problem, ctx->compute_units, 0, forced_splits, &dv, &splits, &t_dma);
+            mfma16dma_plan_split(ra.problem, ctx->compute_units, 0, forced_splits, &dv, &splits, &t_copies);
             // (a product whose plan without copies fits the fixed scratch array fits it in this form too: see dfdx_rocm_gemm_noalloc)
             const size_t piece = mfma16_workspace_bytes(p, v, 2) / 2, most = DFDX_ROCM_NOALLOC_SCRATCH_BYTES;
             if (dv && splits > 1 && !forced_splits && piece * (size_t)splits > most && partials_bytes(p, *plan) <= most)
-                mfma16dma_plan_split(ra.problem, ctx->compute_units, 0, (int)std::max<size_t>(1, most / piece), &dv, &splits, &t_dma);
+                mfma16dma_plan_split(ra.problem, ctx->compute_units, 0, (int)std::max<size_t>(1, most / piece), &dv, &splits, &t_copies);
+            // (copies are not taken for a gain within the estimates' error)
+            t_copies = dv ? t_copies + ra.seconds + (mfma16dma_takes_any_k(dv) ? 0.0 : splits > 1 ? 6.5e-6 : 1.0e-6) : 1e300;
             const bool small_tile = v == mfma16_skinny_variant();
             const double t_staged = t_family * (small_tile ? (ra.off_grid ? 1.0 : 0.6) : ra.off_grid ? 1.4 : 0.95) +
                                     (small_tile ? 0.0 : 2.0 * (double)p.m * (double)p.n * (double)(p.reduce ? 1 : p.nb1 * p.nb2) / 2.2e12);
-            if (dv && t_dma + ra.seconds < std::min(std::min(t_small_here, t_staged), t_bw)) {
+            if (t_copies < std::min(std::min(t_small_here, t_staged), t_bw)) {
                 const Plan plain = *plan;
                 *plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits, true, v, plain.kernel, plain.variant, plain.splits};
             }
         }
+        // (on operands in place with k off 64 the staged tiles run at 0.83 - 1.06 of the estimate: 528 x 1024 x 1325 f16 21.4 us for 25.6,
+        // 2304 x 128 x 1534 in three pieces 16.2 for 15.3; the ring 9.4 both)
+        const double t_plan = plan->realign ? t_copies : plan->kernel == DFDX_ROCM_KERNEL_GEMV ? t_bw : plan->variant == v ? 0.85 * t_family : t_small_here;
+        if (t_ring < t_plan) *plan = ring_plan;
+        return DFDX_ROCM_OK;
+    }
+    if (t_ring < std::min(t_small, t_bw)) {
+        *plan = ring_plan;
         return DFDX_ROCM_OK;
     }
     if (bw) {  // no tiled kernel takes these strides, the multi-vector kernel does
@@ -752,7 +764,7 @@ int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_r
 int gemm_three(dfdx_rocm_ctx *ctx, const GemmProblem &problem, bool *done) {
     *done = false;
     GemmProblem p = problem;
-    if ((p.dtype != DT_F16 && p.dtype != DT_BF16) || p.k % 64) return DFDX_ROCM_OK;
+    if (p.dtype != DT_F16 && p.dtype != DT_BF16) return DFDX_ROCM_OK;
     p.compute_units = ctx->compute_units;
     int dv = 0, splits = 1, dv1 = 0, splits1 = 1;
     double t3 = 1e300, t1 = 1e300;
@@ -764,12 +776,10 @@ int gemm_three(dfdx_rocm_ctx *ctx, const GemmProblem &problem, bool *done) {
     q.nb1 = q.nb2 = 1;
     q.reduce = 0;
     mfma16dma_plan_split(q, ctx->compute_units, 0, 0, &dv1, &splits1, &t1);
-    t1 -= splits1 > 1 ? 6.5e-6 : 1.0e-6;  // (as in make_plan)
-    t3 -= splits > 1 ? 6.5e-6 : 1.0e-6;
     const double t_small = small_supported(q) ? small_time(q, ctx->compute_units) : 1e300;
     // Results that replace those of three calls have the bits of those: the order of the contraction is that of the tiles, so the
     // small kernel and split plans are no match.  (Sums that join what three calls round one by one are free of that.)
-    if (!p.accumulate && (t_small < t1 || splits1 > 1 || splits > 1)) return DFDX_ROCM_OK;
+    if ((!p.accumulate || p.k % 64) && (t_small < t1 || splits1 > 1 || splits > 1)) return DFDX_ROCM_OK;
     if (t3 >= 3.0 * std::min(t1, t_small)) return DFDX_ROCM_OK;
     Plan plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
     if (int e = reserve_partials(ctx, p, plan, false)) return e;
@@ -1113,14 +1123,16 @@ int dfdx_rocm_gemm_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int
     if (kernel) *kernel = plan.kernel;
     if (variant) *variant = plan.kernel == DFDX_ROCM_KERNEL_GEMV ? 0 : plan.variant;  // (a tile variant; the bandwidth kernels have none)
     if (name && name_len) {
+        const bool ring = plan.realign && mfma16dma_takes_any_k(plan.variant - mfma16_dma_first_variant() + 1);  // one of the LDS-DMA kernels too
+        const char *const copied = !plan.realign ? "" : ring ? "_dma_realigned" : "_realigned";
         if (plan.kernel == DFDX_ROCM_KERNEL_MFMA && plan.splits > 1)
             std::snprintf(name, name_len, "%s_%s%s_splitk%d", p.dtype == DT_F32 ? "mfma32" : "mfma16",
-                          p.dtype == DT_F32 ? mfma32_variant_name(plan.variant) : mfma16_variant_name(plan.variant), plan.realign ? "_realigned" : "", plan.splits);
+                          p.dtype == DT_F32 ? mfma32_variant_name(plan.variant) : mfma16_variant_name(plan.variant), copied, plan.splits);
         else if (plan.kernel == DFDX_ROCM_KERNEL_MFMA && p.dtype == DT_F64)
             std::snprintf(name, name_len, "mfma64_%s", mfma64_variant_name(plan.variant));
         else if (plan.kernel == DFDX_ROCM_KERNEL_MFMA)
             std::snprintf(name, name_len, "%s_%s%s", p.dtype == DT_F32 ? "mfma32" : "mfma16",
-                          p.dtype == DT_F32 ? mfma32_variant_name(plan.variant) : mfma16_variant_name(plan.variant), plan.realign ? "_realigned" : "");
+                          p.dtype == DT_F32 ? mfma32_variant_name(plan.variant) : mfma16_variant_name(plan.variant), copied);
         else
             std::snprintf(name, name_len, "%s", plan.kernel != DFDX_ROCM_KERNEL_GEMV ? "generic" : bandwidth_kernel_name(p, plan.variant));
     }

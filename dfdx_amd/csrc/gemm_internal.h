@@ -121,11 +121,12 @@ hipError_t launch_mfma16(const GemmProblem &p, int variant, hipStream_t stream);
 // the shape does not fit (the caller then unfolds).
 hipError_t launch_mfma16_conv(const GemmProblem &p, const ConvPatches &conv, int compute_units, hipStream_t stream);
 
-// ---- LDS-DMA MFMA kernels for 16-bit inputs, K % 64 == 0 (gemm_mfma16_dma.hip) ----
+// ---- LDS-DMA MFMA kernels for 16-bit inputs (gemm_mfma16_dma.hip: K % 64 == 0; gemm_mfma16_ring.hip: any K) ----
 // Reached through the mfma16_* entry points above: their variant ids follow the register-staged ones.
 int mfma16dma_variant_count();
 const char *mfma16dma_variant_name(int variant);
 bool mfma16dma_supported(const GemmProblem &p, int variant);
+bool mfma16dma_takes_any_k(int variant);
 int mfma16dma_pick_variant(const GemmProblem &p, int compute_units);
 hipError_t launch_mfma16dma(const GemmProblem &p, int variant, hipStream_t stream);
 struct DmaParams;

@@ -19,8 +19,10 @@
 // One s_barrier per tile.  Stage hand-over uses explicit s_waitcnt vmcnt/lgkmcnt + s_barrier.
 //
 // Rows/columns past the matrix edge are clamped onto valid addresses (they only feed C entries that are
-// never stored).  There is no k tail here: K % 64 != 0 is served by the register-staged kernel.
+// never stored).  There is no k tail here: K % 64 != 0 is served by gemm_mfma16_ring.hip, whose tiles are planned here too, and by the
+// register-staged kernel.
 #include "gemm_mfma16_dma.h"
+#include "gemm_mfma16_ring.h"
 #include <algorithm>
 
 namespace dfdx_rocm {
@@ -37,8 +39,15 @@ constexpr Variant kVariants[] = {
 #define X(id, bm, bn, wm, wn) {"dma_" #bm "x" #bn "x64_w" #wm "x" #wn, bm, bn, wm, wn},
     DFDX_MFMA16_DMA_VARIANTS(X)
 #undef X
+#define X(id, bm, bn, wm, wn, depth) {"ring_" #bm "x" #bn "x64_w" #wm "x" #wn "_s" #depth, bm, bn, wm, wn},
+    DFDX_MFMA16_RING_VARIANTS(X)  // gemm_mfma16_ring.hip
+#undef X
 };
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
+#define X(...) +1
+constexpr int kNumTiles = 0 DFDX_MFMA16_DMA_VARIANTS(X);
+#undef X
+inline bool is_ring(int variant) { return variant > kNumTiles; }
 
 template <typename T, int BM, int BN, int WM, int WN>
 hipError_t launch_layout(Params p, int compute_units, bool a_kc, bool b_kc, hipStream_t stream) {
@@ -105,13 +114,14 @@ inline bool c_on_grid(const GemmProblem &p, const Variant &v) {
 
 }  // namespace
 
+bool mfma16dma_takes_any_k(int variant) { return is_ring(variant); }
 int mfma16dma_variant_count() { return kNumVariants; }
 const char *mfma16dma_variant_name(int v) { return (v >= 1 && v <= kNumVariants) ? kVariants[v - 1].name : "?"; }
 
 bool mfma16dma_supported(const GemmProblem &p, int variant) {
     if (p.dtype != DT_F16 && p.dtype != DT_BF16) return false;
     if (variant < 1 || variant > kNumVariants) return false;
-    if (p.m < 1 || p.n < 1 || p.k < BK || p.k % BK != 0) return false;
+    if (p.m < 1 || p.n < 1 || p.k < 1 || (!is_ring(variant) && p.k % BK != 0)) return false;
     if (p.m > (1 << 30) || p.n > (1 << 30) || p.k > (1 << 30)) return false;
     if (p.c_cs != 1 && p.n != 1) return false;
     if (p.n > 1 && p.m > 1 && p.c_rs < p.n) return false;
@@ -121,7 +131,7 @@ bool mfma16dma_supported(const GemmProblem &p, int variant) {
     const Variant &v = kVariants[variant - 1];
     if (la.ld * (la.kc ? v.bm : BK) >= (1ll << 30) || lb.ld * (lb.kc ? v.bn : BK) >= (1ll << 30)) return false;
     if (!aligned16(p.a) || !aligned16(p.b)) return false;
-    if (!c_on_grid(p, v) && !(p.ragged && (v.bn / v.waves_n) % 32 == 0)) return false;
+    if (!is_ring(variant) && !c_on_grid(p, v) && !(p.ragged && (v.bn / v.waves_n) % 32 == 0)) return false;
     if (p.batch_count() > 1) {
         if (p.a_b1 % 8 || p.a_b2 % 8 || p.b_b1 % 8 || p.b_b2 % 8) return false;
         if (!p.batches && (p.a_b1 < 0 || p.a_b2 < 0 || p.b_b1 < 0 || p.b_b2 < 0)) return false;
@@ -177,6 +187,37 @@ constexpr VariantModel kModel[] = {
 constexpr double kItemOverhead = 2.0e-6, kLaunchLatency = 2e-6, kCuBandwidth = 24e9, kOperandWeight = 0.32;
 constexpr double kIdleBoost = 0.146, kWsBandwidthCached = 9.5e12, kWsBandwidthHbm = 6.1e12, kWsCached = 128e6;
 constexpr double kSplitLaunch = 7e-6, kSplitPerPiece = 0.25e-6;  // 1024^3: 12.4 us unsplit, 15.9 / 18.0 us in 2 / 4 pieces
+// That model ranks its own tiles and split counts; on products of a few microseconds it runs 1 - 2 us above the clock, and 8 us
+// above it for a split plan.
+constexpr double kAboveClock = 1.0e-6, kAboveClockSplit = 6.5e-6;
+
+// The ring tiles: microseconds per k tile with 1 .. 3 workgroups on a compute unit, per work item, per launch.  Fitted to forced
+// timings of 600 products of m, n = 64 .. 4096 and k = 17 .. 8192 in three layouts (standard deviation 6 %, split plans 10 %).
+// They are taken only where every work item has a place at once: behind a first round the persistent tiles with their larger
+// steps are ahead (1344 x 768 x 3072 f16: 1008 items of 64 x 64 16.9 us, the 256 x 128 tile 15.4; 3072 x 3072 x 128 14.6 and 9.3).
+// Nor over more than 96 k tiles, where the larger tiles' fewer LDS reads have caught up (256 items of 128 x 128 x 4096 f16 36.7 us, the
+// best of the persistent tiles 43.4; x 8192 75.7 and 75.9).  Weight gradients over 4096 rows and more (both operands stored across k),
+// where the persistent tiles take them (whole k tiles), keep the split plans of the persistent tiles, which are fixed points of the sums that ride along with them (ksum): up to 25 % given up
+// at 1024 x 4096 x 1024 (17.8 and 23.7 us), 10 % at 1024 x 8192 x 1024 (29.3 and 32.4).
+// Over the 600 the plan is 1.3 % from the fastest of all tiles and split counts; the plan without the ring was 19 % from it.
+struct RingModel {
+    int per_cu;
+    double k_tile[4], item, launch;
+};
+constexpr int64_t kRingChunk = 96, kRingAcross = 64;
+constexpr RingModel kRing[] = {
+    {2, {0.0, 0.187, 0.390, 0.0}, 2.75, 0.9},    // 64 x 64, four stages
+    {3, {0.0, 0.234, 0.394, 0.572}, 3.30, 0.2},  // 64 x 64, three
+    {2, {0.0, 0.305, 0.610, 0.0}, 4.10, 0.1},    // 128 x 64
+    {1, {0.0, 0.414, 0.0, 0.0}, 4.80, 0.1},      // 128 x 128
+};
+inline double ring_time(const RingModel &r, int cus, int64_t items, int64_t total, bool whole, int64_t chunk, bool a_kc, bool b_kc, int splits, double out_elems) {
+    if (items > (int64_t)cus * r.per_cu || chunk > kRingChunk || (!a_kc && !b_kc && whole && total >= kRingAcross)) return 1e300;
+    const double layout = a_kc && b_kc ? 0.97 : !a_kc && !b_kc ? 1.1 : 1.0;
+    double us = r.launch + r.item + (double)chunk * r.k_tile[(items + cus - 1) / cus] * layout + out_elems * 2.0 / 8e6;
+    if (splits > 1) us += 2.6 + 0.2 * splits + splits * out_elems * 4.0 / 9.5e6;
+    return us * 1e-6;
+}
 }  // namespace
 
 void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_variant, int forced_splits, int *variant,
@@ -186,18 +227,19 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
     const int cus = std::max(1, compute_units);
     const int64_t nbatch = p.reduce ? 1 : p.batch_count();
     const bool may_split = (nbatch == 1 || p.batches > 0) && p.c_cs == 1;
-    const int64_t total_iters = (p.k / BK) * (p.reduce ? p.batch_count() : 1);
+    const int64_t total_iters = ((p.k + BK - 1) / BK) * (p.reduce ? p.batch_count() : 1);
     const bool a_kc = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged).kc, b_kc = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged).kc;
     const double elem = 2.0, out_elems = (double)p.m * p.n * nbatch;
-    double best = 1e300;
+    double best = 1e300, best_ring = 1e300;
+    int ring = 0, ring_splits = 1;
     for (int v = 1; v <= kNumVariants; v++) {
         if (forced_variant > 0 && v != forced_variant) continue;
         if (!mfma16dma_supported(p, v)) continue;
         const Variant &t = kVariants[v - 1];
-        const VariantModel &vm = kModel[v - 1];
+        const VariantModel &vm = kModel[is_ring(v) ? 0 : v - 1];
         // narrow outputs take the BN = 64 tiles; wide ones may take the small 128 x 64 tile (more workgroups for a
         // problem of a few tiles), never the 256 x 64 one
-        if (forced_variant == 0 && (p.n <= 64 ? t.bn > 64 : (t.bn <= 64 && t.bm > 128))) continue;
+        if (forced_variant == 0 && !is_ring(v) && (p.n <= 64 ? t.bn > 64 : (t.bn <= 64 && t.bm > 128))) continue;
         const int64_t tiles = ((p.m + t.bm - 1) / t.bm) * ((p.n + t.bn - 1) / t.bn) * nbatch;
         const double layout = (a_kc && b_kc) ? 1.0 : (!a_kc && !b_kc) ? 0.98 : 0.99;  // transposing LDS reads cost a little
         // candidates 1..16, 20..32, 40..64 (filter gradients of convolutions: a handful of tiles, thousands of k steps)
@@ -208,6 +250,15 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
             const int64_t chunk = (total_iters + s - 1) / s;
             if ((s - 1) * chunk >= total_iters) continue;  // an empty split
             const int64_t items = tiles * s;
+            if (is_ring(v)) {
+                const double time = ring_time(kRing[v - 1 - kNumTiles], cus, items, total_iters, p.k % BK == 0, chunk, a_kc, b_kc, s, out_elems);
+                if (time < best_ring || (forced_variant == v && ring == 0)) {
+                    best_ring = time;
+                    ring = v;
+                    ring_splits = s;
+                }
+                continue;
+            }
             const int64_t grid = std::min<int64_t>(items, (int64_t)cus * vm.per_cu);
             const int64_t conc = (grid + cus - 1) / cus, items_per_wg = (items + grid - 1) / grid;
             const double active = (double)std::min<int64_t>(grid, cus) / cus;
@@ -230,6 +281,12 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
             }
         }
     }
+    if (best < 1e300) best -= *splits > 1 ? kAboveClockSplit : kAboveClock;
+    if (ring && (best_ring < best || *variant == 0)) {
+        best = best_ring;
+        *variant = ring;
+        *splits = ring_splits;
+    }
     if (seconds) *seconds = best;
 }
 
@@ -242,7 +299,7 @@ static void ws_layout(const GemmProblem &p, int variant, int64_t *ld, int64_t *s
     if (ksum_stride) *ksum_stride = ((p.m + v.bm - 1) / v.bm) * v.bm;
 }
 // Workspace slots of the row sums: one per split, sharing tile column and wave.
-static int ksum_slots(int variant, int splits) { return splits * (kVariants[variant - 1].bm / 64) * 8; }
+static int ksum_slots(int variant, int splits) { return is_ring(variant) ? splits : splits * (kVariants[variant - 1].bm / 64) * 8; }
 
 size_t mfma16dma_workspace_bytes(const GemmProblem &p, int variant, int splits) {
     if (splits <= 1) return 0;
@@ -256,24 +313,66 @@ size_t mfma16dma_workspace_bytes(const GemmProblem &p, int variant, int splits) 
 // weight gradient grad_out^T . x after the output transposition) and the contraction is split (the partial sums are
 // combined by the reduce kernel that runs then anyway).
 bool mfma16dma_ksum_supported(const GemmProblem &p, int variant, int splits) {
-    if (!p.ksum || p.ksum_of != KSUM_OF_A || splits <= 1 || !mfma16dma_supported(p, variant)) return false;
+    if (!p.ksum || p.ksum_of != KSUM_OF_A || (splits <= 1 && !is_ring(variant)) || !mfma16dma_supported(p, variant)) return false;
     if (!p.reduce && p.batch_count() != 1 && !p.batches) return false;
     if ((uintptr_t)p.ksum & 1u) return false;
     const Variant &v = kVariants[variant - 1];
-    if ((p.n + v.bn - 1) / v.bn < v.bm / 64) return false;  // too few tile columns to share a tile's pieces
+    if (!is_ring(variant) && (p.n + v.bn - 1) / v.bn < v.bm / 64) return false;  // too few tile columns to share a tile's pieces
     return !classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged).kc && !classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged).kc;
 }
 
 bool mfma16dma_extra_supported(const GemmProblem &p, int variant, int splits) {
     if ((p.accumulate != 0) != (p.extra == EXTRA_FROM) || (p.batch_count() != 1 && !p.reduce) || !mfma16dma_supported(p, variant)) return false;
     if (p.extra != EXTRA_RELU && (!p.with || !aligned16(p.with))) return false;
-    if (splits > 1) return true;  // the reduce kernel applies it
+    if (splits > 1 || is_ring(variant)) return true;  // (split: the reduce kernel applies it)
     const bool a_kc = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged).kc, b_kc = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged).kc;
     return a_kc && b_kc == (p.extra == EXTRA_RELU || p.extra == EXTRA_RESIDUAL);
 }
 
+static hipError_t launch_ring(const GemmProblem &g, int variant, hipStream_t stream) {
+    const Variant &v = kVariants[variant - 1];
+    const OperandLayout la = classify(g.m, g.k, g.a_rs, g.a_cs, g.ragged);
+    const OperandLayout lb = classify(g.n, g.k, g.b_cs, g.b_rs, g.ragged);
+    RingParams p;
+    p.a = (const uint16_t *)g.a; p.b = (const uint16_t *)g.b; p.c = (uint16_t *)g.c; p.bias = (const uint16_t *)g.bias;
+    p.with = (const uint16_t *)g.with; p.ksum = (uint16_t *)g.ksum;
+    p.m = (int)g.m; p.n = (int)g.n; p.k = (int)g.k;
+    p.lda = (int)la.ld; p.ldb = (int)lb.ld;
+    p.ldc = g.m == 1 ? g.n : g.c_rs;
+    p.a_b1 = g.a_b1; p.a_b2 = g.a_b2; p.b_b1 = g.b_b1; p.b_b2 = g.b_b2; p.c_b1 = g.c_b1; p.c_b2 = g.c_b2;
+    p.bias_b1 = g.bias_b1; p.bias_b2 = g.bias_b2; p.ksum_b1 = g.ksum_b1; p.ksum_b2 = g.ksum_b2;
+    p.nb2 = (int)g.nb2;
+    const int nbatch = (int)g.batch_count();
+    p.kbatches = g.reduce ? nbatch : 1;
+    p.tiles_m = (int)((g.m + v.bm - 1) / v.bm);
+    p.tiles_n = (int)((g.n + v.bn - 1) / v.bn);
+    p.tiles_per_batch = p.tiles_m * p.tiles_n;
+    const int outputs = g.reduce ? 1 : nbatch, total_iters = (p.k + BK - 1) / BK * p.kbatches;
+    p.accumulate = g.accumulate; p.bias_mode = g.bias ? g.bias_mode : BIAS_NONE;
+    p.extra = g.extra; p.ksum_accumulate = g.ksum_accumulate;
+    p.group_m = 4;
+    p.splits = std::max(1, g.splits); p.chunk = total_iters; p.ws = p.ws_ksum = nullptr; p.ws_ld = p.ws_split_stride = 0; p.ws_ksum_stride = 0;
+    if (g.ksum && !mfma16dma_ksum_supported(g, variant, g.splits)) return hipErrorInvalidValue;
+    if (g.extra != EXTRA_NONE && !mfma16dma_extra_supported(g, variant, g.splits)) return hipErrorInvalidValue;
+    if (p.splits > 1) {
+        if (!g.workspace || (outputs != 1 && !g.batches)) return hipErrorInvalidValue;
+        p.chunk = (total_iters + p.splits - 1) / p.splits;
+        if ((int64_t)(p.splits - 1) * p.chunk >= total_iters) return hipErrorInvalidValue;
+        p.ws = g.workspace;
+        int64_t ks_stride = 0;
+        ws_layout(g, variant, &p.ws_ld, &p.ws_split_stride, &ks_stride);
+        p.ws_ksum = g.workspace + p.ws_split_stride * p.splits * outputs;
+        p.ws_ksum_stride = (int)ks_stride;
+    }
+    p.items = p.tiles_per_batch * outputs * p.splits;
+    const hipError_t e = launch_mfma16_ring(variant - kNumTiles, g.dtype, p, la.kc, lb.kc, stream);
+    if (e != hipSuccess || p.splits <= 1) return e;
+    return launch_splitk_reduce(g, p.ws_ld, p.ws_split_stride, stream, g.ksum ? p.ws_ksum : nullptr, p.ws_ksum_stride, ksum_slots(variant, p.splits));
+}
+
 hipError_t launch_mfma16dma(const GemmProblem &g, int variant, hipStream_t stream) {
     if (!mfma16dma_supported(g, variant)) return hipErrorInvalidValue;
+    if (is_ring(variant)) return launch_ring(g, variant, stream);
     const Variant &v = kVariants[variant - 1];
     const OperandLayout la = classify(g.m, g.k, g.a_rs, g.a_cs, g.ragged);
     const OperandLayout lb = classify(g.n, g.k, g.b_cs, g.b_rs, g.ragged);

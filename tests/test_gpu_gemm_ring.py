@@ -1,0 +1,85 @@
+"""The 16-bit tiles behind a ring of LDS stages (gemm_mfma16_ring.hip): edges of tiles, partial last k tiles, contractions
+shorter and longer than the ring, batches, and the row sums that ride along."""
+import numpy as np
+import pytest
+
+import oracle
+from dfdx_amd.rocm import KERNEL_MFMA
+from gpu_util import announce, device
+from helpers import assert_within, rng
+from test_gpu_gemm import run_case
+
+pytestmark = pytest.mark.gpu
+TILES = 4
+
+
+def ring_ids():
+    last = device().mfma_variant_count("f16")   # the small-product kernel; the ring tiles are the four in front of it
+    return range(last - TILES, last)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("tile", range(TILES))
+@pytest.mark.parametrize("m,n", [(64, 64), (128, 128), (65, 67), (200, 264), (1, 136), (8, 9)])
+@pytest.mark.parametrize("k", [8, 64, 72, 184, 256, 320, 456])
+def test_operands_along_k(dtype, tile, m, n, k):
+    """1 to 8 k tiles (3 or 4 are in flight), the last one whole or partial; columns of C off the grid of eight."""
+    assert "_ring_" in run_case(dtype, m, k, n, "nt", m > 64, KERNEL_MFMA, ring_ids()[tile], bias=n % 8 == 0, seed=m + k)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("tile", range(TILES))
+@pytest.mark.parametrize("layout,k", [("tn", 1), ("tn", 63), ("tn", 65), ("tn", 259), ("tn", 449), ("nn", 24), ("nn", 328), ("tt", 136)])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_operands_across_k(dtype, tile, layout, k, splits):
+    """The transposing reads: any length of the contraction where both operands lie across it, whole pieces of eight else."""
+    run_case(dtype, 136, k, 72, layout, True, KERNEL_MFMA, ring_ids()[tile], split_k=splits, pads=(8, 8, 8), seed=k)
+    run_case(dtype, 72, k, 200, layout, False, KERNEL_MFMA, ring_ids()[tile], split_k=splits, bias=True, c_colmajor=False, seed=k + 1)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("reduce", [False, True])
+@pytest.mark.parametrize("k", [40, 64, 137])
+def test_batches(dtype, reduce, k):
+    """Batches side by side and summed over (the k loop then restarts in every batch, behind a partial tile)."""
+    dev, g = device(), rng(71 + k)
+    b1, b2, m, n = 2, 3, 72, 80
+    a = oracle.to_storage(g.standard_normal(b1 * b2 * k * m), dtype)
+    b = oracle.to_storage(g.standard_normal(b1 * b2 * k * n), dtype)
+    A = oracle.to_f64(a, dtype).reshape(b1 * b2, k, m).transpose(0, 2, 1)
+    B = oracle.to_f64(b, dtype).reshape(b1 * b2, k, n)
+    want = A @ B
+    if reduce:
+        want = want.sum(axis=0, keepdims=True)
+    da, db = dev.tensor(a, dtype), dev.tensor(b, dtype)
+    for variant in ring_ids():
+        announce("ring batches", dtype, reduce, k, variant)
+        c = dev.zeros(dtype, (want.shape[0], m, n))
+        d = dev.gemm_desc(dtype, m, k, n, da.ptr, (1, m), db.ptr, (n, 1), c.ptr, (n, 1), batch=(b1, b2), a_batch=(b2 * k * m, k * m),
+                          b_batch=(b2 * k * n, k * n), c_batch=(0, 0) if reduce else (b2 * m * n, m * n), reduce_batch=reduce,
+                          kernel=KERNEL_MFMA, variant=variant)
+        dev.gemm(d)
+        got = oracle.to_f64(dev.to_host(c), dtype).reshape(want.shape)
+        ulp = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype]
+        assert_within(dtype, k * (b1 * b2 if reduce else 1), got, want, A, B, extra=ulp * float(np.abs(want).max()), what="ring batches")
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("rows,i,o", [(100, 256, 256), (263, 136, 520), (529, 768, 384), (1344, 768, 768), (2001, 64, 72)])
+def test_bias_gradient_rides_along(dtype, rows, i, o):
+    """Linear's backward on rows that are no multiple of 64: the sums of small whole numbers are exact in f32, so the bias gradient
+    has the one rounding of its result; both gradients against float64."""
+    dev, g = device(), rng(rows)
+    announce("ring row sums", dtype, rows, i, o)
+    x, w = (oracle.to_storage(g.standard_normal(s), dtype) for s in ((rows, i), (o, i)))
+    go = oracle.to_storage(g.integers(-4, 5, size=(rows, o)).astype(np.float64), dtype)
+    dx, dw, dgo = dev.tensor(x, dtype), dev.tensor(w, dtype), dev.tensor(go, dtype)
+    gx, gw, gb = dev.zeros_like_storage(dx), dev.zeros_like_storage(dw), dev.zeros(dtype, (o,))
+    dev.linear_backward(dx, gx, dw, gw, gb, dgo)
+    X, W, G = oracle.to_f64(x, dtype), oracle.to_f64(w, dtype), oracle.to_f64(go, dtype)
+    host = lambda t, shape: oracle.to_f64(dev.to_host(t), dtype).reshape(shape)
+    want = oracle.to_f64(oracle.to_storage(G.sum(axis=0), dtype), dtype)
+    np.testing.assert_array_equal(host(gb, (o,)), want)
+    ulp = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype]
+    assert_within(dtype, rows, host(gw, (o, i)), G.T @ X, G, X, extra=ulp * float(np.abs(G.T @ X).max()), what="weight")
+    assert_within(dtype, o, host(gx, (rows, i)), G @ W, G, W, extra=ulp * float(np.abs(G @ W).max()), what="input")
