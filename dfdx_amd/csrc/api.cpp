@@ -335,7 +335,9 @@ const char *bandwidth_kernel_name(const GemmProblem &p, int which) {
     }
 }
 
-int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProblem &p, Plan *plan) {
+// `seconds` (may be null): the estimate behind an automatic plan of a 16-bit product that the matrix-core tiles take, else 0.
+int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProblem &p, Plan *plan, double *seconds = nullptr) {
+    if (seconds) *seconds = 0.0;
     const bool is16 = p.dtype == DT_F16 || p.dtype == DT_BF16;
     const bool is32 = p.dtype == DT_F32, is64 = p.dtype == DT_F64;
     // split-k: 1 = never (NO_SPLIT_K), n = forced by the caller, 0 = let the planner decide
@@ -414,6 +416,7 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
                 }
             }
             if (t_bw < t_best) *plan = bw_plan;
+            if (seconds) *seconds = std::min(t_best, t_bw);
             return DFDX_ROCM_OK;
         }
     }
@@ -461,6 +464,7 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         // 2304 x 128 x 1534 in three pieces 16.2 for 15.3; the ring 9.4 both)
         const double t_plan = plan->realign ? t_copies : plan->kernel == DFDX_ROCM_KERNEL_GEMV ? t_bw : plan->variant == v ? 0.85 * t_family : t_small_here;
         if (t_ring < t_plan) *plan = ring_plan;
+        if (seconds && is16) *seconds = std::min(t_ring, t_plan);
         return DFDX_ROCM_OK;
     }
     if (t_ring < std::min(t_small, t_bw)) {
@@ -689,9 +693,121 @@ int gemm_beyond(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int extra, 
     }
 }
 
+// Bytes that the matrices of one operand span, matrix by matrix where they lie anywhere (`batches`), else together.
+struct Spans {
+    uintptr_t lo[3], hi[3];
+    int count = 0;
+    void add(const void *ptr, size_t es, int64_t rows, int64_t rs, int64_t cols, int64_t cs, const GemmProblem &p, int64_t b1, int64_t b2) {
+        if (!ptr) return;
+        const int64_t apart = p.batches > 0 ? p.batches : 1;
+        for (int64_t i = 0; i < apart && i < 3; i++) {
+            int64_t from = p.batches > 0 ? (i / p.nb2) * b1 + (i % p.nb2) * b2 : 0, to = from;
+            auto axis = [&](int64_t n, int64_t stride) { (stride < 0 ? from : to) += (n - 1) * stride; };
+            axis(rows, rs);
+            axis(cols, cs);
+            if (p.batches <= 0) {
+                axis(p.nb1, b1);
+                axis(p.nb2, b2);
+            }
+            lo[count] = (uintptr_t)ptr + (uintptr_t)(from * (int64_t)es);
+            hi[count++] = (uintptr_t)ptr + (uintptr_t)((to + 1) * (int64_t)es);
+        }
+    }
+    bool meets(const Spans &o) const {
+        for (int i = 0; i < count; i++)
+            for (int j = 0; j < o.count; j++)
+                if (lo[i] < o.hi[j] && o.lo[j] < hi[i]) return true;
+        return false;
+    }
+};
+
+// May the two products run side by side?  Nothing that one writes may be read or written by the other.
+static bool independent(const GemmProblem &p, const GemmProblem &q) {
+    auto written = [](const GemmProblem &g, Spans(&s)[2]) {
+        const size_t es = dtype_size(g.dtype);
+        s[0].add(g.c, es, g.m, g.c_rs, g.n, g.c_cs, g, g.reduce ? 0 : g.c_b1, g.reduce ? 0 : g.c_b2);
+        s[1].add(g.ksum, es, 1, 0, g.ksum_of == KSUM_OF_B ? g.n : g.m, 1, g, g.ksum_b1, g.ksum_b2);
+    };
+    auto read = [](const GemmProblem &g, Spans(&s)[4]) {
+        const size_t es = dtype_size(g.dtype);
+        s[0].add(g.a, es, g.m, g.a_rs, g.k, g.a_cs, g, g.a_b1, g.a_b2);
+        s[1].add(g.b, es, g.k, g.b_rs, g.n, g.b_cs, g, g.b_b1, g.b_b2);
+        s[2].add(g.with, es, g.m, g.c_rs, g.n, g.c_cs, g, g.reduce ? 0 : g.c_b1, g.reduce ? 0 : g.c_b2);
+        s[3].add(g.bias, es, 1, 0, g.bias_mode == BIAS_PER_ROW ? g.m : g.n, 1, g, g.bias_b1, g.bias_b2);
+    };
+    Spans wp[2], wq[2], rp[4], rq[4];
+    written(p, wp);
+    written(q, wq);
+    read(p, rp);
+    read(q, rq);
+    for (const Spans &w : wp) {
+        for (const Spans &o : wq)
+            if (w.meets(o)) return false;
+        for (const Spans &o : rq)
+            if (w.meets(o)) return false;
+    }
+    for (const Spans &w : wq)
+        for (const Spans &o : rp)
+            if (w.meets(o)) return false;
+    return true;
+}
+
+// The tile on which the two products of a backward pass run faster as one launch than as two, 0 if there is none.  Decided from the
+// shapes and layouts alone, so that a call that joins more of them (the encoder block's) and the calls it stands for agree.
+static int ring_pair_tile(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d1, const GemmProblem &p1, const dfdx_rocm_gemm_desc *d2, const GemmProblem &p2) {
+    if ((p1.dtype != DT_F16 && p1.dtype != DT_BF16) || d1->kernel != DFDX_ROCM_KERNEL_AUTO || d2->kernel != DFDX_ROCM_KERNEL_AUTO) return 0;
+    double together = 1e300, t1 = 0.0, t2 = 0.0;
+    const int tile = mfma16_ring_pair_plan(p1, p2, ctx->compute_units, &together);
+    if (!tile) return 0;
+    Plan plan;
+    if (make_plan(ctx, d1, p1, &plan, &t1) || make_plan(ctx, d2, p2, &plan, &t2)) return 0;
+    // (the second launch and the gap in front of it are not in the estimates)
+    return t1 > 0.0 && t2 > 0.0 && together < t1 + t2 + 1.0e-6 ? tile : 0;
+}
+
+// Two independent products in one launch: pending fills, then the launch.  `sums` of the second one ride along.
+static int run_ring_pair(dfdx_rocm_ctx *ctx, GemmProblem p, GemmProblem q, int tile, bool may_overwrite) {
+    CtxLock lock(ctx->mu);
+    if (int e = settle_operands(ctx, &p, may_overwrite)) return e;
+    if (int e = settle_operands(ctx, &q, /*may_overwrite=*/true)) return e;
+    if (q.ksum) {
+        bool fresh = false;
+        if (int e = settle_output(ctx, q.ksum, (size_t)(q.ksum_of == KSUM_OF_A ? q.m : q.n) * dtype_size(q.dtype), true, &fresh)) return e;
+        q.ksum_accumulate = !fresh;
+    }
+    p.compute_units = q.compute_units = ctx->compute_units;
+    return (int)launch_mfma16_ring_pair(p, q, tile, ctx->stream);
+}
+
+int gemm_two(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, int extra, const void *with, const dfdx_rocm_gemm_desc *second, void *colsum,
+             bool *done) {
+    *done = false;
+    if (int e = bind(ctx)) return e;
+    GemmProblem p, q;
+    if (int e = make_problem(first, &p)) return e;
+    if (int e = make_problem(second, &q, colsum)) return e;
+    if (p.m == 0 || q.m == 0) return DFDX_ROCM_OK;
+    if (colsum && !q.ksum) return DFDX_ROCM_OK;
+    GemmProblem shape = p;
+    shape.accumulate = 1;  // (what the ops that `extra` stands for would do)
+    const int tile = ring_pair_tile(ctx, first, shape, second, q);
+    if (!tile) return DFDX_ROCM_OK;
+    p.extra = extra;
+    p.with = with;
+    if (!independent(p, q)) return DFDX_ROCM_OK;
+    *done = true;
+    return run_ring_pair(ctx, p, q, tile, extra != EXTRA_FROM);
+}
+
 int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_rocm_gemm_desc *second, const void *grad_out, int64_t rows, int64_t cols,
               void *colsum, bool *fused) {
     if (fused) *fused = false;
+    bool done = false;
+    if (int e = gemm_two(ctx, first, EXTRA_NONE, nullptr, second, fused ? colsum : nullptr, &done)) return e;
+    if (done) {
+        if (fused) *fused = colsum != nullptr;
+        return DFDX_ROCM_OK;
+    }
     // (a copy of less than 4 MB costs little more than its launch)
     const bool off = cols % 64 || rows % 64 || ((uintptr_t)grad_out & 15u);
     if ((first->dtype != DFDX_ROCM_F16 && first->dtype != DFDX_ROCM_BF16) || !off || (double)rows * (double)cols < 2097152.0) {
@@ -761,6 +877,37 @@ int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_r
     return DFDX_ROCM_OK;
 }
 
+// Deferred zero fills, as settle_operands, for three products in one.
+static int settle_three(dfdx_rocm_ctx *ctx, GemmProblem *problem) {
+    const GemmProblem p = *problem;
+    const size_t es = dtype_size(p.dtype), c_bytes = (size_t)(p.m * p.n) * es, k_bytes = (size_t)p.m * es;
+    auto at = [&](const void *ptr, int64_t b1, int64_t b2, int i) -> char * {
+        return ptr ? (char *)ptr + (i == 1 ? b2 : i == 2 ? b1 : 0) * (int64_t)es : nullptr;
+    };
+    if (int e = settle(ctx, p.with)) return e;
+    bool fresh[2][3] = {};
+    for (int i = 0; i < 3; i++) {
+        if (int e = settle(ctx, at(p.a, p.a_b1, p.a_b2, i))) return e;
+        if (int e = settle(ctx, at(p.b, p.b_b1, p.b_b2, i))) return e;
+        if (int e = settle(ctx, at(p.bias, p.bias_b1, p.bias_b2, i))) return e;
+        if (i > 0 && p.reduce) continue;
+        if (int e = settle_output(ctx, at(p.c, p.c_b1, p.c_b2, i), c_bytes, p.accumulate, p.extra == EXTRA_FROM ? nullptr : &fresh[0][i])) return e;
+        if (p.ksum)
+            if (int e = settle_output(ctx, at(p.ksum, p.ksum_b1, p.ksum_b2, i), k_bytes, true, &fresh[1][i])) return e;
+    }
+    // gradients are stored where all three count as zero; a mixture is filled after all
+    for (int r = 0; r < 2; r++) {
+        const bool all = fresh[r][0] && fresh[r][1] && fresh[r][2];
+        if (all && r == 0) problem->accumulate = 0;
+        if (all && r == 1) problem->ksum_accumulate = 0;
+        for (int i = 0; i < 3 && !all; i++)
+            if (fresh[r][i])
+                HIP_TRY(launch_zero_fill(r == 0 ? at(p.c, p.c_b1, p.c_b2, i) : at(p.ksum, p.ksum_b1, p.ksum_b2, i), r == 0 ? c_bytes : k_bytes,
+                                         ctx->compute_units, ctx->stream));
+    }
+    return DFDX_ROCM_OK;
+}
+
 int gemm_three(dfdx_rocm_ctx *ctx, const GemmProblem &problem, bool *done) {
     *done = false;
     GemmProblem p = problem;
@@ -783,34 +930,31 @@ int gemm_three(dfdx_rocm_ctx *ctx, const GemmProblem &problem, bool *done) {
     if (t3 >= 3.0 * std::min(t1, t_small)) return DFDX_ROCM_OK;
     Plan plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
     if (int e = reserve_partials(ctx, p, plan, false)) return e;
-    // deferred zero fills: as settle_operands, for each of the three
-    const size_t es = dtype_size(p.dtype), c_bytes = (size_t)(p.m * p.n) * es, k_bytes = (size_t)p.m * es;
-    auto at = [&](const void *ptr, int64_t b1, int64_t b2, int i) -> char * {
-        return ptr ? (char *)ptr + (i == 1 ? b2 : i == 2 ? b1 : 0) * (int64_t)es : nullptr;
-    };
-    if (int e = settle(ctx, p.with)) return e;
-    bool fresh[2][3] = {};
-    for (int i = 0; i < 3; i++) {
-        if (int e = settle(ctx, at(p.a, p.a_b1, p.a_b2, i))) return e;
-        if (int e = settle(ctx, at(p.b, p.b_b1, p.b_b2, i))) return e;
-        if (int e = settle(ctx, at(p.bias, p.bias_b1, p.bias_b2, i))) return e;
-        if (i > 0 && p.reduce) continue;
-        if (int e = settle_output(ctx, at(p.c, p.c_b1, p.c_b2, i), c_bytes, p.accumulate, p.extra == EXTRA_FROM ? nullptr : &fresh[0][i])) return e;
-        if (p.ksum)
-            if (int e = settle_output(ctx, at(p.ksum, p.ksum_b1, p.ksum_b2, i), k_bytes, true, &fresh[1][i])) return e;
-    }
-    // gradients are stored where all three count as zero; a mixture is filled after all
-    for (int r = 0; r < 2; r++) {
-        const bool all = fresh[r][0] && fresh[r][1] && fresh[r][2];
-        if (all && r == 0) p.accumulate = 0;
-        if (all && r == 1) p.ksum_accumulate = 0;
-        for (int i = 0; i < 3 && !all; i++)
-            if (fresh[r][i])
-                HIP_TRY(launch_zero_fill(r == 0 ? at(p.c, p.c_b1, p.c_b2, i) : at(p.ksum, p.ksum_b1, p.ksum_b2, i), r == 0 ? c_bytes : k_bytes,
-                                         ctx->compute_units, ctx->stream));
-    }
+    if (int e = settle_three(ctx, &p)) return e;
     *done = true;
     return run_plan(ctx, p, plan);
+}
+
+int gemm_three_two(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_rocm_gemm_desc *second, void *colsum, const GemmProblem &sum,
+                   const GemmProblem &apart, bool *done) {
+    *done = false;
+    if (int e = bind(ctx)) return e;
+    GemmProblem one, two;
+    if (int e = make_problem(first, &one)) return e;
+    if (int e = make_problem(second, &two, colsum)) return e;
+    if (one.m == 0 || two.m == 0 || !two.ksum) return DFDX_ROCM_OK;
+    one.accumulate = 1;
+    if (!ring_pair_tile(ctx, first, one, second, two)) return DFDX_ROCM_OK;  // (what the calls that this one stands for would do)
+    GemmProblem p = sum, q = apart;
+    double seconds = 0.0;
+    const int tile = mfma16_ring_pair_plan(p, q, ctx->compute_units, &seconds);
+    if (!tile || !independent(p, q)) return DFDX_ROCM_OK;
+    *done = true;
+    CtxLock lock(ctx->mu);
+    if (int e = settle_three(ctx, &p)) return e;
+    if (int e = settle_three(ctx, &q)) return e;
+    p.compute_units = q.compute_units = ctx->compute_units;
+    return (int)launch_mfma16_ring_pair(p, q, tile, ctx->stream);
 }
 
 int gemm_with_colsum(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, void *colsum_b, bool *fused) {

@@ -117,13 +117,27 @@ dfdx_rocm_gemm_desc input_grad(const Shape &s, int64_t i, int64_t o, const void 
     return product(s.dtype, s.T, o, i, gy, o, 1, w, i, 1, gx);
 }
 // grad_w (o, i) and grad_b (o) from x and grad_y, both stored; the sums of grad_y come out of the product where they can
-int weight_grad(dfdx_rocm_ctx *ctx, const Shape &s, int64_t i, int64_t o, const void *x, const void *gy, void *gw, void *gb) {
+dfdx_rocm_gemm_desc weight_product(const Shape &s, int64_t i, int64_t o, const void *x, const void *gy, void *gw) {
     dfdx_rocm_gemm_desc g = product(s.dtype, i, s.T, o, x, 1, i, gy, o, 1, gw);
     g.accumulate = 1;
     g.c_rs = 1; g.c_cs = i;
+    return g;
+}
+int weight_grad(dfdx_rocm_ctx *ctx, const Shape &s, int64_t i, int64_t o, const void *x, const void *gy, void *gw, void *gb) {
+    dfdx_rocm_gemm_desc g = weight_product(s, i, o, x, gy, gw);
     bool done = false;
     if (int e = gemm_with_colsum(ctx, &g, gb, &done)) return e;
     return done ? DFDX_ROCM_OK : dfdx_rocm_bias_backward(ctx, s.dtype, s.T, o, gy, gb);
+}
+// A Linear layer's backward: `gx` is its input gradient with one thing more on the way into it.
+int linear_backward(dfdx_rocm_ctx *ctx, const Shape &s, const dfdx_rocm_gemm_desc &gx, int extra, const void *with, int64_t i, int64_t o, const void *x,
+                    const void *gy, void *gw, void *gb) {
+    const dfdx_rocm_gemm_desc w = weight_product(s, i, o, x, gy, gw);
+    bool done = false;
+    if (int e = gemm_two(ctx, &gx, extra, with, &w, gb, &done)) return e;
+    if (done) return DFDX_ROCM_OK;
+    if (int e = gemm_beyond(ctx, &gx, extra, with)) return e;
+    return weight_grad(ctx, s, i, o, x, gy, gw, gb);
 }
 
 // The products of the query, key and value projections as one launch: same shapes, matrices wherever they are (addresses from
@@ -209,17 +223,14 @@ int backward(dfdx_rocm_ctx *ctx, const Shape &s, const dfdx_rocm_encoder *e, con
     TRY(dfdx_rocm_layer_norm_backward(ctx, s.dtype, s.T, s.d, h2, p[G2], 1e-5, gh2, grads[G2], grads[BE2], grad_out));
     // h2 = Linear2(r1) + n1: gh2 is the gradient of both
     dfdx_rocm_gemm_desc g = input_grad(s, s.ff, s.d, gh2, p[W2], gf1);
-    TRY(gemm_beyond(ctx, &g, EXTRA_MASK, r1));
-    TRY(weight_grad(ctx, s, s.ff, s.d, r1, gh2, grads[W2], grads[B2]));
+    TRY(linear_backward(ctx, s, g, EXTRA_MASK, r1, s.ff, s.d, r1, gh2, grads[W2], grads[B2]));
     g = input_grad(s, s.d, s.ff, gf1, p[W1], gn1);
     g.accumulate = 1;
-    TRY(gemm_beyond(ctx, &g, EXTRA_FROM, gh2));
-    TRY(weight_grad(ctx, s, s.d, s.ff, n1, gf1, grads[W1], grads[B1]));
+    TRY(linear_backward(ctx, s, g, EXTRA_FROM, gh2, s.d, s.ff, n1, gf1, grads[W1], grads[B1]));
     TRY(dfdx_rocm_layer_norm_backward(ctx, s.dtype, s.T, s.d, h1, p[G1], 1e-5, gh1, grads[G1], grads[BE1], gn1));
     // h1 = Linear_o(tok) + x: gh1 is the gradient of both
     g = input_grad(s, s.d, s.d, gh1, p[WO], gtok);
-    TRY(dfdx_rocm_gemm(ctx, &g));
-    TRY(weight_grad(ctx, s, s.d, s.d, tok, gh1, grads[WO], grads[BO]));
+    TRY(linear_backward(ctx, s, g, EXTRA_NONE, nullptr, s.d, s.d, tok, gh1, grads[WO], grads[BO]));
     if (s.fused) {
         TRY(dfdx_rocm_attention_backward(ctx, s.dtype, s.B, s.H, s.S, s.D, q, k, v, s.token, (float)s.scale, tok, gtok, s.token,
                                          (const float *)(saved + l.lse), gq, gk, gv));
@@ -241,20 +252,27 @@ int backward(dfdx_rocm_ctx *ctx, const Shape &s, const dfdx_rocm_encoder *e, con
     }
     // x feeds the three projections and the residual: grad_x is one sum over their 3 d columns, rounded once
     bool summed = false, weights = false;
-    GemmProblem all = three(s.dtype, s.T, s.d, s.d, gq, s.d, 1, p[WQ], s.d, 1, grad_x);
-    all.reduce = 1;
-    all.accumulate = 1;
-    all.extra = EXTRA_FROM;
-    all.with = gh1;
-    if (apart(gq, gk, gv, s.es, &all.a_b1, &all.a_b2) && apart(p[WQ], p[WK], p[WV], s.es, &all.b_b1, &all.b_b2)) TRY(gemm_three(ctx, all, &summed));
-    all = three(s.dtype, s.d, s.T, s.d, gq, 1, s.d, x, s.d, 1, grads[WQ]);  // weight (o, i) += grad_y^T . x, bias += sums of grad_y
+    GemmProblem sum = three(s.dtype, s.T, s.d, s.d, gq, s.d, 1, p[WQ], s.d, 1, grad_x);
+    sum.reduce = 1;
+    sum.accumulate = 1;
+    sum.extra = EXTRA_FROM;
+    sum.with = gh1;
+    const bool may_sum = apart(gq, gk, gv, s.es, &sum.a_b1, &sum.a_b2) && apart(p[WQ], p[WK], p[WV], s.es, &sum.b_b1, &sum.b_b2);
+    GemmProblem all = three(s.dtype, s.d, s.T, s.d, gq, 1, s.d, x, s.d, 1, grads[WQ]);  // weight (o, i) += grad_y^T . x, bias += sums of grad_y
     all.accumulate = 1;
     all.ksum = grads[BQ];
     all.ksum_of = KSUM_OF_A;
     all.ksum_accumulate = 1;
-    if (apart(gq, gk, gv, s.es, &all.a_b1, &all.a_b2) && apart(grads[WQ], grads[WK], grads[WV], s.es, &all.c_b1, &all.c_b2) &&
-        apart(grads[BQ], grads[BK_], grads[BV], s.es, &all.ksum_b1, &all.ksum_b2))
-        TRY(gemm_three(ctx, all, &weights));
+    const bool may_join = apart(gq, gk, gv, s.es, &all.a_b1, &all.a_b2) && apart(grads[WQ], grads[WK], grads[WV], s.es, &all.c_b1, &all.c_b2) &&
+                          apart(grads[BQ], grads[BK_], grads[BV], s.es, &all.ksum_b1, &all.ksum_b2);
+    if (may_sum && may_join) {
+        g = input_grad(s, s.d, s.d, gq, p[WQ], grad_x);
+        const dfdx_rocm_gemm_desc w = weight_product(s, s.d, s.d, x, gq, grads[WQ]);
+        TRY(gemm_three_two(ctx, &g, &w, grads[BQ], sum, all, &summed));
+        weights = summed;
+    }
+    if (may_sum && !summed) TRY(gemm_three(ctx, sum, &summed));
+    if (may_join && !weights) TRY(gemm_three(ctx, all, &weights));
     for (int i = 0; i < 3; i++) {
         const int w = i == 0 ? WQ : i == 1 ? WK : WV;
         const void *gy = i == 0 ? gq : i == 1 ? gk : gv;

@@ -129,6 +129,10 @@ bool mfma16dma_supported(const GemmProblem &p, int variant);
 bool mfma16dma_takes_any_k(int variant);
 int mfma16dma_pick_variant(const GemmProblem &p, int compute_units);
 hipError_t launch_mfma16dma(const GemmProblem &p, int variant, hipStream_t stream);
+// Two products in one launch of the ring tiles: the first with A stored along k, the second with both operands stored across it (a
+// backward pass).  Returns the tile, 0 where they are not taken; `seconds` receives its estimate.
+int mfma16_ring_pair_plan(const GemmProblem &p, const GemmProblem &q, int compute_units, double *seconds);
+hipError_t launch_mfma16_ring_pair(const GemmProblem &p, const GemmProblem &q, int tile, hipStream_t stream);
 struct DmaParams;
 bool mfma16dma_extra_supported(const GemmProblem &p, int variant, int splits);  // can this plan apply p.extra on the way into C?
 hipError_t launch_mfma16dma_extra(int variant, int dtype, int extra, const DmaParams &p, int compute_units, hipStream_t stream);  // gemm_mfma16_dma_extra.hip

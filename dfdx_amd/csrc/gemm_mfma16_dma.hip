@@ -24,6 +24,7 @@
 #include "gemm_mfma16_dma.h"
 #include "gemm_mfma16_ring.h"
 #include <algorithm>
+#include <cmath>
 
 namespace dfdx_rocm {
 namespace {
@@ -329,11 +330,12 @@ bool mfma16dma_extra_supported(const GemmProblem &p, int variant, int splits) {
     return a_kc && b_kc == (p.extra == EXTRA_RELU || p.extra == EXTRA_RESIDUAL);
 }
 
-static hipError_t launch_ring(const GemmProblem &g, int variant, hipStream_t stream) {
+static hipError_t ring_params(const GemmProblem &g, int variant, RingParams &p, bool *a_kc, bool *b_kc) {
     const Variant &v = kVariants[variant - 1];
     const OperandLayout la = classify(g.m, g.k, g.a_rs, g.a_cs, g.ragged);
     const OperandLayout lb = classify(g.n, g.k, g.b_cs, g.b_rs, g.ragged);
-    RingParams p;
+    *a_kc = la.kc;
+    *b_kc = lb.kc;
     p.a = (const uint16_t *)g.a; p.b = (const uint16_t *)g.b; p.c = (uint16_t *)g.c; p.bias = (const uint16_t *)g.bias;
     p.with = (const uint16_t *)g.with; p.ksum = (uint16_t *)g.ksum;
     p.m = (int)g.m; p.n = (int)g.n; p.k = (int)g.k;
@@ -365,9 +367,58 @@ static hipError_t launch_ring(const GemmProblem &g, int variant, hipStream_t str
         p.ws_ksum_stride = (int)ks_stride;
     }
     p.items = p.tiles_per_batch * outputs * p.splits;
-    const hipError_t e = launch_mfma16_ring(variant - kNumTiles, g.dtype, p, la.kc, lb.kc, stream);
+    return hipSuccess;
+}
+
+static hipError_t launch_ring(const GemmProblem &g, int variant, hipStream_t stream) {
+    RingParams p;
+    bool a_kc, b_kc;
+    if (hipError_t e = ring_params(g, variant, p, &a_kc, &b_kc); e != hipSuccess) return e;
+    const hipError_t e = launch_mfma16_ring(variant - kNumTiles, g.dtype, p, a_kc, b_kc, stream);
     if (e != hipSuccess || p.splits <= 1) return e;
     return launch_splitk_reduce(g, p.ws_ld, p.ws_split_stride, stream, g.ksum ? p.ws_ksum : nullptr, p.ws_ksum_stride, ksum_slots(variant, p.splits));
+}
+
+// Work items of both products share the places on the chip; they are handed out as places fall free.
+int mfma16_ring_pair_plan(const GemmProblem &p, const GemmProblem &q, int compute_units, double *seconds) {
+    const int cus = std::max(1, compute_units);
+    int tile = 0;
+    *seconds = 1e300;
+    for (int v = kNumTiles + 1; v <= kNumVariants; v++) {
+        if (!mfma16dma_supported(p, v) || !mfma16dma_supported(q, v)) continue;
+        const OperandLayout pa = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged), pb = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged);
+        if (!pa.kc || classify(q.m, q.k, q.a_rs, q.a_cs, q.ragged).kc || classify(q.n, q.k, q.b_cs, q.b_rs, q.ragged).kc) return 0;
+        if (q.ksum && !mfma16dma_ksum_supported(q, v, 1)) return 0;
+        const Variant &t = kVariants[v - 1];
+        const RingModel &r = kRing[v - 1 - kNumTiles];
+        auto items = [&](const GemmProblem &g) {
+            return (double)((g.m + t.bm - 1) / t.bm) * (double)((g.n + t.bn - 1) / t.bn) * (double)(g.reduce ? 1 : g.batch_count());
+        };
+        auto steps = [&](const GemmProblem &g) { return (double)((g.k + BK - 1) / BK) * (double)(g.reduce ? g.batch_count() : 1); };
+        const double np = items(p), nq = items(q), places = (double)cus * r.per_cu;
+        if (np + nq > 2.0 * places || std::max(steps(p), steps(q)) > kRingChunk) continue;
+        const double k_tile = r.k_tile[(int)std::min((double)r.per_cu, std::ceil((np + nq) / cus))];
+        const double tp = steps(p) * k_tile * (pb.kc ? 0.97 : 1.0) + r.item, tq = steps(q) * k_tile * 1.1 + r.item, longest = std::max(tp, tq);
+        double us = np + nq <= places ? longest : std::max(longest, (np * tp + nq * tq) / places + 0.4 * longest);
+        us += r.launch + 2.0 * ((double)p.m * p.n * (p.reduce ? 1 : p.batch_count()) + (double)q.m * q.n * (q.reduce ? 1 : q.batch_count())) / 8e6;
+        if (us * 1e-6 < *seconds) {
+            *seconds = us * 1e-6;
+            tile = v;
+        }
+    }
+    return tile;
+}
+
+hipError_t launch_mfma16_ring_pair(const GemmProblem &p, const GemmProblem &q, int tile, hipStream_t stream) {
+    if (!is_ring(tile) || p.dtype != q.dtype || !mfma16dma_supported(p, tile) || !mfma16dma_supported(q, tile)) return hipErrorInvalidValue;
+    RingParams rp, rq;
+    bool pa, pb, qa, qb;
+    GemmProblem whole[2] = {p, q};
+    whole[0].splits = whole[1].splits = 1;
+    if (hipError_t e = ring_params(whole[0], tile, rp, &pa, &pb); e != hipSuccess) return e;
+    if (hipError_t e = ring_params(whole[1], tile, rq, &qa, &qb); e != hipSuccess) return e;
+    if (!pa || qa || qb) return hipErrorInvalidValue;
+    return launch_mfma16_ring_two(tile - kNumTiles, p.dtype, rp, rq, pb, stream);
 }
 
 hipError_t launch_mfma16dma(const GemmProblem &g, int variant, hipStream_t stream) {

@@ -25,6 +25,8 @@ struct RingParams {
     X(3, 128, 64, 2, 2, 3)           \
     X(4, 128, 128, 2, 4, 4)
 
+// A backward pass: `p` with A stored along k, `q` with both operands stored across k, in one launch.
+hipError_t launch_mfma16_ring_two(int ring, int dtype, const RingParams &p, const RingParams &q, bool p_b_kc, hipStream_t stream);
 hipError_t launch_mfma16_ring(int ring, int dtype, const RingParams &p, bool a_kc, bool b_kc, hipStream_t stream);
 
 }  // namespace dfdx_rocm

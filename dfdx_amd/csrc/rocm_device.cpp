@@ -26,6 +26,15 @@ bool bad(const void *a, const void *b, const void *c) { return !a || !b || !c; }
 // Can `batch` matrices of `rows` rows, batch stride bs and row stride rs, be seen as one matrix of batch*rows rows?
 bool rows_fold(int64_t batch, int64_t rows, int64_t bs, int64_t rs) { return batch == 1 || bs == rows * rs; }
 
+// The two products of a backward pass: as one launch where that is faster, else one after the other.
+int both(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc &left, const dfdx_rocm_gemm_desc &right) {
+    bool done = false;
+    if (int e = dfdx_rocm::gemm_two(ctx, &left, 0, nullptr, &right, nullptr, &done)) return e;
+    if (done) return DFDX_ROCM_OK;
+    if (int e = dfdx_rocm_gemm(ctx, &left)) return e;
+    return dfdx_rocm_gemm(ctx, &right);
+}
+
 }  // namespace
 
 extern "C" {
@@ -150,14 +159,14 @@ int dfdx_rocm_matmat_batch3_backward(dfdx_rocm_ctx *ctx, int dtype, int64_t batc
     d.a = grad_out; d.a_b1 = m * n; d.a_rs = n; d.a_cs = 1;
     d.b = rhs; d.b_b1 = rs[0]; d.b_rs = rs[2]; d.b_cs = rs[1];
     d.c = grad_lhs; d.c_b1 = ls[0]; d.c_rs = ls[1]; d.c_cs = ls[2];
-    if (int e = dfdx_rocm_gemm(ctx, &d)) return e;
+    const dfdx_rocm_gemm_desc left = d;
     d = blank(dtype, k, m, n);
     d.accumulate = 1;
     d.batch1 = batch;
     d.a = lhs; d.a_b1 = ls[0]; d.a_rs = ls[2]; d.a_cs = ls[1];
     d.b = grad_out; d.b_b1 = m * n; d.b_rs = n; d.b_cs = 1;
     d.c = grad_rhs; d.c_b1 = rs[0]; d.c_rs = rs[1]; d.c_cs = rs[2];
-    return dfdx_rocm_gemm(ctx, &d);
+    return both(ctx, left, d);
 }
 
 // MatMatBatch4Kernel::forward (cpu_kernel.rs:424-448): (B,S,M,K) x (B,S,K,N).
@@ -186,14 +195,14 @@ int dfdx_rocm_matmat_batch4_backward(dfdx_rocm_ctx *ctx, int dtype, int64_t batc
     d.a = grad_out; d.a_b1 = seq * m * n; d.a_b2 = m * n; d.a_rs = n; d.a_cs = 1;
     d.b = rhs; d.b_b1 = rs[0]; d.b_b2 = rs[1]; d.b_rs = rs[3]; d.b_cs = rs[2];
     d.c = grad_lhs; d.c_b1 = ls[0]; d.c_b2 = ls[1]; d.c_rs = ls[2]; d.c_cs = ls[3];
-    if (int e = dfdx_rocm_gemm(ctx, &d)) return e;
+    const dfdx_rocm_gemm_desc left = d;
     d = blank(dtype, k, m, n);
     d.accumulate = 1;
     d.batch1 = batch; d.batch2 = seq;
     d.a = lhs; d.a_b1 = ls[0]; d.a_b2 = ls[1]; d.a_rs = ls[3]; d.a_cs = ls[2];
     d.b = grad_out; d.b_b1 = seq * m * n; d.b_b2 = m * n; d.b_rs = n; d.b_cs = 1;
     d.c = grad_rhs; d.c_b1 = rs[0]; d.c_b2 = rs[1]; d.c_rs = rs[2]; d.c_cs = rs[3];
-    return dfdx_rocm_gemm(ctx, &d);
+    return both(ctx, left, d);
 }
 
 // Linear::try_forward (dfdx/src/nn/layers/linear.rs:82-89) with Bias1D (bias1d.rs:62-78) fused into the store.

@@ -83,3 +83,39 @@ def test_bias_gradient_rides_along(dtype, rows, i, o):
     ulp = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype]
     assert_within(dtype, rows, host(gw, (o, i)), G.T @ X, G, X, extra=ulp * float(np.abs(G.T @ X).max()), what="weight")
     assert_within(dtype, o, host(gx, (rows, i)), G @ W, G, W, extra=ulp * float(np.abs(G @ W).max()), what="input")
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("rows,i,o", [(400, 256, 1024), (96, 128, 128), (529, 768, 768), (1344, 768, 1536), (1344, 768, 3072)])
+def test_two_products_of_a_backward_pass(dtype, rows, i, o):
+    """Launches of both gradients together, of few work items and of more than the chip has places for, into fresh and into
+    accumulated gradients."""
+    dev, g = device(), rng(rows + o)
+    announce("ring pair", dtype, rows, i, o)
+    x, w, go = (oracle.to_storage(g.standard_normal(s), dtype) for s in ((rows, i), (i, o), (rows, o)))
+    dx, dw, dgo = dev.tensor(x, dtype), dev.tensor(w, dtype), dev.tensor(go, dtype)
+    X, W, G = oracle.to_f64(x, dtype), oracle.to_f64(w, dtype), oracle.to_f64(go, dtype)
+    ulp = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype]
+    gx, gw = dev.zeros_many([dx, dw], deferred=True)
+    for times in (1, 2):
+        dev.backward(dx, gx, dw, gw, dgo)
+        for got, a, b, what in ((gx, G, W.T, "lhs"), (gw, X.T, G, "rhs")):
+            want = times * (a @ b)
+            assert_within(dtype, a.shape[1], oracle.to_f64(dev.to_host(got), dtype).reshape(want.shape), want, a, b,
+                          extra=2 * times * ulp * float(np.abs(want).max()), what=what)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("n", [128, 384])
+def test_a_gradient_that_both_products_add_to(dtype, n):
+    """x . x: both gradients go to one buffer, one behind the other."""
+    dev, g = device(), rng(n)
+    announce("ring pair, one gradient", dtype, n)
+    x, go = (oracle.to_storage(g.standard_normal((n, n)), dtype) for _ in range(2))
+    dx, dgo = dev.tensor(x, dtype), dev.tensor(go, dtype)
+    X, G = oracle.to_f64(x, dtype), oracle.to_f64(go, dtype)
+    gx = dev.zeros_like_storage(dx)
+    dev.backward(dx, gx, dx, gx, dgo)
+    want = G @ X.T + X.T @ G
+    ulp = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype]
+    assert_within(dtype, 2 * n, oracle.to_f64(dev.to_host(gx), dtype).reshape(n, n), want, X, G, extra=2 * ulp * float(np.abs(want).max()), what="sum")
