@@ -306,7 +306,7 @@ inline bool use_rank1(const GemmProblem &p) {
 }
 
 // The bandwidth-bound kernels (`Plan::variant` of a DFDX_ROCM_KERNEL_GEMV plan).
-enum { BW_NONE = 0, BW_RANK1 = 1, BW_GEMV_MULTI = 2, BW_GEMV = 3, BW_THIN_MFMA = 4 };
+enum { BW_NONE = 0, BW_RANK1 = 1, BW_GEMV_MULTI = 2, BW_GEMV = 3, BW_THIN_MFMA = 4, BW_ROWS = 5 };
 
 // Which of them takes `p`, if any.  `plain_order`: the caller asked for the contraction order of the tiled kernels
 // (DFDX_ROCM_GEMM_NO_SPLIT_K: the broadcast-rhs forward and grad_lhs, whose results must equal those of the batched
@@ -331,6 +331,7 @@ const char *bandwidth_kernel_name(const GemmProblem &p, int which) {
     case BW_GEMV_MULTI: return "gemv_multi";
     case BW_GEMV: return "gemv";
     case BW_THIN_MFMA: return "thin_k_mfma";
+    case BW_ROWS: return "gemv_rows";
     default: return "none";
     }
 }
@@ -378,18 +379,31 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
     default:
         return DFDX_ROCM_ERR_INVALID_ARG;
     }
-    // The bandwidth-bound kernels first.  The multi-vector form is weighed against the matrix-core plans by estimated
-    // time (the k-sliced small kernel streams a [n][k] matrix faster for most sizes, the tiles a large [k][n] one); the
-    // others have no rival.
-    const int bw = bandwidth_kernel(p, (d->flags & DFDX_ROCM_GEMM_NO_SPLIT_K) != 0);
+    // The bandwidth-bound kernels first.  Of the forms for several vectors those that keep their sums in the vector ALUs are weighed
+    // against the rows form and the matrix-core plans by estimated time (the tiles stream a large [k][n] matrix faster); the rows
+    // form has no rival (1 - 16 vectors against 512 - 16384 rows and columns, 245 products: 1.47 times as fast as the best plan
+    // without it in the mean, 4 x 4091 x 4093 f16 36.5 -> 10.1 us, f32 36.9 -> 15.7, 8 x 4288 x 4288 bf16 14 -> 11) but the
+    // small-product kernel, by estimated time, on rows that lie on the 16-byte grid of a matrix below 8 MB (up to 11 % there, either
+    // way: 8 x 520 x 2635 bf16 3.7 and 4.2 us, 16 x 2048 x 2048 7.0 and 6.8); the others have none.
+    int bw = bandwidth_kernel(p, (d->flags & DFDX_ROCM_GEMM_NO_SPLIT_K) != 0);
     double t_bw = 1e300;
-    if (bw == BW_GEMV_MULTI) {
-        t_bw = gemv_multi_time(p);
-    } else if (bw) {
+    if (bw == BW_GEMV_MULTI) t_bw = gemv_multi_time(p);
+    bool weighed = bw == BW_GEMV_MULTI;
+    if ((bw == BW_NONE || bw == BW_GEMV_MULTI) && !forced_splits && gemv_rows_supported(p)) {
+        // (the other forms take 1.1 times their estimate, 4 x 2048 x 2048 f32 10.2 us and 8.6 as rows, but on matrices that no cache
+        // holds: 8 x 16384 x 16384 f32 218 and 240)
+        const double bytes = (double)std::max(p.m, p.n) * (double)p.k * (double)dtype_size(p.dtype);
+        if (const double t = gemv_rows_time(p); t < (bytes < 268435456.0 ? 1.1 : 1.0) * t_bw) {
+            bw = BW_ROWS;
+            t_bw = t;
+            weighed = bytes < 8e6 && p.k * (int64_t)dtype_size(p.dtype) % 16 == 0;
+        }
+    }
+    if (bw && !weighed) {
         *plan = {DFDX_ROCM_KERNEL_GEMV, bw, 1};
         return DFDX_ROCM_OK;
     }
-    const Plan bw_plan = {DFDX_ROCM_KERNEL_GEMV, BW_GEMV_MULTI, 1};
+    const Plan bw_plan = {DFDX_ROCM_KERNEL_GEMV, bw, 1};
     // The small-product kernel where its estimate beats the family's (the f32 family weighs it among its own variants);
     // not where the caller fixed the order of the contraction.
     const bool may_small = forced_splits == 0 && (is16 || is64) && small_supported(p);
@@ -514,6 +528,7 @@ size_t partials_bytes(const GemmProblem &p, const Plan &plan, Realign *ra) {
                    : mfma16dma_workspace_bytes(p, plan.variant - mfma16_dma_first_variant() + 1, plan.splits);
     if (plan.kernel == DFDX_ROCM_KERNEL_GEMV && plan.variant == BW_GEMV_MULTI) return gemv_multi_workspace_bytes(p);
     if (plan.kernel == DFDX_ROCM_KERNEL_GEMV && plan.variant == BW_GEMV) return gemv_workspace_bytes(p);
+    if (plan.kernel == DFDX_ROCM_KERNEL_GEMV && plan.variant == BW_ROWS) return gemv_rows_workspace_bytes(p);
     return 0;
 }
 
@@ -576,6 +591,7 @@ int run_plan(dfdx_rocm_ctx *ctx, const GemmProblem &problem, const Plan &plan, b
         e = plan.variant == BW_RANK1 ? launch_rank1(p, ctx->stream)
             : plan.variant == BW_GEMV_MULTI ? launch_gemv_multi(p, ctx->stream)
             : plan.variant == BW_GEMV ? launch_gemv(p, ctx->stream)
+            : plan.variant == BW_ROWS ? launch_gemv_rows(p, ctx->stream)
             : plan.variant == BW_THIN_MFMA ? launch_thin_mfma(p, ctx->stream) : hipErrorInvalidValue;
         break;
     case DFDX_ROCM_KERNEL_MFMA:

@@ -206,6 +206,11 @@ bool gemv_multi_supported(const GemmProblem &p);
 size_t gemv_multi_workspace_bytes(const GemmProblem &p);
 double gemv_multi_time(const GemmProblem &p);  // estimated seconds
 hipError_t launch_gemv_multi(const GemmProblem &p, hipStream_t stream);
+// its third form: one to sixteen vectors, both operands stored along k, any alignment, any size of the matrix
+bool gemv_rows_supported(const GemmProblem &p);
+size_t gemv_rows_workspace_bytes(const GemmProblem &p);
+double gemv_rows_time(const GemmProblem &p);  // estimated seconds
+hipError_t launch_gemv_rows(const GemmProblem &p, hipStream_t stream);
 
 // ---- thin contractions with large outputs on the matrix cores (gemm_small.hip): k <= 32, f32 / f16 / bf16, row-major C ----
 bool thin_mfma_supported(const GemmProblem &p);

@@ -8,12 +8,14 @@
 //   "cols"  the matrix is contiguous in j: a thread owns VEC adjacent outputs of every r, the R vector slices sit in LDS
 //           (f32: as f32), the 4 waves of a workgroup take interleaved k, workgroups along grid.y take k slices;
 //   "dots"  the matrix is contiguous in k (a Linear weight viewed transposed): a wave owns 4 outputs j of every r, its
-//           lanes stride over k, each 16-byte piece of a vector is loaded once for the 4 matrix rows.
+//           lanes stride over k, each 16-byte piece of a vector is loaded once for the 4 matrix rows;
+//   "rows"  the same on the matrix cores, up to sixteen vectors, rows anywhere in memory (below).
 // The 16-bit types multiply pairs of k-adjacent values with v_dot2c_f32_f16 / _bf16 (f32 sums, operands stay packed).
 // Partial sums of k slices go to an f32 workspace [slice][r][j] and are combined in slice order (deterministic).
 #include "elem.h"
 #include "gemm_internal.h"
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace dfdx_rocm {
@@ -30,6 +32,7 @@ struct MultiParams {
     int accumulate, has_bias;
     int stream;  // the matrix is read with non-temporal loads: 256 MiB or more, as in the single-vector kernel (gemv.hip)
     float *ws;
+    int unit, period;  // rows form: bytes of the grid that rows are read on; rows that begin alike against it are `period` apart
 };
 template <bool STREAM> __device__ __forceinline__ u32x4 ldm(const void *p) {
     if constexpr (STREAM) return __builtin_nontemporal_load((const u32x4 *)p);
@@ -51,6 +54,8 @@ template <typename T, int N> __device__ __forceinline__ void unpack16(const T *p
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // acc + the products of two values that sit side by side along k in both operands (one dword each).  The 16-bit types
 // take v_dot2c_f32_*: two multiply-adds into an f32 sum per lane and instruction and no widening of the operands, which is
@@ -261,6 +266,96 @@ template <typename T, int R, bool STREAM> __global__ __launch_bounds__(256) void
     }
 }
 
+// The rows form: one to sixteen vectors against a matrix stored along k, its rows anywhere in memory.  A workgroup takes sixteen
+// outputs, its waves steps of 128 bytes of their rows in turn: a matrix core multiplies what a lane's two 16-byte loads bring (row
+// lane % 16, a quarter of the step) as it lies in the registers, so that nothing but the stream of the matrix is left to wait for.
+// Rows of an odd length begin anywhere: a workgroup takes rows that begin alike against the 128-byte lines, every 64th one for an odd
+// length of 16-bit values, and reads all of them in whole lines, the vectors shifted against them (with rows side by side, each load
+// off the grid, 1 x 4091 x 4093 f16 took 13.8 us instead of 9.4, 16379 x 16381 169 instead of 109; on the 16-byte grid only 9.7 and
+// 135).  Four steps of a wave are on their way at once, four waves a workgroup where the rows are short, sixteen where there are few
+// outputs, and k slices where there are fewer than 256 workgroups: 8 x 4096 x 4096 f16 9.4 us (3.6 TB/s), 8 x 16384 x 16384 118 us
+// (4.5 TB/s), f32 17 us and 241 us.
+template <typename T> __device__ __forceinline__ f32x4 rows_mma(u32x4 m, u32x4 v, f32x4 acc);
+template <> __device__ __forceinline__ f32x4 rows_mma<_Float16>(u32x4 m, u32x4 v, f32x4 acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, m), __builtin_bit_cast(f16x8, v), acc, 0, 0, 0);
+}
+template <> __device__ __forceinline__ f32x4 rows_mma<__bf16>(u32x4 m, u32x4 v, f32x4 acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, v), acc, 0, 0, 0);
+}
+template <> __device__ __forceinline__ f32x4 rows_mma<float>(u32x4 m, u32x4 v, f32x4 acc) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(m[e]), __uint_as_float(v[e]), acc, 0, 0, 0);
+    return acc;
+}
+template <bool STREAM> __device__ __forceinline__ u32x4 ldm_any(const void *p) {
+    if constexpr (STREAM) return __builtin_nontemporal_load((const u32x4_unaligned *)p);
+    else return *(const u32x4_unaligned *)p;
+}
+constexpr int rows_step(int elem_bytes) { return 128 / elem_bytes; }
+
+template <typename T, int WAVES, int AHEAD, bool STREAM> __global__ __launch_bounds__(WAVES * 64) void gemv_rows_kernel(const MultiParams p) {
+    constexpr int VEC = Elem<T>::VEC, STEP = rows_step(sizeof(T)), PITCH = 20;
+    __shared__ __align__(16) float part[WAVES][16 * PITCH];
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int l16 = lane % 16, lq = lane / 16;
+    // sixteen outputs whose rows begin alike against the grid: every period-th one
+    const int j0 = (int)blockIdx.x / p.period * 16 * p.period + (int)blockIdx.x % p.period;
+    if (j0 >= p.j) return;
+    const int ahead = (int)(((uintptr_t)((const T *)p.mat + (int64_t)j0 * p.mat_j_stride) & (uintptr_t)(p.unit - 1)) / sizeof(T));
+    const int j = j0 + p.period * l16;
+    const bool has_row = j < p.j, has_vec = l16 < p.r;
+    // step s is the values [s * STEP - ahead, (s + 1) * STEP - ahead); lanes without a row or a vector read the first one's (what
+    // they contribute to is not stored)
+    const T *const row = (const T *)p.mat + (int64_t)(has_row ? j : j0) * p.mat_j_stride + lq * VEC - ahead;
+    const T *const vec = (const T *)p.vec + (int64_t)(has_vec ? l16 : 0) * p.vec_r_stride + lq * VEC - ahead;
+    const int steps = (p.k + ahead + STEP - 1) / STEP, whole = (p.k + ahead) / STEP;
+    const int first = blockIdx.y * p.kchunk, last = min(steps, first + p.kchunk);
+    f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+    auto edge = [&](int s) {  // a step that begins in front of the rows or ends behind them
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int at = s * STEP + h * (STEP / 2) + lq * VEC - ahead;
+            const u32x4 m = row_window<T>((const T *)p.mat + (int64_t)j * p.mat_j_stride, has_row, at, p.k);
+            const u32x4 v = row_window<T>((const T *)p.vec + (int64_t)l16 * p.vec_r_stride, has_vec, at, p.k);
+            acc[h] = rows_mma<T>(m, v, acc[h]);
+        }
+    };
+    const int from = ahead && first == 0 ? 1 : first, to = min(whole, last);
+    int s = from + wave;
+    auto batch = [&](auto full_tag) {  // AHEAD steps, all of which are there (FULL) or some
+        constexpr bool FULL = decltype(full_tag)::value;
+        u32x4 m[AHEAD][2], v[AHEAD][2];
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            const int64_t at = (int64_t)(s + u * WAVES) * STEP;
+            if (!FULL && s + u * WAVES >= to) continue;  // the same in every lane
+#pragma unroll
+            for (int h = 0; h < 2; h++) m[u][h] = ldm_any<STREAM>(row + at + h * (STEP / 2));
+#pragma unroll
+            for (int h = 0; h < 2; h++) v[u][h] = *(const u32x4_unaligned *)(vec + at + h * (STEP / 2));
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            if (!FULL && s + u * WAVES >= to) continue;
+#pragma unroll
+            for (int h = 0; h < 2; h++) acc[h] = rows_mma<T>(m[u][h], v[u][h], acc[h]);
+        }
+    };
+    for (; s + (AHEAD - 1) * WAVES < to; s += AHEAD * WAVES) batch(std::true_type{});
+    if (s < to) batch(std::false_type{});
+    if (from > first && wave == WAVES - 1) edge(0);
+    if (to < last && last == steps && steps > from && wave == WAVES - 2) edge(whole);
+    *(f32x4 *)&part[wave][l16 * PITCH + lq * 4] = acc[0] + acc[1];  // vector l16, outputs lq * 4 .. + 3
+    __syncthreads();
+    const int r = tid / 16, out = j0 + p.period * (tid % 16);
+    if (tid >= 16 * p.r || out >= p.j) return;
+    float v = part[0][r * PITCH + tid % 16];
+#pragma unroll
+    for (int w = 1; w < WAVES; w++) v += part[w][r * PITCH + tid % 16];
+    if (p.kslices > 1) p.ws[((int64_t)blockIdx.y * p.r + r) * p.j + out] = v;
+    else finish<T>(p, r, out, v);
+}
+
 // Eight lanes per output: lane `part` of an output adds the slices part, part + 8, ... (their loads in flight together),
 // then the eight partial sums meet in a fixed tree of three exchanges -- one round trip to the workspace instead of
 // kslices / 8 of them behind one another (64 slices of a 4 x 4096 x 4096 product: 14 -> 9 us for the whole product).
@@ -319,6 +414,7 @@ template <typename T> __global__ __launch_bounds__(256) void gemv_multi_combine_
 struct Shape {
     bool ok, cols;
     MultiParams p;
+    int waves = 0, ahead = 0;  // of the rows form
 };
 
 inline bool al16(const void *q) { return ((uintptr_t)q & 15u) == 0; }
@@ -429,7 +525,104 @@ template <typename T> hipError_t launch_t(const Shape &s, hipStream_t stream) {
     return s.p.r <= 2 ? launch_r<T, 2>(s, stream) : s.p.r <= 4 ? launch_r<T, 4>(s, stream) : launch_r<T, 8>(s, stream);
 }
 
+// ---- the rows form -------------------------------------------------------------------------------------------------------
+int64_t rows_blocks(const MultiParams &p) { return ((int64_t)p.j + 16 * p.period - 1) / (16 * p.period) * p.period; }
+
+Shape classify_rows(const GemmProblem &g) {
+    Shape s{};
+    if (g.dtype == DT_F64 || g.reduce || g.nb1 * g.nb2 != 1 || g.k < 256 || g.k >= (1ll << 30)) return s;  // (k: a few steps)
+    if (g.m >= (1ll << 30) || g.n >= (1ll << 30) || g.c_rs < 1 || g.c_cs < 1) return s;
+    MultiParams &p = s.p;
+    if (g.m <= 16 && g.n > 16) {
+        p.vec = g.a; p.vec_k_stride = g.a_cs; p.vec_r_stride = g.a_rs;
+        p.mat = g.b; p.mat_k_stride = g.b_rs; p.mat_j_stride = g.b_cs;
+        p.out_j_stride = g.c_cs; p.out_r_stride = g.c_rs;
+        p.j = (int)g.n; p.r = (int)g.m;
+        p.bias_j_stride = g.bias_mode == BIAS_PER_COL; p.bias_r_stride = g.bias_mode == BIAS_PER_ROW;
+    } else if (g.n <= 16 && g.m > 16) {
+        p.vec = g.b; p.vec_k_stride = g.b_rs; p.vec_r_stride = g.b_cs;
+        p.mat = g.a; p.mat_k_stride = g.a_cs; p.mat_j_stride = g.a_rs;
+        p.out_j_stride = g.c_rs; p.out_r_stride = g.c_cs;
+        p.j = (int)g.m; p.r = (int)g.n;
+        p.bias_j_stride = g.bias_mode == BIAS_PER_ROW; p.bias_r_stride = g.bias_mode == BIAS_PER_COL;
+    } else {
+        return s;
+    }
+    if (p.mat_k_stride != 1 || p.vec_k_stride != 1 || p.mat_j_stride < 1 || (p.r > 1 && p.vec_r_stride < 1)) return s;
+    if (p.j < 128 || (int64_t)p.r * (int64_t)p.j >= (1ll << 31) - 256) return s;
+    const uintptr_t mask = dtype_size(g.dtype) - 1;
+    if (((uintptr_t)g.a | (uintptr_t)g.b | (uintptr_t)g.c | (uintptr_t)g.bias) & mask) return s;
+    p.out = g.c;
+    p.k = (int)g.k;
+    p.bias = g.bias;
+    p.has_bias = g.bias && g.bias_mode != BIAS_NONE;
+    p.accumulate = g.accumulate;
+    p.stream = (double)p.j * (double)g.k * (double)dtype_size(g.dtype) >= 268435456.0;
+    const int es = (int)dtype_size(g.dtype);
+    p.unit = 128;
+    p.period = 1;
+    while ((p.mat_j_stride * es * p.period) % p.unit) p.period *= 2;
+    const int64_t steps = (p.k + (p.period > 1 || (uintptr_t)p.mat % p.unit ? p.unit / es - 1 : 0) + rows_step(es) - 1) / rows_step(es);
+    const int64_t blocks = rows_blocks(p);
+    s.ahead = steps <= 8 ? 2 : 4;
+    s.waves = steps <= 24 ? 4 : steps <= 48 || blocks >= 512 ? 8 : 16;
+    int slices = 1;
+    while (blocks * slices < 256 && steps / (slices * 2) >= 4 * s.waves) slices *= 2;
+    p.kchunk = (int)((steps + slices - 1) / slices);
+    p.kslices = (int)((steps + p.kchunk - 1) / p.kchunk);
+    s.ok = true;
+    return s;
+}
+
+template <typename T, int WAVES, int AHEAD> void start_rows(const Shape &s, hipStream_t stream) {
+    dim3 grid((unsigned)rows_blocks(s.p), (unsigned)s.p.kslices);
+    if (s.p.stream) gemv_rows_kernel<T, WAVES, AHEAD, true><<<grid, WAVES * 64, 0, stream>>>(s.p);
+    else gemv_rows_kernel<T, WAVES, AHEAD, false><<<grid, WAVES * 64, 0, stream>>>(s.p);
+}
+template <typename T> hipError_t launch_rows_t(const Shape &s, hipStream_t stream) {
+    if (s.waves == 16) start_rows<T, 16, 4>(s, stream);
+    else if (s.waves == 8) start_rows<T, 8, 4>(s, stream);
+    else if (s.ahead == 4) start_rows<T, 4, 4>(s, stream);
+    else start_rows<T, 4, 2>(s, stream);
+    if (s.p.kslices > 1) gemv_multi_combine_kernel<T><<<dim3((unsigned)(((int64_t)s.p.r * s.p.j + 31) / 32)), 256, 0, stream>>>(s.p);
+    return hipGetLastError();
+}
+
 }  // namespace
+
+bool gemv_rows_supported(const GemmProblem &g) { return classify_rows(g).ok; }
+
+// Fitted to 245 products of 1 - 16 vectors and 512 - 16384 rows and columns, on and off the grid (standard deviation 8 %).
+double gemv_rows_time(const GemmProblem &g) {
+    const Shape s = classify_rows(g);
+    if (!s.ok) return 1e300;
+    // (a workgroup's own stream counts where there are few of them: 512 outputs, 32 workgroups)
+    const bool half = g.dtype != DT_F32;
+    const double es = (double)dtype_size(g.dtype), r = (double)s.p.r, mb = (double)s.p.j * (double)s.p.k * es / 1e6;
+    const double blocks = (double)rows_blocks(s.p) * s.p.kslices;
+    const double own = 16e-3 * (double)s.p.k * es / s.p.kslices * std::ceil(blocks / 256.0);
+    const double us = (half ? 2.2 : 2.5) + (s.p.kslices > 1 ? (half ? 2.8 : 1.4) : 0.0) + (s.p.period > 1 ? (half ? 1.3 : 0.8) : 0.0) +
+                      (half ? std::max(mb * (0.225 + 0.0051 * r), own * (0.041 + 0.0018 * r)) - 0.011 * std::max(0.0, mb - 200.0)
+                            : std::max(mb * (0.209 + 0.0063 * r), own * (0.0426 + 0.0015 * r)) - 0.024 * std::max(0.0, mb - 200.0));
+    return us * 1e-6;
+}
+
+size_t gemv_rows_workspace_bytes(const GemmProblem &g) {
+    const Shape s = classify_rows(g);
+    return s.ok && s.p.kslices > 1 ? (size_t)s.p.kslices * s.p.r * s.p.j * sizeof(float) : 0;
+}
+
+hipError_t launch_gemv_rows(const GemmProblem &g, hipStream_t stream) {
+    Shape s = classify_rows(g);
+    if (!s.ok || (s.p.kslices > 1 && !g.workspace)) return hipErrorInvalidValue;
+    s.p.ws = g.workspace;
+    switch (g.dtype) {
+    case DT_F32: return launch_rows_t<float>(s, stream);
+    case DT_F16: return launch_rows_t<_Float16>(s, stream);
+    case DT_BF16: return launch_rows_t<__bf16>(s, stream);
+    default: return hipErrorInvalidValue;
+    }
+}
 
 bool gemv_multi_supported(const GemmProblem &g) {
     Shape s = classify(g);

@@ -1,0 +1,38 @@
+"""One to sixteen vectors against a matrix stored along k, rows anywhere (the rows form of gemv_multi.hip): steps that are whole,
+partial or missing, rows off the 16-byte grid, outputs past the last sixteen, k slices."""
+import numpy as np
+import pytest
+
+import oracle
+from dfdx_amd.rocm import KERNEL_AUTO
+from gpu_util import announce, device
+from helpers import assert_within, rng
+from test_gpu_gemm import run_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rows,k,n", [(2, 1061, 2050), (1, 1063, 1601), (8, 2531, 4099), (16, 1999, 1040), (5, 5001, 517), (13, 12289, 600)])
+@pytest.mark.parametrize("pads", [(0, 0, 0), (3, 5, 1)])
+def test_rows_off_the_grid(dtype, rows, k, n, pads):
+    """Either operand as the matrix; bias, both beta, column-major C; the longest ones in k slices."""
+    assert run_case(dtype, rows, k, n, "nt", False, KERNEL_AUTO, 0, bias=True, pads=pads, seed=k) == "gemv_rows"
+    assert run_case(dtype, n, k, rows, "nt", True, KERNEL_AUTO, 0, pads=pads, seed=k + 1) == "gemv_rows"
+    run_case(dtype, rows, k, n, "nt", True, KERNEL_AUTO, 0, c_colmajor=True, pads=pads, seed=k + 2)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("k", [1024, 1024 + 1, 1024 + 31, 1024 + 32, 1024 + 63, 4096 - 7])
+def test_what_lies_behind_the_contraction_counts_for_nothing(dtype, k):
+    """Rows with a gap of NaN behind each: the partial step takes zeros in their place."""
+    dev, g = device(), rng(k)
+    rows, n, gap = 4, 2056, 9
+    announce("gemv rows gaps", dtype, k)
+    x, w = (oracle.to_storage(np.concatenate([g.standard_normal((r, k)), np.full((r, gap), np.nan)], axis=1), dtype) for r in (rows, n))
+    dx, dw, dc = dev.tensor(x, dtype), dev.tensor(w, dtype), dev.zeros(dtype, (rows, n))
+    dev.gemm(dev.gemm_desc(dtype, rows, k, n, dx.ptr, (k + gap, 1), dw.ptr, (1, k + gap), dc.ptr, (n, 1)))
+    X, W = (oracle.to_f64(t, dtype).reshape(-1, k + gap)[:, :k] for t in (x, w))
+    want = X @ W.T
+    ulp = {"f32": 2.0 ** -24, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype]
+    assert_within(dtype, k, oracle.to_f64(dev.to_host(dc), dtype).reshape(want.shape), want, X, W, extra=ulp * float(np.abs(want).max()), what="rows")
