@@ -559,7 +559,18 @@ template <typename T> bool few_channels(dfdx_rocm_ctx *ctx, int dtype, const Op 
     return true;
 }
 
-// 3 x 3 filters at unit stride with padding 1, f16 / bf16 / f32, channel counts in whole chunks: the kernel that keeps a band
+// Where the band kernels' blocks of 64 output channels are not whole, part of their work is for nothing.  In 16 bits they are ahead
+// all the same (102 shapes of 16 - 512 channels at 14 x 14 - 112 x 112, forward and backward: 1.5 times the speed of the products with
+// a patch matrix in the mean, 512 -> 16 at 28 x 28 181 -> 63 us, 96 -> 96 at 56 x 56 115 -> 54); in f32, which the matrix cores bound,
+// where the narrower side is one block or the chip is half full (8 images: 16 -> 32 at 56 x 56 120 -> 67 us, 256 -> 96 at 56 x 56 494 ->
+// 419, but at 28 x 28 237 -> 275 and 16 images of 512 -> 16 at 14 x 14 92 -> 108).
+bool band_pays(const Conv3x3Problem &c, int compute_units) {
+    if (c.dtype != DT_F32 || (c.chan_out % 64 == 0 && c.chan_in % 16 == 0)) return true;
+    const int64_t hw = (int64_t)c.h * c.w, blocks = (int64_t)((c.chan_out + 63) / 64) * ((hw + 255) / 256) * c.batch;
+    return hw >= 256 && (std::min(c.chan_in, c.chan_out) <= 64 || 2 * blocks >= compute_units);
+}
+
+// 3 x 3 filters at unit stride with padding 1, f16 / bf16 / f32, sixteen channels and more: the kernel that keeps a band
 // of the image in LDS and reads every tap's operand from it (conv3x3.hip).  The filters go through the patch buffer in
 // the order that kernel wants.
 template <typename T>
@@ -571,10 +582,10 @@ bool tiled3x3_forward(dfdx_rocm_ctx *ctx, int dtype, const Op &op, const void *f
     c.batch = op.batch; c.chan_in = op.chan_in; c.chan_out = op.chan_out; c.h = op.h_in; c.w = op.w_in;
     c.img = img; c.filters = filters; c.out = out;
     c.wt = (void *)16;  // any aligned address: the real one needs the lock below
-    if (!conv3x3_supported(c)) return false;
+    if (!conv3x3_supported(c) || !band_pays(c, ctx->compute_units)) return false;
     // Small images in a small batch give that kernel fewer workgroups (64 output channels x 256 pixels x image) than the chip
     // has compute units; one product over the folded batch fills it (f32, batch 32, 256 -> 256 at 14 x 14: 158 us here)
-    const int64_t hw = (int64_t)op.h_in * op.w_in, blocks = (int64_t)(op.chan_out / 64) * ((hw + 255) / 256) * op.batch;
+    const int64_t hw = (int64_t)op.h_in * op.w_in, blocks = (int64_t)((op.chan_out + 63) / 64) * ((hw + 255) / 256) * op.batch;
     if (blocks < ctx->compute_units && hw < 256 && op.batch > 1) return false;
     CtxLock lock(ctx->mu);  // the patch buffer is shared by every conv2d call on this context
     if ((*rc = ensure_patches(ctx, round256(conv3x3_filter_bytes(c))))) return true;
@@ -1156,9 +1167,38 @@ int backward_t(dfdx_rocm_ctx *ctx, int dtype, Op op, const void *img, void *grad
             return (int)launch_conv_few_backward(few, ctx->patches, ctx->stream);
         }
     }
+    // The image gradient of a 3 x 3, unit-stride, padding-1 convolution is such a convolution of grad_out (filters turned
+    // by 180 degrees, channels trading places): f16 / bf16 / f32 run it on the kernel that reads its taps from a band of
+    // grad_out in LDS (conv3x3.hip) instead of the product with the patch matrix, which only the filter gradient needs then.
+    Conv3x3Problem band{};
+    bool use_band = false;
+    if (sizeof(T) <= 4 && op.kernel == 3 && op.stride == 1 && op.padding == 1 && op.dilation == 1 && op.groups == 1 &&
+        op.h_out == op.h_in && op.w_out == op.w_in) {
+        band.dtype = dtype == DFDX_ROCM_F16 ? DT_F16 : dtype == DFDX_ROCM_BF16 ? DT_BF16 : DT_F32;
+        band.chan_in = op.chan_out; band.chan_out = op.chan_in; band.h = op.h_in; band.w = op.w_in;
+        band.batch = op.batch;
+        band.img = grad_out; band.filters = filters; band.out = grad_img;
+        band.accumulate = fresh_img ? 0 : 1; band.transposed_filters = 1;
+        band.wt = (void *)16;  // (placed below)
+        use_band = conv3x3_supported(band) && band_pays(band, ctx->compute_units);
+    }
+    // The filter gradient of such a convolution has its own kernels too (conv3x3_wgrad.hip; 16-bit types: both operands
+    // pixel-major in LDS, fragments through transposing reads; f32: channel-major bands, one value per lane and MFMA).
+    // With both in place the backward pass forms no patch matrix at all.
+    Conv3x3Problem wgrad{};
+    bool use_wgrad = false;
+    if (use_band) {
+        wgrad.dtype = band.dtype;
+        wgrad.batch = op.batch; wgrad.chan_in = op.chan_in; wgrad.chan_out = op.chan_out; wgrad.h = op.h_in; wgrad.w = op.w_in;
+        wgrad.img = img; wgrad.out = const_cast<void *>(grad_out); wgrad.filters = grad_filters;
+        // (f32 with blocks of 64 channels that are not whole: not on few pixels, 16 images of 512 -> 16 at 14 x 14 92 -> 108 us)
+        use_wgrad = conv3x3_wgrad_supported(wgrad, ctx->compute_units) && (sizeof(T) == 2 || hw >= 256 || (op.chan_in % 64 == 0 && op.chan_out % 64 == 0));
+    }
     // (also at unit stride when the image has far fewer channels than the output -- a first layer, 3 -> 64: the forward patch
-    // matrix is O / C times smaller than the one over grad_out, and the products with three rows of filters disappear)
-    if (op.stride > 1 || (int64_t)op.chan_in * 4 <= op.chan_out)
+    // matrix is O / C times smaller than the one over grad_out, and the products with three rows of filters disappear; the band
+    // kernels are ahead of that in 16 bits up to a ratio of sixteen: 8 images of 64 -> 256 at 96 x 96 225 -> 142 us, of 32 -> 512 at
+    // 28 x 28 53 -> 63 us, f32 16 -> 128 at 28 x 28 62 -> 96 us)
+    if (op.stride > 1 || ((int64_t)op.chan_in * 4 <= op.chan_out && !(use_wgrad && sizeof(T) == 2 && op.chan_out < (int64_t)op.chan_in * 16)))
         return strided_backward<T>(ctx, dtype, op, img, grad_img, filters, grad_filters, grad_out, fresh_img);
     if (per_image >= (1ll << 31) || f_elems >= (1ll << 31) || (int64_t)op.chan_in * hp >= (1ll << 31)) return DFDX_ROCM_ERR_UNSUPPORTED;
     CtxLock lock(ctx->mu);  // the patch buffer is shared by every conv2d call on this context
@@ -1182,33 +1222,7 @@ int backward_t(dfdx_rocm_ctx *ctx, int dtype, Op op, const void *img, void *grad
                       chunk <= 32768 && chunk * std::max(op.chan_in, op.chan_out) * hp < (1ll << 31) &&
                       small_unfold_shape<T>(hp, ohw, (int)std::min<int64_t>(chunk, op.batch), &fold_cg, &fold_bg, &fold_lds);
     const size_t img_bytes = (padded || fold) ? round256((size_t)(chunk * op.chan_in * hp) * sizeof(T)) : 0;
-    // The image gradient of a 3 x 3, unit-stride, padding-1 convolution is such a convolution of grad_out (filters turned
-    // by 180 degrees, channels trading places): f16 / bf16 / f32 run it on the kernel that reads its taps from a band of
-    // grad_out in LDS (conv3x3.hip) instead of the product with the patch matrix, which only the filter gradient needs then.
-    Conv3x3Problem band{};
-    bool use_band = false;
-    if (sizeof(T) <= 4 && op.kernel == 3 && op.stride == 1 && op.padding == 1 && op.dilation == 1 && op.groups == 1 &&
-        op.h_out == op.h_in && op.w_out == op.w_in) {
-        band.dtype = dtype == DFDX_ROCM_F16 ? DT_F16 : dtype == DFDX_ROCM_BF16 ? DT_BF16 : DT_F32;
-        band.chan_in = op.chan_out; band.chan_out = op.chan_in; band.h = op.h_in; band.w = op.w_in;
-        band.batch = (int)chunk;
-        band.img = grad_out; band.filters = filters; band.out = grad_img;
-        band.accumulate = fresh_img ? 0 : 1; band.transposed_filters = 1;
-        band.wt = (void *)16;  // (placed below)
-        use_band = conv3x3_supported(band);
-    }
     const size_t wt_bytes = use_band ? round256(conv3x3_filter_bytes(band)) : 0;
-    // The filter gradient of such a convolution has its own kernels too (conv3x3_wgrad.hip; 16-bit types: both operands
-    // pixel-major in LDS, fragments through transposing reads; f32: channel-major bands, one value per lane and MFMA).
-    // With both in place the backward pass forms no patch matrix at all.
-    Conv3x3Problem wgrad{};
-    bool use_wgrad = false;
-    if (use_band) {
-        wgrad.dtype = band.dtype;
-        wgrad.batch = op.batch; wgrad.chan_in = op.chan_in; wgrad.chan_out = op.chan_out; wgrad.h = op.h_in; wgrad.w = op.w_in;
-        wgrad.img = img; wgrad.out = const_cast<void *>(grad_out); wgrad.filters = grad_filters;
-        use_wgrad = conv3x3_wgrad_supported(wgrad, ctx->compute_units);
-    }
     if (use_band && use_wgrad) {
         const size_t ws_bytes = round256(conv3x3_wgrad_workspace_bytes(wgrad, ctx->compute_units));
         if (int rc = ensure_patches(ctx, ws_bytes + wt_bytes)) return rc;

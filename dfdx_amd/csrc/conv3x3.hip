@@ -71,9 +71,9 @@ template <> struct Mma16<float> {};
 
 struct Params {
     const void *img;  // [B][C][H][W]
-    const void *wt;   // [O][9][C]
+    const void *wt;   // [O][9][CP]
     void *out;        // [B][O][H][W]
-    int C, O, H, W, HW;
+    int C, CP, O, H, W, HW;  // CP: channels rounded up to whole chunks
     int nblocks, mblocks;  // pixel blocks per image, blocks of 64 output channels
     int band_rows;         // image rows (with the two halo rows) the LDS band holds
     uint32_t magic_w, magic_pairs;  // ceil(2^32 / W), ceil(2^32 / (W / 2)) (f32: / W again): n / W = umulhi(n, magic_w) for n < 2^24
@@ -81,14 +81,14 @@ struct Params {
 
 // wt[o][tap][c] = filters[o][c][tap] -- or, `transposed` (the image gradient: a convolution of grad_out with the filters
 // turned by 180 degrees, input and output channels trading places), wt[c][tap][o] = filters[o][c][8 - tap].
-// `inner` = the extent of wt's last axis, `outer` = that of its first.
+// `inner` = the extent of wt's last axis without its padding with zeros (`padded`), `outer` = that of its first.
 template <typename E>
-__global__ __launch_bounds__(256) void conv3x3_filters_kernel(const E *__restrict__ f, E *__restrict__ wt, int inner, int outer,
+__global__ __launch_bounds__(256) void conv3x3_filters_kernel(const E *__restrict__ f, E *__restrict__ wt, int inner, int padded, int outer,
                                                               int transposed, int total) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= total) return;
-    const int c = i % inner, tap = (i / inner) % 9, o = i / (9 * inner);
-    wt[i] = transposed ? f[((int64_t)c * outer + o) * 9 + (8 - tap)] : f[((int64_t)o * inner + c) * 9 + tap];
+    const int c = i % padded, tap = (i / padded) % 9, o = i / (9 * padded);
+    wt[i] = c >= inner ? (E)0 : transposed ? f[((int64_t)c * outer + o) * 9 + (8 - tap)] : f[((int64_t)o * inner + c) * 9 + tap];
 }
 
 // UMAX: pixel-pair units of the band a thread may own per chunk (2: four waves per SIMD, 128 registers; 4: two)
@@ -137,7 +137,8 @@ __global__ __launch_bounds__(512, (UMAX * (sizeof(T) == 2 ? 8 : 4) <= 16) ? 4 : 
 
     const char *const image = (const char *)p.img + (int64_t)b * p.C * p.HW * ES;
     const __amdgpu_buffer_rsrc_t planes = __builtin_amdgcn_make_buffer_rsrc((void *)image, 0, p.C * p.HW * ES, 0x00020000);
-    const char *const wrows = (const char *)p.wt + (int64_t)mb * MT * 9 * p.C * ES;
+    const char *const wrows = (const char *)p.wt + (int64_t)mb * MT * 9 * p.CP * ES;
+    const int channels = min(MT, p.O - mb * MT);  // of this block; behind the last one its row is read again, and nothing stored
     const int pairs = W / PPU, units = 4 * rows * pairs;  // units of a band row: pixel pairs (16-bit) or pixels (f32)
 
     // What a thread moves per chunk, worked out once: UMAX pixel-pair units of the band (element offset of channel 0 of
@@ -158,10 +159,11 @@ __global__ __launch_bounds__(512, (UMAX * (sizeof(T) == 2 ? 8 : 4) <= 16) ? 4 : 
     auto request = [&](int c0) {  // the global loads of one chunk: the band first, then the filter pieces
         // buffer loads: the image of this batch entry as the resource, one 32-bit byte offset per lane shared by the eight
         // loads of a unit, the channel plane in the scalar offset; a lane with nothing to load points past the end of the
-        // resource and receives zeros
+        // resource and receives zeros (no such unit, -1, or one of channels behind the last: C is a multiple of UL)
+        const uint32_t end = (uint32_t)((p.C - c0) * p.HW);
 #pragma unroll
         for (int s = 0; s < UMAX; s++) {
-            const uint32_t off = u_src[s] >= 0 ? (uint32_t)u_src[s] * (uint32_t)ES : 0xFFFFFFF0u;
+            const uint32_t off = (uint32_t)u_src[s] < end ? (uint32_t)u_src[s] * (uint32_t)ES : 0xFFFFFFF0u;
 #pragma unroll
             for (int e = 0; e < UL; e++) d[s][e] = __builtin_amdgcn_raw_buffer_load_b32(planes, (int)off, (c0 + e) * p.HW * ES, 0);
         }
@@ -169,8 +171,8 @@ __global__ __launch_bounds__(512, (UMAX * (sizeof(T) == 2 ? 8 : 4) <= 16) ? 4 : 
 #pragma unroll
         for (int s = 0; s < 5; s++) {
             const int q = tid + s * 512;  // 64 rows x 36 pieces, not kept in registers across the chunk
-            const int o = min(q / 36, MT - 1), part = q % 36;
-            piece[s] = *(const u32x4 *)(rowbase + (uint32_t)(((o * 9 + part / 4) * p.C + (part % 4) * (16 / ES)) * ES));
+            const int o = min(q / 36, channels - 1), part = q % 36;
+            piece[s] = *(const u32x4 *)(rowbase + (uint32_t)(((o * 9 + part / 4) * p.CP + (part % 4) * (16 / ES)) * ES));
         }
     };
     auto deposit = [&]() {  // ... into LDS: pixel records of two neighbouring pixels x 8 channels, filter pieces as they are
@@ -208,8 +210,9 @@ __global__ __launch_bounds__(512, (UMAX * (sizeof(T) == 2 ? 8 : 4) <= 16) ? 4 : 
         // ---- 9 taps x (2 x 4) MFMAs; operands swapped so that a lane ends up with 4 consecutive pixels of one channel.
         // Eighteen half taps (two pixel tiles each) in a software pipeline: the fragments of half tap h + 1 are requested
         // from LDS in front of the four MFMAs of half tap h, into the other register set.
-        // (a wave whose 64 pixels all lie past the end of the image -- the last pixel block of an image -- has nothing to multiply)
-        if (n0 + wn0 < p.HW) {
+        // (a wave whose 64 pixels all lie past the end of the image -- the last pixel block of an image -- or whose 32 channels lie
+        // behind the last one has nothing to multiply)
+        if (n0 + wn0 < p.HW && wm0 < channels) {
             u32x4 fa[2], fb[2][2];
             auto read_a = [&](int tap) {
 #pragma unroll
@@ -257,7 +260,7 @@ __global__ __launch_bounds__(512, (UMAX * (sizeof(T) == 2 ? 8 : 4) <= 16) ? 4 : 
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int n = n0 + wn0 + 16 * j + 4 * lq;
-                if (n < p.HW) {
+                if (n < p.HW && wm0 + 16 * i + l16 < channels) {
                     f32x4 v = acc[i][j];
                     if constexpr (ACC) v += *(const f32x4 *)(orow + n);
                     *(f32x4 *)(orow + n) = v;
@@ -286,7 +289,7 @@ __global__ __launch_bounds__(512, (UMAX * (sizeof(T) == 2 ? 8 : 4) <= 16) ? 4 : 
                             v[e] = __uint_as_float(r[0]);
                             v[4 + e] = __uint_as_float(r[1]);
                         }
-                        if (n < p.HW) {
+                        if (n < p.HW && wm0 + 16 * i + l16 < channels) {
                             const u32x4 old = *(const u32x4 *)(orow + n);
 #pragma unroll
                             for (int e = 0; e < 4; e++)
@@ -303,7 +306,7 @@ __global__ __launch_bounds__(512, (UMAX * (sizeof(T) == 2 ? 8 : 4) <= 16) ? 4 : 
                             o[2 + h] = r[1];
                         }
                     }
-                    if (n < p.HW) *(u32x4 *)(orow + n) = o;
+                    if (n < p.HW && wm0 + 16 * i + l16 < channels) *(u32x4 *)(orow + n) = o;
                 }
             }
         } else {
@@ -313,7 +316,7 @@ __global__ __launch_bounds__(512, (UMAX * (sizeof(T) == 2 ? 8 : 4) <= 16) ? 4 : 
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     const int n = n0 + wn0 + 16 * j + 4 * lq;
-                    if (n < p.HW) {  // HW % 4 == 0: all four pixels are in range
+                    if (n < p.HW && wm0 + 16 * i + l16 < channels) {  // HW % 4 == 0: all four pixels are in range
                         float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
                         if constexpr (ACC) {
                             const u32x2 old = *(const u32x2 *)(orow + n);
@@ -335,8 +338,8 @@ __global__ __launch_bounds__(512, (UMAX * (sizeof(T) == 2 ? 8 : 4) <= 16) ? 4 : 
 
 bool conv3x3_supported(const Conv3x3Problem &c) {
     if (c.dtype != DT_F16 && c.dtype != DT_BF16 && c.dtype != DT_F32) return false;
-    const int es = c.dtype == DT_F32 ? 4 : 2, ck = 64 / es;  // element bytes, channels per chunk
-    if (c.batch < 1 || c.chan_in < ck || c.chan_in % ck || c.chan_out < MT || c.chan_out % MT) return false;
+    const int es = c.dtype == DT_F32 ? 4 : 2;  // element bytes
+    if (c.batch < 1 || c.chan_in < 16 || c.chan_in % (16 / es) || c.chan_out < 16) return false;
     if (c.w < 4 || c.w > 254 || c.w % 2 || c.h < 1 || ((int64_t)c.h * c.w) % 4) return false;
     const int64_t hw = (int64_t)c.h * c.w;
     if (hw < 128 || hw >= (1 << 24) || (int64_t)c.chan_in * hw * es >= (1ll << 31)) return false;  // byte offsets of an image fit 31 bits
@@ -348,21 +351,24 @@ bool conv3x3_supported(const Conv3x3Problem &c) {
     return c.batch < 65536 && (hw + NT - 1) / NT < 65536;  // grid.z, grid.y
 }
 
-size_t conv3x3_filter_bytes(const Conv3x3Problem &c) { return (size_t)c.chan_out * 9 * c.chan_in * (c.dtype == DT_F32 ? 4 : 2); }
+namespace {
+int padded_channels(const Conv3x3Problem &c) { const int ck = c.dtype == DT_F32 ? 16 : 32; return (c.chan_in + ck - 1) / ck * ck; }
+}
+size_t conv3x3_filter_bytes(const Conv3x3Problem &c) { return (size_t)c.chan_out * 9 * padded_channels(c) * (c.dtype == DT_F32 ? 4 : 2); }
 
 hipError_t launch_conv3x3(const Conv3x3Problem &c, hipStream_t stream) {
     if (!conv3x3_supported(c)) return hipErrorNotSupported;
-    const int total = c.chan_out * 9 * c.chan_in;
+    const int padded = padded_channels(c), total = c.chan_out * 9 * padded;
     if (c.dtype == DT_F32)
-        conv3x3_filters_kernel<uint32_t><<<(total + 255) / 256, 256, 0, stream>>>((const uint32_t *)c.filters, (uint32_t *)c.wt, c.chan_in, c.chan_out,
+        conv3x3_filters_kernel<uint32_t><<<(total + 255) / 256, 256, 0, stream>>>((const uint32_t *)c.filters, (uint32_t *)c.wt, c.chan_in, padded, c.chan_out,
                                                                                  c.transposed_filters ? 1 : 0, total);
     else
-        conv3x3_filters_kernel<uint16_t><<<(total + 255) / 256, 256, 0, stream>>>((const uint16_t *)c.filters, (uint16_t *)c.wt, c.chan_in, c.chan_out,
+        conv3x3_filters_kernel<uint16_t><<<(total + 255) / 256, 256, 0, stream>>>((const uint16_t *)c.filters, (uint16_t *)c.wt, c.chan_in, padded, c.chan_out,
                                                                                  c.transposed_filters ? 1 : 0, total);
     Params p;
     p.img = c.img; p.wt = c.wt; p.out = c.out;
-    p.C = c.chan_in; p.O = c.chan_out; p.H = c.h; p.W = c.w; p.HW = c.h * c.w;
-    p.nblocks = (p.HW + NT - 1) / NT; p.mblocks = c.chan_out / MT;
+    p.C = c.chan_in; p.CP = padded; p.O = c.chan_out; p.H = c.h; p.W = c.w; p.HW = c.h * c.w;
+    p.nblocks = (p.HW + NT - 1) / NT; p.mblocks = (c.chan_out + MT - 1) / MT;
     p.band_rows = (int)std::min<int64_t>(c.h, (NT - 1) / c.w + 2) + 2;
     const size_t lds = (size_t)A_BYTES + (size_t)p.band_rows * (c.w + 2) * PIX;
     const int per_row = c.dtype == DT_F32 ? c.w : c.w / 2;  // units of a band row

@@ -146,12 +146,13 @@ __global__ __launch_bounds__(NTH, 3) void conv3x3_wgrad_kernel(const Params p) {
     uint32_t dx[UMAX][8], dg[UMAX][8];
     auto request = [&](int item) {  // the global loads of one work item: 8 channels x 2 pixels per unit and band
         const int b = item / p.bands, y0 = (item - b * p.bands) * p.R;
-        const __amdgpu_buffer_rsrc_t xsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.img + ((int64_t)b * p.C + cb * 64) * p.HW), 0, 64 * p.HW * 2, 0x00020000);
-        const __amdgpu_buffer_rsrc_t gsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.go + ((int64_t)b * p.O + ob * 64) * p.HW), 0, 64 * p.HW * 2, 0x00020000);
+        const __amdgpu_buffer_rsrc_t xsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.img + ((int64_t)b * p.C + cb * 64) * p.HW), 0, min(64, p.C - cb * 64) * p.HW * 2, 0x00020000);
+        const __amdgpu_buffer_rsrc_t gsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.go + ((int64_t)b * p.O + ob * 64) * p.HW), 0, min(64, p.O - ob * 64) * p.HW * 2, 0x00020000);
 #pragma unroll
         for (int s = 0; s < UMAX; s++) {
             const int yx = y0 - 1 + xs_row[s], yg = y0 + gs_row[s];
-            // (a unit outside the image, or none at all, points past the end of the resource and receives zeros)
+            // (a unit outside the image, or none at all, points past the end of the resource and receives zeros, as one of channels
+            // behind the last does by itself: they come in whole eights)
             const uint32_t ox = (xs_row[s] >= 0 && yx >= 0 && yx < H) ? (uint32_t)(xs_off[s] + yx * W) * 2u : 0xFFFFFFF0u;
             const uint32_t og = (gs_row[s] >= 0 && yg < H) ? (uint32_t)(gs_off[s] + yg * W) * 2u : 0xFFFFFFF0u;
 #pragma unroll
@@ -231,7 +232,7 @@ __global__ __launch_bounds__(NTH, 3) void conv3x3_wgrad_kernel(const Params p) {
 // each, in slice order, and the eight subtotals meet in LDS in group order: one fixed summation order, whatever the timing.
 template <typename T>
 __global__ __launch_bounds__(256) void conv3x3_wgrad_reduce_kernel(const float *__restrict__ partial,
-                                                                   typename StoredAs<T>::type *__restrict__ grad_filters, int C,
+                                                                   typename StoredAs<T>::type *__restrict__ grad_filters, int C, int O,
                                                                    int cblocks, int combos, int slices, int total) {
     __shared__ f32x4 subtotal[8][32];
     const int lane_elem = threadIdx.x % 32, group = threadIdx.x / 32;
@@ -258,6 +259,7 @@ __global__ __launch_bounds__(256) void conv3x3_wgrad_reduce_kernel(const float *
         for (int g = 1; g < 8; g++) all += subtotal[g][lane_elem];
         const int c = within % 64, o = (within / 64) % 64, tap = within / 4096;
         const int cb = combo % cblocks, ob = combo / cblocks;
+        if (ob * 64 + o >= O || cb * 64 + c >= C) return;  // (C is a multiple of four)
         typename StoredAs<T>::type *dst = grad_filters + ((int64_t)(ob * 64 + o) * C + cb * 64 + c) * 9 + tap;
 #pragma unroll
         for (int e = 0; e < 4; e++) dst[9 * e] = MmaW<T>::from_f32(MmaW<T>::to_f32(dst[9 * e]) + all[e]);
@@ -304,6 +306,9 @@ __global__ __launch_bounds__(NTH, 1) void conv3x3_wgrad_f32_kernel(const ParamsF
     const int combo = blockIdx.x % combos, slice = blockIdx.x / combos;
     const int cb = combo % p.cblocks, ob = combo / p.cblocks;
 
+    // (behind the last channel its band is fetched again; what comes of it is not stored)
+    const int x_chans = min(64, p.C - cb * 64), g_chans = min(64, p.O - ob * 64);
+
     // what this lane fetches for slot 64 seg + lane of any channel: element offset inside the channel's plane, counted
     // from image row y0 - 1, in the low 24 bits and the band row above them
     uint32_t g_unit[SEGS], x_unit[SEGS];
@@ -325,14 +330,14 @@ __global__ __launch_bounds__(NTH, 1) void conv3x3_wgrad_f32_kernel(const ParamsF
     auto begin_request = [&](int item, int stage) {
         const int b = item / p.bands;
         dma_ybase = (item - b * p.bands) * p.RS - 1;
-        xsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.img + ((int64_t)b * p.C + cb * 64) * p.HW), 0, 64 * p.HW * 4, 0x00020000);
-        gsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.go + ((int64_t)b * p.O + ob * 64) * p.HW), 0, 64 * p.HW * 4, 0x00020000);
+        xsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.img + ((int64_t)b * p.C + cb * 64) * p.HW), 0, x_chans * p.HW * 4, 0x00020000);
+        gsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.go + ((int64_t)b * p.O + ob * 64) * p.HW), 0, g_chans * p.HW * 4, 0x00020000);
         dma_dst = smem_addr + (uint32_t)stage * stage_bytes;
         dma_ch = wave;
     };
     auto request_channel = [&]() {  // both bands of channel dma_ch
         if (dma_ch >= 64) return;
-        const int plane = dma_ch * p.HW * 4;
+        const int x_plane = min(dma_ch, x_chans - 1) * p.HW * 4, g_plane = min(dma_ch, g_chans - 1) * p.HW * 4;
         const int row0 = dma_ybase * p.W;
         auto offset_of = [&](uint32_t u) -> int {
             const int y = dma_ybase + (int)(u >> 24);
@@ -342,12 +347,12 @@ __global__ __launch_bounds__(NTH, 1) void conv3x3_wgrad_f32_kernel(const ParamsF
         for (int seg = 0; seg < SEGS; seg++)
             if (seg < g_segs && g_unit[seg] != UNIT_NONE)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(gsrc, (DFDX_LDS void *)(uintptr_t)(dma_dst + (uint32_t)(dma_ch * p.GP + 64 * seg) * 4u), 4,
-                                                         offset_of(g_unit[seg]), plane, 0, 0);
+                                                         offset_of(g_unit[seg]), g_plane, 0, 0);
 #pragma unroll
         for (int seg = 0; seg < SEGS; seg++)
             if (seg < x_segs && x_unit[seg] != UNIT_NONE)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(xsrc, (DFDX_LDS void *)(uintptr_t)(dma_dst + (uint32_t)(64 * p.GP + dma_ch * p.XP + 64 * seg) * 4u), 4,
-                                                         offset_of(x_unit[seg]), plane, 0, 0);
+                                                         offset_of(x_unit[seg]), x_plane, 0, 0);
         dma_ch += 12;
     };
 
@@ -445,7 +450,7 @@ int bank_free_pitch(int n) {  // the smallest odd multiple of 2 that is >= n
 }
 bool make_plan_f32(const Conv3x3Problem &c, int compute_units, PlanF *out) {
     if (c.dtype != DT_F32) return false;
-    if (c.batch < 1 || c.chan_in < 64 || c.chan_in % 64 || c.chan_out < 64 || c.chan_out % 64) return false;
+    if (c.batch < 1 || c.chan_in < 16 || c.chan_in % 4 || c.chan_out < 16) return false;
     if (c.w < 2 || c.h < 1) return false;
     const int64_t hw = (int64_t)c.h * c.w;
     if (hw >= (1 << 22)) return false;  // byte offsets inside a block of 64 planes are 32-bit integers
@@ -462,7 +467,7 @@ bool make_plan_f32(const Conv3x3Problem &c, int compute_units, PlanF *out) {
     if (pl.RS < 1) return false;
     pl.bands = (c.h + pl.RS - 1) / pl.RS;
     pl.lds = (size_t)2 * (pl.GP + pl.XP) * 256;
-    pl.combos = (c.chan_in / 64) * (c.chan_out / 64);
+    pl.combos = ((c.chan_in + 63) / 64) * ((c.chan_out + 63) / 64);
     const int64_t items = (int64_t)c.batch * pl.bands;
     if (items >= (1ll << 31) || pl.combos > 65536) return false;
     pl.slices = (int)std::max<int64_t>(1, std::min<int64_t>(items, std::max(1, compute_units) / pl.combos));
@@ -476,7 +481,7 @@ struct Plan {
 };
 bool make_plan(const Conv3x3Problem &c, int compute_units, Plan *out) {
     if (c.dtype != DT_F16 && c.dtype != DT_BF16) return false;
-    if (c.batch < 1 || c.chan_in < 64 || c.chan_in % 64 || c.chan_out < 64 || c.chan_out % 64) return false;
+    if (c.batch < 1 || c.chan_in < 16 || c.chan_in % 8 || c.chan_out < 16 || c.chan_out % 8) return false;
     if (c.w < 4 || c.w > 254 || c.w % 2 || c.h < 1) return false;
     const int64_t hw = (int64_t)c.h * c.w;
     if (hw >= (1 << 24) || 64 * hw >= (1ll << 30)) return false;
@@ -492,7 +497,7 @@ bool make_plan(const Conv3x3Problem &c, int compute_units, Plan *out) {
     if (8 * (pl.R + 2) * (c.w / 2) > UMAX * NTH) return false;
     pl.lds = (size_t)(KMAX + pl.xrecs) * REC;
     if (pl.lds > 160 * 1024) return false;
-    pl.combos = (c.chan_in / 64) * (c.chan_out / 64);
+    pl.combos = ((c.chan_in + 63) / 64) * ((c.chan_out + 63) / 64);
     const int64_t items = (int64_t)c.batch * pl.bands;
     if (items >= (1ll << 31) || pl.combos > 65536) return false;
     pl.slices = (int)std::max<int64_t>(1, std::min<int64_t>(items, std::max(1, compute_units) / pl.combos));
@@ -522,7 +527,7 @@ hipError_t launch_conv3x3_wgrad_f32(const Conv3x3Problem &c, const PlanF &pl, vo
     p.img = (const float *)c.img; p.go = (const float *)c.out; p.partial = (float *)workspace;
     p.C = c.chan_in; p.O = c.chan_out; p.H = c.h; p.W = c.w; p.HW = c.h * c.w;
     p.RS = pl.RS; p.bands = pl.bands; p.items = c.batch * pl.bands;
-    p.slices = pl.slices; p.cblocks = c.chan_in / 64;
+    p.slices = pl.slices; p.cblocks = (c.chan_in + 63) / 64;
     p.RP = pl.RP; p.Q = pl.Q; p.GP = pl.GP; p.XP = pl.XP;
     p.magic_rp = (uint32_t)(((1ull << 32) + pl.RP - 1) / pl.RP);
     static PerDevice attr_on;
@@ -534,7 +539,7 @@ hipError_t launch_conv3x3_wgrad_f32(const Conv3x3Problem &c, const PlanF &pl, vo
     }
     conv3x3_wgrad_f32_kernel<<<(unsigned)(pl.combos * pl.slices), NTH, pl.lds, stream>>>(p);
     const int total = pl.combos * 9 * 4096;
-    conv3x3_wgrad_reduce_kernel<float><<<total / 128, 256, 0, stream>>>((const float *)workspace, (float *)c.filters, c.chan_in, p.cblocks,
+    conv3x3_wgrad_reduce_kernel<float><<<total / 128, 256, 0, stream>>>((const float *)workspace, (float *)c.filters, c.chan_in, c.chan_out, p.cblocks,
                                                                         pl.combos, pl.slices, total);
     return hipGetLastError();
 }
@@ -551,7 +556,7 @@ hipError_t launch_conv3x3_wgrad(const Conv3x3Problem &c, int compute_units, void
     p.img = (const uint16_t *)c.img; p.go = (const uint16_t *)c.out; p.partial = (float *)workspace;
     p.C = c.chan_in; p.O = c.chan_out; p.H = c.h; p.W = c.w; p.HW = c.h * c.w;
     p.R = pl.R; p.bands = pl.bands; p.items = c.batch * pl.bands;
-    p.slices = pl.slices; p.cblocks = c.chan_in / 64;
+    p.slices = pl.slices; p.cblocks = (c.chan_in + 63) / 64;
     p.kp = pl.kp; p.xrecs = pl.xrecs;
     p.magic_pairs = (uint32_t)(((1ull << 32) + c.w / 2 - 1) / (c.w / 2));
     const unsigned grid = (unsigned)(pl.combos * pl.slices);
@@ -566,7 +571,7 @@ hipError_t launch_conv3x3_wgrad(const Conv3x3Problem &c, int compute_units, void
         }                                                                                                              \
         conv3x3_wgrad_kernel<T><<<grid, NTH, pl.lds, stream>>>(p);                                                     \
         const int total = pl.combos * 9 * 4096;                                                                        \
-        conv3x3_wgrad_reduce_kernel<T><<<total / 128, 256, 0, stream>>>((const float *)workspace, (uint16_t *)c.filters, c.chan_in, \
+        conv3x3_wgrad_reduce_kernel<T><<<total / 128, 256, 0, stream>>>((const float *)workspace, (uint16_t *)c.filters, c.chan_in, c.chan_out, \
                                                                                p.cblocks, pl.combos, pl.slices, total); \
     } while (0)
     if (c.dtype == DT_F16) DFDX_WGRAD(_Float16);

@@ -1,0 +1,45 @@
+"""3 x 3 unit-stride convolutions whose channel counts are no whole blocks of the band kernels (conv3x3.hip, conv3x3_wgrad.hip):
+the last block of outputs and the last chunk of inputs are partial."""
+import numpy as np
+import pytest
+
+import oracle
+from gpu_util import announce, device
+from helpers import rng
+
+pytestmark = pytest.mark.gpu
+EPS = {"f32": 2.0 ** -24, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}
+
+
+def correlate(img, fil):
+    """out[b][o][y][x] = sum of fil[o][c][ky][kx] * img[b][c][y + ky - 1][x + kx - 1] in 64 bits."""
+    pad = np.pad(img, ((0, 0), (0, 0), (1, 1), (1, 1)))
+    h, w = img.shape[2:]
+    return sum(np.einsum("oc,bcyx->boyx", fil[:, :, ky, kx], pad[:, :, ky:ky + h, kx:kx + w]) for ky in range(3) for kx in range(3))
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("cin,cout", [(16, 16), (24, 64), (32, 96), (64, 32), (96, 48), (40, 136), (72, 200), (16, 80)])
+@pytest.mark.parametrize("batch,h,w", [(3, 16, 16), (2, 18, 30)])
+def test_channels_that_are_no_whole_blocks(dtype, cin, cout, batch, h, w):
+    """Forward, image and filter gradients (fresh and accumulated) of whole numbers that every type holds: sums below 2^24 are exact
+    in f32 whatever their order, so each result has the one rounding of its type."""
+    dev, g = device(), rng(cin * cout + w)
+    announce("conv3x3 channels", dtype, cin, cout, batch, h, w)
+    img, fil, go = (g.integers(-3, 4, size=s).astype(np.float64) for s in ((batch, cin, h, w), (cout, cin, 3, 3), (batch, cout, h, w)))
+    dimg, dfil, dgo = (dev.tensor(oracle.to_storage(t, dtype), dtype) for t in (img, fil, go))
+    host = lambda t, shape: oracle.to_f64(dev.to_host(t), dtype).reshape(shape)
+    rounded = lambda v: oracle.to_f64(oracle.to_storage(v, dtype), dtype).reshape(v.shape)
+    out = dev.conv2d_forward(dimg, dfil, stride=1, padding=1)
+    np.testing.assert_array_equal(host(out, go.shape), rounded(correlate(img, fil)))
+    want_img = correlate(go, fil[:, :, ::-1, ::-1].transpose(1, 0, 2, 3))
+    pad = np.pad(img, ((0, 0), (0, 0), (1, 1), (1, 1)))
+    want_fil = np.stack([np.stack([np.einsum("boyx,bcyx->oc", go, pad[:, :, ky:ky + h, kx:kx + w]) for kx in range(3)], -1) for ky in range(3)], -2)
+    gi, gf = dev.zeros_many([dimg, dfil], deferred=True)
+    dev.conv2d_backward(dimg, gi, dfil, gf, dgo, stride=1, padding=1)
+    first_img, first_fil = rounded(want_img), rounded(want_fil)
+    np.testing.assert_array_equal(host(gi, img.shape), first_img)
+    np.testing.assert_array_equal(host(gf, fil.shape), first_fil)
+    dev.conv2d_backward(dimg, gi, dfil, gf, dgo, stride=1, padding=1)  # onto what is there: rounded once more
+    np.testing.assert_array_equal(host(gi, img.shape), rounded(first_img + want_img))
+    np.testing.assert_array_equal(host(gf, fil.shape), rounded(first_fil + want_fil))
