@@ -206,18 +206,83 @@ struct RingModel {
     double k_tile[4], item, launch;
 };
 constexpr int64_t kRingChunk = 96, kRingAcross = 64;
+constexpr double kSecondLaunch = 3.5e-6, kLastRound = 0.6, kShortRound = 12e-6;  // see plan_tail
 constexpr RingModel kRing[] = {
     {2, {0.0, 0.187, 0.390, 0.0}, 2.75, 0.9},    // 64 x 64, four stages
     {3, {0.0, 0.234, 0.394, 0.572}, 3.30, 0.2},  // 64 x 64, three
     {2, {0.0, 0.305, 0.610, 0.0}, 4.10, 0.1},    // 128 x 64
     {1, {0.0, 0.414, 0.0, 0.0}, 4.80, 0.1},      // 128 x 128
 };
-inline double ring_time(const RingModel &r, int cus, int64_t items, int64_t total, bool whole, int64_t chunk, bool a_kc, bool b_kc, int splits, double out_elems) {
-    if (items > (int64_t)cus * r.per_cu || chunk > kRingChunk || (!a_kc && !b_kc && whole && total >= kRingAcross)) return 1e300;
+inline double ring_time(const RingModel &r, int cus, int64_t items, int64_t total, bool whole, int64_t chunk, bool a_kc, bool b_kc, int splits, double out_elems,
+                        int64_t longest = kRingChunk) {
+    if (items > (int64_t)cus * r.per_cu || chunk > longest || (!a_kc && !b_kc && whole && total >= kRingAcross)) return 1e300;
     const double layout = a_kc && b_kc ? 0.97 : !a_kc && !b_kc ? 1.1 : 1.0;
     double us = r.launch + r.item + (double)chunk * r.k_tile[(items + cus - 1) / cus] * layout + out_elems * 2.0 / 8e6;
     if (splits > 1) us += 2.6 + 0.2 * splits + splits * out_elems * 4.0 / 9.5e6;
     return us * 1e-6;
+}
+}  // namespace
+
+// The tiles of a product that has more of them than the chip has places are walked in rounds, and a last round of few tiles leaves
+// the chip idle for as long as a full one takes (0.6 of it: what runs there has the clock and the caches to itself).  Where the ring
+// tiles finish what is left over sooner, the product is cut behind the last full round, along its rows or its columns, into two
+// launches; every 16-bit tile sums in the same order, the bits are the same.  Before, such products took smaller tiles throughout.
+// f16, whole -> cut: 4224^3 177 -> 134 us, 4096 x 2048 x 4352 93 -> 66, 4608 x 1024 x 4096 51 -> 43, 4400 x 8192 x 4096 362 -> 257 (four
+// k pieces before), 8192 x 1024 x 4352 83 -> 69; 50257 x 2048 x 1024 (both across k) 220 -> 200.
+// Not for short rounds (16384 x 256 x 1100 25.7 us whole, 27.0 cut), nor for the tiles of which two share a compute unit, whose rounds
+// have no sharp end; and an uncut plan within 5 % is taken, as the model knows no better (12800 x 3072 x 768: 256 x 256 tiles 73 us, 256
+// x 128 cut 85).
+namespace {
+struct Tail {
+    int variant = 0;            // the ring tile; 0: the product stays whole
+    int64_t cut_m = 0, cut_n = 0;  // rows or columns of the first part (0: not along them)
+    double gain = 0.0;          // seconds less than with a last round as long as a full one (what the model takes it for)
+};
+GemmProblem part_of(const GemmProblem &p, int64_t m0, int64_t m1, int64_t n0, int64_t n1) {
+    GemmProblem q = p;
+    const int64_t es = 2, c_off = (m0 * p.c_rs + n0 * p.c_cs) * es;
+    q.m = m1 - m0;
+    q.n = n1 - n0;
+    q.ksum = nullptr;
+    q.ksum_of = KSUM_NONE;
+    q.a = (const char *)p.a + m0 * p.a_rs * es;
+    q.b = (const char *)p.b + n0 * p.b_cs * es;
+    q.c = (char *)p.c + c_off;
+    if (p.with) q.with = (const char *)p.with + c_off;
+    if (p.bias) q.bias = (const char *)p.bias + (p.bias_mode == BIAS_PER_ROW ? m0 : n0) * es;
+    return q;
+}
+Tail plan_tail(const GemmProblem &p, int variant, int compute_units) {
+    Tail best;
+    if (is_ring(variant) || kModel[variant - 1].per_cu > 1 || p.c_cs != 1 || (p.batch_count() != 1 && !p.reduce)) return best;
+    const Variant &t = kVariants[variant - 1];
+    const int cus = std::max(1, compute_units);
+    const int64_t places = cus;
+    const int64_t tm = (p.m + t.bm - 1) / t.bm, tn = (p.n + t.bn - 1) / t.bn, rounds = tm * tn / places;
+    if (rounds < 1 || tm * tn % places == 0) return best;
+    const int64_t steps = (p.k + BK - 1) / BK * (p.reduce ? p.batch_count() : 1);
+    const bool a_kc = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged).kc, b_kc = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged).kc;
+    const double round_seconds = (double)steps * (2.0 * t.bm * t.bn * BK) / kModel[variant - 1].rate1 + kItemOverhead;
+    if (round_seconds < kShortRound) return best;
+    double soonest = kLastRound * round_seconds;
+    for (int along_n = 0; along_n < 2; along_n++) {
+        const int64_t keep = rounds * places / (along_n ? tm : tn);  // whole rows (columns) of tiles in the full rounds
+        if (keep < 1 || keep >= (along_n ? tn : tm)) continue;
+        const int64_t cut = keep * (along_n ? t.bn : t.bm);
+        const GemmProblem rest = along_n ? part_of(p, 0, p.m, cut, p.n) : part_of(p, cut, p.m, 0, p.n);
+        for (int v = kNumTiles + 1; v <= kNumVariants; v++) {
+            if (!mfma16dma_supported(rest, v) || (p.extra != EXTRA_NONE && !mfma16dma_extra_supported(rest, v, 1))) continue;
+            const Variant &r = kVariants[v - 1];
+            const int64_t items = ((rest.m + r.bm - 1) / r.bm) * ((rest.n + r.bn - 1) / r.bn);
+            const double after = ring_time(kRing[v - 1 - kNumTiles], cus, items, 0, true, steps, a_kc, b_kc, 1, (double)rest.m * (double)rest.n, steps) +
+                                 kSecondLaunch;
+            if (after < soonest) {
+                soonest = after;
+                best = {v, along_n ? 0 : cut, along_n ? cut : 0, round_seconds - after};
+            }
+        }
+    }
+    return best;
 }
 }  // namespace
 
@@ -275,6 +340,8 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
                 time += kSplitLaunch + kSplitPerPiece * s +
                         (ws + out_elems * elem * (1 + p.accumulate)) / (ws <= kWsCached ? kWsBandwidthCached : kWsBandwidthHbm);
             }
+            if (s == 1)
+                if (const Tail tail = plan_tail(p, v, cus); tail.variant) time = 1.05 * (time - tail.gain);
             if (time < best) {
                 best = time;
                 *variant = v;
@@ -424,6 +491,13 @@ hipError_t launch_mfma16_ring_pair(const GemmProblem &p, const GemmProblem &q, i
 hipError_t launch_mfma16dma(const GemmProblem &g, int variant, hipStream_t stream) {
     if (!mfma16dma_supported(g, variant)) return hipErrorInvalidValue;
     if (is_ring(variant)) return launch_ring(g, variant, stream);
+    if (g.splits <= 1) {
+        if (const Tail tail = plan_tail(g, variant, g.compute_units); tail.variant) {
+            const bool rows = tail.cut_m > 0;
+            const hipError_t e = launch_mfma16dma(part_of(g, 0, rows ? tail.cut_m : g.m, 0, rows ? g.n : tail.cut_n), variant, stream);
+            return e != hipSuccess ? e : launch_ring(part_of(g, tail.cut_m, g.m, tail.cut_n, g.n), tail.variant, stream);
+        }
+    }
     const Variant &v = kVariants[variant - 1];
     const OperandLayout la = classify(g.m, g.k, g.a_rs, g.a_cs, g.ragged);
     const OperandLayout lb = classify(g.n, g.k, g.b_cs, g.b_rs, g.ragged);
