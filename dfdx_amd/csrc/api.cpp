@@ -781,8 +781,19 @@ static int ring_pair_tile(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d1, con
     return t1 > 0.0 && t2 > 0.0 && together < t1 + t2 + 1.0e-6 ? tile : 0;
 }
 
+// Would the call `d` run `p` on the small-product kernel?  Products that do and share nothing but what they read are one launch
+// (launch_small_many), with the bits of several.
+static bool plans_small(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProblem &p) {
+    if (d->kernel != DFDX_ROCM_KERNEL_AUTO || !small_supported(p)) return false;
+    Plan plan;
+    if (make_plan(ctx, d, p, &plan) || plan.kernel != DFDX_ROCM_KERNEL_MFMA || plan.realign) return false;
+    const int small = p.dtype == DT_F32 ? mfma32_variant_count() : p.dtype == DT_F64 ? mfma64_small_variant() : mfma16_small_variant();
+    return plan.variant == small && (!p.ksum || small_ksum_supported(p));
+}
+
 // Two independent products in one launch: pending fills, then the launch.  `sums` of the second one ride along.
-static int run_ring_pair(dfdx_rocm_ctx *ctx, GemmProblem p, GemmProblem q, int tile, bool may_overwrite) {
+// `tile`: of the ring, 0: the small-product kernel.
+static int run_pair(dfdx_rocm_ctx *ctx, GemmProblem p, GemmProblem q, int tile, bool may_overwrite) {
     CtxLock lock(ctx->mu);
     if (int e = settle_operands(ctx, &p, may_overwrite)) return e;
     if (int e = settle_operands(ctx, &q, /*may_overwrite=*/true)) return e;
@@ -792,7 +803,9 @@ static int run_ring_pair(dfdx_rocm_ctx *ctx, GemmProblem p, GemmProblem q, int t
         q.ksum_accumulate = !fresh;
     }
     p.compute_units = q.compute_units = ctx->compute_units;
-    return (int)launch_mfma16_ring_pair(p, q, tile, ctx->stream);
+    if (tile) return (int)launch_mfma16_ring_pair(p, q, tile, ctx->stream);
+    const GemmProblem both[2] = {p, q};
+    return (int)launch_small_many(both, 2, ctx->stream);
 }
 
 int gemm_two(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, int extra, const void *with, const dfdx_rocm_gemm_desc *second, void *colsum,
@@ -807,12 +820,12 @@ int gemm_two(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, int extra, co
     GemmProblem shape = p;
     shape.accumulate = 1;  // (what the ops that `extra` stands for would do)
     const int tile = ring_pair_tile(ctx, first, shape, second, q);
-    if (!tile) return DFDX_ROCM_OK;
+    if (!tile && !(plans_small(ctx, first, p) && plans_small(ctx, second, q))) return DFDX_ROCM_OK;
     p.extra = extra;
     p.with = with;
     if (!independent(p, q)) return DFDX_ROCM_OK;
     *done = true;
-    return run_ring_pair(ctx, p, q, tile, extra != EXTRA_FROM);
+    return run_pair(ctx, p, q, tile, extra != EXTRA_FROM);
 }
 
 int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_rocm_gemm_desc *second, const void *grad_out, int64_t rows, int64_t cols,
@@ -927,8 +940,37 @@ static int settle_three(dfdx_rocm_ctx *ctx, GemmProblem *problem) {
 int gemm_three(dfdx_rocm_ctx *ctx, const GemmProblem &problem, bool *done) {
     *done = false;
     GemmProblem p = problem;
-    if (p.dtype != DT_F16 && p.dtype != DT_BF16) return DFDX_ROCM_OK;
     p.compute_units = ctx->compute_units;
+    if (!p.reduce && p.extra == EXTRA_NONE) {
+        GemmProblem one[3] = {p, p, p};
+        const int64_t es = (int64_t)dtype_size(p.dtype);
+        dfdx_rocm_gemm_desc plain;
+        std::memset(&plain, 0, sizeof(plain));  // (an automatic plan)
+        bool small = true;
+        for (int i = 0; i < 3; i++) {
+            auto at = [&](const void *ptr, int64_t b1, int64_t b2) { return ptr ? (char *)ptr + (i == 1 ? b2 : i == 2 ? b1 : 0) * es : nullptr; };
+            GemmProblem &q = one[i];
+            q.batches = 0;
+            q.nb1 = q.nb2 = 1;
+            q.a = at(p.a, p.a_b1, p.a_b2);
+            q.b = at(p.b, p.b_b1, p.b_b2);
+            q.c = at(p.c, p.c_b1, p.c_b2);
+            q.bias = at(p.bias, p.bias_b1, p.bias_b2);
+            q.ksum = at(p.ksum, p.ksum_b1, p.ksum_b2);
+            small = small && plans_small(ctx, &plain, q);
+        }
+        if (small && independent(one[0], one[1]) && independent(one[0], one[2]) && independent(one[1], one[2])) {
+            *done = true;
+            CtxLock lock(ctx->mu);
+            if (int e = settle_three(ctx, &p)) return e;
+            for (GemmProblem &q : one) {
+                q.accumulate = p.accumulate;
+                q.ksum_accumulate = p.ksum_accumulate;
+            }
+            return (int)launch_small_many(one, 3, ctx->stream);
+        }
+    }
+    if (p.dtype != DT_F16 && p.dtype != DT_BF16) return DFDX_ROCM_OK;
     int dv = 0, splits = 1, dv1 = 0, splits1 = 1;
     double t3 = 1e300, t1 = 1e300;
     mfma16dma_plan_split(p, ctx->compute_units, 0, 0, &dv, &splits, &t3);

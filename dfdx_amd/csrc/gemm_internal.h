@@ -195,6 +195,7 @@ bool small_supported(const GemmProblem &p);
 bool small_ksum_supported(const GemmProblem &p);  // p.ksum of A as a second result
 double small_time(const GemmProblem &p, int compute_units);  // estimated seconds
 hipError_t launch_small(const GemmProblem &p, hipStream_t stream);
+hipError_t launch_small_many(const GemmProblem *p, int count, hipStream_t stream);  // two or three independent ones in one launch
 
 // ---- bandwidth-bound vector products (gemv.hip) ----
 bool gemv_supported(const GemmProblem &p);

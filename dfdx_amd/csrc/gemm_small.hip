@@ -124,7 +124,7 @@ template <> struct Small<__bf16> {
 // instructions a longer kernel has to fetch and jump over show (0.3 - 0.6 us on a 64-row Linear layer's gradients).
 // BEYOND: `c_old` and `extra` count.  The plain form has none of it, for the same reason (512 x 2304 x 259 f16 17.5 us with the
 // tests for them, 17.3 without; 16 x 2240 x 12833 f32 51.3 and 50.7).
-template <typename T, int WAVES, bool LONG, bool BEYOND> __global__ __launch_bounds__(WAVES * 64) void gemm_small_kernel(const SmallParams p) {
+template <typename T, int WAVES, bool LONG, bool BEYOND> __device__ __forceinline__ void small_tile(const SmallParams &p, const int block) {
     typedef Small<T> S;
     typedef typename S::acc_t A;
     typedef typename S::acc4 A4;
@@ -134,7 +134,7 @@ template <typename T, int WAVES, bool LONG, bool BEYOND> __global__ __launch_bou
     __shared__ A part_rows[WAVES][16];
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     const int r16 = lane % 16, q = lane / 16;
-    const int tm = blockIdx.x / p.tiles_n, tn = blockIdx.x % p.tiles_n;
+    const int tm = block / p.tiles_n, tn = block % p.tiles_n;
     const int row = tm * 16 + r16, col = tn * 16 + r16;
     const bool row_ok = row < p.m, col_ok = col < p.n;
     const T *ap = (const T *)p.a + (int64_t)(row_ok ? row : 0) * p.a_rs;
@@ -277,6 +277,22 @@ template <typename T, int WAVES, bool LONG, bool BEYOND> __global__ __launch_bou
     }
 }
 
+template <typename T, int WAVES, bool LONG, bool BEYOND> __global__ __launch_bounds__(WAVES * 64) void gemm_small_kernel(const SmallParams p) {
+    small_tile<T, WAVES, LONG, BEYOND>(p, (int)blockIdx.x);
+}
+
+// Two or three products that share nothing but what they read (a backward pass; the three projections of attention) in one launch: at
+// this size a launch costs more than the product behind it.  A product keeps the slices of k, and so the bits, that it has by
+// itself: waves that it has no slice for add zeros.
+struct SmallMany {
+    SmallParams p[3];
+    int first[3];  // block that each begins at; one that is not there begins behind the grid
+};
+template <typename T, int WAVES, bool LONG, bool BEYOND> __global__ __launch_bounds__(WAVES * 64) void gemm_small_many_kernel(const SmallMany s) {
+    const int block = (int)blockIdx.x, i = block >= s.first[2] ? 2 : block >= s.first[1] ? 1 : 0;
+    small_tile<T, WAVES, LONG, BEYOND>(s.p[i], block - s.first[i]);
+}
+
 inline size_t elem_size(int dt) { return dt == DT_F64 ? 8 : dt == DT_F32 ? 4 : 2; }
 // waves per workgroup: slices of at least 32 k; sixteen once each of them has two passes to overlap (not f64, whose two
 // passes of operands fill the 128 registers a lane of such a workgroup may have)
@@ -284,23 +300,37 @@ inline int small_waves(int dtype, int64_t k) {
     return (k >= 2048 && dtype != DT_F64) ? 16 : k >= 256 ? 8 : k >= 128 ? 4 : k >= 64 ? 2 : 1;
 }
 
-template <typename T, bool LONG, bool BEYOND> hipError_t launch_form(const SmallParams &p, int waves, dim3 grid, hipStream_t stream) {
+template <typename T, bool LONG, bool BEYOND, int WAVES> void start(const SmallParams &p, dim3 grid, hipStream_t stream) {
+    gemm_small_kernel<T, WAVES, LONG, BEYOND><<<grid, WAVES * 64, 0, stream>>>(p);
+}
+template <typename T, bool LONG, bool BEYOND, int WAVES> void start(const SmallMany &s, dim3 grid, hipStream_t stream) {
+    gemm_small_many_kernel<T, WAVES, LONG, BEYOND><<<grid, WAVES * 64, 0, stream>>>(s);
+}
+template <typename T, bool LONG, bool BEYOND, typename P> hipError_t launch_form(const P &p, int waves, dim3 grid, hipStream_t stream) {
     switch (waves) {
     case 16:
-        if constexpr (sizeof(T) < 8) gemm_small_kernel<T, 16, LONG, BEYOND><<<grid, 1024, 0, stream>>>(p);
+        if constexpr (sizeof(T) < 8) start<T, LONG, BEYOND, 16>(p, grid, stream);
         else return hipErrorInvalidValue;
         break;
-    case 8: gemm_small_kernel<T, 8, LONG, BEYOND><<<grid, 512, 0, stream>>>(p); break;
-    case 4: gemm_small_kernel<T, 4, LONG, BEYOND><<<grid, 256, 0, stream>>>(p); break;
-    case 2: gemm_small_kernel<T, 2, LONG, BEYOND><<<grid, 128, 0, stream>>>(p); break;
-    default: gemm_small_kernel<T, 1, LONG, BEYOND><<<grid, 64, 0, stream>>>(p); break;
+    case 8: start<T, LONG, BEYOND, 8>(p, grid, stream); break;
+    case 4: start<T, LONG, BEYOND, 4>(p, grid, stream); break;
+    case 2: start<T, LONG, BEYOND, 2>(p, grid, stream); break;
+    default: start<T, LONG, BEYOND, 1>(p, grid, stream); break;
     }
     return hipGetLastError();
 }
-template <typename T> hipError_t launch_t(const SmallParams &p, int waves, dim3 grid, hipStream_t stream) {
-    const bool beyond = p.c_old != p.c || p.extra != EXTRA_NONE;
-    if (p.slice > 16 * Small<T>::KL) return beyond ? launch_form<T, true, true>(p, waves, grid, stream) : launch_form<T, true, false>(p, waves, grid, stream);
+template <typename T, typename P> hipError_t launch_t(const P &p, int waves, int longest, bool beyond, dim3 grid, hipStream_t stream) {
+    if (longest > 16 * Small<T>::KL) return beyond ? launch_form<T, true, true>(p, waves, grid, stream) : launch_form<T, true, false>(p, waves, grid, stream);
     return beyond ? launch_form<T, false, true>(p, waves, grid, stream) : launch_form<T, false, false>(p, waves, grid, stream);
+}
+template <typename P> hipError_t launch_any(int dtype, const P &p, int waves, int longest, bool beyond, dim3 grid, hipStream_t stream) {
+    switch (dtype) {
+    case DT_F32: return launch_t<float>(p, waves, longest, beyond, grid, stream);
+    case DT_F16: return launch_t<_Float16>(p, waves, longest, beyond, grid, stream);
+    case DT_BF16: return launch_t<__bf16>(p, waves, longest, beyond, grid, stream);
+    case DT_F64: return launch_t<double>(p, waves, longest, beyond, grid, stream);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace
@@ -354,8 +384,7 @@ double small_time(const GemmProblem &p, int compute_units) {
     return 2.1e-6 + gather + std::max(std::max(chain, streamed / bandwidth), gather_stream) + c_bytes / c_rate;
 }
 
-hipError_t launch_small(const GemmProblem &g, hipStream_t stream) {
-    if (!small_supported(g) || g.splits > 1) return hipErrorInvalidValue;
+static SmallParams small_params(const GemmProblem &g, int *waves, int *blocks) {
     const size_t es = elem_size(g.dtype);
     const int kl = es == 2 ? 8 : 4;  // k values per lane and step: 16 bytes (f64: 32 bytes as two halves)
     const uintptr_t vmask = 15;
@@ -374,17 +403,42 @@ hipError_t launch_small(const GemmProblem &g, hipStream_t stream) {
     p.c_old = g.extra == EXTRA_FROM ? g.with : g.c;
     p.with = g.with;
     p.extra = g.extra == EXTRA_FROM ? EXTRA_NONE : g.extra;
-    const int waves = small_waves(g.dtype, g.k);
+    *waves = small_waves(g.dtype, g.k);
     const int step = 4 * kl;
-    p.slice = (int)(((g.k + waves - 1) / waves + step - 1) / step * step);
-    const dim3 grid((unsigned)(((g.m + 15) / 16) * p.tiles_n));
-    switch (g.dtype) {
-    case DT_F32: return launch_t<float>(p, waves, grid, stream);
-    case DT_F16: return launch_t<_Float16>(p, waves, grid, stream);
-    case DT_BF16: return launch_t<__bf16>(p, waves, grid, stream);
-    case DT_F64: return launch_t<double>(p, waves, grid, stream);
-    default: return hipErrorInvalidValue;
+    p.slice = (int)(((g.k + *waves - 1) / *waves + step - 1) / step * step);
+    *blocks = (int)((g.m + 15) / 16) * p.tiles_n;
+    return p;
+}
+static bool beyond(const SmallParams &p) { return p.c_old != p.c || p.extra != EXTRA_NONE; }
+
+hipError_t launch_small(const GemmProblem &g, hipStream_t stream) {
+    if (!small_supported(g) || g.splits > 1) return hipErrorInvalidValue;
+    int waves = 0, blocks = 0;
+    const SmallParams p = small_params(g, &waves, &blocks);
+    return launch_any(g.dtype, p, waves, p.slice, beyond(p), dim3((unsigned)blocks), stream);
+}
+
+hipError_t launch_small_many(const GemmProblem *g, int count, hipStream_t stream) {
+    if (count < 2 || count > 3) return hipErrorInvalidValue;
+    SmallMany s;
+    int waves = 0, grid = 0, longest = 0;
+    bool any_beyond = false;
+    for (int i = 0; i < 3; i++) {
+        if (i >= count) {  // never reached
+            s.p[i] = s.p[0];
+            s.first[i] = 1 << 30;
+            continue;
+        }
+        if (g[i].dtype != g[0].dtype || !small_supported(g[i]) || g[i].splits > 1) return hipErrorInvalidValue;
+        int w = 0, blocks = 0;
+        s.p[i] = small_params(g[i], &w, &blocks);
+        s.first[i] = grid;
+        grid += blocks;
+        waves = std::max(waves, w);
+        longest = std::max(longest, s.p[i].slice);
+        any_beyond = any_beyond || beyond(s.p[i]);
     }
+    return launch_any(g[0].dtype, s, waves, longest, any_beyond, dim3((unsigned)grid), stream);
 }
 
 
