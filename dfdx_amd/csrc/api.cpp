@@ -857,7 +857,7 @@ int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_r
         }
         if (int e = make_plan(ctx, d, p[i], &plan[i])) return e;
         // (one matrix each: the batches that a broadcast gradient is summed over step through grad_out by strides of their own)
-        both = both && plan[i].realign && p[i].nb1 * p[i].nb2 == 1 && p[i].a != p[i].b && plan_realign(p[i], &ra) && (p[i].a == grad_out ? ra.a : ra.b);
+        both = both && plan[i].realign && p[i].nb1 * p[i].nb2 == 1 && p[i].a != p[i].b && plan_realign(p[i], &ra) && (p[i].a == grad_out ? ra.a || ra.a_last : ra.b || ra.b_last);
     }
     auto apart = [&]() -> int {
         if (p[0].m)

@@ -52,6 +52,10 @@ struct GemmProblem {
     // of them, and C may lie anywhere.
     bool ragged = false;
     bool a_laid = false, b_laid = false;  // that operand is a copy of launch_realign_shared already
+    // Where the last k tile of an operand lies in a matrix of its own, with the same leading dimension (launch_realign): elements from
+    // its place in the operand to there.
+    bool last_apart = false;
+    int64_t a_last = 0, b_last = 0;
     // split-k (filled in by the planner): `splits` workgroups share one C tile; f32 partials go to `workspace`
     int splits;
     float *workspace;
@@ -92,6 +96,7 @@ static inline GemmProblem transposed(const GemmProblem &p) {
     if (p.bias_mode == BIAS_PER_COL) t.bias_mode = BIAS_PER_ROW;
     else if (p.bias_mode == BIAS_PER_ROW) t.bias_mode = BIAS_PER_COL;
     t.a_laid = p.b_laid; t.b_laid = p.a_laid;
+    t.a_last = p.b_last; t.b_last = p.a_last;
     if (p.ksum_of == KSUM_OF_A) t.ksum_of = KSUM_OF_B;
     else if (p.ksum_of == KSUM_OF_B) t.ksum_of = KSUM_OF_A;
     return t;
@@ -139,7 +144,8 @@ hipError_t launch_mfma16dma_extra(int variant, int dtype, int extra, const DmaPa
 hipError_t launch_mfma16dma_ragged(int variant, int dtype, const DmaParams &p, int compute_units, bool a_kc, bool b_kc, hipStream_t stream);  // gemm_mfma16_dma_ragged.hip
 // ---- operands of the 16-bit types laid out for those kernels (realign.hip) ----
 struct Realign {
-    bool a, b;                 // which operands are copied
+    bool a, b;                 // which operands are copied whole
+    bool a_last, b_last;       // of which the last k tile is copied
     GemmProblem problem;       // what the kernels are given (operand addresses: see realign_into)
     size_t a_bytes, b_bytes;   // space for the copies, multiples of 256
     double seconds;            // estimated time of the copies

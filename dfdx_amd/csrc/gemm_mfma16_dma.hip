@@ -141,6 +141,7 @@ bool mfma16dma_supported(const GemmProblem &p, int variant) {
     const int64_t tiles = ((p.m + v.bm - 1) / v.bm) * ((p.n + v.bn - 1) / v.bn);
     const int64_t blocks = tiles * (p.reduce ? 1 : p.batch_count());
     if (blocks >= (1ll << 31) || p.batch_count() >= (1ll << 31)) return false;
+    if (p.last_apart && (p.batch_count() != 1 || p.k % BK)) return false;
     if (p.k * (p.reduce ? p.batch_count() : 1) >= (1ll << 31)) return false;
     return true;
 }
@@ -419,6 +420,7 @@ static hipError_t ring_params(const GemmProblem &g, int variant, RingParams &p, 
     const int outputs = g.reduce ? 1 : nbatch, total_iters = (p.k + BK - 1) / BK * p.kbatches;
     p.accumulate = g.accumulate; p.bias_mode = g.bias ? g.bias_mode : BIAS_NONE;
     p.extra = g.extra; p.ksum_accumulate = g.ksum_accumulate;
+    p.whole = (int)(g.k / BK) - (g.last_apart ? 1 : 0); p.a_last = g.a_last; p.b_last = g.b_last;
     p.group_m = 4;
     p.splits = std::max(1, g.splits); p.chunk = total_iters; p.ws = p.ws_ksum = nullptr; p.ws_ld = p.ws_split_stride = 0; p.ws_ksum_stride = 0;
     if (g.ksum && !mfma16dma_ksum_supported(g, variant, g.splits)) return hipErrorInvalidValue;
@@ -535,6 +537,8 @@ hipError_t launch_mfma16dma(const GemmProblem &g, int variant, hipStream_t strea
         }
         p.total_blocks *= g.splits;
     }
+    p.apart = g.last_apart ? p.k / BK - 1 : -1;
+    p.a_last = g.a_last; p.b_last = g.b_last;
     p.grid = 0;  // set per kernel instantiation at launch
     p.with = (const uint16_t *)g.with;
     if (g.extra != EXTRA_NONE && !mfma16dma_extra_supported(g, variant, g.splits)) return hipErrorInvalidValue;

@@ -16,6 +16,8 @@ struct RingParams {
     int tiles_m, tiles_n, tiles_per_batch, items;
     int accumulate, bias_mode, extra, ksum_accumulate;
     int group_m, splits, chunk, ws_ksum_stride;
+    int whole;               // k tiles in front of a last one that is not whole, or lies apart: a_last, b_last elements from its place
+    int64_t a_last, b_last;
 };
 
 // X(id, BM, BN, WAVES_M, WAVES_N, stages); ids are 1-based inside this family.

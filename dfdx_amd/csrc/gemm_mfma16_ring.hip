@@ -117,6 +117,10 @@ __device__ __forceinline__ void ring_tile(const RingParams &p, const int index, 
             a_next = a_origin(f_kb);
             b_next = b_origin(f_kb);
         }
+        if (f_kt == p.whole) {
+            a_next += p.a_last;
+            b_next += p.b_last;
+        }
         const int k_left = p.k - f_kt * BK;
         if (k_left >= BK) {
             request_full(st);
@@ -297,7 +301,7 @@ __device__ __forceinline__ void ring_tile(const RingParams &p, const int index, 
     everybody();
     read_tile(fa[0], fb[0]);
     for (int t = 0; t < iters; t += 2) {
-        for (int whole = min(p.k / BK - f_kt, f_left); whole >= 2; whole -= 2, t += 2) {
+        for (int whole = min(p.whole - f_kt, f_left); whole >= 2; whole -= 2, t += 2) {
             step(t, EVEN, std::true_type{});
             step(t + 1, ODD, std::true_type{});
         }

@@ -3,6 +3,8 @@
 //
 // What bounds it: HBM, one read and one write of the operand.  The product behind it is bound by the matrix cores, and the
 // register-staged kernels that take any layout feed them at 0.3 - 0.6 of the LDS-DMA kernels' rate once both are large.
+// An operand on the grid whose rows lie along memory lacks the padding only: its last k tile is copied, with the leading dimension that
+// it has, and the kernels go there for it (2048 x 50257 . 50257 x 1024 f16, the copy 47 -> 6 us).
 // Both operands go in one launch; a thread moves four 16-byte pieces (element-aligned loads, aligned stores) that lie 256
 // pieces apart, so that every wave access is contiguous and four loads are in flight.
 #include "gemm_internal.h"
@@ -61,7 +63,7 @@ inline int64_t up(int64_t v, int64_t to) { return (v + to - 1) / to * to; }
 
 // One operand: `rows` of the product (m or n), strides of it and of the contraction, batch strides.
 struct Operand {
-    bool kc, copy, off;
+    bool kc, copy, off, last;  // last: of the last k tile only
     int64_t lines, lines_out, cols, ld_out, src_ld, n1, n2;  // as the copy walks it
     int64_t pieces() const { return n1 * n2 * lines_out * (ld_out / 8); }
 };
@@ -90,6 +92,13 @@ bool operand(const void *ptr, int64_t rows, int64_t k, int64_t row_stride, int64
     o->off = o->src_ld % 8 != 0 || (!o->kc && rows % 8 != 0) || ((uintptr_t)ptr & 15u) != 0 || (o->n1 > 1 && b1 % 8 != 0) || (o->n2 > 1 && b2 % 8 != 0);
     o->copy = o->off || kp != k;
     if (laid) o->off = o->copy = false;
+    // (one matrix; rows far apart in a view would be a copy of what lies between them)
+    o->last = o->copy && !o->off && !o->kc && nb1 * nb2 == 1 && o->src_ld <= 2 * o->ld_out;
+    if (o->last) {
+        o->lines = k - (kp - 64);
+        o->lines_out = 64;
+        o->ld_out = o->src_ld;
+    }
     return !o->copy || (o->pieces() < (1ll << 31) && o->lines_out < (1ll << 31) && o->ld_out < (1ll << 31));
 }
 void describe(const Operand &o, const void *src, void *dst, int64_t b1, int64_t b2, Side *s) {
@@ -121,8 +130,10 @@ bool plan_realign(const GemmProblem &p, Realign *r) {
     Operand a, b;
     if (!operand(p.a, p.m, p.k, p.a_rs, p.a_cs, p.a_b1, p.a_b2, p.nb1, p.nb2, p.a_laid, &a)) return false;
     if (!operand(p.b, p.n, p.k, p.b_cs, p.b_rs, p.b_b1, p.b_b2, p.nb1, p.nb2, p.b_laid, &b)) return false;
-    r->a = a.copy;
-    r->b = b.copy;
+    r->a = a.copy && !a.last;
+    r->b = b.copy && !b.last;
+    r->a_last = a.last;
+    r->b_last = b.last;
     r->problem = p;
     GemmProblem &q = r->problem;
     q.ragged = true;
@@ -131,16 +142,17 @@ bool plan_realign(const GemmProblem &p, Realign *r) {
     q.k = up(p.k, 64);
     r->a_bytes = r->b_bytes = 0;
     // (planning looks at the addresses' alignment only)
-    if (a.copy) {
+    q.last_apart = a.last || b.last;
+    if (r->a) {
         strides(a, &q.a_rs, &q.a_cs, &q.a_b1, &q.a_b2);
         q.a = (const void *)256;
-        r->a_bytes = (size_t)up(a.pieces() * 16, 256);
     }
-    if (b.copy) {
+    if (r->b) {
         strides(b, &q.b_cs, &q.b_rs, &q.b_b1, &q.b_b2);
         q.b = (const void *)256;
-        r->b_bytes = (size_t)up(b.pieces() * 16, 256);
     }
+    if (a.copy) r->a_bytes = (size_t)up(a.pieces() * 16, 256);
+    if (b.copy) r->b_bytes = (size_t)up(b.pieces() * 16, 256);
     if (r->a_bytes + r->b_bytes > REALIGN_MAX_BYTES) return false;
     r->off_grid = a.off + b.off;
     r->off_grid_k = (a.off && a.kc) + (b.off && b.kc);
@@ -175,13 +187,18 @@ hipError_t launch_realign_shared(const void *src, int64_t rows, int64_t cols, vo
 hipError_t launch_realign(const GemmProblem &p, Realign *r, void *space, hipStream_t stream) {
     Operand a, b;
     if (!operand(p.a, p.m, p.k, p.a_rs, p.a_cs, p.a_b1, p.a_b2, p.nb1, p.nb2, p.a_laid, &a) ||
-        !operand(p.b, p.n, p.k, p.b_cs, p.b_rs, p.b_b1, p.b_b2, p.nb1, p.nb2, p.b_laid, &b) || a.copy != r->a || b.copy != r->b)
+        !operand(p.b, p.n, p.k, p.b_cs, p.b_rs, p.b_b1, p.b_b2, p.nb1, p.nb2, p.b_laid, &b) || (a.copy && !a.last) != r->a || (b.copy && !b.last) != r->b || a.last != r->a_last || b.last != r->b_last)
         return hipErrorInvalidValue;
     Sides both{};
-    describe(a, p.a, space, p.a_b1, p.a_b2, &both.s[0]);
-    describe(b, p.b, (char *)space + r->a_bytes, p.b_b1, p.b_b2, &both.s[1]);
-    r->problem.a = a.copy ? space : p.a;
-    r->problem.b = b.copy ? (char *)space + r->a_bytes : p.b;
+    char *const a_to = (char *)space, *const b_to = a_to + r->a_bytes;
+    const int64_t first = p.k - 1 - (p.k - 1) % 64;  // of the last k tile
+    const uint16_t *const a_from = (const uint16_t *)p.a + (a.last ? first * a.src_ld : 0), *const b_from = (const uint16_t *)p.b + (b.last ? first * b.src_ld : 0);
+    describe(a, a_from, a_to, p.a_b1, p.a_b2, &both.s[0]);
+    describe(b, b_from, b_to, p.b_b1, p.b_b2, &both.s[1]);
+    r->problem.a = r->a ? a_to : p.a;
+    r->problem.b = r->b ? b_to : p.b;
+    r->problem.a_last = a.last ? ((intptr_t)a_to - (intptr_t)a_from) / 2 : 0;
+    r->problem.b_last = b.last ? ((intptr_t)b_to - (intptr_t)b_from) / 2 : 0;
     both.first_blocks = (both.s[0].total + PER_BLOCK - 1) / PER_BLOCK;
     const uint32_t blocks = both.first_blocks + (both.s[1].total + PER_BLOCK - 1) / PER_BLOCK;
     if (blocks == 0) return hipSuccess;
