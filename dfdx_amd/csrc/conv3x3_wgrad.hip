@@ -233,7 +233,7 @@ __global__ __launch_bounds__(NTH, 3) void conv3x3_wgrad_kernel(const Params p) {
 template <typename T>
 __global__ __launch_bounds__(256) void conv3x3_wgrad_reduce_kernel(const float *__restrict__ partial,
                                                                    typename StoredAs<T>::type *__restrict__ grad_filters, int C, int O,
-                                                                   int cblocks, int combos, int slices, int total) {
+                                                                   int cblocks, int combos, int slices, int total, int accumulate) {
     __shared__ f32x4 subtotal[8][32];
     const int lane_elem = threadIdx.x % 32, group = threadIdx.x / 32;
     const int i = blockIdx.x * 128 + lane_elem * 4;  // (combo, tap, o, c), c fastest; total is a multiple of 128
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(256) void conv3x3_wgrad_reduce_kernel(const float *
         if (ob * 64 + o >= O || cb * 64 + c >= C) return;  // (C is a multiple of four)
         typename StoredAs<T>::type *dst = grad_filters + ((int64_t)(ob * 64 + o) * C + cb * 64 + c) * 9 + tap;
 #pragma unroll
-        for (int e = 0; e < 4; e++) dst[9 * e] = MmaW<T>::from_f32(MmaW<T>::to_f32(dst[9 * e]) + all[e]);
+        for (int e = 0; e < 4; e++) dst[9 * e] = MmaW<T>::from_f32(accumulate ? MmaW<T>::to_f32(dst[9 * e]) + all[e] : all[e]);
     }
 }
 
@@ -507,7 +507,7 @@ bool make_plan(const Conv3x3Problem &c, int compute_units, Plan *out) {
 
 }  // namespace
 
-// `c` as for the forward kernel, with `out` = grad_out [batch][chan_out][h][w] and `filters` = grad_filters (accumulated into).
+// `c` as for the forward kernel, with `out` = grad_out [batch][chan_out][h][w] and `filters` = grad_filters (`accumulate`: added to).
 bool conv3x3_wgrad_supported(const Conv3x3Problem &c, int compute_units) {
     Plan pl;
     PlanF plf;
@@ -540,7 +540,7 @@ hipError_t launch_conv3x3_wgrad_f32(const Conv3x3Problem &c, const PlanF &pl, vo
     conv3x3_wgrad_f32_kernel<<<(unsigned)(pl.combos * pl.slices), NTH, pl.lds, stream>>>(p);
     const int total = pl.combos * 9 * 4096;
     conv3x3_wgrad_reduce_kernel<float><<<total / 128, 256, 0, stream>>>((const float *)workspace, (float *)c.filters, c.chan_in, c.chan_out, p.cblocks,
-                                                                        pl.combos, pl.slices, total);
+                                                                        pl.combos, pl.slices, total, c.accumulate);
     return hipGetLastError();
 }
 
@@ -572,7 +572,7 @@ hipError_t launch_conv3x3_wgrad(const Conv3x3Problem &c, int compute_units, void
         conv3x3_wgrad_kernel<T><<<grid, NTH, pl.lds, stream>>>(p);                                                     \
         const int total = pl.combos * 9 * 4096;                                                                        \
         conv3x3_wgrad_reduce_kernel<T><<<total / 128, 256, 0, stream>>>((const float *)workspace, (uint16_t *)c.filters, c.chan_in, c.chan_out, \
-                                                                               p.cblocks, pl.combos, pl.slices, total); \
+                                                                               p.cblocks, pl.combos, pl.slices, total, c.accumulate); \
     } while (0)
     if (c.dtype == DT_F16) DFDX_WGRAD(_Float16);
     else DFDX_WGRAD(__bf16);

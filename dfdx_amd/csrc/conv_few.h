@@ -9,8 +9,8 @@ struct ConvFew {
     int dtype, kernel, stride;
     int batch, chan_in, chan_out, h_in, w_in, h_out, w_out;
     const void *img, *filters, *grad_out;
-    void *out, *grad_img, *grad_filters;  // grad_filters is added to
-    int fresh_img;                        // grad_img is stored instead of added to
+    void *out, *grad_img, *grad_filters;
+    int fresh_img, fresh_filters;         // that gradient is stored instead of added to
     int compute_units;
 };
 

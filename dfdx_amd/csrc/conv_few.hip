@@ -521,7 +521,7 @@ __global__ __launch_bounds__(256, 2) void conv_few_grad_filters_kernel(const Par
 
 // 32 sums per workgroup, the workgroups' shares in eight runs, in order.
 template <typename T>
-__global__ __launch_bounds__(256) void conv_few_grad_filters_add_kernel(const float *ws, int shares, int taps, int chan_out, uint16_t *grad_filters) {
+__global__ __launch_bounds__(256) void conv_few_grad_filters_add_kernel(const float *ws, int shares, int taps, int chan_out, uint16_t *grad_filters, int fresh) {
     __shared__ float part[8][32];
     const int lane = threadIdx.x % 32, run = threadIdx.x / 32, i = blockIdx.x * 32 + lane, n = chan_out * taps;
     const float *src = ws + min(i, n - 1);
@@ -542,7 +542,7 @@ __global__ __launch_bounds__(256) void conv_few_grad_filters_add_kernel(const fl
 #pragma unroll
         for (int r = 1; r < 8; r++) sum += part[r][lane];
         uint16_t *dst = grad_filters + i;
-        *dst = (uint16_t)Mma<T>::pack2(Mma<T>::to_f32(*dst) + sum, 0.0f);
+        *dst = (uint16_t)Mma<T>::pack2(fresh ? sum : Mma<T>::to_f32(*dst) + sum, 0.0f);
     }
 }
 
@@ -636,7 +636,7 @@ template <typename T, int C, int K, int S> hipError_t backward_run(const ConvFew
     const int shares = grad_filters_shares(c), taps = C * K * K;
     conv_few_grad_filters_kernel<T, C, K, S><<<(unsigned)shares, 256, lds, stream>>>(p);
     if (hipError_t e = hipGetLastError()) return e;
-    conv_few_grad_filters_add_kernel<T><<<(unsigned)((c.chan_out * taps + 31) / 32), 256, 0, stream>>>(p.ws, shares, taps, c.chan_out, p.grad_filters);
+    conv_few_grad_filters_add_kernel<T><<<(unsigned)((c.chan_out * taps + 31) / 32), 256, 0, stream>>>(p.ws, shares, taps, c.chan_out, p.grad_filters, c.fresh_filters);
     return hipGetLastError();
 }
 
