@@ -46,8 +46,7 @@ struct DmaParams {
     float *ws_ksum;
     int ws_ksum_stride;
     const uint16_t *with;  // second operand of the EXTRA instances, laid out like c
-    int apart;  // the k tile that lies in matrices of its own, a_last and b_last elements from its place in the operands; -1: none
-    int64_t a_last, b_last;
+    int steps;  // (batch of the contraction, k tile) pairs: the last batch may end early
 };
 
 namespace {
@@ -242,7 +241,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
         w.split = p.splits > 1 ? bidx - w.batch * p.splits : 0;
         // k-loop steps run over (batch, k-tile) pairs; with split-k this item owns steps [it0, it0 + iters)
         w.it0 = w.split * p.chunk;
-        w.iters = min(ktiles * p.kbatches - w.it0, p.chunk);
+        w.iters = min(p.steps - w.it0, p.chunk);
         return w;
     };
 
@@ -285,11 +284,6 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
     auto issue = [&]() {
         const uint32_t st = (uint32_t)f_stage * STAGE_BYTES;
         f_stage ^= 1;
-        if (f_kt == p.apart) {
-            ArgParams *args = late_args();
-            a_next += args->a_last;
-            b_next += args->b_last;
-        }
         ta.issue(a_next, lds_last_a + st);
         tb.issue(b_next, lds_last_b + st);
         if (--f_left == 0) {  // next request belongs to the next work item (if any)

@@ -537,8 +537,18 @@ hipError_t launch_mfma16dma(const GemmProblem &g, int variant, hipStream_t strea
         }
         p.total_blocks *= g.splits;
     }
-    p.apart = g.last_apart ? p.k / BK - 1 : -1;
-    p.a_last = g.a_last; p.b_last = g.b_last;
+    p.steps = total_iters;
+    if (g.last_apart && p.k == BK) {
+        p.a += g.a_last;
+        p.b += g.b_last;
+    } else if (g.last_apart) {
+        // a last k tile that lies apart is one more batch of the contraction, of one tile (a test of the kernel's own for it, once a tile,
+        // cost products of short contractions 0.4 - 0.8 %)
+        p.k -= BK;
+        p.kbatches = p.nb2 = 2;
+        p.a_b2 = (la.kc ? p.k : (int64_t)p.k * p.lda) + g.a_last;
+        p.b_b2 = (lb.kc ? p.k : (int64_t)p.k * p.ldb) + g.b_last;
+    }
     p.grid = 0;  // set per kernel instantiation at launch
     p.with = (const uint16_t *)g.with;
     if (g.extra != EXTRA_NONE && !mfma16dma_extra_supported(g, variant, g.splits)) return hipErrorInvalidValue;
