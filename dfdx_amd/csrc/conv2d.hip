@@ -1243,10 +1243,19 @@ int backward_t(dfdx_rocm_ctx *ctx, int dtype, Op op, const void *img, void *grad
         if (int rc = ensure_patches(ctx, ws_bytes + wt_bytes)) return rc;
         band.batch = op.batch;
         band.wt = (char *)ctx->patches + ws_bytes;
-        HIP_TRY(launch_conv3x3(band, ctx->stream));
+        // The filter gradient first: the filters are laid for the image gradient beside the adding up of its shares.  Not where a gradient
+        // lies on what the kernels in between read.
+        auto meets = [](const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+            return (uintptr_t)a < (uintptr_t)b + b_bytes && (uintptr_t)b < (uintptr_t)a + a_bytes;
+        };
+        const size_t out_bytes = (size_t)op.batch * op.chan_out * ohw * sizeof(T), in_bytes = (size_t)op.batch * op.chan_in * hw * sizeof(T);
+        const bool first = !meets(grad_filters, filter_bytes, filters, filter_bytes) && !meets(grad_filters, filter_bytes, grad_out, out_bytes) &&
+                           !meets(grad_filters, filter_bytes, grad_img, in_bytes);
+        if (!first) HIP_TRY(launch_conv3x3(band, ctx->stream));
         if (int e = take_filters()) return e;
         wgrad.accumulate = !fresh_filters;
-        return ended(launch_conv3x3_wgrad(wgrad, ctx->compute_units, ctx->patches, ctx->stream));
+        if (int e = ended(launch_conv3x3_wgrad(wgrad, ctx->compute_units, ctx->patches, ctx->stream, first ? &band : nullptr))) return e;
+        return first ? (int)launch_conv3x3(band, ctx->stream, /*laid=*/true) : DFDX_ROCM_OK;
     }
     if (pointwise) {
         // Filters [O][C/G] are plain matrices here and both products take them as they lie, transposed through the strides:

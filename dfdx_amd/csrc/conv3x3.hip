@@ -79,16 +79,8 @@ struct Params {
     uint32_t magic_w, magic_pairs;  // ceil(2^32 / W), ceil(2^32 / (W / 2)) (f32: / W again): n / W = umulhi(n, magic_w) for n < 2^24
 };
 
-// wt[o][tap][c] = filters[o][c][tap] -- or, `transposed` (the image gradient: a convolution of grad_out with the filters
-// turned by 180 degrees, input and output channels trading places), wt[c][tap][o] = filters[o][c][8 - tap].
-// `inner` = the extent of wt's last axis without its padding with zeros (`padded`), `outer` = that of its first.
-template <typename E>
-__global__ __launch_bounds__(256) void conv3x3_filters_kernel(const E *__restrict__ f, E *__restrict__ wt, int inner, int padded, int outer,
-                                                              int transposed, int total) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= total) return;
-    const int c = i % padded, tap = (i / padded) % 9, o = i / (9 * padded);
-    wt[i] = c >= inner ? (E)0 : transposed ? f[((int64_t)c * outer + o) * 9 + (8 - tap)] : f[((int64_t)o * inner + c) * 9 + tap];
+template <typename E> __global__ __launch_bounds__(256) void conv3x3_filters_kernel(const Conv3x3Filters a) {
+    conv3x3_lay<E>(a, (int)(blockIdx.x * 256 + threadIdx.x));
 }
 
 // UMAX: pixel-pair units of the band a thread may own per chunk (2: four waves per SIMD, 128 registers; 4: two)
@@ -356,15 +348,20 @@ int padded_channels(const Conv3x3Problem &c) { const int ck = c.dtype == DT_F32 
 }
 size_t conv3x3_filter_bytes(const Conv3x3Problem &c) { return (size_t)c.chan_out * 9 * padded_channels(c) * (c.dtype == DT_F32 ? 4 : 2); }
 
-hipError_t launch_conv3x3(const Conv3x3Problem &c, hipStream_t stream) {
+Conv3x3Filters conv3x3_filters(const Conv3x3Problem &c) {
+    const int padded = padded_channels(c);
+    return {c.filters, c.wt, c.chan_in, padded, c.chan_out, c.transposed_filters ? 1 : 0, c.chan_out * 9 * padded};
+}
+
+hipError_t launch_conv3x3(const Conv3x3Problem &c, hipStream_t stream, bool laid) {
     if (!conv3x3_supported(c)) return hipErrorNotSupported;
-    const int padded = padded_channels(c), total = c.chan_out * 9 * padded;
-    if (c.dtype == DT_F32)
-        conv3x3_filters_kernel<uint32_t><<<(total + 255) / 256, 256, 0, stream>>>((const uint32_t *)c.filters, (uint32_t *)c.wt, c.chan_in, padded, c.chan_out,
-                                                                                 c.transposed_filters ? 1 : 0, total);
-    else
-        conv3x3_filters_kernel<uint16_t><<<(total + 255) / 256, 256, 0, stream>>>((const uint16_t *)c.filters, (uint16_t *)c.wt, c.chan_in, padded, c.chan_out,
-                                                                                 c.transposed_filters ? 1 : 0, total);
+    const int padded = padded_channels(c);
+    if (!laid) {
+        const Conv3x3Filters a = conv3x3_filters(c);
+        const unsigned blocks = (unsigned)((a.total + 255) / 256);
+        if (c.dtype == DT_F32) conv3x3_filters_kernel<uint32_t><<<blocks, 256, 0, stream>>>(a);
+        else conv3x3_filters_kernel<uint16_t><<<blocks, 256, 0, stream>>>(a);
+    }
     Params p;
     p.img = c.img; p.wt = c.wt; p.out = c.out;
     p.C = c.chan_in; p.CP = padded; p.O = c.chan_out; p.H = c.h; p.W = c.w; p.HW = c.h * c.w;

@@ -43,3 +43,20 @@ def test_channels_that_are_no_whole_blocks(dtype, cin, cout, batch, h, w):
     dev.conv2d_backward(dimg, gi, dfil, gf, dgo, stride=1, padding=1)  # onto what is there: rounded once more
     np.testing.assert_array_equal(host(gi, img.shape), rounded(first_img + want_img))
     np.testing.assert_array_equal(host(gf, fil.shape), rounded(first_fil + want_fil))
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+def test_filter_gradient_where_the_filters_lie(dtype):
+    """Added to the filters in place: the image gradient has been formed from them before.  Whole numbers, as above."""
+    dev, g = device(), rng(61)
+    announce("conv3x3, filter gradient onto the filters", dtype)
+    img, fil, go = (g.integers(-3, 4, size=s).astype(np.float64) for s in ((2, 64, 16, 16), (64, 64, 3, 3), (2, 64, 16, 16)))
+    dimg, dfil, dgo = (dev.tensor(oracle.to_storage(t, dtype), dtype) for t in (img, fil, go))
+    apart_img, apart_fil = dev.zeros_many([dimg, dfil], deferred=True)
+    dev.conv2d_backward(dimg, apart_img, dfil, apart_fil, dgo, stride=1, padding=1)
+    onto_img = dev.zeros(dtype, img.shape)
+    want = oracle.to_f64(dev.to_host(apart_fil), dtype) + fil.reshape(-1)
+    dev.conv2d_backward(dimg, onto_img, dfil, dfil, dgo, stride=1, padding=1)
+    np.testing.assert_array_equal(dev.to_host(onto_img), dev.to_host(apart_img))
+    ulp = 0.0 if dtype == "f32" else 2.0 ** -11   # the sum is rounded once more beside the one that stands alone
+    assert np.abs(oracle.to_f64(dev.to_host(dfil), dtype) - want).max() <= 2 * ulp * np.abs(want).max()
