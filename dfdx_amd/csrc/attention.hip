@@ -556,6 +556,22 @@ bool rows_apart(int64_t batch, int64_t heads, int64_t seq, int64_t dim, const in
     }
     return true;
 }
+// Does a row of one of two such views meet a row of the other, which lies `delta` elements behind?  What is left of the distance once the
+// longer strides are taken out lies less than a stride from zero, on either side of it: rows_apart holds.
+bool rows_meet(int64_t batch, int64_t heads, int64_t seq, int64_t dim, const int64_t s[3], int64_t delta) {
+    const int64_t ext[3] = {batch, heads, seq};
+    auto meet = [&](auto &&self, int left, int64_t apart) -> bool {  // `left`: a bit for each axis not taken out yet
+        int top = -1;
+        for (int i = 0; i < 3; i++)
+            if ((left >> i & 1) && ext[i] > 1 && (top < 0 || s[i] > s[top])) top = i;
+        if (top < 0) return apart > -dim && apart < dim;
+        const int64_t steps = apart / s[top] - (apart % s[top] < 0);
+        for (int64_t d = steps; d <= steps + 1; d++)
+            if (d > -ext[top] && d < ext[top] && self(self, left & ~(1 << top), apart - d * s[top])) return true;
+        return false;
+    };
+    return meet(meet, 7, delta);
+}
 
 }  // namespace
 
@@ -653,9 +669,12 @@ int dfdx_rocm_attention_backward(dfdx_rocm_ctx *ctx, int dtype, int64_t batch, i
     p.add_q = !fresh[0]; p.add_k = !fresh[1]; p.add_v = !fresh[2];
     dim3 grid((unsigned)p.total);
     const dim3 block(256);
-    // In one launch where the workgroups of both have a place at once and neither writes what the other reads.
+    // In one launch where the workgroups of both have a place at once and neither writes what the other reads or writes (packed
+    // gradients interleave without meeting; one that two operands share is added to by one launch behind the other).
     auto end = [&](const void *from, const int64_t st[3]) { return (uintptr_t)from + (size_t)((batch - 1) * st[0] + (heads - 1) * st[1] + (seq - 1) * st[2] + dim) * 2; };
     bool apart = 2 * (int64_t)p.total <= (int64_t)ctx->compute_units * (dim == 128 ? 1 : 2);
+    for (const void *ptr : {grad_k, grad_v})
+        apart = apart && !rows_meet(batch, heads, seq, dim, strides, ((intptr_t)ptr - (intptr_t)grad_q) / 2);
     for (int i = 0; i < 3 && apart; i++) {
         const uintptr_t lo = (uintptr_t)grads[i], hi = end(grads[i], strides);
         auto meets = [&](const void *from, uintptr_t to) { return lo < to && (uintptr_t)from < hi; };

@@ -375,7 +375,8 @@ int dfdx_rocm_reshape_backward(dfdx_rocm_ctx *ctx, int dtype, int rank, const in
  * bf16, dim 32, 64 or 128, scale > 0, 16-byte-aligned rows; anything else is
  * DFDX_ROCM_ERR_UNSUPPORTED before anything is launched, and the caller composes
  * the ops above instead.  Backward: grad_q, grad_k, grad_v (strides of q, k, v)
- * are accumulated into.  Rows that are written (out in the forward, the
+ * are accumulated into; a buffer that stands for two or all of them receives
+ * the sum.  Rows that are written (out in the forward, the
  * gradients in the backward) may not overlap, so an axis longer than 1 has no
  * stride of 0 there: DFDX_ROCM_ERR_ALIASED_OUTPUT, before anything is launched.
  * Inputs that are only read (the forward's q, k, v) may be broadcast. */
