@@ -283,9 +283,10 @@ template <> __device__ __forceinline__ f32x4 rows_mma<__bf16>(u32x4 m, u32x4 v, 
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, v), acc, 0, 0, 0);
 }
 template <> __device__ __forceinline__ f32x4 rows_mma<float>(u32x4 m, u32x4 v, f32x4 acc) {
+    f32x4 half[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};  // (short chains: see SUMS)
 #pragma unroll
-    for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(m[e]), __uint_as_float(v[e]), acc, 0, 0, 0);
-    return acc;
+    for (int e = 0; e < 4; e++) half[e / 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(m[e]), __uint_as_float(v[e]), half[e / 2], 0, 0, 0);
+    return acc + (half[0] + half[1]);
 }
 template <bool STREAM> __device__ __forceinline__ u32x4 ldm_any(const void *p) {
     if constexpr (STREAM) return __builtin_nontemporal_load((const u32x4_unaligned *)p);
@@ -310,14 +311,21 @@ template <typename T, int WAVES, int AHEAD, bool STREAM> __global__ __launch_bou
     const T *const vec = (const T *)p.vec + (int64_t)(has_vec ? l16 : 0) * p.vec_r_stride + lq * VEC - ahead;
     const int steps = (p.k + ahead + STEP - 1) / STEP, whole = (p.k + ahead) / STEP;
     const int first = blockIdx.y * p.kchunk, last = min(steps, first + p.kchunk);
-    f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+    // f32: short chains -- a sum for each of the steps in flight, a step's products by themselves (rows_mma), the waves' sums in pairs.
+    // With one chain a wave, 2 x 3072 x 2560 was 2.0 times as far from the sums in 64 bits as the vector-ALU form (2.0e-7, 1.0e-7 now) and
+    // 2 - 16 x 768 x 6000 1.3 times as far as the small-product kernel; 4 % of the time in the mean of 139 shapes, 16 % at most (4099 x
+    // 2635).  In 16 bits the rounding of the result is all that shows.
+    constexpr int SUMS = sizeof(T) == 4 ? AHEAD : 1;
+    f32x4 acc[SUMS][2];
+#pragma unroll
+    for (int u = 0; u < SUMS; u++) acc[u][0] = acc[u][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     auto edge = [&](int s) {  // a step that begins in front of the rows or ends behind them
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const int at = s * STEP + h * (STEP / 2) + lq * VEC - ahead;
             const u32x4 m = row_window<T>((const T *)p.mat + (int64_t)j * p.mat_j_stride, has_row, at, p.k);
             const u32x4 v = row_window<T>((const T *)p.vec + (int64_t)l16 * p.vec_r_stride, has_vec, at, p.k);
-            acc[h] = rows_mma<T>(m, v, acc[h]);
+            acc[0][h] = rows_mma<T>(m, v, acc[0][h]);
         }
     };
     const int from = ahead && first == 0 ? 1 : first, to = min(whole, last);
@@ -338,22 +346,37 @@ template <typename T, int WAVES, int AHEAD, bool STREAM> __global__ __launch_bou
         for (int u = 0; u < AHEAD; u++) {
             if (!FULL && s + u * WAVES >= to) continue;
 #pragma unroll
-            for (int h = 0; h < 2; h++) acc[h] = rows_mma<T>(m[u][h], v[u][h], acc[h]);
+            for (int h = 0; h < 2; h++) acc[u % SUMS][h] = rows_mma<T>(m[u][h], v[u][h], acc[u % SUMS][h]);
         }
     };
     for (; s + (AHEAD - 1) * WAVES < to; s += AHEAD * WAVES) batch(std::true_type{});
     if (s < to) batch(std::false_type{});
     if (from > first && wave == WAVES - 1) edge(0);
     if (to < last && last == steps && steps > from && wave == WAVES - 2) edge(whole);
-    *(f32x4 *)&part[wave][l16 * PITCH + lq * 4] = acc[0] + acc[1];  // vector l16, outputs lq * 4 .. + 3
+#pragma unroll
+    for (int u = SUMS / 2; u > 0; u /= 2)
+#pragma unroll
+        for (int i = 0; i < u; i++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) acc[i][h] += acc[i + u][h];
+    *(f32x4 *)&part[wave][l16 * PITCH + lq * 4] = acc[0][0] + acc[0][1];  // vector l16, outputs lq * 4 .. + 3
     __syncthreads();
     const int r = tid / 16, out = j0 + p.period * (tid % 16);
     if (tid >= 16 * p.r || out >= p.j) return;
-    float v = part[0][r * PITCH + tid % 16];
+    float v[WAVES];
 #pragma unroll
-    for (int w = 1; w < WAVES; w++) v += part[w][r * PITCH + tid % 16];
-    if (p.kslices > 1) p.ws[((int64_t)blockIdx.y * p.r + r) * p.j + out] = v;
-    else finish<T>(p, r, out, v);
+    for (int w = 0; w < WAVES; w++) v[w] = part[w][r * PITCH + tid % 16];
+    if constexpr (sizeof(T) == 4) {  // in pairs
+#pragma unroll
+        for (int half = WAVES / 2; half > 0; half /= 2)
+#pragma unroll
+            for (int w = 0; w < half; w++) v[w] += v[w + half];
+    } else {
+#pragma unroll
+        for (int w = 1; w < WAVES; w++) v[0] += v[w];
+    }
+    if (p.kslices > 1) p.ws[((int64_t)blockIdx.y * p.r + r) * p.j + out] = v[0];
+    else finish<T>(p, r, out, v[0]);
 }
 
 // Eight lanes per output: lane `part` of an output adds the slices part, part + 8, ... (their loads in flight together),
