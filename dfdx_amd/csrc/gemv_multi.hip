@@ -275,6 +275,11 @@ template <typename T, int R, bool STREAM> __global__ __launch_bounds__(256) void
 // 135).  Four steps of a wave are on their way at once, four waves a workgroup where the rows are short, sixteen where there are few
 // outputs, and k slices where there are fewer than 256 workgroups: 8 x 4096 x 4096 f16 9.4 us (3.6 TB/s), 8 x 16384 x 16384 118 us
 // (4.5 TB/s), f32 17 us and 241 us.
+// f32: short chains -- the products of a load by themselves (rows_mma), the waves' sums in pairs.  With one chain a wave, 2 x 3072 x 2560 was
+// 2.0 times as far from the sums in 64 bits as the vector-ALU form (2.0e-7, 1.1e-7 now) and 2 - 16 x 768 x 6000 1.3 times as far as the
+// small-product kernel.  2 % of the time in the mean of 129 shapes, most where sixteen waves no longer share a compute unit with sixteen
+// others (64 registers, 69 now: 4099 x 2635 13.3 -> 15.3 us); the compiler's own choice of registers, up to 208, took 7 %, 12289 x 257 5.2 ->
+// 7.5 us.  In 16 bits the rounding of the result is all that shows.
 template <typename T> __device__ __forceinline__ f32x4 rows_mma(u32x4 m, u32x4 v, f32x4 acc);
 template <> __device__ __forceinline__ f32x4 rows_mma<_Float16>(u32x4 m, u32x4 v, f32x4 acc) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, m), __builtin_bit_cast(f16x8, v), acc, 0, 0, 0);
@@ -283,10 +288,10 @@ template <> __device__ __forceinline__ f32x4 rows_mma<__bf16>(u32x4 m, u32x4 v, 
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, v), acc, 0, 0, 0);
 }
 template <> __device__ __forceinline__ f32x4 rows_mma<float>(u32x4 m, u32x4 v, f32x4 acc) {
-    f32x4 half[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};  // (short chains: see SUMS)
+    f32x4 chain = {0.0f, 0.0f, 0.0f, 0.0f};  // (sixteen products)
 #pragma unroll
-    for (int e = 0; e < 4; e++) half[e / 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(m[e]), __uint_as_float(v[e]), half[e / 2], 0, 0, 0);
-    return acc + (half[0] + half[1]);
+    for (int e = 0; e < 4; e++) chain = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(m[e]), __uint_as_float(v[e]), chain, 0, 0, 0);
+    return acc + chain;
 }
 template <bool STREAM> __device__ __forceinline__ u32x4 ldm_any(const void *p) {
     if constexpr (STREAM) return __builtin_nontemporal_load((const u32x4_unaligned *)p);
@@ -294,7 +299,7 @@ template <bool STREAM> __device__ __forceinline__ u32x4 ldm_any(const void *p) {
 }
 constexpr int rows_step(int elem_bytes) { return 128 / elem_bytes; }
 
-template <typename T, int WAVES, int AHEAD, bool STREAM> __global__ __launch_bounds__(WAVES * 64) void gemv_rows_kernel(const MultiParams p) {
+template <typename T, int WAVES, int AHEAD, bool STREAM> __global__ __launch_bounds__(WAVES * 64, sizeof(T) == 4 ? 7 : 1) void gemv_rows_kernel(const MultiParams p) {
     constexpr int VEC = Elem<T>::VEC, STEP = rows_step(sizeof(T)), PITCH = 20;
     __shared__ __align__(16) float part[WAVES][16 * PITCH];
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -311,21 +316,14 @@ template <typename T, int WAVES, int AHEAD, bool STREAM> __global__ __launch_bou
     const T *const vec = (const T *)p.vec + (int64_t)(has_vec ? l16 : 0) * p.vec_r_stride + lq * VEC - ahead;
     const int steps = (p.k + ahead + STEP - 1) / STEP, whole = (p.k + ahead) / STEP;
     const int first = blockIdx.y * p.kchunk, last = min(steps, first + p.kchunk);
-    // f32: short chains -- a sum for each of the steps in flight, a step's products by themselves (rows_mma), the waves' sums in pairs.
-    // With one chain a wave, 2 x 3072 x 2560 was 2.0 times as far from the sums in 64 bits as the vector-ALU form (2.0e-7, 1.0e-7 now) and
-    // 2 - 16 x 768 x 6000 1.3 times as far as the small-product kernel; 4 % of the time in the mean of 139 shapes, 16 % at most (4099 x
-    // 2635).  In 16 bits the rounding of the result is all that shows.
-    constexpr int SUMS = sizeof(T) == 4 ? AHEAD : 1;
-    f32x4 acc[SUMS][2];
-#pragma unroll
-    for (int u = 0; u < SUMS; u++) acc[u][0] = acc[u][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
     auto edge = [&](int s) {  // a step that begins in front of the rows or ends behind them
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const int at = s * STEP + h * (STEP / 2) + lq * VEC - ahead;
             const u32x4 m = row_window<T>((const T *)p.mat + (int64_t)j * p.mat_j_stride, has_row, at, p.k);
             const u32x4 v = row_window<T>((const T *)p.vec + (int64_t)l16 * p.vec_r_stride, has_vec, at, p.k);
-            acc[0][h] = rows_mma<T>(m, v, acc[0][h]);
+            acc[h] = rows_mma<T>(m, v, acc[h]);
         }
     };
     const int from = ahead && first == 0 ? 1 : first, to = min(whole, last);
@@ -346,20 +344,15 @@ template <typename T, int WAVES, int AHEAD, bool STREAM> __global__ __launch_bou
         for (int u = 0; u < AHEAD; u++) {
             if (!FULL && s + u * WAVES >= to) continue;
 #pragma unroll
-            for (int h = 0; h < 2; h++) acc[u % SUMS][h] = rows_mma<T>(m[u][h], v[u][h], acc[u % SUMS][h]);
+            for (int h = 0; h < 2; h++) acc[h] = rows_mma<T>(m[u][h], v[u][h], acc[h]);
+            if (sizeof(T) == 4 && u % 2) __builtin_amdgcn_sched_barrier(0);  // (two steps' chains at a time, for the registers)
         }
     };
     for (; s + (AHEAD - 1) * WAVES < to; s += AHEAD * WAVES) batch(std::true_type{});
     if (s < to) batch(std::false_type{});
     if (from > first && wave == WAVES - 1) edge(0);
     if (to < last && last == steps && steps > from && wave == WAVES - 2) edge(whole);
-#pragma unroll
-    for (int u = SUMS / 2; u > 0; u /= 2)
-#pragma unroll
-        for (int i = 0; i < u; i++)
-#pragma unroll
-            for (int h = 0; h < 2; h++) acc[i][h] += acc[i + u][h];
-    *(f32x4 *)&part[wave][l16 * PITCH + lq * 4] = acc[0][0] + acc[0][1];  // vector l16, outputs lq * 4 .. + 3
+    *(f32x4 *)&part[wave][l16 * PITCH + lq * 4] = acc[0] + acc[1];  // vector l16, outputs lq * 4 .. + 3
     __syncthreads();
     const int r = tid / 16, out = j0 + p.period * (tid % 16);
     if (tid >= 16 * p.r || out >= p.j) return;
