@@ -325,6 +325,26 @@ int bandwidth_kernel(const GemmProblem &p, bool plain_order) {
     return thin_mfma_supported(p) ? BW_THIN_MFMA : BW_NONE;
 }
 
+// The same with the rows form of gemv_multi.hip among them.  Of the forms for several vectors those that keep their sums in the vector ALUs
+// are weighed against the rows form and the matrix-core plans by estimated time (the tiles stream a large [k][n] matrix faster); the rows
+// form has no rival (1 - 16 vectors against 512 - 16384 rows and columns, 245 products: 1.47 times as fast as the best plan
+// without it in the mean, 4 x 4091 x 4093 f16 36.5 -> 10.1 us, f32 36.9 -> 15.7, 8 x 4288 x 4288 bf16 14 -> 11) but the
+// small-product kernel, by estimated time, on rows that lie on the 16-byte grid of a matrix below 8 MB (up to 11 % there, either
+// way: 8 x 520 x 2635 bf16 3.7 and 4.2 us, 16 x 2048 x 2048 7.0 and 6.8); the others have none.  `seconds`: the estimate where it has rivals,
+// else 0.
+int bandwidth_plan(const GemmProblem &p, bool plain_order, bool may_rows, double *seconds) {
+    *seconds = 0.0;
+    const int bw = bandwidth_kernel(p, plain_order);
+    if (bw == BW_GEMV_MULTI) *seconds = gemv_multi_time(p);
+    if ((bw != BW_NONE && bw != BW_GEMV_MULTI) || !may_rows || !gemv_rows_supported(p)) return bw;
+    // (the other forms take 1.1 times their estimate, 4 x 2048 x 2048 f32 10.2 us and 8.6 as rows, but on matrices that no cache
+    // holds: 8 x 16384 x 16384 f32 218 and 240)
+    const double t = gemv_rows_time(p), bytes = (double)std::max(p.m, p.n) * (double)p.k * (double)dtype_size(p.dtype);
+    if (bw == BW_GEMV_MULTI && t >= (bytes < 268435456.0 ? 1.1 : 1.0) * *seconds) return bw;
+    *seconds = bytes < 8e6 && p.k * (int64_t)dtype_size(p.dtype) % 16 == 0 ? t : 0.0;
+    return BW_ROWS;
+}
+
 const char *bandwidth_kernel_name(const GemmProblem &p, int which) {
     switch (which) {
     case BW_RANK1: return p.k == 1 ? "rank1" : "thin_k";
@@ -348,7 +368,8 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         *plan = {DFDX_ROCM_KERNEL_GENERIC, 0, 1};
         return DFDX_ROCM_OK;
     case DFDX_ROCM_KERNEL_GEMV: {  // the bandwidth-bound kernels, forced: the caller's choice outranks the order flag
-        const int bw = bandwidth_kernel(p, false);
+        double unused;
+        const int bw = bandwidth_plan(p, false, true, &unused);
         if (!bw) return DFDX_ROCM_ERR_UNSUPPORTED;
         *plan = {DFDX_ROCM_KERNEL_GEMV, bw, 1};
         return DFDX_ROCM_OK;
@@ -379,30 +400,14 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
     default:
         return DFDX_ROCM_ERR_INVALID_ARG;
     }
-    // The bandwidth-bound kernels first.  Of the forms for several vectors those that keep their sums in the vector ALUs are weighed
-    // against the rows form and the matrix-core plans by estimated time (the tiles stream a large [k][n] matrix faster); the rows
-    // form has no rival (1 - 16 vectors against 512 - 16384 rows and columns, 245 products: 1.47 times as fast as the best plan
-    // without it in the mean, 4 x 4091 x 4093 f16 36.5 -> 10.1 us, f32 36.9 -> 15.7, 8 x 4288 x 4288 bf16 14 -> 11) but the
-    // small-product kernel, by estimated time, on rows that lie on the 16-byte grid of a matrix below 8 MB (up to 11 % there, either
-    // way: 8 x 520 x 2635 bf16 3.7 and 4.2 us, 16 x 2048 x 2048 7.0 and 6.8); the others have none.
-    int bw = bandwidth_kernel(p, (d->flags & DFDX_ROCM_GEMM_NO_SPLIT_K) != 0);
+    // The bandwidth-bound kernels first.
     double t_bw = 1e300;
-    if (bw == BW_GEMV_MULTI) t_bw = gemv_multi_time(p);
-    bool weighed = bw == BW_GEMV_MULTI;
-    if ((bw == BW_NONE || bw == BW_GEMV_MULTI) && !forced_splits && gemv_rows_supported(p)) {
-        // (the other forms take 1.1 times their estimate, 4 x 2048 x 2048 f32 10.2 us and 8.6 as rows, but on matrices that no cache
-        // holds: 8 x 16384 x 16384 f32 218 and 240)
-        const double bytes = (double)std::max(p.m, p.n) * (double)p.k * (double)dtype_size(p.dtype);
-        if (const double t = gemv_rows_time(p); t < (bytes < 268435456.0 ? 1.1 : 1.0) * t_bw) {
-            bw = BW_ROWS;
-            t_bw = t;
-            weighed = bytes < 8e6 && p.k * (int64_t)dtype_size(p.dtype) % 16 == 0;
-        }
-    }
-    if (bw && !weighed) {
+    const int bw = bandwidth_plan(p, (d->flags & DFDX_ROCM_GEMM_NO_SPLIT_K) != 0, !forced_splits, &t_bw);
+    if (bw && t_bw == 0.0) {
         *plan = {DFDX_ROCM_KERNEL_GEMV, bw, 1};
         return DFDX_ROCM_OK;
     }
+    if (!bw) t_bw = 1e300;
     const Plan bw_plan = {DFDX_ROCM_KERNEL_GEMV, bw, 1};
     // The small-product kernel where its estimate beats the family's (the f32 family weighs it among its own variants);
     // not where the caller fixed the order of the contraction.

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import oracle
-from dfdx_amd.rocm import KERNEL_AUTO
+from dfdx_amd.rocm import KERNEL_AUTO, KERNEL_GEMV
 from gpu_util import announce, device
 from helpers import assert_within, rng
 from test_gpu_gemm import run_case
@@ -65,3 +65,13 @@ def test_f32_sums_are_short_chains(k):
     want = x.astype(np.float64) @ w.astype(np.float64).T
     far = lambda got: np.linalg.norm(got - want)
     assert far(dev.to_host(dc).reshape(rows, n)) <= 1.15 * far(chains(x, w, 32))
+
+
+@pytest.mark.parametrize("dtype,rows,k,n", [("f16", 16, 4096, 4096), ("f16", 4, 4093, 4091), ("f32", 4, 4093, 1091), ("f16", 8, 4096, 4096)])
+def test_the_kernel_that_a_plan_names_can_be_asked_for(dtype, rows, k, n):
+    dev = device()
+    plan = lambda kernel: dev.gemm_plan(dev.gemm_desc(dtype, rows, k, n, 256, (k, 1), 512, (1, k), 1024, (n, 1), kernel=kernel))
+    assert plan(KERNEL_AUTO)[2] == "gemv_rows" and plan(KERNEL_AUTO)[0] == KERNEL_GEMV
+    assert plan(KERNEL_GEMV) == plan(KERNEL_AUTO)
+    if n < 2000:
+        assert run_case(dtype, rows, k, n, "nt", True, KERNEL_GEMV, 0, seed=k) == "gemv_rows"
