@@ -420,7 +420,9 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         int dv = 0, splits = 1;
         double t_dma = 1e300;
         mfma16dma_plan_split(p, ctx->compute_units, 0, forced_splits, &dv, &splits, &t_dma);
-        if (dv && p.k % 64) {  // (one of the tiles that take any k: weighed against the families below)
+        bool only_ring = dv && mfma16dma_takes_any_k(dv);
+        for (int v = 1; only_ring && !mfma16dma_takes_any_k(v); v++) only_ring = !mfma16dma_supported(p, v);
+        if (only_ring) {  // (k off the tile or C off the grid: weighed against the families below, copies among them)
             t_ring = t_dma;
             ring_plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
         } else if (dv) {
@@ -482,7 +484,7 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         // (on operands in place with k off 64 the staged tiles run at 0.83 - 1.06 of the estimate: 528 x 1024 x 1325 f16 21.4 us for 25.6,
         // 2304 x 128 x 1534 in three pieces 16.2 for 15.3; the ring 9.4 both)
         const double t_plan = plan->realign ? t_copies : plan->kernel == DFDX_ROCM_KERNEL_GEMV ? t_bw : plan->variant == v ? 0.85 * t_family : t_small_here;
-        if (t_ring < t_plan) *plan = ring_plan;
+        if (t_ring <= t_plan) *plan = ring_plan;
         if (seconds && is16) *seconds = std::min(t_ring, t_plan);
         return DFDX_ROCM_OK;
     }

@@ -119,3 +119,15 @@ def test_a_gradient_that_both_products_add_to(dtype, n):
     want = G @ X.T + X.T @ G
     ulp = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype]
     assert_within(dtype, 2 * n, oracle.to_f64(dev.to_host(gx), dtype).reshape(n, n), want, X, G, extra=2 * ulp * float(np.abs(want).max()), what="sum")
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("m,k,n,want", [
+    (2048, 64, 367, "mfma16_64x64x64_w2x2"), (520, 128, 1001, "mfma16_64x64x64_w2x2"), (8, 16384, 257, "gemv_multi"),
+    (1000, 8192, 63, "mfma16_ring_64x64x64_w2x2_s4_splitk10"), (300, 2048, 1025, "ring"),
+])
+def test_results_off_the_grid_have_rivals(dtype, m, k, n, want):
+    """Whole k tiles and a C that only the ring takes of the LDS-DMA kernels: the other families are weighed too."""
+    dev = device()
+    name = dev.gemm_plan(dev.gemm_desc(dtype, m, k, n, 256, (k, 1), 512, (1, k), 1024, (n, 1)))[2]
+    assert want == name or (want == "ring" and "_ring_" in name and "_realigned" not in name), name
