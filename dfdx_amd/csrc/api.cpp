@@ -296,6 +296,7 @@ struct Plan {
     bool realign = false;
     int staged = 0;
     int plain_kernel = 0, plain_variant = 0, plain_splits = 1;
+    GemmCut cut;
 };
 
 // Rank-1 updates and k = 2 stream their rows on the vector ALUs; from k = 3 on the matrix-core form of the thin
@@ -378,9 +379,11 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         int v = d->variant;
         if (is16 && (v == 0 || (v >= mfma16_dma_first_variant() && v != mfma16_small_variant()))) {  // LDS-DMA family: tile and split count together
             int dv = 0, splits = 1;
-            mfma16dma_plan_split(p, ctx->compute_units, v ? v - mfma16_dma_first_variant() + 1 : 0, forced_splits, &dv, &splits);
+            GemmCut cut;
+            mfma16dma_plan_split(p, ctx->compute_units, v ? v - mfma16_dma_first_variant() + 1 : 0, forced_splits, &dv, &splits, nullptr, &cut);
             if (dv) {
                 *plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
+                plan->cut = cut;
                 return DFDX_ROCM_OK;
             }
             if (v) return DFDX_ROCM_ERR_UNSUPPORTED;
@@ -419,14 +422,17 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
     if (is16) {
         int dv = 0, splits = 1;
         double t_dma = 1e300;
-        mfma16dma_plan_split(p, ctx->compute_units, 0, forced_splits, &dv, &splits, &t_dma);
+        GemmCut cut;
+        mfma16dma_plan_split(p, ctx->compute_units, 0, forced_splits, &dv, &splits, &t_dma, &cut);
         bool only_ring = dv && mfma16dma_takes_any_k(dv);
         for (int v = 1; only_ring && !mfma16dma_takes_any_k(v); v++) only_ring = !mfma16dma_supported(p, v);
         if (only_ring) {  // (k off the tile or C off the grid: weighed against the families below, copies among them)
             t_ring = t_dma;
             ring_plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
         } else if (dv) {
-            *plan = t_small < t_dma ? small_plan : Plan{DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
+            *plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
+            plan->cut = cut;
+            if (t_small < t_dma) *plan = small_plan;
             double t_best = std::min(t_small, t_dma);
             int skinny_splits = 1;
             double t_skinny = 1e300;
@@ -466,11 +472,12 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         double t_copies = 1e300;
         if (realignable) {
             int dv = 0, splits = 1;
-            mfma16dma_plan_split(ra.problem, ctx->compute_units, 0, forced_splits, &dv, &splits, &t_copies);
+            GemmCut cut;
+            mfma16dma_plan_split(ra.problem, ctx->compute_units, 0, forced_splits, &dv, &splits, &t_copies, &cut);
             // (a product whose plan without copies fits the fixed scratch array fits it in this form too: see dfdx_rocm_gemm_noalloc)
             const size_t piece = mfma16_workspace_bytes(p, v, 2) / 2, most = DFDX_ROCM_NOALLOC_SCRATCH_BYTES;
             if (dv && splits > 1 && !forced_splits && piece * (size_t)splits > most && partials_bytes(p, *plan) <= most)
-                mfma16dma_plan_split(ra.problem, ctx->compute_units, 0, (int)std::max<size_t>(1, most / piece), &dv, &splits, &t_copies);
+                mfma16dma_plan_split(ra.problem, ctx->compute_units, 0, (int)std::max<size_t>(1, most / piece), &dv, &splits, &t_copies, &cut);
             // (copies are not taken for a gain within the estimates' error)
             t_copies = dv ? t_copies + ra.seconds + (mfma16dma_takes_any_k(dv) ? 0.0 : splits > 1 ? 6.5e-6 : 1.0e-6) : 1e300;
             const bool small_tile = v == mfma16_skinny_variant();
@@ -478,7 +485,7 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
                                     (small_tile ? 0.0 : 2.0 * (double)p.m * (double)p.n * (double)(p.reduce ? 1 : p.nb1 * p.nb2) / 2.2e12);
             if (t_copies < std::min(std::min(t_small_here, t_staged), t_bw)) {
                 const Plan plain = *plan;
-                *plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits, true, v, plain.kernel, plain.variant, plain.splits};
+                *plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits, true, v, plain.kernel, plain.variant, plain.splits, cut};
             }
         }
         // (on operands in place with k off 64 the staged tiles run at 0.83 - 1.06 of the estimate: 528 x 1024 x 1325 f16 21.4 us for 25.6,
@@ -591,6 +598,7 @@ int run_plan(dfdx_rocm_ctx *ctx, const GemmProblem &problem, const Plan &plan, b
     }
     if (plan.realign) p = ra.problem;
     if (plan.kernel == DFDX_ROCM_KERNEL_MFMA && plan.splits > 1) p.splits = plan.splits;
+    p.cut = plan.cut;
     hipError_t e;
     switch (plan.kernel) {
     case DFDX_ROCM_KERNEL_GENERIC: e = launch_generic(p, ctx->stream); break;
@@ -640,7 +648,11 @@ bool extra_supported(const GemmProblem &p, const Plan &plan) {
     const bool is16 = p.dtype == DT_F16 || p.dtype == DT_BF16;
     if (is16 && plan.variant == mfma16_small_variant()) return true;
     if (p.dtype == DT_F64 && plan.variant == mfma64_small_variant()) return true;
-    if (is16 && plan.variant >= mfma16_dma_first_variant()) return mfma16dma_extra_supported(p, plan.variant - mfma16_dma_first_variant() + 1, plan.splits);
+    if (is16 && plan.variant >= mfma16_dma_first_variant()) {
+        GemmProblem whole = p;
+        whole.cut = plan.cut;
+        return mfma16dma_extra_supported(whole, plan.variant - mfma16_dma_first_variant() + 1, plan.splits);
+    }
     return plan.splits > 1;  // the reduce kernel does it
 }
 
@@ -980,7 +992,8 @@ int gemm_three(dfdx_rocm_ctx *ctx, const GemmProblem &problem, bool *done) {
     if (p.dtype != DT_F16 && p.dtype != DT_BF16) return DFDX_ROCM_OK;
     int dv = 0, splits = 1, dv1 = 0, splits1 = 1;
     double t3 = 1e300, t1 = 1e300;
-    mfma16dma_plan_split(p, ctx->compute_units, 0, 0, &dv, &splits, &t3);
+    GemmCut cut;
+    mfma16dma_plan_split(p, ctx->compute_units, 0, 0, &dv, &splits, &t3, &cut);
     if (!dv || (p.ksum && !mfma16dma_ksum_supported(p, dv, splits)) || (p.extra != EXTRA_NONE && !mfma16dma_extra_supported(p, dv, splits)))
         return DFDX_ROCM_OK;
     GemmProblem q = p;
@@ -994,6 +1007,7 @@ int gemm_three(dfdx_rocm_ctx *ctx, const GemmProblem &problem, bool *done) {
     if ((!p.accumulate || p.k % 64) && (t_small < t1 || splits1 > 1 || splits > 1)) return DFDX_ROCM_OK;
     if (t3 >= 3.0 * std::min(t1, t_small)) return DFDX_ROCM_OK;
     Plan plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
+    plan.cut = cut;
     if (int e = reserve_partials(ctx, p, plan, false)) return e;
     if (int e = settle_three(ctx, &p)) return e;
     *done = true;
@@ -1344,6 +1358,10 @@ int dfdx_rocm_gemm_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int
                           p.dtype == DT_F32 ? mfma32_variant_name(plan.variant) : mfma16_variant_name(plan.variant), copied);
         else
             std::snprintf(name, name_len, "%s", plan.kernel != DFDX_ROCM_KERNEL_GEMV ? "generic" : bandwidth_kernel_name(p, plan.variant));
+        if (plan.cut.variant) {
+            const size_t at = std::strlen(name);
+            std::snprintf(name + at, name_len - at, "+%s", mfma16dma_variant_name(plan.cut.variant));
+        }
     }
     return DFDX_ROCM_OK;
 }

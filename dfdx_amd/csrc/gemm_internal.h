@@ -17,6 +17,13 @@ enum { KSUM_NONE = 0, KSUM_OF_A = 1, KSUM_OF_B = 2 };
 
 // One strided, batched GEMM:  C[b][i,j] = (accumulate ? C : 0) + bias + sum_k A[b][i,k] * B[b][k,j].
 // Strides are in elements.  With `reduce` set, all nb1*nb2 batches are summed into one C.
+// A 16-bit product in two launches (plan_tail in gemm_mfma16_dma.hip): its first `m` rows or `n` columns (the other is 0) on the planned tile,
+// what lies behind them on the LDS-DMA variant `variant` (0: the product is one launch).
+struct GemmCut {
+    int variant = 0;
+    int64_t m = 0, n = 0;
+};
+
 struct GemmProblem {
     int dtype;
     int accumulate;
@@ -56,6 +63,7 @@ struct GemmProblem {
     // its place in the operand to there.
     bool last_apart = false;
     int64_t a_last = 0, b_last = 0;
+    GemmCut cut;  // filled in from the plan: automatic ones only, a tile that the caller asks for is that tile
     // split-k (filled in by the planner): `splits` workgroups share one C tile; f32 partials go to `workspace`
     int splits;
     float *workspace;
@@ -165,9 +173,10 @@ size_t bias_backward_copy_partials(int compute_units, int64_t rows, int64_t cols
 hipError_t launch_bias_backward_copy(int dtype, int compute_units, int64_t rows, int64_t cols, const void *go, void *copy, int64_t ld, int64_t rows_out,
                                      void *grad_bias, bool fresh, float *partial, hipStream_t stream);
 // Split-k planning for the LDS-DMA kernels: picks tile variant and split count together.  `forced_splits`
-// > 0 overrides the count (clamped to what the k extent allows).  `seconds` (may be null) receives the estimate.
+// > 0 overrides the count (clamped to what the k extent allows).  `seconds` (may be null) receives the estimate, `cut` (may be null)
+// whether the estimate is for two launches; a forced variant is not cut.
 void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_variant, int forced_splits, int *variant,
-                          int *splits, double *seconds = nullptr);
+                          int *splits, double *seconds = nullptr, GemmCut *cut = nullptr);
 size_t mfma16dma_workspace_bytes(const GemmProblem &p, int variant, int splits);
 bool mfma16dma_ksum_supported(const GemmProblem &p, int variant, int splits);  // can this plan also produce p.ksum?
 

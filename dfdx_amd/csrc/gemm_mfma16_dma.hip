@@ -235,9 +235,8 @@ inline double ring_time(const RingModel &r, int cus, int64_t items, int64_t tota
 // x 128 cut 85).
 namespace {
 struct Tail {
-    int variant = 0;            // the ring tile; 0: the product stays whole
-    int64_t cut_m = 0, cut_n = 0;  // rows or columns of the first part (0: not along them)
-    double gain = 0.0;          // seconds less than with a last round as long as a full one (what the model takes it for)
+    GemmCut cut;
+    double gain = 0.0;  // seconds less than with a last round as long as a full one (what the model takes it for)
 };
 GemmProblem part_of(const GemmProblem &p, int64_t m0, int64_t m1, int64_t n0, int64_t n1) {
     GemmProblem q = p;
@@ -246,6 +245,7 @@ GemmProblem part_of(const GemmProblem &p, int64_t m0, int64_t m1, int64_t n0, in
     q.n = n1 - n0;
     q.ksum = nullptr;
     q.ksum_of = KSUM_NONE;
+    q.cut = {};
     q.a = (const char *)p.a + m0 * p.a_rs * es;
     q.b = (const char *)p.b + n0 * p.b_cs * es;
     q.c = (char *)p.c + c_off;
@@ -279,7 +279,7 @@ Tail plan_tail(const GemmProblem &p, int variant, int compute_units) {
                                  kSecondLaunch;
             if (after < soonest) {
                 soonest = after;
-                best = {v, along_n ? 0 : cut, along_n ? cut : 0, round_seconds - after};
+                best = {{v, along_n ? 0 : cut, along_n ? cut : 0}, round_seconds - after};
             }
         }
     }
@@ -288,7 +288,8 @@ Tail plan_tail(const GemmProblem &p, int variant, int compute_units) {
 }  // namespace
 
 void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_variant, int forced_splits, int *variant,
-                          int *splits, double *seconds) {
+                          int *splits, double *seconds, GemmCut *cut) {
+    GemmCut best_cut;
     *variant = 0;
     *splits = 1;
     const int cus = std::max(1, compute_units);
@@ -341,10 +342,12 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
                 time += kSplitLaunch + kSplitPerPiece * s +
                         (ws + out_elems * elem * (1 + p.accumulate)) / (ws <= kWsCached ? kWsBandwidthCached : kWsBandwidthHbm);
             }
-            if (s == 1)
-                if (const Tail tail = plan_tail(p, v, cus); tail.variant) time = 1.05 * (time - tail.gain);
+            Tail tail;
+            if (s == 1 && forced_variant == 0)
+                if (tail = plan_tail(p, v, cus); tail.cut.variant) time = 1.05 * (time - tail.gain);
             if (time < best) {
                 best = time;
+                best_cut = tail.cut;
                 *variant = v;
                 *splits = s;
             }
@@ -353,9 +356,11 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
     if (best < 1e300) best -= *splits > 1 ? kAboveClockSplit : kAboveClock;
     if (ring && (best_ring < best || *variant == 0)) {
         best = best_ring;
+        best_cut = {};
         *variant = ring;
         *splits = ring_splits;
     }
+    if (cut) *cut = best_cut;
     if (seconds) *seconds = best;
 }
 
@@ -393,6 +398,7 @@ bool mfma16dma_ksum_supported(const GemmProblem &p, int variant, int splits) {
 bool mfma16dma_extra_supported(const GemmProblem &p, int variant, int splits) {
     if ((p.accumulate != 0) != (p.extra == EXTRA_FROM) || (p.batch_count() != 1 && !p.reduce) || !mfma16dma_supported(p, variant)) return false;
     if (p.extra != EXTRA_RELU && (!p.with || !aligned16(p.with))) return false;
+    if (p.cut.variant && !mfma16dma_extra_supported(part_of(p, p.cut.m, p.m, p.cut.n, p.n), p.cut.variant, 1)) return false;
     if (splits > 1 || is_ring(variant)) return true;  // (split: the reduce kernel applies it)
     const bool a_kc = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged).kc, b_kc = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged).kc;
     return a_kc && b_kc == (p.extra == EXTRA_RELU || p.extra == EXTRA_RESIDUAL);
@@ -493,12 +499,13 @@ hipError_t launch_mfma16_ring_pair(const GemmProblem &p, const GemmProblem &q, i
 hipError_t launch_mfma16dma(const GemmProblem &g, int variant, hipStream_t stream) {
     if (!mfma16dma_supported(g, variant)) return hipErrorInvalidValue;
     if (is_ring(variant)) return launch_ring(g, variant, stream);
-    if (g.splits <= 1) {
-        if (const Tail tail = plan_tail(g, variant, g.compute_units); tail.variant) {
-            const bool rows = tail.cut_m > 0;
-            const hipError_t e = launch_mfma16dma(part_of(g, 0, rows ? tail.cut_m : g.m, 0, rows ? g.n : tail.cut_n), variant, stream);
-            return e != hipSuccess ? e : launch_ring(part_of(g, tail.cut_m, g.m, tail.cut_n, g.n), tail.variant, stream);
-        }
+    if (g.cut.variant) {
+        const GemmProblem rest = part_of(g, g.cut.m, g.m, g.cut.n, g.n);
+        if (g.splits > 1 || g.ksum || !is_ring(g.cut.variant) || !mfma16dma_supported(rest, g.cut.variant) ||
+            (g.extra != EXTRA_NONE && !mfma16dma_extra_supported(rest, g.cut.variant, 1)))
+            return hipErrorInvalidValue;
+        const hipError_t e = launch_mfma16dma(part_of(g, 0, g.cut.m ? g.cut.m : g.m, 0, g.cut.n ? g.cut.n : g.n), variant, stream);
+        return e != hipSuccess ? e : launch_ring(rest, g.cut.variant, stream);
     }
     const Variant &v = kVariants[variant - 1];
     const OperandLayout la = classify(g.m, g.k, g.a_rs, g.a_cs, g.ragged);
