@@ -696,17 +696,12 @@ int run_with_colsum(dfdx_rocm_ctx *ctx, GemmProblem &p, Plan &plan, bool *fused)
 
 namespace dfdx_rocm {
 
-int gemm_beyond(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int extra, const void *with) {
-    if (int e = bind(ctx)) return e;
-    GemmProblem p;
-    if (int e = make_problem(desc, &p)) return e;
-    if (p.m == 0) return DFDX_ROCM_OK;
-    // C and `with` are one contiguous matrix each: what the separate ops below walk
-    if (p.nb1 * p.nb2 != 1 || p.c_cs != 1 || p.c_rs != p.n || (extra && (p.accumulate != 0) != (extra == EXTRA_FROM)) ||
-        (extra > EXTRA_RELU && !with))
-        return DFDX_ROCM_ERR_INVALID_ARG;
-    Plan plan;
-    if (int e = make_plan(ctx, desc, p, &plan)) return e;
+// What gemm_beyond asks of a product: C and `with` are one contiguous matrix each, which the separate ops walk.
+static bool beyond_ok(const GemmProblem &p, int extra, const void *with) {
+    return p.nb1 * p.nb2 == 1 && p.c_cs == 1 && p.c_rs == p.n && (!extra || (p.accumulate != 0) == (extra == EXTRA_FROM)) && (extra <= EXTRA_RELU || with);
+}
+
+static int run_beyond(dfdx_rocm_ctx *ctx, GemmProblem &p, Plan &plan, int extra, const void *with) {
     if (int e = reserve_partials(ctx, p, plan, false)) return e;
     p.extra = extra;
     p.with = with;
@@ -726,6 +721,17 @@ int gemm_beyond(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int extra, 
     case EXTRA_MASK: return relu_mask(ctx, p.dtype, len, with, p.c);
     default: return DFDX_ROCM_OK;
     }
+}
+
+int gemm_beyond(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int extra, const void *with) {
+    if (int e = bind(ctx)) return e;
+    GemmProblem p;
+    if (int e = make_problem(desc, &p)) return e;
+    if (p.m == 0) return DFDX_ROCM_OK;
+    if (!beyond_ok(p, extra, with)) return DFDX_ROCM_ERR_INVALID_ARG;
+    Plan plan;
+    if (int e = make_plan(ctx, desc, p, &plan)) return e;
+    return run_beyond(ctx, p, plan, extra, with);
 }
 
 // Bytes that the matrices of one operand span, matrix by matrix where they lie anywhere (`batches`), else together.
@@ -787,27 +793,50 @@ static bool independent(const GemmProblem &p, const GemmProblem &q) {
     return true;
 }
 
+// A call's product and its plan, which is made once, when it is first asked for.
+struct Product {
+    const dfdx_rocm_gemm_desc *desc;
+    GemmProblem p;
+    Plan plan;
+    double seconds = 0.0;
+    bool planned = false;
+    int need_plan(dfdx_rocm_ctx *ctx) {
+        if (planned) return DFDX_ROCM_OK;
+        if (int e = make_plan(ctx, desc, p, &plan, &seconds)) return e;
+        planned = true;
+        return DFDX_ROCM_OK;
+    }
+};
+
 // The tile on which the two products of a backward pass run faster as one launch than as two, 0 if there is none.  Decided from the
 // shapes and layouts alone, so that a call that joins more of them (the encoder block's) and the calls it stands for agree.
-static int ring_pair_tile(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d1, const GemmProblem &p1, const dfdx_rocm_gemm_desc *d2, const GemmProblem &p2) {
-    if ((p1.dtype != DT_F16 && p1.dtype != DT_BF16) || d1->kernel != DFDX_ROCM_KERNEL_AUTO || d2->kernel != DFDX_ROCM_KERNEL_AUTO) return 0;
-    double together = 1e300, t1 = 0.0, t2 = 0.0;
-    const int tile = mfma16_ring_pair_plan(p1, p2, ctx->compute_units, &together);
+static int ring_pair_tile(dfdx_rocm_ctx *ctx, Product &one, Product &two) {
+    if ((one.p.dtype != DT_F16 && one.p.dtype != DT_BF16) || one.desc->kernel != DFDX_ROCM_KERNEL_AUTO || two.desc->kernel != DFDX_ROCM_KERNEL_AUTO) return 0;
+    double together = 1e300;
+    const int tile = mfma16_ring_pair_plan(one.p, two.p, ctx->compute_units, &together);
     if (!tile) return 0;
-    Plan plan;
-    if (make_plan(ctx, d1, p1, &plan, &t1) || make_plan(ctx, d2, p2, &plan, &t2)) return 0;
+    double t1 = 0.0;
+    if (one.p.accumulate) {
+        if (one.need_plan(ctx)) return 0;
+        t1 = one.seconds;
+    } else {  // (the ops that a product with one thing more stands for accumulate)
+        GemmProblem added = one.p;
+        added.accumulate = 1;
+        Plan unused;
+        if (make_plan(ctx, one.desc, added, &unused, &t1)) return 0;
+    }
+    if (two.need_plan(ctx)) return 0;
     // (the second launch and the gap in front of it are not in the estimates)
-    return t1 > 0.0 && t2 > 0.0 && together < t1 + t2 + 1.0e-6 ? tile : 0;
+    return t1 > 0.0 && two.seconds > 0.0 && together < t1 + two.seconds + 1.0e-6 ? tile : 0;
 }
 
-// Would the call `d` run `p` on the small-product kernel?  Products that do and share nothing but what they read are one launch
+// Would the call run on the small-product kernel?  Products that do and share nothing but what they read are one launch
 // (launch_small_many), with the bits of several.
-static bool plans_small(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProblem &p) {
-    if (d->kernel != DFDX_ROCM_KERNEL_AUTO || !small_supported(p)) return false;
-    Plan plan;
-    if (make_plan(ctx, d, p, &plan) || plan.kernel != DFDX_ROCM_KERNEL_MFMA || plan.realign) return false;
-    const int small = p.dtype == DT_F32 ? mfma32_variant_count() : p.dtype == DT_F64 ? mfma64_small_variant() : mfma16_small_variant();
-    return plan.variant == small && (!p.ksum || small_ksum_supported(p));
+static bool plans_small(dfdx_rocm_ctx *ctx, Product &x) {
+    if (x.desc->kernel != DFDX_ROCM_KERNEL_AUTO || !small_supported(x.p)) return false;
+    if (x.need_plan(ctx) || x.plan.kernel != DFDX_ROCM_KERNEL_MFMA || x.plan.realign) return false;
+    const int small = x.p.dtype == DT_F32 ? mfma32_variant_count() : x.p.dtype == DT_F64 ? mfma64_small_variant() : mfma16_small_variant();
+    return x.plan.variant == small && (!x.p.ksum || small_ksum_supported(x.p));
 }
 
 // Two independent products in one launch: pending fills, then the launch.  `sums` of the second one ride along.
@@ -827,69 +856,84 @@ static int run_pair(dfdx_rocm_ctx *ctx, GemmProblem p, GemmProblem q, int tile, 
     return (int)launch_small_many(both, 2, ctx->stream);
 }
 
-int gemm_two(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, int extra, const void *with, const dfdx_rocm_gemm_desc *second, void *colsum,
-             bool *done) {
+// Both products as one launch where that is expected to be faster: *done.  When not, nothing has been touched.
+static int join_two(dfdx_rocm_ctx *ctx, Product &one, int extra, const void *with, Product &two, bool colsum, bool *done) {
     *done = false;
-    if (int e = bind(ctx)) return e;
-    GemmProblem p, q;
-    if (int e = make_problem(first, &p)) return e;
-    if (int e = make_problem(second, &q, colsum)) return e;
-    if (p.m == 0 || q.m == 0) return DFDX_ROCM_OK;
-    if (colsum && !q.ksum) return DFDX_ROCM_OK;
-    GemmProblem shape = p;
-    shape.accumulate = 1;  // (what the ops that `extra` stands for would do)
-    const int tile = ring_pair_tile(ctx, first, shape, second, q);
-    if (!tile && !(plans_small(ctx, first, p) && plans_small(ctx, second, q))) return DFDX_ROCM_OK;
+    if (one.p.m == 0 || two.p.m == 0 || (colsum && !two.p.ksum)) return DFDX_ROCM_OK;
+    const int tile = ring_pair_tile(ctx, one, two);
+    if (!tile && !(plans_small(ctx, one) && plans_small(ctx, two))) return DFDX_ROCM_OK;
+    GemmProblem p = one.p;
     p.extra = extra;
     p.with = with;
-    if (!independent(p, q)) return DFDX_ROCM_OK;
+    if (!independent(p, two.p)) return DFDX_ROCM_OK;
     *done = true;
-    return run_pair(ctx, p, q, tile, extra != EXTRA_FROM);
+    return run_pair(ctx, p, two.p, tile, extra != EXTRA_FROM);
+}
+
+// One behind the other.
+static int run_apart(dfdx_rocm_ctx *ctx, Product &one, int extra, const void *with, Product &two, bool *fused) {
+    if (one.p.m) {
+        if (int e = one.need_plan(ctx)) return e;
+        if (int e = extra == EXTRA_NONE ? run_planned(ctx, one.p, one.plan) : run_beyond(ctx, one.p, one.plan, extra, with)) return e;
+    }
+    if (!two.p.m) return DFDX_ROCM_OK;
+    if (int e = two.need_plan(ctx)) return e;
+    return run_with_colsum(ctx, two.p, two.plan, fused);
+}
+
+int gemm_two(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, int extra, const void *with, const dfdx_rocm_gemm_desc *second, void *colsum, bool *fused) {
+    *fused = false;
+    if (int e = bind(ctx)) return e;
+    Product one{first}, two{second};
+    if (int e = make_problem(first, &one.p)) return e;
+    if (int e = make_problem(second, &two.p, colsum)) return e;
+    if (one.p.m && extra != EXTRA_NONE && !beyond_ok(one.p, extra, with)) return DFDX_ROCM_ERR_INVALID_ARG;
+    bool done = false;
+    if (int e = join_two(ctx, one, extra, with, two, colsum != nullptr, &done)) return e;
+    if (!done) return run_apart(ctx, one, extra, with, two, fused);
+    *fused = colsum != nullptr;
+    return DFDX_ROCM_OK;
 }
 
 int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_rocm_gemm_desc *second, const void *grad_out, int64_t rows, int64_t cols,
               void *colsum, bool *fused) {
-    if (fused) *fused = false;
+    bool taken = false;  // (without `fused` no sums are asked for)
+    if (!fused) {
+        fused = &taken;
+        colsum = nullptr;
+    }
+    *fused = false;
+    if (int e = bind(ctx)) return e;
+    Product x[2] = {{first}, {second}};
+    if (int e = make_problem(first, &x[0].p)) return e;
+    if (int e = make_problem(second, &x[1].p, colsum)) return e;
     bool done = false;
-    if (int e = gemm_two(ctx, first, EXTRA_NONE, nullptr, second, fused ? colsum : nullptr, &done)) return e;
+    if (int e = join_two(ctx, x[0], EXTRA_NONE, nullptr, x[1], colsum != nullptr, &done)) return e;
     if (done) {
-        if (fused) *fused = colsum != nullptr;
+        *fused = colsum != nullptr;
         return DFDX_ROCM_OK;
     }
+    auto apart = [&]() { return run_apart(ctx, x[0], EXTRA_NONE, nullptr, x[1], fused); };
     // (a copy of less than 4 MB costs little more than its launch)
     const bool off = cols % 64 || rows % 64 || ((uintptr_t)grad_out & 15u);
-    if ((first->dtype != DFDX_ROCM_F16 && first->dtype != DFDX_ROCM_BF16) || !off || (double)rows * (double)cols < 2097152.0) {
-        if (int e = dfdx_rocm_gemm(ctx, first)) return e;
-        return fused ? gemm_with_colsum(ctx, second, colsum, fused) : dfdx_rocm_gemm(ctx, second);
-    }
-    if (int e = bind(ctx)) return e;
-    GemmProblem p[2];
-    Plan plan[2];
+    if ((first->dtype != DFDX_ROCM_F16 && first->dtype != DFDX_ROCM_BF16) || !off || (double)rows * (double)cols < 2097152.0) return apart();
     Realign ra;
     bool both = true;
-    for (int i = 0; i < 2; i++) {
-        const dfdx_rocm_gemm_desc *d = i ? second : first;
-        if (int e = make_problem(d, &p[i], i && fused ? colsum : nullptr)) return e;
-        if (p[i].m == 0) {
+    for (Product &i : x) {
+        if (i.p.m == 0) {
             both = false;
             continue;
         }
-        if (int e = make_plan(ctx, d, p[i], &plan[i])) return e;
+        if (int e = i.need_plan(ctx)) return e;
         // (one matrix each: the batches that a broadcast gradient is summed over step through grad_out by strides of their own)
-        both = both && plan[i].realign && p[i].nb1 * p[i].nb2 == 1 && p[i].a != p[i].b && plan_realign(p[i], &ra) && (p[i].a == grad_out ? ra.a || ra.a_last : ra.b || ra.b_last);
+        both = both && i.plan.realign && i.p.nb1 * i.p.nb2 == 1 && i.p.a != i.p.b && plan_realign(i.p, &ra) && (i.p.a == grad_out ? ra.a || ra.a_last : ra.b || ra.b_last);
     }
-    auto apart = [&]() -> int {
-        if (p[0].m)
-            if (int e = run_planned(ctx, p[0], plan[0])) return e;
-        if (!p[1].m) return DFDX_ROCM_OK;
-        return fused ? run_with_colsum(ctx, p[1], plan[1], fused) : run_planned(ctx, p[1], plan[1]);
-    };
     CtxLock lock(ctx->mu);  // the copy lives in the patch buffer until the second product has been launched
     int64_t ld = 0;
     const size_t bytes = realign_shared_bytes(rows, cols, &ld);
     if (!both || bytes == 0 || (bytes > ctx->patches_bytes && !grow_for_copies(ctx, ensure_patches, bytes))) return apart();
     // each product with grad_out replaced by the copy: the space of its own copy is not asked for
-    GemmProblem q[2] = {p[0], p[1]};
+    GemmProblem q[2] = {x[0].p, x[1].p};
     for (int i = 0; i < 2; i++) {
         q[i].ksum = nullptr;
         q[i].ksum_of = KSUM_NONE;
@@ -902,11 +946,11 @@ int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_r
             q[i].b = ctx->patches;
             q[i].b_laid = true;
         }
-        Plan reserved = plan[i];
+        Plan reserved = x[i].plan;
         if (int e = reserve_partials(ctx, q[i], reserved, false)) return e;
         if (!reserved.realign) return apart();
     }
-    const size_t sums_bytes = fused && colsum ? bias_backward_copy_partials(ctx->compute_units, rows, cols, ld) : 0;
+    const size_t sums_bytes = colsum ? bias_backward_copy_partials(ctx->compute_units, rows, cols, ld) : 0;
     const bool sums = sums_bytes > 0 && (sums_bytes <= ctx->workspace_bytes || grow_for_copies(ctx, ensure_workspace, sums_bytes));
     if (int e = settle(ctx, grad_out)) return e;
     if (sums) {  // on the way into the copy; their partials are done with the workspace before the products write it
@@ -920,7 +964,7 @@ int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_r
     }
     for (int i = 0; i < 2; i++) {
         if (int e = settle_operands(ctx, &q[i], /*may_overwrite=*/true)) return e;
-        if (int e = run_plan(ctx, q[i], plan[i])) return e;
+        if (int e = run_plan(ctx, q[i], x[i].plan)) return e;
     }
     return DFDX_ROCM_OK;
 }
@@ -976,7 +1020,9 @@ int gemm_three(dfdx_rocm_ctx *ctx, const GemmProblem &problem, bool *done) {
             q.c = at(p.c, p.c_b1, p.c_b2);
             q.bias = at(p.bias, p.bias_b1, p.bias_b2);
             q.ksum = at(p.ksum, p.ksum_b1, p.ksum_b2);
-            small = small && plans_small(ctx, &plain, q);
+            if (!small) continue;
+            Product x{&plain, q};
+            small = plans_small(ctx, x);
         }
         if (small && independent(one[0], one[1]) && independent(one[0], one[2]) && independent(one[1], one[2])) {
             *done = true;
@@ -1018,12 +1064,11 @@ int gemm_three_two(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const d
                    const GemmProblem &apart, bool *done) {
     *done = false;
     if (int e = bind(ctx)) return e;
-    GemmProblem one, two;
-    if (int e = make_problem(first, &one)) return e;
-    if (int e = make_problem(second, &two, colsum)) return e;
-    if (one.m == 0 || two.m == 0 || !two.ksum) return DFDX_ROCM_OK;
-    one.accumulate = 1;
-    if (!ring_pair_tile(ctx, first, one, second, two)) return DFDX_ROCM_OK;  // (what the calls that this one stands for would do)
+    Product one{first}, two{second};
+    if (int e = make_problem(first, &one.p)) return e;
+    if (int e = make_problem(second, &two.p, colsum)) return e;
+    if (one.p.m == 0 || two.p.m == 0 || !two.p.ksum) return DFDX_ROCM_OK;
+    if (!ring_pair_tile(ctx, one, two)) return DFDX_ROCM_OK;  // (what the calls that this one stands for would do)
     GemmProblem p = sum, q = apart;
     double seconds = 0.0;
     const int tile = mfma16_ring_pair_plan(p, q, ctx->compute_units, &seconds);

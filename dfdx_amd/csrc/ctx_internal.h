@@ -85,10 +85,10 @@ int gemm_beyond(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int extra, 
 // copy onto the 16-byte grid is copied once, with the column sums taken on the way.
 int gemm_pair(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, const dfdx_rocm_gemm_desc *second, const void *grad_out, int64_t rows, int64_t cols,
               void *colsum, bool *fused);
-// Two independent products -- `first` with one thing more on the way into C (gemm_beyond), `second` with the column sums of B
-// (gemm_with_colsum; colsum may be null) -- as one launch, where that is expected to be faster.  *done tells whether it ran; when not,
-// nothing has been touched.
-int gemm_two(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, int extra, const void *with, const dfdx_rocm_gemm_desc *second, void *colsum, bool *done);
+// Two products -- `first` with one thing more on the way into C (gemm_beyond), `second` with the column sums of B (gemm_with_colsum;
+// colsum may be null, *fused tells whether they are in it) -- as one launch where they are independent and that is expected to be faster,
+// else one behind the other.
+int gemm_two(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *first, int extra, const void *with, const dfdx_rocm_gemm_desc *second, void *colsum, bool *fused);
 // Three products of the same shape in one launch (GemmProblem::batches = 3, or their sum: `reduce`), where the LDS-DMA kernels take
 // them and one launch is expected to be faster than three.  *done tells whether it ran; when not, nothing has been touched.
 int gemm_three(dfdx_rocm_ctx *ctx, const struct GemmProblem &problem, bool *done);

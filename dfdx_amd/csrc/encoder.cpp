@@ -135,9 +135,7 @@ int linear_backward(dfdx_rocm_ctx *ctx, const Shape &s, const dfdx_rocm_gemm_des
     const dfdx_rocm_gemm_desc w = weight_product(s, i, o, x, gy, gw);
     bool done = false;
     if (int e = gemm_two(ctx, &gx, extra, with, &w, gb, &done)) return e;
-    if (done) return DFDX_ROCM_OK;
-    if (int e = gemm_beyond(ctx, &gx, extra, with)) return e;
-    return weight_grad(ctx, s, i, o, x, gy, gw, gb);
+    return done ? DFDX_ROCM_OK : dfdx_rocm_bias_backward(ctx, s.dtype, s.T, o, gy, gb);
 }
 
 // The products of the query, key and value projections as one launch: same shapes, matrices wherever they are (addresses from

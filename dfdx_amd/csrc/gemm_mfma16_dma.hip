@@ -300,6 +300,22 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
     const double elem = 2.0, out_elems = (double)p.m * p.n * nbatch;
     double best = 1e300, best_ring = 1e300;
     int ring = 0, ring_splits = 1;
+    // candidates 1..16, 20..32, 40..64 (filter gradients of convolutions: a handful of tiles, thousands of k steps), with their k steps
+    struct Pieces {
+        int splits;
+        int64_t chunk;
+    } pieces[32];
+    int count = 0;
+    {
+        int forced_s = forced_splits > 0 ? (int)std::min<int64_t>(forced_splits, total_iters) : 0;
+        while (forced_s > 1 && (forced_s - 1) * ((total_iters + forced_s - 1) / forced_s) >= total_iters) forced_s--;  // no empty split
+        for (int s = forced_s ? forced_s : 1; s <= (forced_s ? forced_s : 64); s += (s < 16 ? 1 : s < 32 ? 4 : 8)) {
+            if (s > 1 && (!may_split || (forced_splits == 0 && total_iters < 4 * (int64_t)s))) break;
+            const int64_t chunk = (total_iters + s - 1) / s;
+            if ((s - 1) * chunk >= total_iters) continue;  // an empty split
+            pieces[count++] = {s, chunk};
+        }
+    }
     for (int v = 1; v <= kNumVariants; v++) {
         if (forced_variant > 0 && v != forced_variant) continue;
         if (!mfma16dma_supported(p, v)) continue;
@@ -310,15 +326,11 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
         if (forced_variant == 0 && !is_ring(v) && (p.n <= 64 ? t.bn > 64 : (t.bn <= 64 && t.bm > 128))) continue;
         const int64_t tiles = ((p.m + t.bm - 1) / t.bm) * ((p.n + t.bn - 1) / t.bn) * nbatch;
         const double layout = (a_kc && b_kc) ? 1.0 : (!a_kc && !b_kc) ? 0.98 : 0.99;  // transposing LDS reads cost a little
-        // candidates 1..16, 20..32, 40..64 (filter gradients of convolutions: a handful of tiles, thousands of k steps)
-        int forced_s = forced_splits > 0 ? (int)std::min<int64_t>(forced_splits, total_iters) : 0;
-        while (forced_s > 1 && (forced_s - 1) * ((total_iters + forced_s - 1) / forced_s) >= total_iters) forced_s--;  // no empty split
-        for (int s = forced_s ? forced_s : 1; s <= (forced_s ? forced_s : 64); s += (s < 16 ? 1 : s < 32 ? 4 : 8)) {
-            if (s > 1 && (!may_split || (forced_splits == 0 && total_iters / s < 4))) break;
-            const int64_t chunk = (total_iters + s - 1) / s;
-            if ((s - 1) * chunk >= total_iters) continue;  // an empty split
-            const int64_t items = tiles * s;
+        for (int i = 0; i < count; i++) {
+            const int s = pieces[i].splits;
+            const int64_t chunk = pieces[i].chunk, items = tiles * s;
             if (is_ring(v)) {
+                if (forced_variant == 0 && items > (int64_t)cus * kRing[v - 1 - kNumTiles].per_cu) break;
                 const double time = ring_time(kRing[v - 1 - kNumTiles], cus, items, total_iters, p.k % BK == 0, chunk, a_kc, b_kc, s, out_elems);
                 if (time < best_ring || (forced_variant == v && ring == 0)) {
                     best_ring = time;
@@ -327,8 +339,8 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
                 }
                 continue;
             }
-            const int64_t grid = std::min<int64_t>(items, (int64_t)cus * vm.per_cu);
-            const int64_t conc = (grid + cus - 1) / cus, items_per_wg = (items + grid - 1) / grid;
+            const int grid = (int)std::min<int64_t>(items, (int64_t)cus * vm.per_cu), conc = (grid + cus - 1) / cus;
+            const int64_t items_per_wg = items == grid ? 1 : (items + grid - 1) / grid;
             const double active = (double)std::min<int64_t>(grid, cus) / cus;
             const double cu_rate = (conc >= 2 ? vm.rate2 : vm.rate1) * layout * (1.0 + kIdleBoost * (1.0 - active));
             const double t_mma = chunk * (2.0 * t.bm * t.bn * BK) / (cu_rate / conc);

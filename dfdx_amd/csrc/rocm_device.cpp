@@ -28,11 +28,8 @@ bool rows_fold(int64_t batch, int64_t rows, int64_t bs, int64_t rs) { return bat
 
 // The two products of a backward pass: as one launch where that is faster, else one after the other.
 int both(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc &left, const dfdx_rocm_gemm_desc &right) {
-    bool done = false;
-    if (int e = dfdx_rocm::gemm_two(ctx, &left, 0, nullptr, &right, nullptr, &done)) return e;
-    if (done) return DFDX_ROCM_OK;
-    if (int e = dfdx_rocm_gemm(ctx, &left)) return e;
-    return dfdx_rocm_gemm(ctx, &right);
+    bool unused = false;
+    return dfdx_rocm::gemm_two(ctx, &left, 0, nullptr, &right, nullptr, &unused);
 }
 
 }  // namespace
