@@ -28,6 +28,28 @@ def announce(*what):
     sys.stdout.flush()
 
 
+def launches(prepare):
+    """Launches of the call that ``prepare(dev)`` returns, on a context of its own: the nodes of the graph it is captured into, behind
+    one run by itself (so that the workspaces have their sizes)."""
+    import torch
+
+    from dfdx_amd import Rocm
+    from test_gpu_encoder_block import graph_nodes
+
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        own = Rocm(0)
+        run = prepare(own)
+        run()
+        own.synchronize()
+        n = graph_nodes(run, stream)
+        own.synchronize()
+    del run
+    own.close()
+    return n
+
+
 def make_operand(g, rows, cols, transposed, dtype, pad=0, scale=1.0, dist="normal"):
     """Storage + strides of a (rows, cols) matrix view; `transposed` stores it as (cols, rows)."""
     r, c = (cols, rows) if transposed else (rows, cols)

@@ -7,7 +7,7 @@ import torch
 
 import oracle
 from helpers import rng
-from gpu_util import announce, device
+from gpu_util import announce, device, launches
 from test_gpu_attention_fused import reference
 from test_gpu_encoder_block import graph_nodes
 
@@ -29,6 +29,16 @@ def backward(dev, dtype, st, B, H, S, D, in_place=False):
     return [oracle.to_f64(dev.to_host(t), dtype) for t in (gq, gk, gv)]
 
 
+def count(dtype, B, H, S, D):
+    """Launches of the backward."""
+    def prepare(dev):
+        q, k, v, gq, gk, gv = (dev.zeros(dtype, (B, H, S, D)) for _ in range(6))
+        go = dev.zeros(dtype, (B, S, H * D))
+        out, lse = dev.attention_forward(q, k, v, D ** -0.5)
+        return lambda: dev.attention_backward(q, gq, k, gk, v, gv, D ** -0.5, out, go, lse)
+    return launches(prepare)
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("H,S,D", [(2, 1, 64), (3, 63, 32), (2, 64, 64), (2, 65, 128), (2, 100, 64), (1, 129, 128), (4, 197, 64), (1, 257, 32)])
 def test_one_launch_and_two_agree(dtype, H, S, D):
@@ -37,6 +47,7 @@ def test_one_launch_and_two_agree(dtype, H, S, D):
     n = many * S * H * D
     st = [oracle.to_storage(g.standard_normal(n) * w, dtype) for w in (2.0, 2.0, 1.0, 1.0)]
     announce("attention backward, joined", dtype, H, S, D, many)
+    assert [count(dtype, B, H, S, D) for B in (1, many)] == [1, 2]
     few, all_ = backward(dev, dtype, st, 1, H, S, D), backward(dev, dtype, st, many, H, S, D)
     eps = 2.0 ** -11 if dtype == "f16" else 2.0 ** -8
     for name, a, b in zip(("dq", "dk", "dv"), few, all_):

@@ -5,7 +5,7 @@ import pytest
 
 import oracle
 from dfdx_amd.rocm import KERNEL_MFMA
-from gpu_util import announce, device
+from gpu_util import announce, device, launches
 from helpers import assert_within, rng
 from test_gpu_gemm import run_case
 
@@ -104,6 +104,11 @@ def test_two_products_of_a_backward_pass(dtype, rows, i, o):
             assert_within(dtype, a.shape[1], oracle.to_f64(dev.to_host(got), dtype).reshape(want.shape), want, a, b,
                           extra=2 * times * ulp * float(np.abs(want).max()), what=what)
 
+    def prepare(own):
+        x, w, go, gx, gw = (own.zeros(dtype, s) for s in ((rows, i), (i, o), (rows, o), (rows, i), (i, o)))
+        return lambda: own.backward(x, gx, w, gw, go)
+    assert launches(prepare) == 1
+
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("n", [128, 384])
@@ -118,6 +123,11 @@ def test_a_gradient_that_both_products_add_to(dtype, n):
     dev.backward(dx, gx, dx, gx, dgo)
     want = G @ X.T + X.T @ G
     ulp = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype]
+
+    def prepare(own, shared):
+        x, go, gx, gy = (own.zeros(dtype, (n, n)) for _ in range(4))
+        return lambda: own.backward(x, gx, x, gx if shared else gy, go)
+    assert [launches(lambda own: prepare(own, shared)) for shared in (True, False)] == [2, 1]
     assert_within(dtype, 2 * n, oracle.to_f64(dev.to_host(gx), dtype).reshape(n, n), want, X, G, extra=2 * ulp * float(np.abs(want).max()), what="sum")
 
 
