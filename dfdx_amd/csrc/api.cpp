@@ -369,8 +369,8 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         *plan = {DFDX_ROCM_KERNEL_GENERIC, 0, 1};
         return DFDX_ROCM_OK;
     case DFDX_ROCM_KERNEL_GEMV: {  // the bandwidth-bound kernels, forced: the caller's choice outranks the order flag
-        double unused;
-        const int bw = bandwidth_plan(p, false, true, &unused);
+        // (the rows form by its id, or where no other form takes the product)
+        const int other = bandwidth_kernel(p, false), bw = (!other || d->variant == BW_ROWS) && gemv_rows_supported(p) ? BW_ROWS : other;
         if (!bw) return DFDX_ROCM_ERR_UNSUPPORTED;
         *plan = {DFDX_ROCM_KERNEL_GEMV, bw, 1};
         return DFDX_ROCM_OK;
@@ -1389,7 +1389,8 @@ int dfdx_rocm_gemm_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc, int
     if (p.m != 0)
         if (int e = make_plan(ctx, desc, p, &plan)) return e;
     if (kernel) *kernel = plan.kernel;
-    if (variant) *variant = plan.kernel == DFDX_ROCM_KERNEL_GEMV ? 0 : plan.variant;  // (a tile variant; the bandwidth kernels have none)
+    // (a tile variant; of the bandwidth kernels, which the shape and the layout choose, one beside another has an id)
+    if (variant) *variant = plan.kernel == DFDX_ROCM_KERNEL_GEMV && plan.variant != BW_ROWS ? 0 : plan.variant;
     if (name && name_len) {
         const bool ring = plan.realign && mfma16dma_takes_any_k(plan.variant - mfma16_dma_first_variant() + 1);  // one of the LDS-DMA kernels too
         const char *const copied = !plan.realign ? "" : ring ? "_dma_realigned" : "_realigned";

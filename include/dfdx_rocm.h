@@ -177,7 +177,7 @@ typedef struct dfdx_rocm_gemm_desc {
     const void *bias;
     int32_t reduce_batch;
     int32_t kernel;  /* DFDX_ROCM_KERNEL_* ; 0 = automatic */
-    int32_t variant; /* tile variant inside the family; 0 = automatic */
+    int32_t variant; /* variant inside the family, as a plan reports it (a tile; 5: the rows form of KERNEL_GEMV); 0 = automatic */
     int32_t flags;   /* DFDX_ROCM_GEMM_* bits below; 0 = defaults */
 } dfdx_rocm_gemm_desc;
 

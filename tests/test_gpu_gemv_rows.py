@@ -69,9 +69,12 @@ def test_f32_sums_are_short_chains(k):
 
 @pytest.mark.parametrize("dtype,rows,k,n", [("f16", 16, 4096, 4096), ("f16", 4, 4093, 4091), ("f32", 4, 4093, 1091), ("f16", 8, 4096, 4096)])
 def test_the_kernel_that_a_plan_names_can_be_asked_for(dtype, rows, k, n):
+    """By the id that the plan reports; without one the vector-ALU form comes first, where there is one."""
     dev = device()
-    plan = lambda kernel: dev.gemm_plan(dev.gemm_desc(dtype, rows, k, n, 256, (k, 1), 512, (1, k), 1024, (n, 1), kernel=kernel))
-    assert plan(KERNEL_AUTO)[2] == "gemv_rows" and plan(KERNEL_AUTO)[0] == KERNEL_GEMV
-    assert plan(KERNEL_GEMV) == plan(KERNEL_AUTO)
+    plan = lambda *how: dev.gemm_plan(dev.gemm_desc(dtype, rows, k, n, 256, (k, 1), 512, (1, k), 1024, (n, 1), kernel=how[0], variant=how[1]))
+    kernel, variant, name = plan(KERNEL_AUTO, 0)
+    assert (kernel, name) == (KERNEL_GEMV, "gemv_rows")
+    assert plan(kernel, variant) == (kernel, variant, name)
+    assert plan(kernel, 0)[2] == ("gemv_multi" if k % 8 == 0 and rows <= 8 else "gemv_rows")
     if n < 2000:
-        assert run_case(dtype, rows, k, n, "nt", True, KERNEL_GEMV, 0, seed=k) == "gemv_rows"
+        assert run_case(dtype, rows, k, n, "nt", True, kernel, variant, seed=k) == "gemv_rows"
