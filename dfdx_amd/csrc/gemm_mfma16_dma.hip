@@ -207,6 +207,7 @@ struct RingModel {
     double k_tile[4], item, launch;
 };
 constexpr int64_t kRingChunk = 96, kRingAcross = 64;
+constexpr double kSecondRound = 2.0;  // see mfma16_ring_pair_plan (microseconds)
 constexpr double kSecondLaunch = 3.5e-6, kLastRound = 0.6, kShortRound = 12e-6;  // see plan_tail
 constexpr RingModel kRing[] = {
     {2, {0.0, 0.187, 0.390, 0.0}, 2.75, 0.9},    // 64 x 64, four stages
@@ -466,7 +467,16 @@ static hipError_t launch_ring(const GemmProblem &g, int variant, hipStream_t str
     return launch_splitk_reduce(g, p.ws_ld, p.ws_split_stride, stream, g.ksum ? p.ws_ksum : nullptr, p.ws_ksum_stride, ksum_slots(variant, p.splits));
 }
 
-// Work items of both products share the places on the chip; they are handed out as places fall free.
+// When the last of `longer` items of `t_longer`, which go first, and `shorter` ones of `t_shorter` ends, of more items than places and at
+// most twice as many.
+static double two_rounds(double longer, double shorter, double t_longer, double t_shorter, double places) {
+    if (longer >= places) return longer > places ? 2.0 * t_longer : t_longer + t_shorter;
+    const double free = places - longer;  // short items go there twice before a long one ends
+    return shorter <= 2.0 * free ? std::max(t_longer, 2.0 * t_shorter) : t_longer + t_shorter;
+}
+
+// Work items of both products share the places on the chip; they are handed out as places fall free.  With one place a compute unit the rounds
+// have a sharp end, and the average says too little: 39 x (448 x 80 . 80 x 448) bf16, 312 items, 17.4 us apart and 19.2 joined.
 int mfma16_ring_pair_plan(const GemmProblem &p, const GemmProblem &q, int compute_units, double *seconds) {
     const int cus = std::max(1, compute_units);
     int tile = 0;
@@ -487,6 +497,7 @@ int mfma16_ring_pair_plan(const GemmProblem &p, const GemmProblem &q, int comput
         const double k_tile = r.k_tile[(int)std::min((double)r.per_cu, std::ceil((np + nq) / cus))];
         const double tp = steps(p) * k_tile * (pb.kc ? 0.97 : 1.0) + r.item, tq = steps(q) * k_tile * 1.1 + r.item, longest = std::max(tp, tq);
         double us = np + nq <= places ? longest : std::max(longest, (np * tp + nq * tq) / places + 0.4 * longest);
+        if (r.per_cu == 1 && np + nq > places) us = std::max(us, two_rounds(tp >= tq ? np : nq, tp >= tq ? nq : np, longest, std::min(tp, tq), places) + kSecondRound);
         us += r.launch + 2.0 * ((double)p.m * p.n * (p.reduce ? 1 : p.batch_count()) + (double)q.m * q.n * (q.reduce ? 1 : q.batch_count())) / 8e6;
         if (us * 1e-6 < *seconds) {
             *seconds = us * 1e-6;

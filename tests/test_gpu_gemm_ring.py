@@ -111,6 +111,34 @@ def test_two_products_of_a_backward_pass(dtype, rows, i, o):
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("batch,m,k,n,expected", [
+    (39, 448, 80, 448, 1), (43, 256, 256, 256, 1), (25, 200, 136, 264, 1),   # more work items than the chip has places for
+    (54, 512, 80, 512, 2), (77, 320, 128, 320, 2),                           # no tile whose second round is worth it
+])
+def test_batches_of_a_backward_pass(dtype, batch, m, k, n, expected):
+    """The right operand stored along k, as attention's keys are."""
+    dev, g = device(), rng(batch + m)
+    announce("ring pair, batches", dtype, batch, m, k, n)
+    x, wt, go = (oracle.to_storage(g.standard_normal(s), dtype) for s in ((batch, m, k), (batch, n, k), (batch, m, n)))
+    shapes = ((batch, m, k), (batch, n, k), (batch, m, n), (batch, m, k), (batch, n, k))
+    turned = lambda t: t.permute(0, 2, 1)
+    dx, dw, dgo = dev.tensor(x, dtype), dev.tensor(wt, dtype), dev.tensor(go, dtype)
+    gx, gw = dev.zeros_many([dx, dw], deferred=True)
+    dev.backward(dx, gx, turned(dw), turned(gw), dgo)
+    X, W, G = oracle.to_f64(x, dtype), oracle.to_f64(wt, dtype), oracle.to_f64(go, dtype)
+    ulp = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype]
+    for got, a, b, what in ((gx, G, W, "lhs"), (gw, G.transpose(0, 2, 1), X, "rhs")):
+        want = a @ b
+        assert_within(dtype, a.shape[2], oracle.to_f64(dev.to_host(got), dtype)[:want.size].reshape(want.shape), want, a, b,
+                      extra=ulp * float(np.abs(want).max()), what=what)
+
+    def prepare(own):
+        x, w, go, gx, gw = (own.zeros(dtype, s) for s in shapes)
+        return lambda: own.backward(x, gx, turned(w), turned(gw), go)
+    assert launches(prepare) == expected
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("n", [128, 384])
 def test_a_gradient_that_both_products_add_to(dtype, n):
     """x . x: both gradients go to one buffer, one behind the other."""
