@@ -456,6 +456,7 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
                       : is16 ? mfma16_plan_splits(p, v, ctx->compute_units, forced_splits) : 1};
         if (!is32) t_family = is16 ? mfma16_staged_time(p, v, plan->splits, ctx->compute_units) : mfma64_time(p, v, ctx->compute_units);
         Realign ra;
+        ra.off_grid = ra.off_grid_k = 0;
         const bool realignable = is16 && plan_realign(p, &ra);
         // The small-product kernel's estimate holds for rows on the 16-byte grid; an operand stored along k whose rows are off it
         // is gathered value by value (f16, 76 x 6298 x 100, both such: 62 us for an estimate of 13, 13 us in 64 x 64 tiles;
@@ -470,7 +471,11 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         // 2340 x 3033 150 and 52, 530 x 3231 x 1057 84 and 28, 6928 x 106 x 7330 80 and 43; and where the line leaves the
         // staged kernels: 1000^3 12.0 and 18.8, 304 x 611 x 4120 11.0 and 16.4, 448 x 315 x 4890 13.2 and 14.5.
         double t_copies = 1e300;
-        if (realignable) {
+        const bool small_tile = v == mfma16_skinny_variant();
+        const double t_staged = t_family * (small_tile ? (ra.off_grid ? 1.0 : 0.6) : ra.off_grid ? 1.4 : 0.95) +
+                                (small_tile ? 0.0 : 2.0 * (double)p.m * (double)p.n * (double)(p.reduce ? 1 : p.nb1 * p.nb2) / 2.2e12);
+        const double t_uncopied = std::min(std::min(t_small_here, t_staged), t_bw);
+        if (realignable && ra.seconds + mfma16dma_least_time() < t_uncopied) {
             int dv = 0, splits = 1;
             GemmCut cut;
             mfma16dma_plan_split(ra.problem, ctx->compute_units, 0, forced_splits, &dv, &splits, &t_copies, &cut);
@@ -480,10 +485,7 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
                 mfma16dma_plan_split(ra.problem, ctx->compute_units, 0, (int)std::max<size_t>(1, most / piece), &dv, &splits, &t_copies, &cut);
             // (copies are not taken for a gain within the estimates' error)
             t_copies = dv ? t_copies + ra.seconds + (mfma16dma_takes_any_k(dv) ? 0.0 : splits > 1 ? 6.5e-6 : 1.0e-6) : 1e300;
-            const bool small_tile = v == mfma16_skinny_variant();
-            const double t_staged = t_family * (small_tile ? (ra.off_grid ? 1.0 : 0.6) : ra.off_grid ? 1.4 : 0.95) +
-                                    (small_tile ? 0.0 : 2.0 * (double)p.m * (double)p.n * (double)(p.reduce ? 1 : p.nb1 * p.nb2) / 2.2e12);
-            if (t_copies < std::min(std::min(t_small_here, t_staged), t_bw)) {
+            if (t_copies < t_uncopied) {
                 const Plan plain = *plan;
                 *plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits, true, v, plain.kernel, plain.variant, plain.splits, cut};
             }

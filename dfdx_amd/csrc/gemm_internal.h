@@ -177,6 +177,7 @@ hipError_t launch_bias_backward_copy(int dtype, int compute_units, int64_t rows,
 // whether the estimate is for two launches; a forced variant is not cut.
 void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_variant, int forced_splits, int *variant,
                           int *splits, double *seconds = nullptr, GemmCut *cut = nullptr);
+double mfma16dma_least_time();  // no estimate is below it
 size_t mfma16dma_workspace_bytes(const GemmProblem &p, int variant, int splits);
 bool mfma16dma_ksum_supported(const GemmProblem &p, int variant, int splits);  // can this plan also produce p.ksum?
 

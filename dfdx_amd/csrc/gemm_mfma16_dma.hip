@@ -119,31 +119,41 @@ bool mfma16dma_takes_any_k(int variant) { return is_ring(variant); }
 int mfma16dma_variant_count() { return kNumVariants; }
 const char *mfma16dma_variant_name(int v) { return (v >= 1 && v <= kNumVariants) ? kVariants[v - 1].name : "?"; }
 
-bool mfma16dma_supported(const GemmProblem &p, int variant) {
+// What the family asks of a product whatever the tile (a planner looks at it once); the operands' layouts are left in `la` and `lb`.
+static bool takes(const GemmProblem &p, OperandLayout *la, OperandLayout *lb) {
     if (p.dtype != DT_F16 && p.dtype != DT_BF16) return false;
-    if (variant < 1 || variant > kNumVariants) return false;
-    if (p.m < 1 || p.n < 1 || p.k < 1 || (!is_ring(variant) && p.k % BK != 0)) return false;
+    if (p.m < 1 || p.n < 1 || p.k < 1) return false;
     if (p.m > (1 << 30) || p.n > (1 << 30) || p.k > (1 << 30)) return false;
     if (p.c_cs != 1 && p.n != 1) return false;
     if (p.n > 1 && p.m > 1 && p.c_rs < p.n) return false;
-    const OperandLayout la = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged);
-    const OperandLayout lb = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged);
-    if (!la.ok || !lb.ok) return false;
-    const Variant &v = kVariants[variant - 1];
-    if (la.ld * (la.kc ? v.bm : BK) >= (1ll << 30) || lb.ld * (lb.kc ? v.bn : BK) >= (1ll << 30)) return false;
+    *la = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged);
+    *lb = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged);
+    if (!la->ok || !lb->ok) return false;
     if (!aligned16(p.a) || !aligned16(p.b)) return false;
-    if (!is_ring(variant) && !c_on_grid(p, v) && !(p.ragged && (v.bn / v.waves_n) % 32 == 0)) return false;
     if (p.batch_count() > 1) {
         if (p.a_b1 % 8 || p.a_b2 % 8 || p.b_b1 % 8 || p.b_b2 % 8) return false;
         if (!p.batches && (p.a_b1 < 0 || p.a_b2 < 0 || p.b_b1 < 0 || p.b_b2 < 0)) return false;
         if (p.bias_b1 % 8 || p.bias_b2 % 8) return false;
     }
-    const int64_t tiles = ((p.m + v.bm - 1) / v.bm) * ((p.n + v.bn - 1) / v.bn);
-    const int64_t blocks = tiles * (p.reduce ? 1 : p.batch_count());
-    if (blocks >= (1ll << 31) || p.batch_count() >= (1ll << 31)) return false;
+    if (p.batch_count() >= (1ll << 31)) return false;
     if (p.last_apart && (p.batch_count() != 1 || p.k % BK)) return false;
     if (p.k * (p.reduce ? p.batch_count() : 1) >= (1ll << 31)) return false;
     return true;
+}
+static int64_t tile_count(const GemmProblem &p, const Variant &v) {
+    return ((p.m + v.bm - 1) >> __builtin_ctz(v.bm)) * ((p.n + v.bn - 1) >> __builtin_ctz(v.bn));  // (powers of two)
+}
+static bool takes_on(const GemmProblem &p, int variant, const OperandLayout &la, const OperandLayout &lb) {
+    const Variant &v = kVariants[variant - 1];
+    if (!is_ring(variant) && p.k % BK != 0) return false;
+    if (la.ld * (la.kc ? v.bm : BK) >= (1ll << 30) || lb.ld * (lb.kc ? v.bn : BK) >= (1ll << 30)) return false;
+    if (!is_ring(variant) && !c_on_grid(p, v) && !(p.ragged && (v.bn / v.waves_n) % 32 == 0)) return false;
+    return tile_count(p, v) * (p.reduce ? 1 : p.batch_count()) < (1ll << 31);
+}
+
+bool mfma16dma_supported(const GemmProblem &p, int variant) {
+    OperandLayout la, lb;
+    return variant >= 1 && variant <= kNumVariants && takes(p, &la, &lb) && takes_on(p, variant, la, lb);
 }
 
 int mfma16dma_pick_variant(const GemmProblem &p, int compute_units) {
@@ -288,16 +298,22 @@ Tail plan_tail(const GemmProblem &p, int variant, int compute_units) {
 }
 }  // namespace
 
+double mfma16dma_least_time() { return kItemOverhead + kLaunchLatency - kAboveClock; }
+
 void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_variant, int forced_splits, int *variant,
                           int *splits, double *seconds, GemmCut *cut) {
     GemmCut best_cut;
     *variant = 0;
     *splits = 1;
+    if (cut) *cut = {};
+    if (seconds) *seconds = 1e300;
+    OperandLayout la, lb;
+    if (!takes(p, &la, &lb)) return;
     const int cus = std::max(1, compute_units);
     const int64_t nbatch = p.reduce ? 1 : p.batch_count();
     const bool may_split = (nbatch == 1 || p.batches > 0) && p.c_cs == 1;
     const int64_t total_iters = ((p.k + BK - 1) / BK) * (p.reduce ? p.batch_count() : 1);
-    const bool a_kc = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged).kc, b_kc = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged).kc;
+    const bool a_kc = la.kc, b_kc = lb.kc;
     const double elem = 2.0, out_elems = (double)p.m * p.n * nbatch;
     double best = 1e300, best_ring = 1e300;
     int ring = 0, ring_splits = 1;
@@ -319,13 +335,13 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
     }
     for (int v = 1; v <= kNumVariants; v++) {
         if (forced_variant > 0 && v != forced_variant) continue;
-        if (!mfma16dma_supported(p, v)) continue;
+        if (!takes_on(p, v, la, lb)) continue;
         const Variant &t = kVariants[v - 1];
         const VariantModel &vm = kModel[is_ring(v) ? 0 : v - 1];
         // narrow outputs take the BN = 64 tiles; wide ones may take the small 128 x 64 tile (more workgroups for a
         // problem of a few tiles), never the 256 x 64 one
         if (forced_variant == 0 && !is_ring(v) && (p.n <= 64 ? t.bn > 64 : (t.bn <= 64 && t.bm > 128))) continue;
-        const int64_t tiles = ((p.m + t.bm - 1) / t.bm) * ((p.n + t.bn - 1) / t.bn) * nbatch;
+        const int64_t tiles = tile_count(p, t) * nbatch;
         const double layout = (a_kc && b_kc) ? 1.0 : (!a_kc && !b_kc) ? 0.98 : 0.99;  // transposing LDS reads cost a little
         for (int i = 0; i < count; i++) {
             const int s = pieces[i].splits;
