@@ -575,14 +575,28 @@ Shape classify_rows(const GemmProblem &g) {
     p.accumulate = g.accumulate;
     p.stream = (double)p.j * (double)g.k * (double)dtype_size(g.dtype) >= 268435456.0;
     const int es = (int)dtype_size(g.dtype);
-    p.unit = 128;
-    p.period = 1;
-    while ((p.mat_j_stride * es * p.period) % p.unit) p.period *= 2;
+    // Sixteen rows that begin alike against the lines may lie far apart: of few rows most workgroups would then have a few (218 x 6077 f16, of
+    // 64 workgroups with 3 or 4 rows each 8.7 us, of 16 on the 16-byte grid 6.6; 1087 x 7177 15.6 and 12.5; 934 x 4323, nine tenths of
+    // the places taken, 9.9 and 9.8) -- but not of short rows, which the number of workgroups is good for (131 x 2055 5.3 and 5.8).
+    for (p.unit = 128;; p.unit /= 2) {
+        p.period = 1;
+        while ((p.mat_j_stride * es * p.period) % p.unit) p.period *= 2;
+        if (p.unit == 16 || p.period == 1 || g.k * es < 5120 || 10 * (int64_t)p.j >= 9 * 16 * rows_blocks(p)) break;
+    }
     const int64_t steps = (p.k + (p.period > 1 || (uintptr_t)p.mat % p.unit ? p.unit / es - 1 : 0) + rows_step(es) - 1) / rows_step(es);
     const int64_t blocks = rows_blocks(p);
     s.ahead = steps <= 8 ? 2 : 4;
     s.waves = steps <= 24 ? 4 : steps <= 48 || blocks >= 512 ? 8 : 16;
     int slices = 1;
+    if (blocks < 128 && steps >= 48 && 4 * steps >= 3 * blocks) {
+        // Few outputs of long rows: up to sixteen slices, each with a step for every one of four waves at least, 16 waves a compute unit in
+        // all.  49 shapes of 128 - 1300 outputs, 1 - 16 vectors, k of 1500 - 16384: 0.63 of the time of sixteen waves and a slice for
+        // every 64 steps at the least (16 x 198 x 7040 bf16 14.6 -> 6.5 us, 9 x 475 x 15104 f16 16.9 -> 9.1, 13 x 160 x 3136 f32 12.7 -> 5.8); below
+        // 48 steps the second launch costs more than it gives (4 x 276 x 1728 bf16 4.6 us, in four slices 5.4;
+        // 6 x 1562 x 1600 f32, 98 workgroups, 7.4 and 7.8).
+        while (slices < 16 && blocks * slices * 2 <= 640 && steps / (slices * 2) >= 4) slices *= 2;
+        s.waves = steps / slices < 8 ? 4 : 8;
+    }
     while (blocks * slices < 256 && steps / (slices * 2) >= 4 * s.waves) slices *= 2;
     p.kchunk = (int)((steps + slices - 1) / slices);
     p.kslices = (int)((steps + p.kchunk - 1) / p.kchunk);

@@ -23,11 +23,22 @@ def test_rows_off_the_grid(dtype, rows, k, n, pads):
 
 
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rows,k,n", [(12, 6077, 218), (16, 5493, 453), (13, 14271, 151), (2, 7680, 250), (9, 15104, 130), (3, 3071, 128), (3, 3073, 129),
+                                      (7, 2559, 257), (7, 2561, 1087), (16, 8190, 1024)])
+@pytest.mark.parametrize("pads", [(0, 0, 0), (3, 5, 1)])
+def test_few_outputs_of_long_rows(dtype, rows, k, n, pads):
+    """Up to sixteen k slices of four waves and more, rows on the 16-byte grid instead of the lines; at the lengths where either begins."""
+    for m_, n_, acc in ((rows, n, False), (n, rows, True)):
+        assert run_case(dtype, m_, k, n_, "nt", acc, KERNEL_GEMV, 5, pads=pads, seed=k + acc) == "gemv_rows"
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("k", [1024, 1024 + 1, 1024 + 31, 1024 + 32, 1024 + 63, 4096 - 7])
-def test_what_lies_behind_the_contraction_counts_for_nothing(dtype, k):
+@pytest.mark.parametrize("n", [2056, 200])
+def test_what_lies_behind_the_contraction_counts_for_nothing(dtype, k, n):
     """Rows with a gap of NaN behind each: the partial step takes zeros in their place."""
     dev, g = device(), rng(k)
-    rows, n, gap = 4, 2056, 9
+    rows, gap = 4, 9
     announce("gemv rows gaps", dtype, k)
     x, w = (oracle.to_storage(np.concatenate([g.standard_normal((r, k)), np.full((r, gap), np.nan)], axis=1), dtype) for r in (rows, n))
     dx, dw, dc = dev.tensor(x, dtype), dev.tensor(w, dtype), dev.zeros(dtype, (rows, n))
