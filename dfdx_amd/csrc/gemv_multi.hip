@@ -631,7 +631,8 @@ double gemv_rows_time(const GemmProblem &g) {
     const double es = (double)dtype_size(g.dtype), r = (double)s.p.r, mb = (double)s.p.j * (double)s.p.k * es / 1e6;
     const double blocks = (double)rows_blocks(s.p) * s.p.kslices;
     const double own = 16e-3 * (double)s.p.k * es / s.p.kslices * std::ceil(blocks / 256.0);
-    const double us = (half ? 2.2 : 2.5) + (s.p.kslices > 1 ? (half ? 2.8 : 1.4) : 0.0) + (s.p.period > 1 ? (half ? 1.3 : 0.8) : 0.0) +
+    const bool few = rows_blocks(s.p) < 128;  // (f32: two slices of many workgroups, or up to sixteen of few)
+    const double us = (half ? 2.2 : 2.5) + (s.p.kslices > 1 ? (half || few ? 2.8 : 1.4) : 0.0) + (s.p.period > 1 ? (half ? 1.3 : 0.8) : 0.0) +
                       (half ? std::max(mb * (0.225 + 0.0051 * r), own * (0.041 + 0.0018 * r)) - 0.011 * std::max(0.0, mb - 200.0)
                             : std::max(mb * (0.209 + 0.0063 * r), own * (0.0426 + 0.0015 * r)) - 0.024 * std::max(0.0, mb - 200.0));
     return us * 1e-6;
