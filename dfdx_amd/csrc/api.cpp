@@ -416,6 +416,11 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
     // not where the caller fixed the order of the contraction.
     const bool may_small = forced_splits == 0 && (is16 || is64) && small_supported(p);
     const double t_small = may_small ? small_time(p, ctx->compute_units) : 1e300;
+    // Against the ring tiles: a short contraction that four waves share takes less than the estimate, which is of long ones, most of all where
+    // values that lie across k are gathered (512 x 208 x 200 tn f16 4.2 us for 4.9, the ring 5.1 for 4.5; 104 x 64 x 384 tn 3.3 and 4.0, 256 x 96 x
+    // 1971 nt 3.9 and 4.6; of 82 products that the ring had taken from this kernel 15 were slower there by 4 - 24 %, all of them such; none that
+    // adds to C).
+    const double t_short = is16 && p.k < 256 && !p.accumulate ? (p.a_cs != 1 || p.b_rs != 1 ? 1.0e-6 : 0.4e-6) : 0.0;
     const Plan small_plan = {DFDX_ROCM_KERNEL_MFMA, is16 ? mfma16_small_variant() : mfma64_small_variant(), 1};
     Plan ring_plan = {};
     double t_ring = 1e300;
@@ -432,7 +437,7 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         } else if (dv) {
             *plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
             plan->cut = cut;
-            if (t_small < t_dma) *plan = small_plan;
+            if (t_small - (mfma16dma_takes_any_k(dv) ? t_short : 0.0) < t_dma) *plan = small_plan;
             double t_best = std::min(t_small, t_dma);
             int skinny_splits = 1;
             double t_skinny = 1e300;
@@ -492,12 +497,12 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         }
         // (on operands in place with k off 64 the staged tiles run at 0.83 - 1.06 of the estimate: 528 x 1024 x 1325 f16 21.4 us for 25.6,
         // 2304 x 128 x 1534 in three pieces 16.2 for 15.3; the ring 9.4 both)
-        const double t_plan = plan->realign ? t_copies : plan->kernel == DFDX_ROCM_KERNEL_GEMV ? t_bw : plan->variant == v ? 0.85 * t_family : t_small_here;
+        const double t_plan = plan->realign ? t_copies : plan->kernel == DFDX_ROCM_KERNEL_GEMV ? t_bw : plan->variant == v ? 0.85 * t_family : t_small_here - t_short;
         if (t_ring <= t_plan) *plan = ring_plan;
         if (seconds && is16) *seconds = std::min(t_ring, t_plan);
         return DFDX_ROCM_OK;
     }
-    if (t_ring < std::min(t_small, t_bw)) {
+    if (t_ring < std::min(t_small - t_short, t_bw)) {
         *plan = ring_plan;
         return DFDX_ROCM_OK;
     }

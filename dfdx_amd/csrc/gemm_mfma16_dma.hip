@@ -383,7 +383,11 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
         }
     }
     if (best < 1e300) best -= *splits > 1 ? kAboveClockSplit : kAboveClock;
-    if (ring && (best_ring < best || *variant == 0)) {
+    // A large C behind a few k tiles is bound by its stores, which the persistent tiles overlap with the next item: the ring's estimate lacks
+    // up to 1.2 us there, theirs is 0.9 too high (7040 x 64 x 512 f16 5.1 us and 6.5 for estimates of 6.2 and 5.7, 512 x 256 x 5248 6.7 and
+    // 8.0; 30 such products 1.05 - 1.26 times as long; where C is added to the two are level, and below 2.2 million values the ring is ahead).
+    const double stores = p.k <= 6 * BK && !p.accumulate && out_elems >= 2.2e6 ? 1.5e-6 : 0.0;
+    if (ring && (best_ring + stores < best || *variant == 0)) {
         best = best_ring;
         best_cut = {};
         *variant = ring;

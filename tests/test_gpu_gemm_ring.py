@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import oracle
-from dfdx_amd.rocm import KERNEL_MFMA
+from dfdx_amd.rocm import KERNEL_AUTO, KERNEL_MFMA
 from gpu_util import announce, device, launches
 from helpers import assert_within, rng
 from test_gpu_gemm import run_case
@@ -161,7 +161,7 @@ def test_a_gradient_that_both_products_add_to(dtype, n):
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("m,k,n,want", [
-    (2048, 64, 367, "mfma16_64x64x64_w2x2"), (520, 128, 1001, "mfma16_64x64x64_w2x2"), (8, 16384, 257, "gemv_multi"),
+    (2048, 64, 367, "mfma16_64x64x64_w2x2"), (520, 128, 1001, "mfma16_64x64x64_w2x2"), (8, 16384, 257, "gemv_rows"),
     (1000, 8192, 63, "mfma16_ring_64x64x64_w2x2_s4_splitk10"), (300, 2048, 1025, "ring"),
 ])
 def test_results_off_the_grid_have_rivals(dtype, m, k, n, want):
@@ -169,3 +169,14 @@ def test_results_off_the_grid_have_rivals(dtype, m, k, n, want):
     dev = device()
     name = dev.gemm_plan(dev.gemm_desc(dtype, m, k, n, 256, (k, 1), 512, (1, k), 1024, (n, 1)))[2]
     assert want == name or (want == "ring" and "_ring_" in name and "_realigned" not in name), name
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("m,k,n,layout,accumulate,want", [
+    (7040, 64, 512, "nn", False, "_dma_128x128"), (512, 256, 5248, "tn", False, "_dma_128x128"),   # many stores behind a few k tiles
+    (7040, 64, 512, "nn", True, "_ring_"), (1152, 64, 640, "nn", False, "_ring_"), (7040, 512, 512, "nn", False, "_ring_"),
+    (512, 208, 200, "tn", False, "_small_"), (104, 64, 384, "tn", False, "_small_"), (256, 96, 1971, "nt", False, "_small_"),   # short contractions
+    (512, 288, 200, "tn", False, "_ring_"), (512, 208, 200, "tn", True, "_ring_"),
+])
+def test_where_the_ring_has_rivals(dtype, m, k, n, layout, accumulate, want):
+    assert want in run_case(dtype, m, k, n, layout, accumulate, KERNEL_AUTO, 0, seed=m + n)
