@@ -587,6 +587,11 @@ bool tiled3x3_forward(dfdx_rocm_ctx *ctx, int dtype, const Op &op, const void *f
     // has compute units; one product over the folded batch fills it (f32, batch 32, 256 -> 256 at 14 x 14: 158 us here)
     const int64_t hw = (int64_t)op.h_in * op.w_in, blocks = (int64_t)((op.chan_out + 63) / 64) * ((hw + 255) / 256) * op.batch;
     if (blocks < ctx->compute_units && hw < 256 && op.batch > 1) return false;
+    // Half a chunk of channels (16, 24) and little to do: the product that forms its patches itself (implicit_forward) is one launch, this
+    // kernel two (16 bits: 8 images of 16 -> 64 at 32 x 32 8.1 and 10.2 us, 16 -> 128 at 40 x 40 8.8 and 10.3, but 16 -> 96 at 56 x 56 12.8 and 10.4)
+    if (sizeof(T) == 2 && op.chan_in < 32 && 18.0 * (double)op.batch * (double)hw * op.chan_in * op.chan_out < 4.75e8 &&
+        (op.w_out % 8 == 0 || op.w_out >= 24) && ((uintptr_t)filters & 15u) == 0)
+        return false;
     CtxLock lock(ctx->mu);  // the patch buffer is shared by every conv2d call on this context
     if ((*rc = ensure_patches(ctx, round256(conv3x3_filter_bytes(c))))) return true;
     c.wt = ctx->patches;
@@ -1211,9 +1216,13 @@ int backward_t(dfdx_rocm_ctx *ctx, int dtype, Op op, const void *img, void *grad
     }
     // (also at unit stride when the image has far fewer channels than the output -- a first layer, 3 -> 64: the forward patch
     // matrix is O / C times smaller than the one over grad_out, and the products with three rows of filters disappear; the band
-    // kernels are ahead of that in 16 bits up to a ratio of sixteen: 8 images of 64 -> 256 at 96 x 96 225 -> 142 us, of 32 -> 512 at
-    // 28 x 28 53 -> 63 us, f32 16 -> 128 at 28 x 28 62 -> 96 us)
-    if (op.stride > 1 || ((int64_t)op.chan_in * 4 <= op.chan_out && !(use_wgrad && sizeof(T) == 2 && op.chan_out < (int64_t)op.chan_in * 16)))
+    // kernels are ahead of that in 16 bits up to a ratio of sixteen where a workgroup's walk over the output channels is short or there are
+    // enough of them: 8 images of 64 -> 256 at 96 x 96 225 -> 142 us, of 16 -> 128 at 40 x 40 34 -> 32, but 4 images of 48 -> 512 at 32 x 32, 16
+    // workgroups, 35 -> 62 us, of 128 -> 512 50 -> 70; 8 of 32 -> 512 at 28 x 28 53 -> 63 us, f32 16 -> 128 at 28 x 28 62 -> 96 us)
+    const int64_t band_blocks = (int64_t)((op.chan_in + 63) / 64) * ((hw + 255) / 256) * op.batch;
+    const bool band_ahead = use_wgrad && sizeof(T) == 2 && op.chan_out < (int64_t)op.chan_in * 16 &&
+                            (4 * band_blocks >= op.chan_out || (op.chan_out <= 128 && op.batch > 1));
+    if (op.stride > 1 || ((int64_t)op.chan_in * 4 <= op.chan_out && !band_ahead))
         return strided_backward<T>(ctx, dtype, op, img, grad_img, filters, grad_filters, grad_out, fresh_img);
     if (per_image >= (1ll << 31) || f_elems >= (1ll << 31) || (int64_t)op.chan_in * hp >= (1ll << 31)) return DFDX_ROCM_ERR_UNSUPPORTED;
     CtxLock lock(ctx->mu);  // the patch buffer is shared by every conv2d call on this context

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import oracle
-from gpu_util import announce, device
+from gpu_util import announce, device, launches
 from helpers import rng
 
 pytestmark = pytest.mark.gpu
@@ -20,7 +20,7 @@ def correlate(img, fil):
 
 @pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("cin,cout", [(16, 16), (24, 64), (32, 96), (64, 32), (96, 48), (40, 136), (72, 200), (16, 80)])
-@pytest.mark.parametrize("batch,h,w", [(3, 16, 16), (2, 18, 30)])
+@pytest.mark.parametrize("batch,h,w", [(3, 16, 16), (2, 18, 30), (3, 18, 20)])
 def test_channels_that_are_no_whole_blocks(dtype, cin, cout, batch, h, w):
     """Forward, image and filter gradients (fresh and accumulated) of whole numbers that every type holds: sums below 2^24 are exact
     in f32 whatever their order, so each result has the one rounding of its type."""
@@ -60,3 +60,29 @@ def test_filter_gradient_where_the_filters_lie(dtype):
     np.testing.assert_array_equal(dev.to_host(onto_img), dev.to_host(apart_img))
     ulp = 0.0 if dtype == "f32" else 2.0 ** -11   # the sum is rounded once more beside the one that stands alone
     assert np.abs(oracle.to_f64(dev.to_host(dfil), dtype) - want).max() <= 2 * ulp * np.abs(want).max()
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("batch,cin,cout,hw,forward", [(8, 16, 64, 32, 1), (8, 24, 96, 32, 1), (8, 16, 96, 56, 2), (8, 32, 64, 32, 2), (3, 16, 64, 20, 2)])
+def test_little_to_do_is_one_launch(dtype, batch, cin, cout, hw, forward):
+    """Half a chunk of channels: the band kernel, behind the launch that lays the filters, only where there is enough to do."""
+    announce("conv3x3, launches", dtype, batch, cin, cout, hw)
+
+    def prepare(dev):
+        img, fil = dev.zeros(dtype, (batch, cin, hw, hw)), dev.zeros(dtype, (cout, cin, 3, 3))
+        return lambda: dev.conv2d_forward(img, fil, stride=1, padding=1)
+    assert launches(prepare) == forward
+
+
+@pytest.mark.parametrize("batch,cin,cout,hw,band", [(4, 48, 512, 32, False), (4, 128, 512, 32, False), (8, 64, 256, 14, False), (1, 16, 128, 32, False),
+                                                    (2, 16, 128, 32, True), (8, 64, 256, 96, True), (64, 32, 256, 20, True)])
+def test_many_output_channels_and_few_pixels(batch, cin, cout, hw, band):
+    """Backward: three launches with the band kernels (shares of the filter gradient, their sums beside the filters, the image gradient);
+    with the patch matrix of the image there are the patches, two products and the fold."""
+    announce("conv3x3 backward, launches", batch, cin, cout, hw)
+
+    def prepare(dev):
+        img, fil, go = (dev.zeros("f16", s) for s in ((batch, cin, hw, hw), (cout, cin, 3, 3), (batch, cout, hw, hw)))
+        gi, gf = (dev.zeros("f16", t.shape) for t in (img, fil))
+        return lambda: dev.conv2d_backward(img, gi, fil, gf, go, stride=1, padding=1)
+    assert (launches(prepare) <= 3) == band
