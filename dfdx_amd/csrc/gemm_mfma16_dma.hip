@@ -208,10 +208,14 @@ constexpr double kAboveClock = 1.0e-6, kAboveClockSplit = 6.5e-6;
 // They are taken only where every work item has a place at once: behind a first round the persistent tiles with their larger
 // steps are ahead (1344 x 768 x 3072 f16: 1008 items of 64 x 64 16.9 us, the 256 x 128 tile 15.4; 3072 x 3072 x 128 14.6 and 9.3).
 // Nor over more than 96 k tiles, where the larger tiles' fewer LDS reads have caught up (256 items of 128 x 128 x 4096 f16 36.7 us, the
-// best of the persistent tiles 43.4; x 8192 75.7 and 75.9).  Weight gradients over 4096 rows and more (both operands stored across k),
-// where the persistent tiles take them (whole k tiles), keep the split plans of the persistent tiles, which are fixed points of the sums that ride along with them (ksum): up to 25 % given up
-// at 1024 x 4096 x 1024 (17.8 and 23.7 us), 10 % at 1024 x 8192 x 1024 (29.3 and 32.4).
-// Over the 600 the plan is 1.3 % from the fastest of all tiles and split counts; the plan without the ring was 19 % from it.
+// best of the persistent tiles 43.4; x 8192 75.7 and 75.9).
+// kRingAcross is no line between two speeds: weight gradients over 4096 rows and more (both operands stored across k, whole k tiles) keep
+// the split plans of the persistent tiles, so that those which carry a layer's bias gradient along (ksum) stay reached and tested at the
+// sizes they were built for (test_gpu_linear.py names them); the ring takes 17.8 us for 23.7 at 1024 x 4096 x 1024 and 29.3 for 32.4 at 1024 x 8192 x
+// 1024, and has not been measured beyond 8192 rows.
+// Over the 600, launched again and again on operands that the last-level cache holds, the plan is 1.3 % from the fastest of all tiles and
+// split counts; the plan without the ring was 19 % from it.  In a chain of launches the operands may come from memory: behind the launch that
+// writes its first operand, 3152 x 3072 x 768 f16 takes 34 us on the 128 x 128 tile for an estimate of 25.
 struct RingModel {
     int per_cu;
     double k_tile[4], item, launch;

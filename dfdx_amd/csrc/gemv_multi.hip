@@ -272,8 +272,8 @@ template <typename T, int R, bool STREAM> __global__ __launch_bounds__(256) void
 // Rows of an odd length begin anywhere: a workgroup takes rows that begin alike against the 128-byte lines, every 64th one for an odd
 // length of 16-bit values, and reads all of them in whole lines, the vectors shifted against them (with rows side by side, each load
 // off the grid, 1 x 4091 x 4093 f16 took 13.8 us instead of 9.4, 16379 x 16381 169 instead of 109; on the 16-byte grid only 9.7 and
-// 135).  Four steps of a wave are on their way at once, four waves a workgroup where the rows are short, sixteen where there are few
-// outputs, and k slices where there are fewer than 256 workgroups: 8 x 4096 x 4096 f16 9.4 us (3.6 TB/s), 8 x 16384 x 16384 118 us
+// 135).  Four steps of a wave are on their way at once, four waves a workgroup where the rows are short, up to sixteen where there are few
+// outputs, and k slices where there are fewer than 256 workgroups (classify_rows): 8 x 4096 x 4096 f16 9.4 us (3.6 TB/s), 8 x 16384 x 16384 118 us
 // (4.5 TB/s), f32 17 us and 241 us.
 // f32: short chains -- the products of a load by themselves (rows_mma), the waves' sums in pairs.  With one chain a wave, 2 x 3072 x 2560 was
 // 2.0 times as far from the sums in 64 bits as the vector-ALU form (2.0e-7, 1.1e-7 now) and 2 - 16 x 768 x 6000 1.3 times as far as the
