@@ -331,18 +331,28 @@ int bandwidth_kernel(const GemmProblem &p, bool plain_order) {
 // form has no rival (1 - 16 vectors against 512 - 16384 rows and columns, 245 products: 1.47 times as fast as the best plan
 // without it in the mean, 4 x 4091 x 4093 f16 36.5 -> 10.1 us, f32 36.9 -> 15.7, 8 x 4288 x 4288 bf16 14 -> 11) but the
 // small-product kernel, by estimated time, on rows that lie on the 16-byte grid of a matrix below 8 MB (up to 11 % there, either
-// way: 8 x 520 x 2635 bf16 3.7 and 4.2 us, 16 x 2048 x 2048 7.0 and 6.8); the others have none.  `seconds`: the estimate where it has rivals,
-// else 0.
-int bandwidth_plan(const GemmProblem &p, bool plain_order, bool may_rows, double *seconds) {
+// way: 8 x 520 x 2635 bf16 3.7 and 4.2 us, 16 x 2048 x 2048 7.0 and 6.8), and but the LDS-DMA tiles (`tiles_only`) on such rows of a larger one in
+// 16 bits, which a vector more costs nothing (16 x 14208 x 8384 bf16 84 us and 52, 16 x 10304 x 4355 f16 43 and 22, 8 x 7680 x 8960 36 and 30; 57
+// products of 1 - 16 rows: 1.11 times the better of the two on this form alone, 1.02 with 0.85 of its estimate against theirs, 0.95 from 96 MB on); the
+// others have none.
+// `seconds`: the estimate where it has rivals, else 0.
+int bandwidth_plan(const GemmProblem &p, bool plain_order, bool may_rows, double *seconds, bool *tiles_only) {
     *seconds = 0.0;
+    *tiles_only = false;
     const int bw = bandwidth_kernel(p, plain_order);
     if (bw == BW_GEMV_MULTI) *seconds = gemv_multi_time(p);
     if ((bw != BW_NONE && bw != BW_GEMV_MULTI) || !may_rows || !gemv_rows_supported(p)) return bw;
     // (the other forms take 1.1 times their estimate, 4 x 2048 x 2048 f32 10.2 us and 8.6 as rows, but on matrices that no cache
-    // holds: 8 x 16384 x 16384 f32 218 and 240)
+    // holds: 8 x 16384 x 16384 f32 218 and 240; in 16 bits they are ahead of all others there, 2 x 12920 x 12288 f16 57 us, 68 as rows, 71 on the ring
+    // tiles, 8 x 11008 x 16768 89, 103 and 101)
     const double t = gemv_rows_time(p), bytes = (double)std::max(p.m, p.n) * (double)p.k * (double)dtype_size(p.dtype);
+    if (bw == BW_GEMV_MULTI && bytes >= 268435456.0 && dtype_size(p.dtype) == 2) {
+        *seconds = 0.0;
+        return bw;
+    }
     if (bw == BW_GEMV_MULTI && t >= (bytes < 268435456.0 ? 1.1 : 1.0) * *seconds) return bw;
-    *seconds = bytes < 8e6 && p.k * (int64_t)dtype_size(p.dtype) % 16 == 0 ? t : 0.0;
+    *tiles_only = bytes >= 8e6 && mfma16dma_supported(p, mfma16dma_variant_count());
+    *seconds = *tiles_only ? (bytes < 96e6 ? 0.85 : 0.95) * t : bytes < 8e6 && p.k * (int64_t)dtype_size(p.dtype) % 16 == 0 ? t : 0.0;
     return BW_ROWS;
 }
 
@@ -405,7 +415,22 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
     }
     // The bandwidth-bound kernels first.
     double t_bw = 1e300;
-    const int bw = bandwidth_plan(p, (d->flags & DFDX_ROCM_GEMM_NO_SPLIT_K) != 0, !forced_splits, &t_bw);
+    bool tiles_only = false;
+    const int bw = bandwidth_plan(p, (d->flags & DFDX_ROCM_GEMM_NO_SPLIT_K) != 0, !forced_splits, &t_bw, &tiles_only);
+    if (tiles_only) {
+        // what the tiles' estimates lack on few rows: the matrix streams past the caches once (238 MB 52 us for an estimate of 32)
+        const double t_stream = 3.0e-6 + (double)(p.m + p.n) * (double)p.k * (double)dtype_size(p.dtype) / 4.6e12;
+        int dv = 0, splits = 1;
+        double t_dma = 1e300;
+        GemmCut cut;
+        mfma16dma_plan_split(p, ctx->compute_units, 0, 0, &dv, &splits, &t_dma, &cut);
+        *plan = {DFDX_ROCM_KERNEL_GEMV, bw, 1};
+        if (dv && std::max(t_dma, t_stream) < t_bw) {
+            *plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
+            plan->cut = cut;
+        }
+        return DFDX_ROCM_OK;
+    }
     if (bw && t_bw == 0.0) {
         *plan = {DFDX_ROCM_KERNEL_GEMV, bw, 1};
         return DFDX_ROCM_OK;

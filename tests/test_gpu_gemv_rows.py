@@ -83,9 +83,22 @@ def test_the_kernel_that_a_plan_names_can_be_asked_for(dtype, rows, k, n):
     """By the id that the plan reports; without one the vector-ALU form comes first, where there is one."""
     dev = device()
     plan = lambda *how: dev.gemm_plan(dev.gemm_desc(dtype, rows, k, n, 256, (k, 1), 512, (1, k), 1024, (n, 1), kernel=how[0], variant=how[1]))
-    kernel, variant, name = plan(KERNEL_AUTO, 0)
-    assert (kernel, name) == (KERNEL_GEMV, "gemv_rows")
-    assert plan(kernel, variant) == (kernel, variant, name)
+    assert plan(*plan(KERNEL_AUTO, 0)[:2]) == plan(KERNEL_AUTO, 0)
+    kernel, variant, name = plan(KERNEL_GEMV, 5)
+    assert (kernel, variant, name) == (KERNEL_GEMV, 5, "gemv_rows")
     assert plan(kernel, 0)[2] == ("gemv_multi" if k % 8 == 0 and rows <= 8 else "gemv_rows")
     if n < 2000:
         assert run_case(dtype, rows, k, n, "nt", True, kernel, variant, seed=k) == "gemv_rows"
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("rows,k,n,pad,want", [
+    (16, 10304, 4355, 0, "_ring_"), (8, 8960, 7680, 0, "_ring_"), (12, 5376, 4438, 0, "_ring_"),   # rows on the grid of a large matrix
+    (16, 10304, 4355, 4, "gemv_rows"), (16, 10301, 4355, 0, "gemv_rows"), (8, 2048, 2744, 0, "gemv_rows"),
+    (2, 12920, 12288, 0, "gemv_multi"), (8, 16768, 11008, 0, "gemv_multi"), (16, 16768, 11008, 0, "_ring_"),   # beyond the caches
+])
+def test_rivals_on_large_matrices(dtype, rows, k, n, pad, want):
+    dev = device()
+    name = dev.gemm_plan(dev.gemm_desc(dtype, rows, k, n, 256, (k + pad, 1), 512, (1, k + pad), 1024, (n, 1)))[2]
+    announce("gemv rows, rivals", dtype, rows, k, n, pad, name)
+    assert want in name, name
