@@ -574,17 +574,19 @@ size_t partials_bytes(const GemmProblem &p, const Plan &plan, Realign *ra) {
                    : mfma16dma_workspace_bytes(p, plan.variant - mfma16_dma_first_variant() + 1, plan.splits);
     if (plan.kernel == DFDX_ROCM_KERNEL_GEMV && plan.variant == BW_GEMV_MULTI) return gemv_multi_workspace_bytes(p);
     if (plan.kernel == DFDX_ROCM_KERNEL_GEMV && plan.variant == BW_GEMV) return gemv_workspace_bytes(p);
-    if (plan.kernel == DFDX_ROCM_KERNEL_GEMV && plan.variant == BW_ROWS) return gemv_rows_workspace_bytes(p);
+    if (plan.kernel == DFDX_ROCM_KERNEL_GEMV && plan.variant == BW_ROWS) return plan.splits ? gemv_rows_workspace_bytes(p) : 0;  // (0: in one piece)
     return 0;
 }
 
 // Space that the call could do without is not asked for while the stream is being captured into a graph, nor where as much has been
 // refused since memory was last freed.
+bool capturing(dfdx_rocm_ctx *ctx) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess) (void)hipGetLastError();
+    return status != hipStreamCaptureStatusNone;
+}
 bool grow_for_copies(dfdx_rocm_ctx *ctx, int (*ensure)(dfdx_rocm_ctx *, size_t), size_t bytes) {
-    if (bytes >= ctx->copies_refused) return false;
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess) (void)hipGetLastError();
-    if (capturing != hipStreamCaptureStatusNone) return false;
+    if (bytes >= ctx->copies_refused || capturing(ctx)) return false;
     if (ensure(ctx, bytes) == DFDX_ROCM_OK) return true;
     ctx->copies_refused = bytes;
     return false;
@@ -611,6 +613,17 @@ int reserve_partials(dfdx_rocm_ctx *ctx, const GemmProblem &problem, Plan &plan,
         plan = plain;
     }
     const size_t need = partials_bytes(p, plan);
+    // Products that kernels without partial sums had before the ring tiles and the rows form: captured with no space they run in one piece.
+    const bool ring = plan.kernel == DFDX_ROCM_KERNEL_MFMA && (p.dtype == DT_F16 || p.dtype == DT_BF16) && plan.variant >= mfma16_dma_first_variant() &&
+                      plan.variant != mfma16_small_variant() && mfma16dma_takes_any_k(plan.variant - mfma16_dma_first_variant() + 1);
+    const bool rows = plan.kernel == DFDX_ROCM_KERNEL_GEMV && plan.variant == BW_ROWS;
+    if (need && !static_scratch && (ring || rows)) {
+        CtxLock lock(ctx->mu);
+        if (need > ctx->workspace_bytes && capturing(ctx)) {
+            plan.splits = ring ? 1 : 0;
+            return DFDX_ROCM_OK;
+        }
+    }
     return need ? partials_buffer(ctx, need, static_scratch, &unused) : DFDX_ROCM_OK;
 }
 

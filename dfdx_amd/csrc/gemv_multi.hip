@@ -645,8 +645,12 @@ size_t gemv_rows_workspace_bytes(const GemmProblem &g) {
 
 hipError_t launch_gemv_rows(const GemmProblem &g, hipStream_t stream) {
     Shape s = classify_rows(g);
-    if (!s.ok || (s.p.kslices > 1 && !g.workspace)) return hipErrorInvalidValue;
+    if (!s.ok) return hipErrorInvalidValue;
     s.p.ws = g.workspace;
+    if (!g.workspace) {  // in one piece
+        s.p.kchunk *= s.p.kslices;
+        s.p.kslices = 1;
+    }
     switch (g.dtype) {
     case DT_F32: return launch_rows_t<float>(s, stream);
     case DT_F16: return launch_rows_t<_Float16>(s, stream);

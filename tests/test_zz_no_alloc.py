@@ -156,3 +156,48 @@ def test_captured_into_a_graph_with_a_cold_context(m, k, n, at):
             own.synchronize()
             assert np.array_equal(own.to_host(out).view(np.uint16), dev.to_host(want).view(np.uint16))
     own.close()
+
+
+@pytest.mark.parametrize("dtype,m,k,n,at,plan", [("f16", 12, 6077, 218, False, "gemv_rows"), ("f32", 3, 9001, 300, False, "gemv_rows"),
+                                                 ("bf16", 8, 2496, 384, True, "_ring_64x64x64_w2x2_s4_splitk"), ("f16", 16, 10304, 1091, False, "_ring_64x64x64_w2x2_s4_splitk")])
+def test_a_cold_context_captures_in_one_piece(dtype, m, k, n, at, plan):
+    """Slices of the contraction on kernels that took such products from others without partial sums: where there is no space for the sums and
+    none can be had, one piece."""
+    import torch
+
+    from dfdx_amd import Rocm
+
+    dev, g = device(), rng(k)
+    a, astr = make_operand(g, m, k, at, dtype)
+    b, bstr = make_operand(g, k, n, not at, dtype)
+    da, db = dev.tensor(a, dtype), dev.tensor(b, dtype)
+    desc = lambda d, c: d.gemm_desc(dtype, m, k, n, da.ptr, astr, db.ptr, bstr, c.ptr, (n, 1))
+    name = dev.gemm_plan(desc(dev, da))[2]
+    announce("captured, cold", dtype, (m, k, n), name)
+    assert plan in name, name
+    dev.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        own = Rocm(0)
+        out = own.zeros(dtype, (m, n))
+        own.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            own.gemm(desc(own, out))
+        A, B = values(a, dtype, (m, k), astr), values(b, dtype, (k, n), bstr)
+        want = A @ B
+        ulp = {"f32": 2.0 ** -24, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dtype]
+        for _ in range(3):
+            out.storage.fill_(0x55)
+            graph.replay()
+            own.synchronize()
+            assert_within(dtype, k, oracle.to_f64(own.to_host(out), dtype).reshape(m, n), want, A, B, extra=ulp * float(np.abs(want).max()), what=name)
+    own.close()
+
+
+@pytest.mark.parametrize("dtype,m,k,n", [("f16", 12, 6077, 218), ("f32", 16, 7744, 1100), ("bf16", 1090, 7177, 16), ("f16", 16, 10304, 1091)])
+def test_few_rows_in_slices(dtype, m, k, n):
+    """The partial sums of up to sixteen slices, or of the ring tiles' pieces, of one to sixteen rows fit the array."""
+    name = device().gemm_plan(device().gemm_desc(dtype, m, k, n, 256, (k, 1), 512, (1, k), 1024, (n, 1)))[2]
+    assert "gemv_rows" in name or "_ring_" in name, name
+    both_entries(dtype, m, k, n, (False, True), True, seed=k, expect_split=False)
