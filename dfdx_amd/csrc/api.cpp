@@ -455,7 +455,7 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         GemmCut cut;
         mfma16dma_plan_split(p, ctx->compute_units, 0, forced_splits, &dv, &splits, &t_dma, &cut);
         bool only_ring = dv && mfma16dma_takes_any_k(dv);
-        for (int v = 1; only_ring && !mfma16dma_takes_any_k(v); v++) only_ring = !mfma16dma_supported(p, v);
+        for (int v = 1; only_ring && v <= mfma16dma_variant_count(); v++) only_ring = mfma16dma_takes_any_k(v) || !mfma16dma_supported(p, v);
         // (a C on the 8-byte grid only: of the persistent tiles one stores it as it is, the 128 x 64 one; all others with the
         // element-aligned stores of the plans below.  2048 x 1024 x 50260 f16 342 us and 208, 4096 x 1024 x 4092 51 and 36.)
         const int64_t ldc = p.m == 1 ? p.n : p.c_rs;

@@ -1013,14 +1013,14 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
 
 #undef DFDX_LEFT
 
-// X(id, BM, BN, WAVES_M, WAVES_N); ids are 1-based inside this family.
+// X(id, BM, BN, WAVES_M, WAVES_N); ids are 1-based inside this family and shared with the ring tiles (gemm_mfma16_ring.h).
 #define DFDX_MFMA16_DMA_VARIANTS(X) \
     X(1, 256, 256, 2, 4)            \
     X(2, 256, 128, 4, 2)            \
     X(3, 128, 128, 2, 4)            \
     X(4, 256, 64, 4, 2)             \
     X(5, 128, 64, 2, 4)             \
-    X(6, 256, 192, 4, 2)
+    X(10, 256, 192, 4, 2)
 
 // Persistent launch: as many workgroups as the chip holds at once (what LDS and registers allow per compute
 // unit, rounded to a multiple of the 8 XCDs so that work item i and i + grid land on the same XCD), or one per

@@ -24,6 +24,7 @@
 #include "gemm_mfma16_dma.h"
 #include "gemm_mfma16_ring.h"
 #include <algorithm>
+#include <array>
 #include <cmath>
 
 namespace dfdx_rocm {
@@ -34,21 +35,24 @@ namespace {
 struct Variant {
     const char *name;
     int bm, bn, waves_m, waves_n;
+    bool ring;  // a tile of gemm_mfma16_ring.hip
 };
 
-constexpr Variant kVariants[] = {
-#define X(id, bm, bn, wm, wn) {"dma_" #bm "x" #bn "x64_w" #wm "x" #wn, bm, bn, wm, wn},
+// Ids are those of the two lists, which count through both: a caller may ask for a tile by its id, so new ones go behind.
+#define X(...) +1
+constexpr int kNumVariants = 0 DFDX_MFMA16_DMA_VARIANTS(X) DFDX_MFMA16_RING_VARIANTS(X);
+#undef X
+constexpr std::array<Variant, kNumVariants> kVariants = [] {
+    std::array<Variant, kNumVariants> v{};
+#define X(id, bm, bn, wm, wn) v[id - 1] = {"dma_" #bm "x" #bn "x64_w" #wm "x" #wn, bm, bn, wm, wn, false};
     DFDX_MFMA16_DMA_VARIANTS(X)
 #undef X
-#define X(id, bm, bn, wm, wn, depth) {"ring_" #bm "x" #bn "x64_w" #wm "x" #wn "_s" #depth, bm, bn, wm, wn},
-    DFDX_MFMA16_RING_VARIANTS(X)  // gemm_mfma16_ring.hip
+#define X(id, bm, bn, wm, wn, depth) v[id - 1] = {"ring_" #bm "x" #bn "x64_w" #wm "x" #wn "_s" #depth, bm, bn, wm, wn, true};
+    DFDX_MFMA16_RING_VARIANTS(X)
 #undef X
-};
-constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
-#define X(...) +1
-constexpr int kNumTiles = 0 DFDX_MFMA16_DMA_VARIANTS(X);
-#undef X
-inline bool is_ring(int variant) { return variant > kNumTiles; }
+    return v;
+}();
+inline bool is_ring(int variant) { return kVariants[variant - 1].ring; }
 
 template <typename T, int BM, int BN, int WM, int WN>
 hipError_t launch_layout(Params p, int compute_units, bool a_kc, bool b_kc, hipStream_t stream) {
@@ -196,12 +200,13 @@ struct VariantModel {
     int per_cu;           // workgroups resident per compute unit (LDS and register limits)
     double rate1, rate2;  // flop/s of a compute unit with 1 / with >= 2 resident workgroups
 };
-constexpr VariantModel kModel[] = {
+constexpr VariantModel kModel[kNumVariants] = {
     {1, 5.50e12, 5.50e12},  // 256x256
     {1, 4.40e12, 4.40e12},  // 256x128
     {2, 3.00e12, 4.25e12},  // 128x128
     {1, 3.60e12, 3.60e12},  // 256x64
     {2, 2.20e12, 2.90e12},  // 128x64
+    {}, {}, {}, {},         // (ring tiles)
     {1, 5.00e12, 5.00e12},  // 256x192
 };
 constexpr double kItemOverhead = 2.0e-6, kLaunchLatency = 2e-6, kCuBandwidth = 24e9, kOperandWeight = 0.32;
@@ -236,12 +241,14 @@ struct RingModel {
 constexpr int64_t kRingChunk = 96, kRingAcross = 64;
 constexpr double kSecondRound = 2.0;  // see mfma16_ring_pair_plan (microseconds)
 constexpr double kSecondLaunch = 3.5e-6, kLastRound = 0.6, kShortRound = 12e-6;  // see plan_tail
-constexpr RingModel kRing[] = {
-    {1, {0.0, 0.349, 0.0, 0.0}, 5.00, 0.1},      // 192 x 64
+constexpr RingModel kRing[kNumVariants] = {
+    {}, {}, {}, {}, {},                          // (persistent tiles)
     {2, {0.0, 0.187, 0.390, 0.0}, 2.75, 0.9},    // 64 x 64, four stages
     {3, {0.0, 0.234, 0.394, 0.572}, 3.30, 0.2},  // 64 x 64, three
     {2, {0.0, 0.305, 0.610, 0.0}, 4.10, 0.1},    // 128 x 64
     {1, {0.0, 0.414, 0.0, 0.0}, 4.80, 0.1},      // 128 x 128
+    {},                                          // (256 x 192)
+    {1, {0.0, 0.349, 0.0, 0.0}, 5.00, 0.1},      // 192 x 64
 };
 inline double ring_time(const RingModel &r, int cus, int64_t items, int64_t total, bool whole, int64_t chunk, bool a_kc, bool b_kc, int splits, double out_elems,
                         int64_t longest = kRingChunk) {
@@ -300,11 +307,11 @@ Tail plan_tail(const GemmProblem &p, int variant, int compute_units) {
         if (keep < 1 || keep >= (along_n ? tn : tm)) continue;
         const int64_t cut = keep * (along_n ? t.bn : t.bm);
         const GemmProblem rest = along_n ? part_of(p, 0, p.m, cut, p.n) : part_of(p, cut, p.m, 0, p.n);
-        for (int v = kNumTiles + 1; v <= kNumVariants; v++) {
-            if (!mfma16dma_supported(rest, v) || (p.extra != EXTRA_NONE && !mfma16dma_extra_supported(rest, v, 1))) continue;
+        for (int v = 1; v <= kNumVariants; v++) {
+            if (!is_ring(v) || !mfma16dma_supported(rest, v) || (p.extra != EXTRA_NONE && !mfma16dma_extra_supported(rest, v, 1))) continue;
             const Variant &r = kVariants[v - 1];
             const int64_t items = ((rest.m + r.bm - 1) / r.bm) * ((rest.n + r.bn - 1) / r.bn);
-            const double after = ring_time(kRing[v - 1 - kNumTiles], cus, items, 0, true, steps, a_kc, b_kc, 1, (double)rest.m * (double)rest.n, steps) +
+            const double after = ring_time(kRing[v - 1], cus, items, 0, true, steps, a_kc, b_kc, 1, (double)rest.m * (double)rest.n, steps) +
                                  kSecondLaunch;
             if (after < soonest) {
                 soonest = after;
@@ -355,7 +362,7 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
         if (forced_variant > 0 && v != forced_variant) continue;
         if (!takes_on(p, v, la, lb)) continue;
         const Variant &t = kVariants[v - 1];
-        const VariantModel &vm = kModel[is_ring(v) ? 0 : v - 1];
+        const VariantModel &vm = kModel[v - 1];
         // narrow outputs take the BN = 64 tiles; wide ones may take the small 128 x 64 tile (more workgroups for a
         // problem of a few tiles), never the 256 x 64 one
         if (forced_variant == 0 && !is_ring(v) && (p.n <= 64 ? t.bn > 64 : (t.bn <= 64 && t.bm > 128))) continue;
@@ -367,8 +374,8 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
             const int s = pieces[i].splits;
             const int64_t chunk = pieces[i].chunk, items = tiles * s;
             if (is_ring(v)) {
-                if (forced_variant == 0 && items > (int64_t)cus * kRing[v - 1 - kNumTiles].per_cu) break;
-                const double time = ring_time(kRing[v - 1 - kNumTiles], cus, items, total_iters, p.k % BK == 0, chunk, a_kc, b_kc, s, out_elems);
+                if (forced_variant == 0 && items > (int64_t)cus * kRing[v - 1].per_cu) break;
+                const double time = ring_time(kRing[v - 1], cus, items, total_iters, p.k % BK == 0, chunk, a_kc, b_kc, s, out_elems);
                 if (time < best_ring || (forced_variant == v && ring == 0)) {
                     best_ring = time;
                     ring = v;
@@ -503,7 +510,7 @@ static hipError_t launch_ring(const GemmProblem &g, int variant, hipStream_t str
     RingParams p;
     bool a_kc, b_kc;
     if (hipError_t e = ring_params(g, variant, p, &a_kc, &b_kc); e != hipSuccess) return e;
-    const hipError_t e = launch_mfma16_ring(variant - kNumTiles, g.dtype, p, a_kc, b_kc, stream);
+    const hipError_t e = launch_mfma16_ring(variant, g.dtype, p, a_kc, b_kc, stream);
     if (e != hipSuccess || p.splits <= 1) return e;
     return launch_splitk_reduce(g, p.ws_ld, p.ws_split_stride, stream, g.ksum ? p.ws_ksum : nullptr, p.ws_ksum_stride, ksum_slots(variant, p.splits));
 }
@@ -522,8 +529,8 @@ int mfma16_ring_pair_plan(const GemmProblem &p, const GemmProblem &q, int comput
     const int cus = std::max(1, compute_units);
     int tile = 0;
     *seconds = 1e300;
-    for (int v = kNumTiles + 1; v <= kNumVariants; v++) {
-        if (!mfma16dma_supported(p, v) || !mfma16dma_supported(q, v)) continue;
+    for (int v = 1; v <= kNumVariants; v++) {
+        if (!is_ring(v) || !mfma16dma_supported(p, v) || !mfma16dma_supported(q, v)) continue;
         const OperandLayout pa = classify(p.m, p.k, p.a_rs, p.a_cs, p.ragged), pb = classify(p.n, p.k, p.b_cs, p.b_rs, p.ragged);
         if (!pa.kc || classify(q.m, q.k, q.a_rs, q.a_cs, q.ragged).kc || classify(q.n, q.k, q.b_cs, q.b_rs, q.ragged).kc) return 0;
         if (q.ksum && !mfma16dma_ksum_supported(q, v, 1)) return 0;
@@ -531,7 +538,7 @@ int mfma16_ring_pair_plan(const GemmProblem &p, const GemmProblem &q, int comput
         // (not in 192 x 64 tiles: an estimate that ranks single products of theirs has 2048 x 768 . 768 x 768 and its weight gradient at less than
         // 14.9 us, the time of 64 x 64 tiles; they take 22.9)
         if (t.bm == 192) continue;
-        const RingModel &r = kRing[v - 1 - kNumTiles];
+        const RingModel &r = kRing[v - 1];
         auto items = [&](const GemmProblem &g) {
             return (double)((g.m + t.bm - 1) / t.bm) * (double)((g.n + t.bn - 1) / t.bn) * (double)(g.reduce ? 1 : g.batch_count());
         };
@@ -560,7 +567,7 @@ hipError_t launch_mfma16_ring_pair(const GemmProblem &p, const GemmProblem &q, i
     if (hipError_t e = ring_params(whole[0], tile, rp, &pa, &pb); e != hipSuccess) return e;
     if (hipError_t e = ring_params(whole[1], tile, rq, &qa, &qb); e != hipSuccess) return e;
     if (!pa || qa || qb) return hipErrorInvalidValue;
-    return launch_mfma16_ring_two(tile - kNumTiles, p.dtype, rp, rq, pb, stream);
+    return launch_mfma16_ring_two(tile, p.dtype, rp, rq, pb, stream);
 }
 
 hipError_t launch_mfma16dma(const GemmProblem &g, int variant, hipStream_t stream) {

@@ -20,13 +20,13 @@ struct RingParams {
     int64_t a_last, b_last;
 };
 
-// X(id, BM, BN, WAVES_M, WAVES_N, stages); ids are 1-based inside this family.
+// X(id, BM, BN, WAVES_M, WAVES_N, stages); ids go on behind and between those of gemm_mfma16_dma.h.
 #define DFDX_MFMA16_RING_VARIANTS(X) \
-    X(1, 192, 64, 4, 2, 4)           \
-    X(2, 64, 64, 2, 2, 4)            \
-    X(3, 64, 64, 2, 2, 3)            \
-    X(4, 128, 64, 2, 2, 3)           \
-    X(5, 128, 128, 2, 4, 4)
+    X(6, 64, 64, 2, 2, 4)            \
+    X(7, 64, 64, 2, 2, 3)            \
+    X(8, 128, 64, 2, 2, 3)           \
+    X(9, 128, 128, 2, 4, 4)          \
+    X(11, 192, 64, 4, 2, 4)
 
 // A backward pass: `p` with A stored along k, `q` with both operands stored across k, in one launch.
 hipError_t launch_mfma16_ring_two(int ring, int dtype, const RingParams &p, const RingParams &q, bool p_b_kc, hipStream_t stream);

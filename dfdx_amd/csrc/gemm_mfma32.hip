@@ -10,11 +10,11 @@
 // which is all the instruction needs.
 //
 // Preconditions (mfma32_supported): C unit column stride; A and B each have a unit
-// stride.  Two kernels: the LDS-DMA form further down (256 x 256 tiles, operands on the
-// 16-byte grid, K % 32 == 0) for the largest products, and the register-staged 64 x 64
-// tile, which the ring tiles (gemm_mfma32_ring.hip) have left what they cannot address:
-// 32 rows of an operand further apart than 4 GB.  Off the grid it runs its WINDOW
-// instantiation.
+// stride.  Two kernels: the LDS-DMA form further down (operands on the 16-byte grid,
+// K % 32 == 0), whose 256 x 256 tile is planned for the largest products, and the
+// register-staged tiles, which the ring tiles (gemm_mfma32_ring.hip) have left what they
+// cannot address (64 rows of a k-contiguous operand, or 32 k of the other kind, 4 GB apart or
+// more) and callers that ask for them.  Off the grid they run their WINDOW instantiations.
 #include "gemm_internal.h"
 #include "elem.h"
 #include "gemm_mfma32_ring.h"
@@ -558,9 +558,16 @@ struct Variant {
     bool small;  // the 16 x 16 tile with the contraction cut over the waves (gemm_small.hip: any strides, no batch)
     int ring;    // a tile of gemm_mfma32_ring.hip (any k, any alignment), else 0
 };
+// Ids are places in this list (1-based), and a caller may ask for a tile by its id: new ones go behind these, in front of the small one.
 constexpr Variant kVariants[] = {
+    {"256x256x32_w2x4", 256, 256, 32, 2, 4, false},
+    {"256x256x32_w2x2", 256, 256, 32, 2, 2, false},
+    {"256x128x32_w2x2", 256, 128, 32, 2, 2, false},
+    {"128x128x32_w2x2", 128, 128, 32, 2, 2, false},
+    {"128x64x32_w4x1", 128, 64, 32, 4, 1, false},
     {"64x64x32_w2x2", 64, 64, 32, 2, 2, false},
     {"dma_256x256x32_w2x4", 256, 256, 32, 2, 4, true},
+    {"dma_128x128x32_w2x2", 128, 128, 32, 2, 2, true},
 #define X(id, bm, bn, wm, wn, depth) {"ring_" #bm "x" #bn "x32_w" #wm "x" #wn "_s" #depth, bm, bn, 32, wm, wn, false, false, id},
     DFDX_MFMA32_RING_VARIANTS(X)
 #undef X
@@ -702,8 +709,16 @@ struct Cost32 {
     int places;  // of a compute unit, where its workgroups end together and the next ones come in pairs: half of what a last round leaves free is lost
 };
 constexpr Cost32 kCost32[kNumVariants] = {
-    {4.6, 0.64, 2.6, 6.1, 3.0, 1.2, 0},   // register-staged: for what the ring cannot address; slower everywhere but on one k tile
+    // register-staged, where no ring tile takes the product (`planned`): the 64 x 64 one fitted, the others at their rates against it
+    // on 4096^3 (130, 126, 117, 118 and 104 TFLOP/s for its 101)
+    {4.6, 8.0, 2.6, 6.1, 3.0, 1.2, 0},
+    {4.6, 8.3, 2.6, 6.1, 3.0, 1.2, 0},
+    {4.6, 4.4, 2.6, 6.1, 3.0, 1.2, 0},
+    {4.6, 2.2, 2.6, 6.1, 3.0, 1.2, 0},
+    {4.6, 1.25, 2.6, 6.1, 3.0, 1.2, 0},
+    {4.6, 0.64, 2.6, 6.1, 3.0, 1.2, 0},
     {8.1, 7.53, 5.4, 7.4, 7.8, 0.0, 0},
+    {8.1, 2.05, 5.4, 7.4, 7.8, 0.0, 0},  // (0.92 of the rate of the 256 x 256 one; planned like the register-staged ones)
     {4.2, 0.498, 2.8, 8.9, 4.3, 0.066, 0},
     {5.1, 0.962, 2.5, 8.6, 5.0, 0.072, 2},
     {},
@@ -786,11 +801,19 @@ size_t mfma32_workspace_bytes(const GemmProblem &p, int variant, int splits) {
     return (size_t)stride * splits * sizeof(float);
 }
 
+// The register-staged tiles and the smaller LDS-DMA one are planned only where no ring tile takes the product.
+static bool planned(int variant, bool ring) {
+    const Variant &v = kVariants[variant - 1];
+    return v.ring || v.small || (v.dma && v.bm == 256) || !ring;
+}
+
 int mfma32_pick_variant(const GemmProblem &p, int compute_units, int forced_splits, double *seconds) {
     int best = 0;
     double best_time = 1e300;
+    bool ring = false;
+    for (int v = 1; v <= kNumVariants; v++) ring = ring || (kVariants[v - 1].ring && mfma32_supported(p, v));
     for (int v = 1; v <= kNumVariants; v++) {
-        if (!mfma32_supported(p, v)) continue;
+        if (!planned(v, ring) || !mfma32_supported(p, v)) continue;
         // the small kernel adds its k slices in an order of its own: not where the caller asked for the plain k order
         // (nor for large products, except those of a few rows or columns: one row of 16 x 16 tiles streams the large
         // operand once, 16 x 8192 x 8192: 67 us against 103 us on the split 64 x 64 tiles)
@@ -862,8 +885,14 @@ static hipError_t launch_tiles(const Params &p, int variant, bool a_kc, bool b_k
     return p.window ? launch_layout<BM, BN, 32, WM, WN, true>(p, la.kc, lb.kc, stream)               \
                     : launch_layout<BM, BN, 32, WM, WN, false>(p, la.kc, lb.kc, stream)
     switch (variant) {
-    case 1: DFDX_TILE(64, 64, 2, 2);
-    case 2: return launch_dma_layout<256, 256, 2, 4>(p, la.kc, lb.kc, stream);
+    case 1: DFDX_TILE(256, 256, 2, 4);
+    case 2: DFDX_TILE(256, 256, 2, 2);
+    case 3: DFDX_TILE(256, 128, 2, 2);
+    case 4: DFDX_TILE(128, 128, 2, 2);
+    case 5: DFDX_TILE(128, 64, 4, 1);
+    case 6: DFDX_TILE(64, 64, 2, 2);
+    case 7: return launch_dma_layout<256, 256, 2, 4>(p, la.kc, lb.kc, stream);
+    case 8: return launch_dma_layout<128, 128, 2, 2>(p, la.kc, lb.kc, stream);
     default: return hipErrorInvalidValue;
     }
 #undef DFDX_TILE

@@ -10,7 +10,7 @@ from helpers import assert_within, rng
 from test_gpu_gemm import run_case
 
 pytestmark = pytest.mark.gpu
-STAGED, RING = 1, (3, 4)   # the register-staged tile, and the 64 x 64 and 128 x 64 ones in front of the small-product kernel
+STAGED, RING = 6, (9, 10)   # the register-staged 64 x 64 tile, and the 64 x 64 and 128 x 64 ones in front of the small-product kernel
 
 
 @pytest.mark.parametrize("variant", RING)

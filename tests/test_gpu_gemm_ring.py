@@ -10,12 +10,15 @@ from helpers import assert_within, rng
 from test_gpu_gemm import run_case
 
 pytestmark = pytest.mark.gpu
-TILES = 4
+TILES = 5
 
 
 def ring_ids():
-    last = device().mfma_variant_count("f16")   # the small-product kernel; the ring tiles are the four in front of it
-    return range(last - TILES, last)
+    dev = device()
+    plan = lambda v: dev.gemm_plan(dev.gemm_desc("f16", 256, 256, 256, 256, (256, 1), 512, (256, 1), 1024, (256, 1), kernel=KERNEL_MFMA, variant=v))[2]
+    ids = [v for v in range(1, dev.mfma_variant_count("f16")) if "_ring_" in plan(v)]
+    assert len(ids) == TILES
+    return ids
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
