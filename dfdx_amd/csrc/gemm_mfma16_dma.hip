@@ -23,6 +23,7 @@
 // register-staged kernel.
 #include "gemm_mfma16_dma.h"
 #include "gemm_mfma16_ring.h"
+#include "../../include/dfdx_rocm.h"
 #include <algorithm>
 #include <array>
 #include <cmath>
@@ -373,6 +374,8 @@ void mfma16dma_plan_split(const GemmProblem &p, int compute_units, int forced_va
         for (int i = 0; i < count; i++) {
             const int s = pieces[i].splits;
             const int64_t chunk = pieces[i].chunk, items = tiles * s;
+            // (256 x 192 with no more partial sums than the entry point that allocates nothing has space for: the plans that it stands in for fit)
+            if (!is_ring(v) && t.bn == 192 && s > 1 && forced_splits == 0 && mfma16dma_workspace_bytes(p, v, s) > (size_t)DFDX_ROCM_NOALLOC_SCRATCH_BYTES) break;
             if (is_ring(v)) {
                 if (forced_variant == 0 && items > (int64_t)cus * kRing[v - 1].per_cu) break;
                 const double time = ring_time(kRing[v - 1], cus, items, total_iters, p.k % BK == 0, chunk, a_kc, b_kc, s, out_elems);

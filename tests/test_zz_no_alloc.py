@@ -121,6 +121,15 @@ def test_operands_off_the_grid(dtype, m, k, n, layout, accumulate, copies):
     both_entries(dtype, m, k, n, layout, accumulate, seed=m + k, expect_split=False, check_oracle=m * k * n < 1 << 33)
 
 
+@pytest.mark.parametrize("dtype,m,k,n,layout,accumulate", [
+    ("f16", 512, 5056, 4416, (True, False), True), ("bf16", 1344, 4416, 4032, (True, False), True), ("bf16", 6400, 5568, 896, (False, True), False),
+    ("f16", 1472, 4224, 3968, (False, False), False), ("bf16", 1472, 12160, 2624, (False, False), False),
+])
+def test_pieces_of_large_tiles_fit(dtype, m, k, n, layout, accumulate):
+    """Products that 256 x 192 tiles would take in pieces of 42 to 47 MB, and other tiles in less."""
+    both_entries(dtype, m, k, n, layout, accumulate, seed=m + k, expect_split=False, check_oracle=False)
+
+
 @pytest.mark.parametrize("m,k,n,at", [(2049, 1153, 1031, False), (261, 6795, 871, True), (2305, 1024, 2051, False)])
 def test_captured_into_a_graph_with_a_cold_context(m, k, n, at):
     """A context that has no buffer yet allocates none while its stream is captured: the operands are read where they lie (a split
