@@ -297,6 +297,7 @@ struct Plan {
     int staged = 0;
     int plain_kernel = 0, plain_variant = 0, plain_splits = 1;
     GemmCut cut;
+    bool pieces_asked = false;  // the caller asked for this number of pieces
 };
 
 // Rank-1 updates and k = 2 stream their rows on the vector ALUs; from k = 3 on the matrix-core form of the thin
@@ -625,7 +626,8 @@ int reserve_partials(dfdx_rocm_ctx *ctx, const GemmProblem &problem, Plan &plan,
         plan = plain;
     }
     const size_t need = partials_bytes(p, plan);
-    // Products that kernels without partial sums had before the ring tiles and the rows form: captured with no space they run in one piece.
+    // Products that kernels without partial sums had before the ring tiles and the rows form, and any that f32 tiles are planned to take in
+    // pieces: captured with no space they run in one piece.  An f32 product keeps the pieces that the caller asked for.
     const bool ring = plan.kernel == DFDX_ROCM_KERNEL_MFMA &&
                       (p.dtype == DT_F32 || ((p.dtype == DT_F16 || p.dtype == DT_BF16) && plan.variant >= mfma16_dma_first_variant() &&
                                              plan.variant != mfma16_small_variant() && mfma16dma_takes_any_k(plan.variant - mfma16_dma_first_variant() + 1)));
@@ -633,6 +635,7 @@ int reserve_partials(dfdx_rocm_ctx *ctx, const GemmProblem &problem, Plan &plan,
     if (need && !static_scratch && (ring || rows)) {
         CtxLock lock(ctx->mu);
         if (need > ctx->workspace_bytes && capturing(ctx)) {
+            if (plan.pieces_asked && p.dtype == DT_F32) return DFDX_ROCM_ERR_SCRATCH_TOO_SMALL;
             plan.splits = ring ? 1 : 0;
             return DFDX_ROCM_OK;
         }
@@ -1425,6 +1428,7 @@ int dfdx_rocm_gemm(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc) {
     if (p.m == 0) return DFDX_ROCM_OK;
     Plan plan;  // from the product as the caller states it: a pending zero fill of C must not change which kernel runs
     if (int e = make_plan(ctx, desc, p, &plan)) return e;
+    plan.pieces_asked = ((desc->flags >> 8) & 0xff) != 0;
     return run_planned(ctx, p, plan);
 }
 

@@ -210,8 +210,9 @@ int dfdx_rocm_gemm(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *desc);
  * operand is touched (the caller may then lower or forbid the split through
  * `flags`, or call dfdx_rocm_gemm with the same descriptor).
  * dfdx_rocm_gemm on a stream that is being captured into a graph does the same
- * with the buffer that the context has by then, and runs few rows and small
- * tiles in one piece where it has no space for several: call once before the
+ * with the buffer that the context has by then, and runs few rows, small
+ * tiles and f32 products in one piece where it has no space for several (an f32
+ * product whose pieces SPLIT_K asks for is refused there): call once before the
  * capture for the plan with copies and pieces.
  * Nothing in the array has to start at zero: every partial sum that is read
  * has been written by the same call.  All calls on one GPU share the array,

@@ -204,6 +204,45 @@ def test_a_cold_context_captures_in_one_piece(dtype, m, k, n, at, plan):
     own.close()
 
 
+@pytest.mark.parametrize("m,k,n,variant", [(704, 874, 512, 0), (512, 1024, 512, 4), (512, 1024, 512, 7)])
+def test_pieces_that_were_asked_for_are_not_dropped(m, k, n, variant):
+    """f32 in three pieces because the caller says so: captured with no space it is refused, not run in another order."""
+    import torch
+
+    from dfdx_amd import Rocm
+
+    dev, g = device(), rng(k)
+    a, astr = make_operand(g, m, k, False, "f32")
+    b, bstr = make_operand(g, k, n, True, "f32")
+    da, db, want = dev.tensor(a, "f32"), dev.tensor(b, "f32"), dev.zeros("f32", (m, n))
+    desc = lambda d, c, **kw: d.gemm_desc("f32", m, k, n, da.ptr, astr, db.ptr, bstr, c.ptr, (n, 1), kernel=2, variant=variant, **kw)
+    name = dev.gemm_plan(desc(dev, want, split_k=3))[2]
+    announce("captured, cold, pieces asked for", (m, k, n), name)
+    assert "splitk3" in name, name
+    dev.gemm(desc(dev, want, split_k=3))
+    dev.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        own = Rocm(0)
+        out, other = own.zeros("f32", (m, n)), own.zeros("f32", (m, n))
+        own.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            with pytest.raises(RocmError) as err:
+                own.gemm(desc(own, out, split_k=3))
+            own.gemm(desc(own, other, no_split_k=True))
+        assert err.value.code == ERR_SCRATCH_TOO_SMALL
+        for _ in range(3):
+            graph.replay()
+            own.synchronize()
+            assert not own.to_host(out).any() and own.to_host(other).any()
+        own.gemm(desc(own, out, split_k=3))   # outside a capture the space is had
+        own.synchronize()
+        assert np.array_equal(own.to_host(out).view(np.uint32), dev.to_host(want).view(np.uint32))
+        del graph
+    own.close()
+
+
 @pytest.mark.parametrize("dtype,m,k,n", [("f16", 12, 6077, 218), ("f32", 16, 7744, 1100), ("bf16", 1090, 7177, 16), ("f16", 16, 10304, 1091)])
 def test_few_rows_in_slices(dtype, m, k, n):
     """The partial sums of up to sixteen slices, or of the ring tiles' pieces, of one to sixteen rows fit the array."""
