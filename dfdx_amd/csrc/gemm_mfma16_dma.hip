@@ -234,29 +234,31 @@ constexpr double kAboveClock = 1.0e-6, kAboveClockSplit = 6.5e-6;
 // 256): 3152 x 3072 x 768 f16 nt 26.8 -> 24.3 us, 2080 x 3968 x 1472 nn 36.1 -> 32.5, 512 x 4480 x 5440 tn 40.8 -> 37.2; 3152 x 768 x 3072 25.2 ->
 // 20.0, 2432 x 1344 x 3712 38.0 -> 32.6, 2048 x 896 x 5864 31.3 -> 26.0.  Of 796 products 124 changed plans, to 1.10 times the speed (geometric
 // mean); the largest loss was 11 % (3016 x 768 x 5696 tn, added to C).  192 x 64 is fitted like its neighbour, 7 % under the clock on a
-// full chip; split plans of the two that have a compute unit to themselves are 5.8 us above their parts, not 2.6.
+// full chip, and 4 % above that fit: of 298 products that took it at the fit 17 had been faster by more than 3 % on another tile (most of
+// them on 64 x 64 ones, at level estimates), 6 so, at the same speed in the mean.  What a split plan takes above its parts (`split`) grows
+// with the tile: 2.1 - 3.1 us on 64 x 64, 3.9 on 128 x 64, 6.4 on 128 x 128 and 5.3 on 192 x 64 in the middle of 250 forced timings.
 struct RingModel {
     int per_cu;
-    double k_tile[4], item, launch;
+    double k_tile[4], item, launch, split;
 };
 constexpr int64_t kRingChunk = 96, kRingAcross = 64;
 constexpr double kSecondRound = 2.0;  // see mfma16_ring_pair_plan (microseconds)
 constexpr double kSecondLaunch = 3.5e-6, kLastRound = 0.6, kShortRound = 12e-6;  // see plan_tail
 constexpr RingModel kRing[kNumVariants] = {
-    {}, {}, {}, {}, {},                          // (persistent tiles)
-    {2, {0.0, 0.187, 0.390, 0.0}, 2.75, 0.9},    // 64 x 64, four stages
-    {3, {0.0, 0.234, 0.394, 0.572}, 3.30, 0.2},  // 64 x 64, three
-    {2, {0.0, 0.305, 0.610, 0.0}, 4.10, 0.1},    // 128 x 64
-    {1, {0.0, 0.414, 0.0, 0.0}, 4.80, 0.1},      // 128 x 128
-    {},                                          // (256 x 192)
-    {1, {0.0, 0.349, 0.0, 0.0}, 5.00, 0.1},      // 192 x 64
+    {}, {}, {}, {}, {},                               // (persistent tiles)
+    {2, {0.0, 0.187, 0.390, 0.0}, 2.75, 0.9, 2.6},    // 64 x 64, four stages
+    {3, {0.0, 0.234, 0.394, 0.572}, 3.30, 0.2, 2.6},  // 64 x 64, three
+    {2, {0.0, 0.305, 0.610, 0.0}, 4.10, 0.1, 2.6},    // 128 x 64
+    {1, {0.0, 0.414, 0.0, 0.0}, 4.80, 0.1, 5.8},      // 128 x 128
+    {},                                               // (256 x 192)
+    {1, {0.0, 0.363, 0.0, 0.0}, 5.20, 0.1, 5.2},      // 192 x 64
 };
 inline double ring_time(const RingModel &r, int cus, int64_t items, int64_t total, bool whole, int64_t chunk, bool a_kc, bool b_kc, int splits, double out_elems,
                         int64_t longest = kRingChunk) {
     if (items > (int64_t)cus * r.per_cu || chunk > longest || (!a_kc && !b_kc && whole && total >= kRingAcross)) return 1e300;
     const double layout = a_kc && b_kc ? 0.97 : !a_kc && !b_kc ? 1.1 : 1.0;
     double us = r.launch + r.item + (double)chunk * r.k_tile[(items + cus - 1) / cus] * layout + out_elems * 2.0 / 8e6;
-    if (splits > 1) us += (r.per_cu == 1 ? 5.8 : 2.6) + 0.2 * splits + splits * out_elems * 4.0 / 9.5e6;
+    if (splits > 1) us += r.split + 0.2 * splits + splits * out_elems * 4.0 / 9.5e6;
     return us * 1e-6;
 }
 }  // namespace

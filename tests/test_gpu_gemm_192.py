@@ -41,3 +41,12 @@ def test_where_they_are_taken(dtype, layout, m, k, n, want):
 @pytest.mark.parametrize("rows,i,o", [(1792, 2496, 1080), (4608, 1152, 5056)])
 def test_row_sums(dtype, rows, i, o):
     bias_gradient_rides_along(dtype, rows, i, o)
+
+
+@pytest.mark.parametrize("dtype,layout,m,k,n,accumulate,never", [
+    ("f16", "tn", 1216, 2165, 1664, False, "_192x64x64"),
+])
+def test_where_another_tile_is_left(dtype, layout, m, k, n, accumulate, never):
+    """Products that were faster on the tile before."""
+    name = run_case(dtype, m, k, n, layout, accumulate, KERNEL_AUTO, 0, seed=m)
+    assert never not in name or "_dma_" in name, name
