@@ -450,6 +450,7 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
     const Plan small_plan = {DFDX_ROCM_KERNEL_MFMA, is16 ? mfma16_small_variant() : mfma64_small_variant(), 1};
     Plan ring_plan = {};
     double t_ring = 1e300;
+    bool narrow = false;
     if (is16) {
         int dv = 0, splits = 1;
         double t_dma = 1e300;
@@ -460,7 +461,7 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         // (a C on the 8-byte grid only: of the persistent tiles one stores it as it is, the 128 x 64 one; all others with the
         // element-aligned stores of the plans below.  2048 x 1024 x 50260 f16 342 us and 208, 4096 x 1024 x 4092 51 and 36.)
         const int64_t ldc = p.m == 1 ? p.n : p.c_rs;
-        const bool narrow = dv && (p.n % 8 || ldc % 8 || ((uintptr_t)p.c & 15u) || p.c_b1 % 8 || p.c_b2 % 8);
+        narrow = dv && (p.n % 8 || ldc % 8 || ((uintptr_t)p.c & 15u) || p.c_b1 % 8 || p.c_b2 % 8);
         if (only_ring || narrow) {  // (k off the tile or C off the grid: weighed against the families below, copies among them)
             t_ring = t_dma;
             ring_plan = {DFDX_ROCM_KERNEL_MFMA, dv + mfma16_dma_first_variant() - 1, splits};
@@ -512,10 +513,13 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
         // 0.6 of it with operands on the 16-byte grid and at 0.9 - 1.6 off it, the larger tiles at about 1 and 1.4 - 3, and those
         // write a large C at 2.2 TB/s.  f16, staged and on copies: 2048 x 50257 x 1024 563 and 325 us, 4095^3 293 and 143, 1315 x
         // 2340 x 3033 150 and 52, 530 x 3231 x 1057 84 and 28, 6928 x 106 x 7330 80 and 43; and where the line leaves the
-        // staged kernels: 1000^3 12.0 and 18.8, 304 x 611 x 4120 11.0 and 16.4, 448 x 315 x 4890 13.2 and 14.5.
+        // staged kernels: 1000^3 12.0 and 18.8, 304 x 611 x 4120 11.0 and 16.4, 448 x 315 x 4890 13.2 and 14.5.  In pieces the larger tiles
+        // take 1.45 of the estimate on the grid and 2.1 - 2.9 off it (84 products; 3778 x 7038 x 256 bf16 nn 104 us for 37, 43 on copies), and
+        // 2.2 - 3.5 where only C is off it (2304 x 576 x 8188 f16 nt + C 70 us for 29, the 128 x 64 LDS-DMA tile 40).
         double t_copies = 1e300;
         const bool small_tile = v == mfma16_skinny_variant();
-        const double t_staged = t_family * (small_tile ? (ra.off_grid ? 1.0 : 0.6) : ra.off_grid ? 1.4 : 0.95) +
+        const bool large_pieces = is16 && !small_tile && mfma16_plan_splits(p, v, ctx->compute_units, forced_splits) > 1;
+        const double t_staged = t_family * (small_tile ? (ra.off_grid ? 1.0 : 0.6) : large_pieces ? (ra.off_grid ? 2.4 : 1.45) : narrow ? 2.2 : ra.off_grid ? 1.4 : 0.95) +
                                 (small_tile ? 0.0 : 2.0 * (double)p.m * (double)p.n * (double)(p.reduce ? 1 : p.nb1 * p.nb2) / 2.2e12);
         const double t_uncopied = std::min(std::min(t_small_here, t_staged), t_bw);
         if (realignable && ra.seconds + mfma16dma_least_time() < t_uncopied) {
@@ -534,8 +538,10 @@ int make_plan(dfdx_rocm_ctx *ctx, const dfdx_rocm_gemm_desc *d, const GemmProble
             }
         }
         // (on operands in place with k off 64 the staged tiles run at 0.83 - 1.06 of the estimate: 528 x 1024 x 1325 f16 21.4 us for 25.6,
-        // 2304 x 128 x 1534 in three pieces 16.2 for 15.3; the ring 9.4 both)
-        const double t_plan = plan->realign ? t_copies : plan->kernel == DFDX_ROCM_KERNEL_GEMV ? t_bw : plan->variant == v ? 0.85 * t_family : t_small_here - t_short;
+        // 2304 x 128 x 1534 in three pieces 16.2 for 15.3; the ring 9.4 both; not so the larger ones in pieces, nor where C alone
+        // is off the grid)
+        const double t_place = large_pieces || (narrow && !small_tile) ? t_staged : 0.85 * t_family;
+        const double t_plan = plan->realign ? t_copies : plan->kernel == DFDX_ROCM_KERNEL_GEMV ? t_bw : plan->variant == v ? t_place : t_small_here - t_short;
         if (t_ring <= t_plan) *plan = ring_plan;
         if (seconds && is16) *seconds = std::min(t_ring, t_plan);
         return DFDX_ROCM_OK;
