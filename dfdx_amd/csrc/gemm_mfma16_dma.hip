@@ -237,18 +237,24 @@ constexpr double kAboveClock = 1.0e-6, kAboveClockSplit = 6.5e-6;
 // full chip, and 4 % above that fit: of 298 products that took it at the fit 17 had been faster by more than 3 % on another tile (most of
 // them on 64 x 64 ones, at level estimates), 6 so, at the same speed in the mean.  What a split plan takes above its parts (`split`) grows
 // with the tile: 2.1 - 3.1 us on 64 x 64, 3.9 on 128 x 64, 6.4 on 128 x 128 and 5.3 on 192 x 64 in the middle of 250 forced timings.
+// `cold` is a k tile of a workgroup that has its compute unit to itself and walks kCold of them or more: on operands that the launch in
+// front has written, which come from beyond the L2 caches, the two tiles that three stages have on their way do not cover what one takes.
+// 128 x 64, 0.31 us on operands launched again and again, 0.53 in an encoder block's forward: its second product of 1752 x 3072 x 768 f16
+// 27.7 us where 128 x 128 in three pieces takes 16.7 + 1.8 more in the launch behind, 2007 x 4096 x 1024 34.8 and 25.0 + 1.3.  One plan has to do
+// for both (the block leaves the bits of its ops), so the figure lies between, just where that product changes tiles; on fewer k tiles it
+// would send products to 128 x 64 in three pieces, which are slower (1833 x 2112 x 640 14.7 -> 18.9).
 struct RingModel {
     int per_cu;
-    double k_tile[4], item, launch, split;
+    double k_tile[4], item, launch, split, cold;
 };
-constexpr int64_t kRingChunk = 96, kRingAcross = 64;
+constexpr int64_t kRingChunk = 96, kRingAcross = 64, kCold = 48;
 constexpr double kSecondRound = 2.0;  // see mfma16_ring_pair_plan (microseconds)
 constexpr double kSecondLaunch = 3.5e-6, kLastRound = 0.6, kShortRound = 12e-6;  // see plan_tail
 constexpr RingModel kRing[kNumVariants] = {
     {}, {}, {}, {}, {},                               // (persistent tiles)
     {2, {0.0, 0.187, 0.390, 0.0}, 2.75, 0.9, 2.6},    // 64 x 64, four stages
     {3, {0.0, 0.234, 0.394, 0.572}, 3.30, 0.2, 2.6},  // 64 x 64, three
-    {2, {0.0, 0.305, 0.610, 0.0}, 4.10, 0.1, 2.6},    // 128 x 64
+    {2, {0.0, 0.305, 0.610, 0.0}, 4.10, 0.1, 2.6, 0.35},  // 128 x 64
     {1, {0.0, 0.414, 0.0, 0.0}, 4.80, 0.1, 5.8},      // 128 x 128
     {},                                               // (256 x 192)
     {1, {0.0, 0.363, 0.0, 0.0}, 5.20, 0.1, 5.2},      // 192 x 64
@@ -257,7 +263,8 @@ inline double ring_time(const RingModel &r, int cus, int64_t items, int64_t tota
                         int64_t longest = kRingChunk) {
     if (items > (int64_t)cus * r.per_cu || chunk > longest || (!a_kc && !b_kc && whole && total >= kRingAcross)) return 1e300;
     const double layout = a_kc && b_kc ? 0.97 : !a_kc && !b_kc ? 1.1 : 1.0;
-    double us = r.launch + r.item + (double)chunk * r.k_tile[(items + cus - 1) / cus] * layout + out_elems * 2.0 / 8e6;
+    const double k_tile = items <= cus && chunk >= kCold ? std::max(r.cold, r.k_tile[1]) : r.k_tile[(items + cus - 1) / cus];
+    double us = r.launch + r.item + (double)chunk * k_tile * layout + out_elems * 2.0 / 8e6;
     if (splits > 1) us += r.split + 0.2 * splits + splits * out_elems * 4.0 / 9.5e6;
     return us * 1e-6;
 }

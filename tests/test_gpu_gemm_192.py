@@ -46,6 +46,7 @@ def test_row_sums(dtype, rows, i, o):
 @pytest.mark.parametrize("dtype,layout,m,k,n,accumulate,never", [
     ("bf16", "nn", 3778, 7038, 256, False, "_128x128x64_w2x2"), ("f16", "tn", 896, 7076, 512, False, "_128x128x64_w2x2"),
     ("f16", "nt", 2304, 576, 8188, True, "_256x256x64_w2x4"), ("f16", "tn", 1216, 2165, 1664, False, "_192x64x64"),
+    ("f16", "nt", 1998, 4096, 1024, False, "_ring_128x64x64"), ("f16", "nt", 1752, 3072, 768, False, "_ring_128x64x64"),   # (in a chain of launches)
 ])
 def test_where_another_tile_is_left(dtype, layout, m, k, n, accumulate, never):
     """Products that were faster on the tile before: by up to 2.4 times than in pieces on the large register-staged tiles."""
