@@ -1,10 +1,12 @@
 """The native half of the Python front-end (csrc/host.cpp): what its entry points take as arguments and refuse, without a GPU."""
 import ctypes
 
+from types import SimpleNamespace
+
 import pytest
 import torch
 
-from dfdx_amd import View
+from dfdx_amd import EncoderBlock, View
 from dfdx_amd.rocm import Encoder, _load_host
 
 INVALID = -1   # DFDX_ROCM_ERR_INVALID_ARG: what a null context gets
@@ -55,3 +57,16 @@ def test_parameters():
         assert host.parameters(raw, p | {"p3": wrong}, "f16", specs) is None
     with pytest.raises(KeyError):
         host.parameters(raw, {}, "f16", specs)
+
+
+def test_parameters_with_strides_in_a_list():
+    """A View's strides may be any sequence; what is refused stays refused."""
+    host = _load_host()
+    p = {f"p{i}": View(torch.zeros(64, dtype=torch.uint8), "f16", (4, 2), [2, 1] if i == 3 else (2, 1)) for i in range(16)}
+    plan = SimpleNamespace(raw=bytes(Encoder(1, 0, 2, 3, 4, 5, 6)), params=tuple((n, (4, 2), (2, 1)) for n in p))
+    block = SimpleNamespace(dev=SimpleNamespace(_f=host), p=p, dtype="f16")
+    desc = Encoder.from_buffer_copy(EncoderBlock._desc(block, plan))
+    assert list(desc.params) == [v.ptr for v in p.values()] and (desc.batch, desc.d_ff) == (2, 6)
+    p["p3"].strides = [1, 4]
+    with pytest.raises(AssertionError):
+        EncoderBlock._desc(block, plan)
