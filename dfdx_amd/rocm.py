@@ -133,9 +133,6 @@ def load_library() -> ctypes.CDLL:
     return _lib
 
 
-_PACK = {n: struct.Struct(f"{n}q").pack for n in range(1, 9)}
-
-
 def _load_host():
     """The native half of this front-end (csrc/host.cpp): the entry points a training or inference step goes through, as functions
     that take addresses, Views and tuples of numbers as they are.  Needs torch's libraries, so torch is imported before."""
@@ -148,8 +145,13 @@ def _load_host():
 
 
 def _i64s(v) -> bytes:
-    """A small int64_t array as an argument: the call reads it while the bytes object lives."""
-    return _PACK[len(v)](*v)
+    """An int64_t array as an argument: the call reads it while the bytes object lives."""
+    return struct.pack(f"{len(v)}q", *v)
+
+
+def _axes(v):
+    """One number per axis as an argument: a tuple as it is, unless it is longer than the native module takes (the library refuses such ranks)."""
+    return tuple(v) if len(v) <= 8 else _i64s(v)
 
 
 @dataclass
@@ -557,12 +559,12 @@ class Rocm:
         if x.strides == _row_major(x.shape):
             return View(x.storage, x.dtype, new_shape, _row_major(new_shape), x.offset, x.owner)
         out = self.empty(x.dtype, new_shape)
-        self._check(self._f.reshape_forward(self._at, DTYPES[x.dtype], len(x.shape), tuple(x.shape), tuple(x.strides), x, out))
+        self._check(self._f.reshape_forward(self._at, DTYPES[x.dtype], len(x.shape), _axes(x.shape), _axes(x.strides), x, out))
         return out
 
     def reshape_backward(self, x: View, grad_inp: View, grad_out: View):
         """Backward of a copying reshape: grad_inp (laid out like x's storage) += grad_out through x's strides."""
-        self._check(self._f.reshape_backward(self._at, DTYPES[x.dtype], len(x.shape), tuple(x.shape), tuple(x.strides), grad_inp, grad_out))
+        self._check(self._f.reshape_backward(self._at, DTYPES[x.dtype], len(x.shape), _axes(x.shape), _axes(x.strides), grad_inp, grad_out))
 
     def attention_supported(self, dtype: str, head_dim: int) -> bool:
         """Whether the fused attention takes this element type and head dimension (else: matmul, softmax, matmul)."""

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from dfdx_amd import EncoderBlock, View
-from dfdx_amd.rocm import Encoder, _load_host
+from dfdx_amd.rocm import Encoder, Rocm, RocmError, _load_host, load_library
 
 INVALID = -1   # DFDX_ROCM_ERR_INVALID_ARG: what a null context gets
 
@@ -70,3 +70,15 @@ def test_parameters_with_strides_in_a_list():
     p["p3"].strides = [1, 4]
     with pytest.raises(AssertionError):
         EncoderBlock._desc(block, plan)
+
+
+@pytest.mark.parametrize("rank", [8, 9, 12])
+def test_reshapes_of_many_axes_are_refused_by_the_library(rank):
+    """Nine axes are no error of the call's form: the library refuses them (here, without a context, eight as well)."""
+    x = View(torch.zeros(64, dtype=torch.uint8), "f32", (1,) * (rank - 1) + (2,), (2,) * rank)
+    check = SimpleNamespace(lib=load_library())
+    dev = SimpleNamespace(_f=_load_host(), _at=0, empty=lambda dtype, shape: x, _check=lambda code: Rocm._check(check, code))
+    for call in (lambda: Rocm.reshape_forward(dev, x, (2,)), lambda: Rocm.reshape_backward(dev, x, x, x)):
+        with pytest.raises(RocmError) as err:
+            call()
+        assert err.value.code == INVALID
