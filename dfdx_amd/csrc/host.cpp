@@ -189,20 +189,24 @@ PyObject *make_view(PyTypeObject *cls, PyObject *storage, PyObject *dtype, PyObj
     return nullptr;
 }
 
-PyObject *row_major(PyObject *shape, int64_t *count) {  // strides of a tuple of extents, and their product
+// Strides of a tuple of extents, and the bytes of as many elements of `size` bytes (at least 16).  Numbers beyond 64 bits are an
+// OverflowError, also on the way to a product of zero.
+PyObject *row_major(PyObject *shape, int64_t size, int64_t *bytes) {
     const Py_ssize_t n = PyTuple_GET_SIZE(shape);
     PyObject *strides = PyTuple_New(n);
     int64_t step = 1;
     for (Py_ssize_t i = n - 1; strides && i >= 0; i--) {
         PyTuple_SET_ITEM(strides, i, PyLong_FromLongLong(step));
         const int64_t e = PyLong_AsLongLong(PyTuple_GET_ITEM(shape, i));
-        if (e == -1 && PyErr_Occurred()) {
-            Py_DECREF(strides);
-            return nullptr;
-        }
-        step *= e;
+        if (!(e == -1 && PyErr_Occurred()) && __builtin_mul_overflow(step, e, &step)) PyErr_SetString(PyExc_OverflowError, "more elements than 64 bits count");
+        if (PyErr_Occurred()) Py_CLEAR(strides);
     }
-    *count = step;
+    if (!strides) return nullptr;
+    if (__builtin_mul_overflow(step, size, bytes)) {
+        PyErr_SetString(PyExc_OverflowError, "more bytes than 64 bits count");
+        Py_CLEAR(strides);
+    }
+    *bytes = std::max<int64_t>(*bytes, 16);
     return strides;
 }
 
@@ -221,11 +225,10 @@ PyObject *py_allocator(PyObject *, PyObject *ordinal) { return PyCFunction_New(&
 PyObject *py_empty(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (n != 4 || !PyType_Check(args[0]) || !PyTuple_Check(args[3])) return PyErr_Format(PyExc_TypeError, "empty(View, ordinal, dtype, shape)");
     const int64_t es = item_size(args[2]), dev = PyLong_AsLongLong(args[1]);
-    int64_t count = 0;
-    PyObject *strides = es < 0 || PyErr_Occurred() ? nullptr : row_major(args[3], &count);
+    int64_t bytes = 0;
+    PyObject *strides = es < 0 || PyErr_Occurred() ? nullptr : row_major(args[3], es, &bytes);
     if (!strides) return nullptr;
-    PyObject *view = make_view((PyTypeObject *)args[0], guarded([&] { return THPVariable_Wrap(allocate(dev, std::max<int64_t>(count * es, 16))); }), args[2],
-                               args[3], strides, Py_None);
+    PyObject *view = make_view((PyTypeObject *)args[0], guarded([&] { return THPVariable_Wrap(allocate(dev, bytes)); }), args[2], args[3], strides, Py_None);
     Py_DECREF(strides);
     return view;
 }
@@ -268,10 +271,11 @@ PyObject *py_carve(PyObject *, PyObject *const *args, Py_ssize_t n) {
         Part &p = parts.back();
         if (!p.dtype || !p.shape) return done(nullptr);
         const int64_t es = item_size(p.dtype);
-        int64_t elements = 0;
-        if (es < 0 || !(p.strides = row_major(p.shape, &elements))) return done(nullptr);
-        p.bytes = std::max<int64_t>(elements * es, 16);
-        total += (p.bytes + 255) / 256 * 256;
+        if (es < 0 || !(p.strides = row_major(p.shape, es, &p.bytes))) return done(nullptr);
+        if (__builtin_add_overflow(total, p.bytes, &total) || __builtin_add_overflow(total, -p.bytes & 255, &total)) {
+            PyErr_SetString(PyExc_OverflowError, "more bytes than 64 bits count");
+            return done(nullptr);
+        }
     }
     ordinal = PyObject_GetAttr(dev, s_ordinal);
     at = PyObject_GetAttr(dev, s_at);

@@ -82,3 +82,15 @@ def test_reshapes_of_many_axes_are_refused_by_the_library(rank):
         with pytest.raises(RocmError) as err:
             call()
         assert err.value.code == INVALID
+
+
+@pytest.mark.parametrize("shape", [(1 << 32, 1 << 32), (1 << 62,), (1 << 21, 1 << 21, 1 << 21), (3, 1 << 62)])
+def test_sizes_beyond_64_bits(shape):
+    """No allocation of what is left of the product: 2^64 elements are not none."""
+    host, like = _load_host(), View(torch.zeros(16, dtype=torch.uint8), "f32", shape, (1,) * len(shape))
+    with pytest.raises(OverflowError):
+        host.empty(View, 0, "f32", shape)
+    with pytest.raises(OverflowError):
+        host.carve(SimpleNamespace(ordinal=0, _at=0), View, None, [like], True)
+    with pytest.raises(OverflowError):   # (each of them fits)
+        host.carve(SimpleNamespace(ordinal=0, _at=0), View, None, [View(like.storage, "f64", (1 << 59,), (1,))] * 2, True)
