@@ -139,8 +139,8 @@ def _load_host():
     try:
         from . import _host
     except ImportError as e:
-        raise FileNotFoundError(f"{os.path.join(_HERE, '_host.so')} is missing or does not load ({e}): build it with `make -C dfdx_amd/csrc` "
-                                "(or __graft_entry__.build())") from e
+        raise FileNotFoundError(f"the extension module _host in {_HERE} is missing or does not load ({e}): build it with `make -C dfdx_amd/csrc` "
+                                "(or __graft_entry__.build()), with the interpreter and the torch that run this") from e
     return _host
 
 

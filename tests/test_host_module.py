@@ -1,6 +1,7 @@
 """The native half of the Python front-end (csrc/host.cpp): what its entry points take as arguments and refuse, without a GPU."""
 import ctypes
-
+import os
+import subprocess
 from types import SimpleNamespace
 
 import pytest
@@ -94,3 +95,11 @@ def test_sizes_beyond_64_bits(shape):
         host.carve(SimpleNamespace(ordinal=0, _at=0), View, None, [like], True)
     with pytest.raises(OverflowError):   # (each of them fits)
         host.carve(SimpleNamespace(ordinal=0, _at=0), View, None, [View(like.storage, "f64", (1 << 59,), (1,))] * 2, True)
+
+
+def test_the_library_builds_without_python():
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "dfdx_amd", "csrc")
+    plan = lambda *args: subprocess.run(["make", "-n", "-B", "-C", csrc, *args], capture_output=True, text=True)
+    with_python, without = plan(), plan("PYTHON=/nonexistent")
+    assert with_python.returncode == without.returncode == 0
+    assert "host.cpp" in with_python.stdout and "host.cpp" not in without.stdout and "libdfdx_rocm.so" in without.stdout
