@@ -1,5 +1,5 @@
 """The image gradient of strided first layers by rows of cells (conv_few.hip): ends of tiles of 16 columns and of groups of four
-rows, one to four chunks of 16 channels, both tile counts, and what infinities at the edges of tiles reach."""
+rows, one to four chunks of 16 channels, both tile counts, more groups than workgroups walk at once, and what infinities reach."""
 import pytest
 import torch
 
@@ -52,3 +52,44 @@ def test_an_infinity_at_an_edge(k, w, col):
     # (formed again position by position: the sums in another order, of cout * k * k terms of 8 at the most behind an f16 rounding)
     a, b = (torch.where(reach, 0, r).float() for r in results)
     assert bool(((a - b).abs() <= 2.0 ** -10 * a.abs() + cout * k * k * 8 * 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("batch,cin,cout,h,w,k", [(1100, 3, 16, 8, 32, 7), (1100, 3, 64, 7, 32, 3), (1100, 3, 10, 8, 160, 3), (700, 3, 64, 14, 144, 5)])
+def test_several_groups_a_workgroup(dtype, batch, cin, cout, h, w, k):
+    """Two workgroups a compute unit walk what is more than 512 groups: the next group's rows on their way under this one's sums."""
+    dev, gen = device(), torch.Generator(device="cuda").manual_seed(cout + k)
+    announce("conv few rows, walked", dtype, batch, cin, cout, h, w, k)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=gen).to(TYPES[dtype])
+    x, f, g = rnd(batch, cin, h, w), rnd(cout, cin, k, k) / 8, rnd(batch, cout, (h + 1) // 2, w // 2)
+    assert batch * -(-g.shape[2] // 4) > 1024
+    image = lambda f, g: torch.nn.grad.conv2d_input(x.shape, f.double().cpu(), g.double().cpu(), stride=2, padding=k // 2)
+    want, mag = image(f, g), image(f.abs(), g.abs())
+    for fresh in (True, False):
+        old = rnd(*x.shape)
+        gi, gf = dev.zeros_many([view(x, dtype), view(f, dtype)], deferred=True) if fresh else (view(old.clone(), dtype), view(torch.zeros_like(f), dtype))
+        dev.conv2d_backward(view(x, dtype), gi, view(f, dtype), gf, view(g, dtype), stride=2, padding=k // 2)
+        dev.settle_zeros()
+        check("grad_img", gi.storage.view(TYPES[dtype]).reshape(x.shape), want, mag, cout * k * k, dtype, None if fresh else old)
+
+
+@pytest.mark.parametrize("cout,w", [(16, 32), (64, 32), (16, 160), (64, 160)])
+def test_an_infinity_in_an_early_group(cout, w):
+    """The groups that a workgroup walks behind one that it has formed again are what they are without it, bit for bit."""
+    dev, dtype, batch, h, k = device(), "f16", 1100, 8, 7
+    announce("conv few rows, infinity early", cout, w)
+    gen = torch.Generator(device="cuda").manual_seed(w)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=gen).to(TYPES[dtype])
+    x, f, g = rnd(batch, 3, h, w), rnd(cout, 3, k, k) / 8, rnd(batch, cout, h // 2, w // 2)
+    images = [0, 1, 77, 300, 511, 512, 600]   # one group of four rows each
+    results = []
+    for value in (0.0, float("inf")):
+        g[images, cout - 1, 2, w // 2 - 1] = value
+        gi, gf = dev.zeros_many([view(x, dtype), view(f, dtype)], deferred=True)
+        dev.conv2d_backward(view(x, dtype), gi, view(f, dtype), gf, view(g, dtype), stride=2, padding=k // 2)
+        dev.settle_zeros()
+        results.append(gi.storage.view(TYPES[dtype]).reshape(x.shape).clone())
+    others = torch.ones(batch, dtype=torch.bool, device="cuda")
+    others[images] = False
+    assert torch.equal(results[0][others], results[1][others]) and bool(torch.isfinite(results[0]).all())
+    assert bool((~torch.isfinite(results[1][images])).flatten(1).any(1).all())

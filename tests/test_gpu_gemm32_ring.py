@@ -83,6 +83,27 @@ def test_plans(m, k, n, layout, want):
     assert want in dev.gemm_plan(dev.gemm_desc("f32", m, k, n, 256, a, 512, b, 1024, (n, 1), kernel=KERNEL_AUTO))[2]
 
 
+@pytest.mark.parametrize("ld,tile", [(16777148, "_ring_64x64"), (16777152, "_64x64x32_w2x2")])
+def test_rows_too_far_apart_for_the_ring(ld, tile):
+    """64 rows of a k-contiguous operand (as many as a tile has, whatever m is) have to lie within 32 bits of bytes: beyond, the register-staged
+    tile is planned."""
+    import torch
+    dev, (m, k, n) = device(), (5, 100, 72)
+    gen = torch.Generator(device="cuda").manual_seed(ld)
+    a = torch.zeros((m - 1) * ld + k, device="cuda")
+    rows = a.as_strided((m, k), (ld, 1))
+    rows.copy_(torch.randn(m, k, device="cuda", generator=gen))
+    b, c = torch.randn(k, n, device="cuda", generator=gen), torch.zeros(m, n, device="cuda")
+    desc = dev.gemm_desc("f32", m, k, n, a.data_ptr(), (ld, 1), b.data_ptr(), (n, 1), c.data_ptr(), (n, 1), kernel=KERNEL_MFMA, no_split_k=True)
+    name = dev.gemm_plan(desc)[2]
+    announce("f32, rows far apart", ld, name)
+    assert tile in name and ("_ring_" in tile) == ("_ring_" in name), name
+    dev.gemm(desc)
+    dev.synchronize()
+    A, B = rows.double().cpu().numpy(), b.double().cpu().numpy()
+    assert_within("f32", k, c.double().cpu().numpy(), A @ B, A, B, what=name)
+
+
 def test_captured_with_no_space_for_partial_sums():
     """A cold context: a product that is planned in pieces runs in one, and replays."""
     import torch

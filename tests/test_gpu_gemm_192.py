@@ -28,6 +28,18 @@ def test_any_contraction(dtype, layout, m, k, n):
     run_case(dtype, m, k, n, layout, True, KERNEL_MFMA, variant, seed=k)
 
 
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("layout,m,k,n,splits", [
+    ("nt", 6144, 64, 4224, 1), ("nn", 6100, 192, 4224, 1), ("nn", 6144, 64, 4232, 1), ("tn", 6144, 192, 4168, 1),   # (the last two off the 128-byte lines)
+    ("tn", 3584, 192, 2688, 3), ("nt", 3600, 512, 2624, 4),
+])
+def test_several_items_a_workgroup(layout, m, k, n, splits, accumulate):
+    """More than two rounds of items, of one k tile and more each: a tile's stores leave under the next one's loads."""
+    (variant,) = tiles(device(), "f16", "_dma_256x192x64")
+    assert -(-m // 256) * -(-n // 192) * splits > 512
+    assert "_dma_256x192x64" in run_case("f16", m, k, n, layout, accumulate, KERNEL_MFMA, variant, split_k=splits, seed=m + n)
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("layout,m,k,n,want", [
     ("nt", 3152, 768, 3072, "_dma_256x192"), ("tn", 2168, 1472, 4840, "_dma_256x192"), ("nt", 3152, 3072, 768, "_ring_192x64"),
@@ -46,7 +58,7 @@ def test_row_sums(dtype, rows, i, o):
 @pytest.mark.parametrize("dtype,layout,m,k,n,accumulate,never", [
     ("bf16", "nn", 3778, 7038, 256, False, "_128x128x64_w2x2"), ("f16", "tn", 896, 7076, 512, False, "_128x128x64_w2x2"),
     ("f16", "nt", 2304, 576, 8188, True, "_256x256x64_w2x4"), ("f16", "tn", 1216, 2165, 1664, False, "_192x64x64"),
-    ("f16", "nt", 1998, 4096, 1024, False, "_ring_128x64x64"), ("f16", "nt", 1752, 3072, 768, False, "_ring_128x64x64"),   # (in a chain of launches)
+    ("f16", "nt", 1998, 4096, 1024, False, "_ring_128x64x64"),   # (slower in a chain of launches)
 ])
 def test_where_another_tile_is_left(dtype, layout, m, k, n, accumulate, never):
     """Products that were faster on the tile before: by up to 2.4 times than in pieces on the large register-staged tiles."""
