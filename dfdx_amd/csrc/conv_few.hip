@@ -1005,6 +1005,9 @@ template <typename T, int C, int K, int TILES> hipError_t grad_img_rows_run(cons
 template <typename T, int C, int K, int S> hipError_t backward_run(const ConvFew &c, void *workspace, hipStream_t stream) {
     bool rows = false;
     if constexpr (S == 2) {
+        // Rows of up to seven tiles: with eight, filters of 7 x 7 on three channels leave no room for the votes (81920 + 16 bytes, and two
+        // workgroups share 160 KB).  Smaller filters and one channel would fit with eight; rows beyond 112 were not measured for them and
+        // take the kernel below, as all rows did before.
         if (c.w_out <= 112) {
             rows = true;
             if (hipError_t e = c.w_out <= 64 ? grad_img_rows_run<T, C, K, 4>(c, stream) : grad_img_rows_run<T, C, K, 7>(c, stream)) return e;

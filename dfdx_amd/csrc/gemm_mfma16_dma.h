@@ -636,7 +636,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, dma_waves_per_simd(BM, BN, W
             [[maybe_unused]] const int after = (lq_after * 16 + (quarter == 3 ? l16 ^ 8 : l16)) * 4;
             // (rows of a lane lie 8 or 16 apart: all of them start on the same half of a word)
             [[maybe_unused]] const bool odd = (((uintptr_t)cbase >> 1) + (uint32_t)l16 * (uint32_t)p.ldc & 1) != 0;
-            [[maybe_unused]] const bool words = (((uintptr_t)cbase >> 1 | (uint32_t)p.ldc) & 1) == 0;  // (all rows of the problem, then)
+            // (all rows of the problem, then; tiles of 96 columns a wave take no others, see takes_on)
+            [[maybe_unused]] const bool words = TN == 6 || (((uintptr_t)cbase >> 1 | (uint32_t)p.ldc) & 1) == 0;
             [[maybe_unused]] auto right = [&](uint32_t x) -> uint32_t { return (uint32_t)__builtin_amdgcn_ds_bpermute(after, (int)x); };
             // The general form: bounds checks, either bias, beta = 1 with the old value loaded where it is used (edge
             // tiles, per-row bias, very large ldc).

@@ -159,7 +159,9 @@ static bool takes_on(const GemmProblem &p, int variant, const OperandLayout &la,
     const Variant &v = kVariants[variant - 1];
     if (!is_ring(variant) && p.k % BK != 0) return false;
     if (la.ld * (la.kc ? v.bm : BK) >= (1ll << 30) || lb.ld * (lb.kc ? v.bn : BK) >= (1ll << 30)) return false;
-    if (!is_ring(variant) && !c_on_grid(p, v) && !(p.ragged && (v.bn / v.waves_n) % 32 == 0)) return false;
+    // (wave tiles of 96 columns store half lines: beside a C off the grid the others are ahead, and their instances have no odd rows)
+    const int wave_columns = v.bn / v.waves_n;
+    if (!is_ring(variant) && !c_on_grid(p, v) && !(p.ragged && wave_columns % 32 == 0 && wave_columns != 96)) return false;
     return tile_count(p, v) * (p.reduce ? 1 : p.batch_count()) < (1ll << 31);
 }
 
